@@ -10,7 +10,7 @@
 //   mie_terms        per (size, 8 orders): a_n, b_n, contraction operand, series partials
 //                                                              (src/lmie_core.c:453-652)
 //   mie_sums         series per size                          (src/lmie_core.c:537-596)
-//   mie_coefs        per size with forward tangents (tangent passes)
+//   mie_tan_*        the same with the derivatives along x and m
 //   angular_mix      S sums on the 16-bit matrix cores (split operands), Stokes in
 //                    FP64, weighted sums per angle            (src/lmie_core.c:658-791)
 //   angular_f64      the same on the FP64 matrix cores
@@ -169,6 +169,8 @@ __device__ __forceinline__ cd cmul(cd a, cd b) { return cd{a.r * b.r - a.i * b.i
 __device__ __forceinline__ cd cscale(cd a, double s) { return cd{a.r * s, a.i * s}; }
 __device__ __forceinline__ cd cconj(cd a) { return cd{a.r, -a.i}; }
 __device__ __forceinline__ double cabs2(cd a) { return a.r * a.r + a.i * a.i; }
+__device__ __forceinline__ double cdot(cd a, cd b) { return a.r * b.r + a.i * b.i; }   // Re(conj(a) b)
+__device__ __forceinline__ double cim(cd a, cd b) { return a.r * b.i - a.i * b.r; }    // Im(conj(a) b)
 // Smith's division: scaled by the larger component of the divisor, so no
 // intermediate overflows where |b|^2 would.
 __device__ __forceinline__ cd cdiv(cd a, cd b) {
@@ -531,242 +533,8 @@ __global__ void gsf_table_b(const gsf_table_B *cases) {
 
 
 // ---------------------------------------------------------------------------
-// Per-size Mie coefficients.  One thread per size point (NT tangent channels
-// carried alongside).  Downward D_n(z) from n2 (stored for n <= n1) and
-// downward ratio r_n = psi_n / psi_{n-1} from r_{n1} = 0 (stored), then one
-// upward sweep for psi_n, chi_n, a_n, b_n, the series and the A operand
-// (src/lmie_core.c:298-652).  Scratch rows are [n][Np] so every access of a
-// wave is one contiguous 512-byte (or 1 KiB) line.
-struct CoefArgs {
-     int N, Np, n1max;
-     const double *x;           // [Np]
-     const double *sx, *cx;     // [Np] sin x, cos x (from the host's C library, as the reference)
-     const int *n1, *n2;        // [Np]
-     const int *kfill;          // [Np / TILE] rows to zero-fill up to
-     double mr, mi;
-     int nt;                    // tangent channels in this pass
-     const double *dx;          // [nt][Np]
-     const double *dm;          // [nt][2]
-     double *scrD;              // [(1 + nt)][2][n1max + 1][Np]
-     double *scrR;              // [(1 + nt)][n1max + 1][Np]
-     double *A;                 // base planes [4][Kp][Np]
-     double *At[4];             // tangent planes of this pass, each [4][Kp][Np]
-     int Kp;
-     double *S;                 // series [4][Np]: ext, sca, |c_bak|^2, asym
-     double *St[4];             // tangent series of this pass, each [4][Np]
-     int write_base;            // write A and S of the base channel
-     double *CB;                // reverse-pass checkpoint: c_bak series [2][Np] or NULL
-};
-
-// Used for passes that carry tangent channels (NT >= 1); the value channel
-// alone goes through mie_chains / mie_terms / mie_sums.
-template <int NT>
-__global__ __launch_bounds__(64) void mie_coefs(CoefArgs p) {
-     // separately rounded operations in the reference's order and association
-     // (src/lmie_core.c:298-611): the real recurrences reproduce the
-     // reference's bits; complex divisions use Smith's scaling (ulp-level
-     // differences that the downward recurrences damp)
-#pragma clang fp contract(off)
-     int i = blockIdx.x * blockDim.x + threadIdx.x;
-     if (i >= p.Np) return;
-     const size_t Np = p.Np, plane = (size_t) p.Kp * Np, srow = (size_t) (p.n1max + 1) * Np;
-     int kf = p.kfill[i / TILE];
-     if (i >= p.N) {
-          // padded columns: zero operand rows and series
-          for (int r = 0; r < kf; ++r)
-               for (int c = 0; c < 4; ++c) {
-                    if (p.write_base) p.A[c * plane + r * Np + i] = 0.;
-                    for (int t = 0; t < NT; ++t) p.At[t][c * plane + r * Np + i] = 0.;
-               }
-          for (int q = 0; q < 4; ++q) {
-               if (p.write_base) p.S[q * Np + i] = 0.;
-               for (int t = 0; t < NT; ++t) p.St[t][q * Np + i] = 0.;
-          }
-          return;
-     }
-     const double x = p.x[i];
-     const int n1 = p.n1[i], n2 = p.n2[i];
-     const cd m = cmk(p.mr, -p.mi);
-     const cd z = cscale(m, x);
-     const cd m2 = cmul(m, m);
-     cd dz[NT > 0 ? NT : 1], dmv[NT > 0 ? NT : 1];
-     double dxv[NT > 0 ? NT : 1];
-#pragma unroll
-     for (int t = 0; t < NT; ++t) {
-          dxv[t] = p.dx[t * Np + i];
-          dmv[t] = cmk(p.dm[2 * t], p.dm[2 * t + 1]);
-          dz[t] = cadd(cscale(dmv[t], x), cscale(m, dxv[t]));
-     }
-     double *Dre = p.scrD, *Dim = p.scrD + srow, *R = p.scrR;
-
-     // downward D_j(z) = (j+1)/z - 1 / (D_{j+1} + (j+1)/z), D_{n2} = 0
-     cd D = cmk(0., 0.), dD[NT > 0 ? NT : 1];
-#pragma unroll
-     for (int t = 0; t < NT; ++t) dD[t] = cmk(0., 0.);
-     for (int j = n2 - 1; j >= 1; --j) {
-          const cd c1 = cdiv(cmk(j + 1., 0.), z);
-          const cd c2 = cadd(D, c1);
-          D = csub(c1, crecip(c2));
-#pragma unroll
-          for (int t = 0; t < NT; ++t) {
-               const cd c5 = cmul(cdiv(cscale(c1, -1.), z), dz[t]);
-               dD[t] = cadd(c5, cdiv(cadd(dD[t], c5), cmul(c2, c2)));
-          }
-          if (j <= n1) {
-               Dre[j * Np + i] = D.r;
-               Dim[j * Np + i] = D.i;
-#pragma unroll
-               for (int t = 0; t < NT; ++t) {
-                    p.scrD[(size_t) (1 + t) * 2 * srow + j * Np + i] = dD[t].r;
-                    p.scrD[(size_t) (1 + t) * 2 * srow + srow + j * Np + i] = dD[t].i;
-               }
-          }
-     }
-     // downward ratio r_j = 1 / ((2j+1)/x - r_{j+1}), r_{n1} = 0
-     {
-          double r = 0., dr[NT > 0 ? NT : 1];
-#pragma unroll
-          for (int t = 0; t < NT; ++t) dr[t] = 0.;
-          R[n1 * Np + i] = 0.;
-#pragma unroll
-          for (int t = 0; t < NT; ++t) p.scrR[(size_t) (1 + t) * srow + n1 * Np + i] = 0.;
-          for (int j = n1 - 1; j >= 1; --j) {
-               const double c = (2. * j + 1.) / x;
-               const double rn = 1. / (c - r);
-               const double a2 = -c / x, a3 = rn * rn;
-#pragma unroll
-               for (int t = 0; t < NT; ++t) {
-                    dr[t] = -(a2 * dxv[t] - dr[t]) * a3;
-                    p.scrR[(size_t) (1 + t) * srow + j * Np + i] = dr[t];
-               }
-               r = rn;
-               R[j * Np + i] = r;
-          }
-     }
-     // upward sweep
-     const double sx = p.sx[i], cx = p.cx[i];
-     const double ax = 1. / x;
-     double psi0 = sx, chi0 = cx, chi1 = ax * cx + sx;
-     double dpsi0[NT > 0 ? NT : 1], dchi0[NT > 0 ? NT : 1], dchi1[NT > 0 ? NT : 1];
-#pragma unroll
-     for (int t = 0; t < NT; ++t) {
-          const double a2l = -ax / x * dxv[t];
-          dpsi0[t] = dxv[t] * cx;
-          dchi0[t] = dxv[t] * -sx;
-          dchi1[t] = a2l * cx + ax * dchi0[t] + dxv[t] * cx;
-     }
-     double se = 0., ss = 0., sg = 0.;
-     cd cb = cmk(0., 0.), ap = cmk(0., 0.), bp = cmk(0., 0.);
-     double dse[NT > 0 ? NT : 1], dss[NT > 0 ? NT : 1], dsg[NT > 0 ? NT : 1];
-     cd dcb[NT > 0 ? NT : 1], dap[NT > 0 ? NT : 1], dbp[NT > 0 ? NT : 1];
-#pragma unroll
-     for (int t = 0; t < NT; ++t) {
-          dse[t] = dss[t] = dsg[t] = 0.;
-          dcb[t] = dap[t] = dbp[t] = cmk(0., 0.);
-     }
-     double sgn = -1.;
-     for (int j = 1; j <= n1; ++j) {
-          const double r = R[j * Np + i];
-          const double psi = r * psi0;
-          const cd Dj = cmk(Dre[j * Np + i], Dim[j * Np + i]);
-          const double jx = j / x;
-          const cd zj = cmk(psi, chi1), zjm = cmk(psi0, chi0);
-          // a_j with u = D_j / m + j / x; b_j with v = m D_j + j / x
-          const cd u = cadd(cdiv(Dj, m), cmk(jx, 0.));
-          const cd v = cadd(cmul(m, Dj), cmk(jx, 0.));
-          const cd na = csub(cscale(u, psi), cmk(psi0, 0.)), da = csub(cmul(u, zj), zjm);
-          const cd nb = csub(cscale(v, psi), cmk(psi0, 0.)), db = csub(cmul(v, zj), zjm);
-          const cd a = cdiv(na, da), b = cdiv(nb, db);
-          const double fv1 = 2. * j + 1., fv2 = (j + 1.) / j, fv4 = fv1 / (j * (j + 1.));
-          const double fv3m = j > 1 ? (j + 1.) / ((double) j / (j - 1.)) : 0.;
-          const double fv4m = j > 1 ? (2. * j - 1.) / ((j - 1.) * j) : 0.;
-          (void) fv2;
-          se += fv1 * (a.r + b.r);
-          ss += fv1 * (cabs2(a) + cabs2(b));
-          cb = cadd(cb, cscale(csub(a, b), fv1 * sgn));
-          if (j > 1)
-               sg += fv3m * ((ap.r * a.r + ap.i * a.i) + (bp.r * b.r + bp.i * b.i)) + fv4m * (ap.r * bp.r + ap.i * bp.i);
-          if (p.write_base) {
-               const size_t o = (size_t) (j - 1) * Np + i;
-               p.A[o] = fv4 * (a.r + b.r);
-               p.A[plane + o] = fv4 * (a.i + b.i);
-               p.A[2 * plane + o] = fv4 * (a.r - b.r);
-               p.A[3 * plane + o] = fv4 * (a.i - b.i);
-          }
-#pragma unroll
-          for (int t = 0; t < NT; ++t) {
-               const double drt = p.scrR[(size_t) (1 + t) * srow + j * Np + i];
-               const double dpsi = drt * psi0 + r * dpsi0[t];
-               const cd dD = cmk(p.scrD[(size_t) (1 + t) * 2 * srow + j * Np + i],
-                                 p.scrD[(size_t) (1 + t) * 2 * srow + srow + j * Np + i]);
-               const double djx = -jx * dxv[t] / x;
-               const cd dzj = cmk(dpsi, dchi1[t]), dzjm = cmk(dpsi0[t], dchi0[t]);
-               // du = dD/m - D dm / m^2 + d(j/x); dv = dm D + m dD + d(j/x)
-               const cd du = cadd(csub(cdiv(dD, m), cmul(cdiv(Dj, m2), dmv[t])), cmk(djx, 0.));
-               const cd dv = cadd(cadd(cmul(dmv[t], Dj), cmul(m, dD)), cmk(djx, 0.));
-               const cd dna = csub(cadd(cscale(du, psi), cscale(u, dpsi)), cmk(dpsi0[t], 0.));
-               const cd dda = csub(cadd(cmul(du, zj), cmul(u, dzj)), dzjm);
-               const cd dnb = csub(cadd(cscale(dv, psi), cscale(v, dpsi)), cmk(dpsi0[t], 0.));
-               const cd ddb = csub(cadd(cmul(dv, zj), cmul(v, dzj)), dzjm);
-               const cd dat = csub(cdiv(dna, da), cdiv(cmul(na, dda), cmul(da, da)));
-               const cd dbt = csub(cdiv(dnb, db), cdiv(cmul(nb, ddb), cmul(db, db)));
-               dse[t] += fv1 * (dat.r + dbt.r);
-               dss[t] += fv1 * 2. * ((a.r * dat.r + a.i * dat.i) + (b.r * dbt.r + b.i * dbt.i));
-               dcb[t] = cadd(dcb[t], cscale(csub(dat, dbt), fv1 * sgn));
-               if (j > 1)
-                    dsg[t] += fv3m * (dap[t].r * a.r + dap[t].i * a.i + ap.r * dat.r + ap.i * dat.i +
-                                      dbp[t].r * b.r + dbp[t].i * b.i + bp.r * dbt.r + bp.i * dbt.i) +
-                              fv4m * (dap[t].r * bp.r + dap[t].i * bp.i + ap.r * dbp[t].r + ap.i * dbp[t].i);
-               const size_t o = (size_t) (j - 1) * Np + i;
-               p.At[t][o] = fv4 * (dat.r + dbt.r);
-               p.At[t][plane + o] = fv4 * (dat.i + dbt.i);
-               p.At[t][2 * plane + o] = fv4 * (dat.r - dbt.r);
-               p.At[t][3 * plane + o] = fv4 * (dat.i - dbt.i);
-               dap[t] = dat;
-               dbp[t] = dbt;
-               // advance tangent recurrences
-               const double c = fv1 / x;
-               const double dchi2 = -c * dxv[t] / x * chi1 + c * dchi1[t] - dchi0[t];
-               dchi0[t] = dchi1[t];
-               dchi1[t] = dchi2;
-               dpsi0[t] = dpsi;
-          }
-          ap = a;
-          bp = b;
-          sgn = -sgn;
-          const double chi2 = fv1 / x * chi1 - chi0;
-          chi0 = chi1;
-          chi1 = chi2;
-          psi0 = psi;
-     }
-     // zero rows n1 .. kf-1 so the contraction can run whole chunks
-     for (int r = n1; r < kf; ++r) {
-          const size_t o = (size_t) r * Np + i;
-          for (int c = 0; c < 4; ++c) {
-               if (p.write_base) p.A[c * plane + o] = 0.;
-#pragma unroll
-               for (int t = 0; t < NT; ++t) p.At[t][c * plane + o] = 0.;
-          }
-     }
-     if (p.CB) {
-          p.CB[i] = cb.r;
-          p.CB[Np + i] = cb.i;
-     }
-     if (p.write_base) {
-          p.S[i] = se;
-          p.S[Np + i] = ss;
-          p.S[2 * Np + i] = cabs2(cb);
-          p.S[3 * Np + i] = sg;
-     }
-#pragma unroll
-     for (int t = 0; t < NT; ++t) {
-          p.St[t][i] = dse[t];
-          p.St[t][Np + i] = dss[t];
-          p.St[t][2 * Np + i] = 2. * (cb.r * dcb[t].r + cb.i * dcb[t].i);
-          p.St[t][3 * Np + i] = dsg[t];
-     }
-}
-
+// Per-size Mie coefficients.
+//
 // Element i of row `row` of a [rows][Np] array: the row pointer is uniform
 // over the wave (row and the base are), the lane's byte offset a 32-bit
 // register, so each load is one scalar-based address and no 64-bit lane
@@ -807,7 +575,7 @@ __device__ __forceinline__ double rcp_s3(double q) {
 }
 
 // ---------------------------------------------------------------------------
-// Value channel in three kernels: mie_chains runs the three recurrences that
+// Three kernels: mie_chains runs the three recurrences that
 // are serial in n, two threads per size in different waves (the D chain; the
 // ratio chain and then the psi, chi chain); mie_terms forms a_n, b_n, the
 // contraction operand and the partial series sums in parallel, one thread
@@ -824,8 +592,13 @@ struct ChainArgs {
      double *D;                 // [n2rows][Np][2]: D_j (re, im) at row j
      double *PC;                // [2][n1max + 1][Np]: U_j (psi_j = s U_j), chi_j at row j
      double *PS;                // [Np]: s
+     double *Dz, *PQ;           // TAN: dD_j/dz as D; [2][Np] p and q of psi' (see mie_tan_terms)
 };
 
+// TAN: forward tangents follow (mie_tan_terms): the D chain carries dD_j/dz too,
+// dD_j/dz = c' + (dD_{j+1}/dz + c') / w_j^2 with c' = -(j+1)/z^2, beside the
+// chain of w, which stays the longer dependence.
+template <bool TAN>
 __device__ __forceinline__ void mie_chains_body(ChainArgs p) {
 #pragma clang fp contract(off)
      const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -843,9 +616,17 @@ __device__ __forceinline__ void mie_chains_body(ChainArgs p) {
           // recurrence damps its last-bit differences.
           const cd z = cscale(cmk(p.mr, -p.mi), x), iz = crecip(z);
           cd w = cscale(iz, (double) n2);
+          cd dz = cmk(0., 0.);
+          const cd iz2 = cmul(iz, iz);
           for (int j = n2 - 1; j >= 1; --j) {
                const cd c1 = cscale(iz, j + 1.), e = cscale(iz, 2. * j + 1.);
                const double q = rcp_s3(__builtin_fma(w.r, w.r, w.i * w.i));
+               if constexpr (TAN) {
+                    const cd dc = cscale(iz2, -(j + 1.)), r = cmk(w.r * q, -w.i * q), r2 = cmul(r, r), t = cadd(dz, dc);
+                    dz = cmk(__builtin_fma(t.r, r2.r, __builtin_fma(-t.i, r2.i, dc.r)),
+                             __builtin_fma(t.r, r2.i, __builtin_fma(t.i, r2.r, dc.i)));
+                    if (j <= dtop) ((double2 *) p.Dz)[j * Np + i] = double2{dz.r, dz.i};
+               }
                if (j <= dtop)
                     Dv[j * Np + i] = double2{__builtin_fma(-w.r, q, c1.r), __builtin_fma(w.i, q, c1.i)};
                w = cmk(__builtin_fma(-w.r, q, e.r), __builtin_fma(w.i, q, e.i));
@@ -882,9 +663,16 @@ __device__ __forceinline__ void mie_chains_body(ChainArgs p) {
                ub = un;
           }
      }
-     p.PS[i] = sx / ub;
+     const double s = sx / ub;
+     p.PS[i] = s;
+     if constexpr (TAN) {               // chi0 = chi_{n1}, ua = U_1
+          const double q = -s / chi0;
+          p.PQ[i] = (cx - sx * ax + s * ua - q * cx) / sx;
+          p.PQ[Np + i] = q;
+     }
 }
-__global__ __launch_bounds__(64) void mie_chains(ChainArgs p) { mie_chains_body(p); }
+template <bool TAN>
+__global__ __launch_bounds__(64) void mie_chains(ChainArgs p) { mie_chains_body<TAN>(p); }
 struct mie_chains_B {
      ChainArgs p;
      unsigned gx, gy;
@@ -892,11 +680,11 @@ struct mie_chains_B {
 __global__ __launch_bounds__(64) void mie_chains_b(const mie_chains_B *cases) {
      const mie_chains_B a = cases[blockIdx.z];
      if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     mie_chains_body(a.p);
+     mie_chains_body<false>(a.p);
 }
 
 
-// a_j, b_j (src/lmie_core.c:557-583), operations as mie_coefs
+// a_j, b_j (src/lmie_core.c:557-583)
 __device__ __forceinline__ void mie_ab_jx(double jx, cd m, cd im, cd Dj, double psi, double psi0, double chi1,
                                           double chi0, cd *a, cd *b) {
 #pragma clang fp contract(off)
@@ -1163,6 +951,209 @@ __global__ __launch_bounds__(256) void mie_sums_b(const mie_sums_B *cases) {
 
 
 // ---------------------------------------------------------------------------
+// Forward tangents of the per-size coefficients.  a_n and b_n depend on the
+// inputs through the size parameter x and, analytically, through the complex
+// m, so the derivatives along x (HX) and along m (HM) give those of every
+// direction.  mie_chains<true> carries dD_j/dz along the D chain; everything
+// else is closed per order from the kept D, U and chi:
+//   chi'_j = chi_{j-1} - (j/x) chi_j,
+//   psi'_j = psi_{j-1} - (j/x) psi_j + p psi_j + q chi_j,
+// where psi_j = s U_j is the chain's psi, cut at psi_{n1} = 0: its derivative
+// in x solves the same recurrence up to a solution p psi + q chi, fixed by the
+// cut (psi'_{n1} = 0: q = -psi_{n1-1} / chi_{n1}) and by psi'_0 = cos x.
+// One thread per (size, 8 orders), as mie_terms; the previous order is formed
+// again for the g series.  Bound: FP64 VALU (about 400 operations per (size,
+// order) with both derivatives) and the operand planes it writes, 32 bytes per
+// (size, order) and operand set.
+struct TanArgs {
+     int N, Np, n1max, n2rows, Kp, ng;
+     const double *ft;          // order_factors rows over 0 .. n1max + 1
+     const double *x;
+     const int *n1, *kfill;
+     double mr, mi;
+     const double *D, *Dz, *PC, *PS, *PQ;   // from mie_chains: D_j and dD_j/dz [n2rows][Np][2], U and chi, s, [2][Np] p and q
+     double *A[3];              // operand planes [4][Kp][Np] of the value, then of d/dx, d/dm as present
+     double *part;              // [rows][ng][Np]: the value's se, ss, cb (re, im), sg, then mie_tan_sums's rows
+};
+
+template <bool HX, bool HM>
+__global__ __launch_bounds__(64) void mie_tan_terms(TanArgs p) {
+     constexpr int NB = 1 + HX + HM, BM = HX ? 2 : 1;
+     const int i = blockIdx.x * 64 + threadIdx.x, g = blockIdx.y;
+     const size_t Np = p.Np, plane = (size_t) p.Kp * Np, gp = (size_t) p.ng * Np, ld = (size_t) p.n1max + 2;
+     const int kf = p.kfill[i / TILE];
+     const int n1 = i < p.N ? p.n1[i] : 0;
+     const int j0 = 8 * g + 1, j1 = min(8 * g + 8, n1);
+     if (j0 <= j1) {
+          const double x = p.x[i], ax = 1. / x, sc = p.PS[i], pc = p.PQ[i], qc = p.PQ[Np + i];
+          const cd m = cmk(p.mr, -p.mi), im = crecip(m), m2 = cmul(m, m);
+          const double2 *Dv = (const double2 *) p.D, *Dz = (const double2 *) p.Dz;
+          const double *U = p.PC, *Chi = p.PC + (size_t) (p.n1max + 1) * Np;
+          const unsigned o8 = (unsigned) i * 8u, o16 = (unsigned) i * 16u;
+          // psi, chi and their derivatives of the order before the first one formed
+          const int js = g ? j0 - 1 : 1;
+          double ps = sc * ld_row(U, js - 1, Np, o8), ch = ld_row(Chi, js - 1, Np, o8), dps, dch;
+          if (g) {
+               const double jx = (js - 1) * ax;
+               dps = sc * ld_row(U, js - 2, Np, o8) - jx * ps + (pc * ps + qc * ch);
+               dch = ld_row(Chi, js - 2, Np, o8) - jx * ch;
+          } else {
+               dps = ch;                 // psi_0 = sin x, chi_0 = cos x
+               dch = -ps;
+          }
+          double se = 0., ss = 0., sg = 0., xe = 0., xs = 0., xg = 0., mg = 0., mgi = 0.;
+          cd cb = cmk(0., 0.), xb = cb, me = cb, ms = cb, mb = cb;
+          cd ap = cb, bp = cb, axp = cb, bxp = cb, amp = cb, bmp = cb;
+          const int jl = min(8 * g + 8, p.n1max);       // uniform: the group's last row
+          double un = ld_row(U, js, Np, o8), cn = ld_row(Chi, js, Np, o8);
+          double2 dn = ld_row(Dv, js, Np, o16), zn = ld_row(Dz, js, Np, o16);
+          for (int j = js; j <= jl; ++j) {
+               const double ps0 = ps, ch0 = ch, dps0 = dps, dch0 = dch;
+               ps = sc * un;
+               ch = cn;
+               const cd D = cmk(dn.x, dn.y), Dd = cmk(zn.x, zn.y);
+               // the next row, ahead of its use (clamped to the arrays)
+               const int jn = min(j + 1, jl), kn = min(jn, p.n2rows - 1);
+               un = ld_row(U, jn, Np, o8);
+               cn = ld_row(Chi, jn, Np, o8);
+               dn = ld_row(Dv, kn, Np, o16);
+               zn = ld_row(Dz, kn, Np, o16);
+               if (j > j1) continue;
+               const double jx = j * ax, jxx = -jx * ax;
+               dps = ps0 - jx * ps + (pc * ps + qc * ch);
+               dch = ch0 - jx * ch;
+               const cd zj = cmk(ps, ch), zp = cmk(ps0, ch0);
+               const cd Di = cmul(D, im);               // D / m
+               const cd u = cadd(Di, cmk(jx, 0.)), v = cadd(cmul(m, D), cmk(jx, 0.));
+               const cd da = csub(cmul(u, zj), zp), db = csub(cmul(v, zj), zp);
+               const cd a = cdiv_nr(csub(cscale(u, ps), cmk(ps0, 0.)), da), b = cdiv_nr(csub(cscale(v, ps), cmk(ps0, 0.)), db);
+               const cd ra = cdiv_nr(cmk(1., 0.), da), rb = cdiv_nr(cmk(1., 0.), db);
+               cd atx = cmk(0., 0.), btx = atx, atm = atx, btm = atx;
+               if constexpr (HX) {
+                    // (u_x psi + u psi' - psi'_{j-1} - a (u_x zeta + u zeta' - zeta'_{j-1})) / da
+                    const cd dz = cmk(dps, dch), dzp = cmk(dps0, dch0);
+                    const cd ux = cadd(Dd, cmk(jxx, 0.)), vx = cadd(cmul(m2, Dd), cmk(jxx, 0.));
+                    const cd na = csub(cadd(cscale(ux, ps), cscale(u, dps)), cmk(dps0, 0.));
+                    const cd nb = csub(cadd(cscale(vx, ps), cscale(v, dps)), cmk(dps0, 0.));
+                    const cd ea = csub(cadd(cmul(ux, zj), cmul(u, dz)), dzp), eb = csub(cadd(cmul(vx, zj), cmul(v, dz)), dzp);
+                    atx = cmul(csub(na, cmul(a, ea)), ra);
+                    btx = cmul(csub(nb, cmul(b, eb)), rb);
+               }
+               if constexpr (HM) {
+                    // u_m (psi - a zeta) / da, u_m = (x D' - D/m) / m, v_m = D + m x D'
+                    const cd xd = cscale(Dd, x);
+                    const cd um = cmul(csub(xd, Di), im), vm = cadd(D, cmul(m, xd));
+                    atm = cmul(cmul(um, csub(cmk(ps, 0.), cmul(a, zj))), ra);
+                    btm = cmul(cmul(vm, csub(cmk(ps, 0.), cmul(b, zj))), rb);
+               }
+               if (j >= j0) {
+                    const double f1 = 2. * j + 1., fs = (j & 1) ? -f1 : f1;
+                    const double f3 = p.ft[FT_FV3M * ld + j], f4 = p.ft[FT_FV4M * ld + j], fa = p.ft[FT_FV4 * ld + j];
+                    const size_t o = (size_t) (j - 1) * Np + i;
+                    auto put = [&](double *A, cd s, cd t) {
+                         A[o] = fa * (s.r + t.r);
+                         A[plane + o] = fa * (s.i + t.i);
+                         A[2 * plane + o] = fa * (s.r - t.r);
+                         A[3 * plane + o] = fa * (s.i - t.i);
+                    };
+                    se += f1 * (a.r + b.r);
+                    ss += f1 * (cabs2(a) + cabs2(b));
+                    cb = cadd(cb, cscale(csub(a, b), fs));
+                    sg += f3 * (cdot(ap, a) + cdot(bp, b)) + f4 * cdot(ap, bp);
+                    put(p.A[0], a, b);
+                    if constexpr (HX) {
+                         xe += f1 * (atx.r + btx.r);
+                         xs += f1 * 2. * (cdot(a, atx) + cdot(b, btx));
+                         xb = cadd(xb, cscale(csub(atx, btx), fs));
+                         xg += f3 * (cdot(axp, a) + cdot(ap, atx) + cdot(bxp, b) + cdot(bp, btx)) +
+                               f4 * (cdot(axp, bp) + cdot(ap, bxp));
+                         put(p.A[1], atx, btx);
+                    }
+                    if constexpr (HM) {
+                         // complex sums: the derivative along t is Re(t (.))
+                         me = cadd(me, cscale(cadd(atm, btm), f1));
+                         ms = cadd(ms, cscale(cadd(cmul(cconj(a), atm), cmul(cconj(b), btm)), 2. * f1));
+                         mb = cadd(mb, cscale(csub(atm, btm), fs));
+                         mg += f3 * (cdot(amp, a) + cdot(ap, atm) + cdot(bmp, b) + cdot(bp, btm)) +
+                               f4 * (cdot(amp, bp) + cdot(ap, bmp));
+                         mgi += f3 * (cim(amp, a) - cim(ap, atm) + cim(bmp, b) - cim(bp, btm)) +
+                                f4 * (cim(amp, bp) - cim(ap, bmp));
+                         put(p.A[BM], atm, btm);
+                    }
+               }
+               ap = a;
+               bp = b;
+               if constexpr (HX) { axp = atx; bxp = btx; }
+               if constexpr (HM) { amp = atm; bmp = btm; }
+          }
+          double *pt = p.part + (size_t) g * Np + i;
+          pt[0] = se; pt[gp] = ss; pt[2 * gp] = cb.r; pt[3 * gp] = cb.i; pt[4 * gp] = sg;
+          if constexpr (HX) {
+               pt += 5 * gp;
+               pt[0] = xe; pt[gp] = xs; pt[2 * gp] = xb.r; pt[3 * gp] = xb.i; pt[4 * gp] = xg;
+          }
+          if constexpr (HM) {
+               pt += 5 * gp;
+               pt[0] = me.r; pt[gp] = me.i; pt[2 * gp] = ms.r; pt[3 * gp] = ms.i;
+               pt[4 * gp] = mb.r; pt[5 * gp] = mb.i; pt[6 * gp] = mg; pt[7 * gp] = mgi;
+          }
+     }
+     // operand rows of orders beyond n1 (up to the tile's depth) are zero
+     for (int r = max(8 * g, n1); r < min(8 * g + 8, kf); ++r)
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+#pragma unroll
+               for (int c = 0; c < 4; ++c) p.A[b][c * plane + (size_t) r * Np + i] = 0.;
+}
+
+// Series per size from the group partials (as mie_sums): S [4][Np] of the
+// value (ext, sca, |c_bak|^2, asym), then 4 rows of d/dx (HX), then 4 rows
+// each of the derivatives along Re m and Im m (HM).
+template <bool HX, bool HM>
+__global__ __launch_bounds__(256) void mie_tan_sums(const double *part, int N, int Np, int ng, const int *n1, double *S) {
+     constexpr int R = 5 + 5 * HX + 8 * HM;
+     __shared__ double red[R][8][32];
+     const int il = threadIdx.x & 31, l = threadIdx.x >> 5, i = blockIdx.x * 32 + il;
+     const size_t gp = (size_t) ng * Np;
+     double v[R];
+#pragma unroll
+     for (int q = 0; q < R; ++q) v[q] = 0.;
+     if (i < Np) {
+          const int gn = i < N ? (n1[i] + 7) / 8 : 0;
+          for (int g = l; g < gn; g += 8) {
+               const double *pt = part + (size_t) g * Np + i;
+#pragma unroll
+               for (int q = 0; q < R; ++q) v[q] += pt[q * gp];
+          }
+     }
+#pragma unroll
+     for (int q = 0; q < R; ++q) red[q][l][il] = v[q];
+     __syncthreads();
+     if (l || i >= Np) return;
+#pragma unroll
+     for (int q = 0; q < R; ++q) {
+          v[q] = red[q][0][il];
+          for (int k = 1; k < 8; ++k) v[q] += red[q][k][il];
+     }
+     const size_t n = Np;
+     const cd cb = cmk(v[2], v[3]);
+     double *s = S + i;
+     s[0] = v[0]; s[n] = v[1]; s[2 * n] = cabs2(cb); s[3 * n] = v[4];
+     if constexpr (HX) {
+          s += 4 * n;
+          s[0] = v[5]; s[n] = v[6]; s[2 * n] = 2. * cdot(cb, cmk(v[7], v[8])); s[3 * n] = v[9];
+     }
+     if constexpr (HM) {
+          constexpr int q = 5 + 5 * HX;
+          const cd mb = cmk(v[q + 4], v[q + 5]);
+          s += 4 * n;
+          s[0] = v[q]; s[n] = v[q + 2]; s[2 * n] = 2. * cdot(cb, mb); s[3 * n] = v[q + 6];
+          s += 4 * n;
+          s[0] = -v[q + 1]; s[n] = -v[q + 3]; s[2 * n] = 2. * cim(mb, cb); s[3 * n] = v[q + 7];
+     }
+}
+
+// ---------------------------------------------------------------------------
 // Weighted sums over sizes: out[k] = sum_i u_k[i] v_k[i] (+ sum_i u2_k[i] v2_k[i]),
 // one workgroup per output, fixed-order tree reduction (deterministic).
 struct DotJob {
@@ -1217,34 +1208,8 @@ __global__ __launch_bounds__(256) void weighted_dots_b(const weighted_dots_B *ca
 
 
 // ---------------------------------------------------------------------------
-// Angular contraction, FP64 matrix cores.
-//
-// For a tile of sizes i and positive angles j the four complex sums
-//   sp+ = sum_n S_n (pi+tau)_n   sm+ = sum_n T_n (pi-tau)_n
-//   sp- = sum_n s_n S_n (pi-tau)_n   sm- = sum_n s_n T_n (pi+tau)_n,
-// S_n = fv4 (a+b), T_n = fv4 (a-b), s_n = (-1)^(n-1) (the -mu mirror,
-// src/lmie_core.c:617-652,682-686), are 8 real GEMM accumulators of
-// v_mfma_f64_16x16x4 (operand lane layout: A[i][k] in lane i + 16 k, B[k][j] in
-// lane j + 16 k; result D[l/16 + 4 v][l % 16] in lane l, element v -- checked by
-// lmie_gpu_selftest_mfma_f64).  The
-// epilogue forms S1, S2 and the four matrix elements (src/lmie_core.c:726-749),
-// weights them by f_i and reduces over the sizes of the workgroup; partials per
-// block of sizes go to HBM and are summed by reduce_parts.
-struct AngArgs {
-     int Np, Kp, Hp, H, Q;
-     const double *A[3];        // base planes, tangent planes (channel 0, 1 of the pass)
-     const double *Bp, *Bm;     // [Kp][Hp]
-     const int *ktile;          // rows to contract per size tile of TM
-     const double *W[4];        // weight channels [Np]: f, then weight-only tangents
-     const double *WT[2];       // tangent df [Np]
-     const double *f;           // base weight (for f dP of tangents)
-     int tiles_per_block;       // size tiles per workgroup
-     double *part;              // [gridDim.y][nch][4][Q]
-     double *save2;             // [4][N][Q] per-size matrix (save_control 1) or NULL
-     int N;
-     double *sst;               // reverse-pass checkpoint [Np][Hp][8]: sp+, sm+, sp-, sm- (re, im) or NULL
-};
-
+// Stokes elements of one (size, angle) from the sums sp = S1 + S2, sm = S1 - S2
+// (src/lmie_core.c:726-749), and their tangents.
 __device__ __forceinline__ void stokes(double spr, double spi, double smr, double smi, double P[4]) {
      const double s1r = .5 * (spr + smr), s1i = .5 * (spi + smi);
      const double s2r = .5 * (spr - smr), s2i = .5 * (spi - smi);
@@ -1270,200 +1235,6 @@ __device__ __forceinline__ void stokes_tan(double spr, double spi, double smr, d
      dP[2] = -(dq1 - dq2) * .5;
      dP[3] = dxi;
 }
-
-template <int WM, int WN, int NT, int NW>
-__global__ __launch_bounds__(256) void angular_f64(AngArgs p) {
-     constexpr int TM = 32 * WM, TN = 32 * WN;
-     constexpr int SA = TM + 16, SB = TN + 16;       // LDS row strides (bank spread)
-     constexpr int NC = 1 + NT;
-     __shared__ double sA[NC * 4 * KC * SA];
-     __shared__ double sB[2 * KC * SB];
-     constexpr int NE = (NW + NT) > 0 ? (NW + NT) : 1;
-     __shared__ double sR[NE * 8 * 32 * WN];
-
-     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-     const int wm = wave & 1, wn = wave >> 1;
-     const int l16 = lane & 15, lg = lane >> 4;
-     const int jt0 = blockIdx.x * TN;
-     const int tile0 = blockIdx.y * p.tiles_per_block;
-     const size_t Np = p.Np, Hp = p.Hp, plane = (size_t) p.Kp * Np;
-
-     double ew[NE][WN][8];
-#pragma unroll
-     for (int c = 0; c < NW + NT; ++c)
-#pragma unroll
-          for (int b = 0; b < WN; ++b)
-#pragma unroll
-               for (int q = 0; q < 8; ++q) ew[c][b][q] = 0.;
-
-     for (int tt = 0; tt < p.tiles_per_block; ++tt) {
-          const int tile = tile0 + tt;
-          const int it0 = tile * TM;
-          if (it0 >= p.Np) break;
-          const int kmax = p.ktile[tile];
-          v4d acc[NC][WM][WN][8];
-#pragma unroll
-          for (int c = 0; c < NC; ++c)
-#pragma unroll
-               for (int a = 0; a < WM; ++a)
-#pragma unroll
-                    for (int b = 0; b < WN; ++b)
-#pragma unroll
-                         for (int q = 0; q < 8; ++q) acc[c][a][b][q] = v4d{0., 0., 0., 0.};
-
-          for (int k0 = 0; k0 < kmax; k0 += KC) {
-               __syncthreads();
-               // stage A: NC*4 planes x KC rows x TM sizes
-               for (int e = threadIdx.x; e < NC * 4 * KC * (TM / 2); e += 256) {
-                    const int col2 = e % (TM / 2), rest = e / (TM / 2);
-                    const int row = rest % KC, pl = rest / KC;
-                    const int c = pl / 4, comp = pl % 4;
-                    const double2 v = *(const double2 *) (p.A[c] + comp * plane + (size_t) (k0 + row) * Np + it0 + 2 * col2);
-                    *(double2 *) (sA + (pl * KC + row) * SA + 2 * col2) = v;
-               }
-               for (int e = threadIdx.x; e < 2 * KC * (TN / 2); e += 256) {
-                    const int col2 = e % (TN / 2), rest = e / (TN / 2);
-                    const int row = rest % KC, pm = rest / KC;
-                    const double *src = pm ? p.Bm : p.Bp;
-                    const double2 v = *(const double2 *) (src + (size_t) (k0 + row) * Hp + jt0 + 2 * col2);
-                    *(double2 *) (sB + (pm * KC + row) * SB + 2 * col2) = v;
-               }
-               __syncthreads();
-#pragma unroll
-               for (int ks = 0; ks < KC / 4; ++ks) {
-                    const int r = ks * 4 + lg;                   // this lane's k row
-                    const double sg = ((k0 + r) & 1) ? -1. : 1.;   // s_n, n = k0 + r + 1
-                    double bp[WN], bm[WN];
-#pragma unroll
-                    for (int b = 0; b < WN; ++b) {
-                         const int jc = wn * 16 * WN + 16 * b + l16;
-                         bp[b] = sB[r * SB + jc];
-                         bm[b] = sB[(KC + r) * SB + jc];
-                    }
-#pragma unroll
-                    for (int c = 0; c < NC; ++c)
-#pragma unroll
-                         for (int a = 0; a < WM; ++a) {
-                              const int ic = wm * 16 * WM + 16 * a + l16;
-                              const double Sr = sA[((c * 4 + 0) * KC + r) * SA + ic];
-                              const double Si = sA[((c * 4 + 1) * KC + r) * SA + ic];
-                              const double Tr = sA[((c * 4 + 2) * KC + r) * SA + ic];
-                              const double Ti = sA[((c * 4 + 3) * KC + r) * SA + ic];
-#pragma unroll
-                              for (int b = 0; b < WN; ++b) {
-                                   v4d *q = acc[c][a][b];
-                                   q[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(Sr, bp[b], q[0], 0, 0, 0);
-                                   q[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(Si, bp[b], q[1], 0, 0, 0);
-                                   q[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(Tr, bm[b], q[2], 0, 0, 0);
-                                   q[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(Ti, bm[b], q[3], 0, 0, 0);
-                                   q[4] = __builtin_amdgcn_mfma_f64_16x16x4f64(sg * Sr, bm[b], q[4], 0, 0, 0);
-                                   q[5] = __builtin_amdgcn_mfma_f64_16x16x4f64(sg * Si, bm[b], q[5], 0, 0, 0);
-                                   q[6] = __builtin_amdgcn_mfma_f64_16x16x4f64(sg * Tr, bp[b], q[6], 0, 0, 0);
-                                   q[7] = __builtin_amdgcn_mfma_f64_16x16x4f64(sg * Ti, bp[b], q[7], 0, 0, 0);
-                              }
-                         }
-               }
-          }
-          // epilogue: Stokes elements, weights, reduction over this lane's sizes
-#pragma unroll
-          for (int a = 0; a < WM; ++a)
-#pragma unroll
-               for (int v = 0; v < 4; ++v) {
-                    const int i = it0 + wm * 16 * WM + 16 * a + lg + 4 * v;
-                    double wv[NW > 0 ? NW : 1], wt[NT > 0 ? NT : 1];
-#pragma unroll
-                    for (int c = 0; c < NW; ++c) wv[c] = p.W[c][i];
-#pragma unroll
-                    for (int t = 0; t < NT; ++t) wt[t] = p.WT[t][i];
-                    const double f0 = p.f[i];
-#pragma unroll
-                    for (int b = 0; b < WN; ++b) {
-                         const v4d *q = acc[0][a][b];
-                         double Pp[4], Pm[4];
-                         stokes(q[0][v], q[1][v], q[2][v], q[3][v], Pp);
-                         stokes(q[4][v], q[5][v], q[6][v], q[7][v], Pm);
-#pragma unroll
-                         for (int c = 0; c < NW; ++c)
-#pragma unroll
-                              for (int k = 0; k < 4; ++k) {
-                                   ew[c][b][k] += wv[c] * Pp[k];
-                                   ew[c][b][4 + k] += wv[c] * Pm[k];
-                              }
-#pragma unroll
-                         for (int t = 0; t < NT; ++t) {
-                              const v4d *d = acc[1 + t][a][b];
-                              double dPp[4], dPm[4];
-                              stokes_tan(q[0][v], q[1][v], q[2][v], q[3][v], d[0][v], d[1][v], d[2][v], d[3][v], dPp);
-                              stokes_tan(q[4][v], q[5][v], q[6][v], q[7][v], d[4][v], d[5][v], d[6][v], d[7][v], dPm);
-#pragma unroll
-                              for (int k = 0; k < 4; ++k) {
-                                   ew[NW + t][b][k] += wt[t] * Pp[k] + f0 * dPp[k];
-                                   ew[NW + t][b][4 + k] += wt[t] * Pm[k] + f0 * dPm[k];
-                              }
-                         }
-                         if (p.sst) {
-                              const int j = jt0 + wn * 16 * WN + 16 * b + l16;
-                              double *o = p.sst + ((size_t) i * p.Hp + j) * 8;
-#pragma unroll
-                              for (int c = 0; c < 8; ++c) o[c] = q[c][v];
-                         }
-                         if (p.save2 && i < p.N) {
-                              const int j = jt0 + wn * 16 * WN + 16 * b + l16;
-                              if (j < p.H) {
-#pragma unroll
-                                   for (int k = 0; k < 4; ++k) {
-                                        p.save2[((size_t) k * p.N + i) * p.Q + p.H + j] = Pp[k];
-                                        p.save2[((size_t) k * p.N + i) * p.Q + p.H - 1 - j] = Pm[k];
-                                   }
-                              }
-                         }
-                    }
-               }
-     }
-     // reduce over the 4 lane groups (same angle column), then over the two
-     // waves sharing the columns, then write this block's partial
-#pragma unroll
-     for (int c = 0; c < NW + NT; ++c)
-#pragma unroll
-          for (int b = 0; b < WN; ++b)
-#pragma unroll
-               for (int q = 0; q < 8; ++q) {
-                    double s = ew[c][b][q];
-                    s += __shfl_xor(s, 16);
-                    s += __shfl_xor(s, 32);
-                    ew[c][b][q] = s;
-               }
-     __syncthreads();
-     if (wm == 1 && lg == 0) {
-#pragma unroll
-          for (int c = 0; c < NW + NT; ++c)
-#pragma unroll
-               for (int b = 0; b < WN; ++b)
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) sR[((c * WN + b) * 8 + q) * 32 + wn * 16 + l16] = ew[c][b][q];
-     }
-     __syncthreads();
-     if (wm == 0 && lg == 0) {
-          const int nch = NW + NT;
-          double *out = p.part + (size_t) blockIdx.y * nch * 4 * p.Q;
-#pragma unroll
-          for (int b = 0; b < WN; ++b) {
-               const int j = jt0 + wn * 16 * WN + 16 * b + l16;
-               if (j < p.H) {
-#pragma unroll
-                    for (int c = 0; c < NW + NT; ++c)
-#pragma unroll
-                         for (int k = 0; k < 4; ++k) {
-                              const double vp = ew[c][b][k] + sR[((c * WN + b) * 8 + k) * 32 + wn * 16 + l16];
-                              const double vm = ew[c][b][4 + k] + sR[((c * WN + b) * 8 + 4 + k) * 32 + wn * 16 + l16];
-                              out[((size_t) c * 4 + k) * p.Q + p.H + j] = vp;
-                              out[((size_t) c * 4 + k) * p.Q + p.H - 1 - j] = vm;
-                         }
-               }
-          }
-     }
-}
-
 
 // Staging of one LDS stage of a blocked split operand: plane-major rows of
 // `cols` 16-byte columns, [plane][group of 8][column], `rows` = planes x G rows
@@ -2831,16 +2602,11 @@ __global__ __launch_bounds__(64) void rev_carry_b(const rev_carry_B *cases) {
 }
 
 
-// Sum of the per-block partials per (pass channel, element, angle); channel c
-// of the pass goes to channel map.g[c] of the output.
-struct ChMap {
-     int g[6];
-};
-
+// Sum of the per-tile partials per (channel, element, angle).
 // Eight lanes per output element, each summing every eighth block, then the
 // eight partials in a fixed order: deterministic, and eight times the
 // threads of a plain per-element loop.
-__device__ __forceinline__ void reduce_parts_body(const double *part, int nblk, int nchp, int Q, ChMap map, double *out) {
+__device__ __forceinline__ void reduce_parts_body(const double *part, int nblk, int nchp, int Q, double *out) {
      const int per = nchp * 4 * Q;
      const int e = blockIdx.x * 32 + (threadIdx.x >> 3), l = threadIdx.x & 7;
      double s = 0.;
@@ -2859,23 +2625,21 @@ __device__ __forceinline__ void reduce_parts_body(const double *part, int nblk, 
      s += __shfl_xor(s, 2);
      s += __shfl_xor(s, 4);
      if (e >= per || l) return;
-     const int c = e / (4 * Q), rem = e % (4 * Q);
-     out[(size_t) map.g[c] * 4 * Q + rem] = s;
+     out[e] = s;
 }
-__global__ __launch_bounds__(256) void reduce_parts(const double *part, int nblk, int nchp, int Q, ChMap map, double *out) { reduce_parts_body(part, nblk, nchp, Q, map, out); }
+__global__ __launch_bounds__(256) void reduce_parts(const double *part, int nblk, int nchp, int Q, double *out) { reduce_parts_body(part, nblk, nchp, Q, out); }
 struct reduce_parts_B {
      const double *part;
      int nblk;
      int nchp;
      int Q;
-     ChMap map;
      double *out;
      unsigned gx, gy;
 };
 __global__ __launch_bounds__(256) void reduce_parts_b(const reduce_parts_B *cases) {
      const reduce_parts_B a = cases[blockIdx.z];
      if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     reduce_parts_body(a.part, a.nblk, a.nchp, a.Q, a.map, a.out);
+     reduce_parts_body(a.part, a.nblk, a.nchp, a.Q, a.out);
 }
 
 
@@ -3217,13 +2981,15 @@ struct Workspace {
      std::vector<double> hguess;     // host staging of the Gauss root guesses
      std::vector<int2> htask;        // host staging of the contraction task list
      hipEvent_t ev[2 * LMIE_N_TIMERS + 2];
-     Buf x, sx, cx, f, n1, n2, kfill, ktile32, ktile64, dx, dm, dft, dfw;
-     Buf guess, mu, w, Bp, Bm, B16, A16, T, scrD, scrR, A, S, part, pf, E, coefs, dots, dotjobs, save2, order;
+     Buf x, sx, cx, f, n1, n2, kfill, ktile32, ktile64;
+     Buf wrow, comb;                // weight rows and directions of the raw channels
+     Buf guess, mu, w, Bp, Bm, B16, A16, T, A, S, part, pfraw, pf, E, coefs, dots, dotjobs, save2, order;
      std::vector<double> hsc;       // host staging of sin x, cos x
      // reverse-pass checkpoint and buffers
      Buf CB, sst, pfbar, bar, fang, mbar, fbar, gbar, expart;
      Buf wts, scal, L16, R16, Gf, G16, Uf, tasks;   // mixed reverse pass
-     Buf chD, chPC, chPS, chPart, revScan;   // per-size recurrences of the value channel
+     Buf chD, chPC, chPS, chPart, revScan;   // per-size recurrences
+     Buf chDz, chPQ;                // and what their tangents need
      Buf ftab;                      // order_factors of the value channel
      Buf sw, s1, s2;                // save_control 2: channel weights, saved per-size arrays
      Buf bargs, bup, bdown;         // per-case arguments and staging of a batch launched from here
@@ -3338,287 +3104,281 @@ struct Timer {
      }
 };
 
-// The FP64 contraction of a pass without tangent channels, with its operand
-// stages moved by direct loads (global_load_lds_dwordx4, 16 bytes a lane
-// straight into LDS, no registers) into ST LDS buffers: stages up to ST - 1
-// ahead load while the matrix cores work on this one, one barrier per stage.
-// One size tile per workgroup, the largest size tiles first.  On 32 x 32
-// tiles (WM = WN = 1) each wave holds 8 accumulators of 16 x 16 in ordinary
-// registers and two workgroups share a CU; with 16 accumulators (64 x 32
-// tiles) the compiler keeps them in ordinary registers across the stage loop
-// and copies them to the matrix-core registers and back at every stage,
-// which costs as much as the loads saved.  The products and their order are
-// those of angular_f64; the partials are per size tile (angular_f64 sums four
-// tiles per partial), so the sums group differently (1e-15 relative).
-template <int WM, int WN, int NW, int ST, int OCC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC))) void angular_f64_dma(AngArgs p) {
-     constexpr int TM = 32 * WM, TN = 32 * WN;
-     constexpr int SA = TM + 16, SB = TN + 16;       // LDS row strides (bank spread)
-     constexpr int AST = 4 * KC * SA, BST = 2 * KC * SB;
-     // direct loads one wave issues per stage (its vmcnt events)
-     constexpr int NLOAD = KC + KC / 2;
-     static_assert(TM * 8 <= 1024 && TN * 8 <= 1024 && KC % 4 == 0, "a row is one direct load of at most 64 lanes");
-     static_assert(ST == 2 || ST == 3, "stages");
-     static_assert(NLOAD < 64, "vmcnt field");
-     __shared__ double sA[ST * AST];
-     __shared__ double sB[ST * BST];
-     double *sR = sA;                    // [NW][WN][8][32], after the stages
-     static_assert(NW * 8 * 32 * WN <= ST * AST, "epilogue buffer");
+// ---------------------------------------------------------------------------
+// Angular contraction, FP64 matrix cores.
+//
+// For a tile of sizes i and positive angles j the four complex sums
+//   sp+ = sum_n S_n (pi+tau)_n   sm+ = sum_n T_n (pi-tau)_n
+//   sp- = sum_n s_n S_n (pi-tau)_n   sm- = sum_n s_n T_n (pi+tau)_n,
+// S_n = fv4 (a+b), T_n = fv4 (a-b), s_n = (-1)^(n-1) (the -mu mirror,
+// src/lmie_core.c:617-652,682-686), are 8 real GEMM accumulators of
+// v_mfma_f64_16x16x4 (operand lane layout: A[i][k] in lane i + 16 k, B[k][j] in
+// lane j + 16 k; result D[l/16 + 4 v][l % 16] in lane l, element v -- checked by
+// lmie_gpu_selftest_mfma_f64).
+//
+// Forward tangents: every direction's derivative of the sums is
+//   dS = dx_i S_x + dm S_m,
+// with S_x the derivative along the size parameter and S_m the (complex,
+// analytic) derivative along m, so two further operand sets (HX, HM) serve
+// any number of directions.  The epilogue forms the elements P and their
+// derivatives along x, Re m and Im m, and sums them over the sizes with one
+// weight row per raw channel: rows 0 .. nP-1 of W weigh P (the density, its
+// tangents), rows nP .. nP+nX-1 weigh dP/dx (f dx_i of each direction that
+// moves x), and the two last channels are dP/dRe m and dP/dIm m with the
+// weight of row 0.  combine_channels forms the directions from the sums.
+//
+// What bounds it: the FP64 matrix cores (64 cycles per instruction and SIMD).
+// A wave owns one 16 x 16 block with all its sums in registers (8
+// accumulators per operand set); WM x WN waves share an LDS tile of 16 WM
+// sizes x 16 WN angles, filled by direct loads (global_load_lds_dwordx4, 64
+// lanes x 16 bytes straight into LDS) ST - 1 stages of KS orders ahead, one
+// barrier per stage; a wave waits only for its own loads of the stage.  The
+// products' LDS reads are 16 consecutive doubles per lane group, so rows need
+// no padding.  (size tile, angle tile) tasks come from a host-built list dealt
+// over the XCDs.  Partials per size tile: part[tile][channel][4][Q].
+struct F64Args {
+     int Np, Kp, Hp, H, Q, N;
+     const double *A[3];        // operand planes [4][Kp][Np] of the value, then of d/dx, d/dm as present
+     const double *Bp, *Bm;     // [Kp][Hp]
+     const int *ktile;          // rows to contract per size tile
+     const int2 *task;          // (size tile, angle tile), (-1, -1) none
+     const double *W;           // [nP + nX][Np] weight rows, row 0 the density
+     int nP, nX;
+     double *part;              // [size tiles][channels][4][Q]
+     double *save2;             // [4][N][Q] per-size matrix (save_control 1) or NULL
+     double *sst;               // reverse-pass checkpoint [Np][Hp][8]: sp+, sm+, sp-, sm- (re, im) or NULL
+};
 
+// waits until at most n of this wave's vector memory operations are in
+// flight (vmcnt in bits 3:0 and 15:14; lgkmcnt and expcnt left open)
+template <int n>
+__device__ __forceinline__ void wait_vm() {
+     static_assert(n < 64, "vmcnt field");
+     __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
+}
+
+template <int WM, int WN, bool HX, bool HM, int KS, int ST, int OCC>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OCC))) void angular_f64(F64Args p) {
+     constexpr int NB = 1 + HX + HM, NW = WM * WN, TM = 16 * WM, TN = 16 * WN;
+     constexpr int ASTG = NB * 4 * KS * TM, STG = ASTG + 2 * KS * TN;
+     constexpr int NL = STG / (128 * NW);             // direct loads per wave and stage
+     static_assert(STG % (128 * NW) == 0 && ASTG % 128 == 0 && KS % 4 == 0, "whole 1 KiB loads");
+     static_assert(ST >= 2 && ST <= 4 && NL * (ST - 2) < 64, "stages");
+     constexpr int CHB = 8 * WM * TN;                 // epilogue buffer per channel
+     constexpr int CAP = ST * STG / CHB;              // channels per flush
+     __shared__ double sh[ST * STG];
+
+     const int2 tk = p.task[blockIdx.x];
+     if (tk.x < 0) return;
      const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-     const int wm = wave & 1, wn = wave >> 1;
+     const int wm = wave % WM, wn = wave / WM;
      const int l16 = lane & 15, lg = lane >> 4;
-     const int jt0 = blockIdx.x * TN;
-     const int tile = gridDim.y - 1 - blockIdx.y;
-     const int it0 = tile * TM;
+     const int tile = tk.x, it0 = tile * TM, jt0 = tk.y * TN;
      const size_t Np = p.Np, Hp = p.Hp, plane = (size_t) p.Kp * Np;
-     const int nch = p.ktile[tile] / KC;
+     const int nch = p.ktile[tile] / KS;
 
-     // stage of orders k0 .. k0 + KC - 1 into buffer b_: A rows (plane, order)
-     // of TM sizes and B rows ((pi+tau) / (pi-tau), order) of TN angles, one
-     // direct load per row, rows dealt over the four waves
-     auto stage_load = [&](int b_, int k0) {
+     // this lane's source of each of the wave's loads at stage 0, and the step
+     // to the next stage
+     const double *src[NL];
+     size_t step[NL];
 #pragma unroll
-          for (int u = 0; u < KC; ++u) {
-               const int row = wave + 4 * u, pl = row / KC, r = row % KC;
-               if (lane < TM / 2)
-                    __builtin_amdgcn_global_load_lds(
-                         (const void *) (p.A[0] + pl * plane + (size_t) (k0 + r) * Np + it0 + 2 * lane),
-                         (lds_ptr) (sA + b_ * AST + row * SA), 16, 0, 0);
+     for (int u = 0; u < NL; ++u) {
+          const int c = wave + NW * u;
+          if (c < ASTG / 128) {
+               const int e = c * 128 + 2 * lane, row = e / TM, pl = row / KS;
+               const double *base = p.A[0];
+               if (NB > 1 && pl >= 4) base = p.A[1];
+               if (NB > 2 && pl >= 8) base = p.A[2];
+               src[u] = base + (size_t) (pl & 3) * plane + (size_t) (row % KS) * Np + it0 + e % TM;
+               step[u] = (size_t) KS * Np;
+          } else {
+               const int e = c * 128 - ASTG + 2 * lane, row = e / TN;
+               src[u] = (row / KS ? p.Bm : p.Bp) + (size_t) (row % KS) * Hp + jt0 + e % TN;
+               step[u] = (size_t) KS * Hp;
           }
+     }
+     auto stage_load = [&](int buf) {
 #pragma unroll
-          for (int u = 0; u < KC / 2; ++u) {
-               const int row = wave + 4 * u, pm = row / KC, r = row % KC;
-               const double *src = pm ? p.Bm : p.Bp;
-               if (lane < TN / 2)
-                    __builtin_amdgcn_global_load_lds((const void *) (src + (size_t) (k0 + r) * Hp + jt0 + 2 * lane),
-                                                     (lds_ptr) (sB + b_ * BST + row * SB), 16, 0, 0);
+          for (int u = 0; u < NL; ++u) {
+               __builtin_amdgcn_global_load_lds((const void *) src[u], (lds_ptr) (sh + buf * STG + (wave + NW * u) * 128), 16, 0, 0);
+               src[u] += step[u];
           }
      };
 
-     v4d acc[WM][WN][8];
+     v4d acc[NB][8];
 #pragma unroll
-     for (int a = 0; a < WM; ++a)
+     for (int b = 0; b < NB; ++b)
 #pragma unroll
-          for (int b = 0; b < WN; ++b)
-#pragma unroll
-               for (int q = 0; q < 8; ++q) acc[a][b][q] = v4d{0., 0., 0., 0.};
+          for (int q = 0; q < 8; ++q) acc[b][q] = v4d{0., 0., 0., 0.};
 
-     // stages 0 .. ST - 2 in flight before the first is computed
+     // s_n of this lane's orders (k0 + 4 ks + lg + 1: alternate lane groups)
+     const unsigned long long sgn = (unsigned long long) (lg & 1) << 63;
+     auto flip = [&](double v) { return __longlong_as_double((long long) ((unsigned long long) __double_as_longlong(v) ^ sgn)); };
 #pragma unroll
      for (int k = 0; k < ST - 1; ++k)
-          if (k < nch) stage_load(k, k * KC);
+          if (k < nch) stage_load(k);
+     int buf = 0, nbuf = ST - 1;
      for (int kc = 0; kc < nch; ++kc) {
-          const int buf = kc % ST, k0 = kc * KC;
-          // this wave's rows of the stage have landed (the younger stage may
-          // stay in flight: the loads complete in order), then everyone's;
-          // every wave is also done with the buffer of stage kc - 1, which
-          // takes stage kc + ST - 1
-          // (vmcnt in bits 3:0 and 15:14, lgkmcnt and expcnt left open)
-          if (ST == 3 && kc + 1 < nch) __builtin_amdgcn_s_waitcnt(0x0F70 | (NLOAD & 15) | ((NLOAD >> 4) << 14));
-          else __builtin_amdgcn_s_waitcnt(0);
+          // this wave's loads of the stage have landed (they complete in order;
+          // the younger stages stay in flight), then everyone's; every wave is
+          // also done with the buffer of stage kc - 1, which takes stage
+          // kc + ST - 1
+          const int young = nch - 1 - kc;
+          if (ST >= 4 && young >= 2) wait_vm<NL * (ST >= 4 ? 2 : 0)>();
+          else if (ST >= 3 && young >= 1) wait_vm<NL>();
+          else wait_vm<0>();
           __builtin_amdgcn_s_barrier();
           __asm__ volatile("" ::: "memory");
-          if (kc + ST - 1 < nch) stage_load((kc + ST - 1) % ST, (kc + ST - 1) * KC);
-          const double *a0 = sA + buf * AST, *b0 = sB + buf * BST;
+          if (kc + ST - 1 < nch) stage_load(nbuf);
+          const double *a0 = sh + buf * STG + lg * TM + 16 * wm + l16;
+          const double *b0 = sh + buf * STG + ASTG + lg * TN + 16 * wn + l16;
 #pragma unroll
-          for (int ks = 0; ks < KC / 4; ++ks) {
-               const int r = ks * 4 + lg;                   // this lane's k row
-               const double sg = ((k0 + r) & 1) ? -1. : 1.;   // s_n, n = k0 + r + 1
-               // the -mu products take s_n on the angle operand: the same
-               // products as s_n on the size operand (a sign), fewer multiplies
-               double bp[WN], bm[WN], sbp[WN], sbm[WN];
+          for (int ks = 0; ks < KS / 4; ++ks) {
+               // the -mu products take s_n on the angle operand
+               const double bp = b0[4 * ks * TN], bm = b0[(KS + 4 * ks) * TN];
+               const double sbp = flip(bp), sbm = flip(bm);
 #pragma unroll
-               for (int b = 0; b < WN; ++b) {
-                    const int jc = wn * 16 * WN + 16 * b + l16;
-                    bp[b] = b0[r * SB + jc];
-                    bm[b] = b0[(KC + r) * SB + jc];
-                    sbp[b] = sg * bp[b];
-                    sbm[b] = sg * bm[b];
-               }
-#pragma unroll
-               for (int a = 0; a < WM; ++a) {
-                    const int ic = wm * 16 * WM + 16 * a + l16;
-                    const double Sr = a0[(0 * KC + r) * SA + ic];
-                    const double Si = a0[(1 * KC + r) * SA + ic];
-                    const double Tr = a0[(2 * KC + r) * SA + ic];
-                    const double Ti = a0[(3 * KC + r) * SA + ic];
-#pragma unroll
-                    for (int b = 0; b < WN; ++b) {
-                         v4d *q = acc[a][b];
-                         q[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(Sr, bp[b], q[0], 0, 0, 0);
-                         q[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(Si, bp[b], q[1], 0, 0, 0);
-                         q[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(Tr, bm[b], q[2], 0, 0, 0);
-                         q[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(Ti, bm[b], q[3], 0, 0, 0);
-                         q[4] = __builtin_amdgcn_mfma_f64_16x16x4f64(Sr, sbm[b], q[4], 0, 0, 0);
-                         q[5] = __builtin_amdgcn_mfma_f64_16x16x4f64(Si, sbm[b], q[5], 0, 0, 0);
-                         q[6] = __builtin_amdgcn_mfma_f64_16x16x4f64(Tr, sbp[b], q[6], 0, 0, 0);
-                         q[7] = __builtin_amdgcn_mfma_f64_16x16x4f64(Ti, sbp[b], q[7], 0, 0, 0);
-                    }
+               for (int b = 0; b < NB; ++b) {
+                    const double Sr = a0[((4 * b + 0) * KS + 4 * ks) * TM], Si = a0[((4 * b + 1) * KS + 4 * ks) * TM];
+                    const double Tr = a0[((4 * b + 2) * KS + 4 * ks) * TM], Ti = a0[((4 * b + 3) * KS + 4 * ks) * TM];
+                    v4d *q = acc[b];
+                    q[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(Sr, bp, q[0], 0, 0, 0);
+                    q[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(Si, bp, q[1], 0, 0, 0);
+                    q[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(Tr, bm, q[2], 0, 0, 0);
+                    q[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(Ti, bm, q[3], 0, 0, 0);
+                    q[4] = __builtin_amdgcn_mfma_f64_16x16x4f64(Sr, sbm, q[4], 0, 0, 0);
+                    q[5] = __builtin_amdgcn_mfma_f64_16x16x4f64(Si, sbm, q[5], 0, 0, 0);
+                    q[6] = __builtin_amdgcn_mfma_f64_16x16x4f64(Tr, sbp, q[6], 0, 0, 0);
+                    q[7] = __builtin_amdgcn_mfma_f64_16x16x4f64(Ti, sbp, q[7], 0, 0, 0);
                }
           }
+          buf = buf + 1 == ST ? 0 : buf + 1;
+          nbuf = nbuf + 1 == ST ? 0 : nbuf + 1;
      }
 
-     // epilogue: Stokes elements, weights, reduction over this lane's sizes
-     double ew[NW][WN][8];
-#pragma unroll
-     for (int c = 0; c < NW; ++c)
-#pragma unroll
-          for (int b = 0; b < WN; ++b)
-#pragma unroll
-               for (int q = 0; q < 8; ++q) ew[c][b][q] = 0.;
-#pragma unroll
-     for (int a = 0; a < WM; ++a)
+     // epilogue: Stokes elements, weighted sums over this wave's 16 sizes (four
+     // per lane, then the four lane groups), over the WM waves of a column in
+     // a fixed order through LDS
+     const int i0 = it0 + 16 * wm + lg, j = jt0 + 16 * wn + l16;
+     if (p.sst || p.save2) {
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
-               const int i = it0 + wm * 16 * WM + 16 * a + lg + 4 * v;
-               double wv[NW];
+               const int i = i0 + 4 * v;
+               if (p.sst) {
+                    double *o = p.sst + ((size_t) i * Hp + j) * 8;
 #pragma unroll
-               for (int c = 0; c < NW; ++c) wv[c] = p.W[c][i];
-#pragma unroll
-               for (int b = 0; b < WN; ++b) {
-                    const v4d *q = acc[a][b];
+                    for (int c = 0; c < 8; ++c) o[c] = acc[0][c][v];
+               }
+               if (p.save2 && i < p.N && j < p.H) {
                     double Pp[4], Pm[4];
-                    stokes(q[0][v], q[1][v], q[2][v], q[3][v], Pp);
-                    stokes(q[4][v], q[5][v], q[6][v], q[7][v], Pm);
+                    stokes(acc[0][0][v], acc[0][1][v], acc[0][2][v], acc[0][3][v], Pp);
+                    stokes(acc[0][4][v], acc[0][5][v], acc[0][6][v], acc[0][7][v], Pm);
 #pragma unroll
-                    for (int c = 0; c < NW; ++c)
-#pragma unroll
-                         for (int k = 0; k < 4; ++k) {
-                              ew[c][b][k] += wv[c] * Pp[k];
-                              ew[c][b][4 + k] += wv[c] * Pm[k];
-                         }
-                    if (p.sst) {
-                         const int j = jt0 + wn * 16 * WN + 16 * b + l16;
-                         double *o = p.sst + ((size_t) i * p.Hp + j) * 8;
-#pragma unroll
-                         for (int c = 0; c < 8; ++c) o[c] = q[c][v];
-                    }
-                    if (p.save2 && i < p.N) {
-                         const int j = jt0 + wn * 16 * WN + 16 * b + l16;
-                         if (j < p.H) {
-#pragma unroll
-                              for (int k = 0; k < 4; ++k) {
-                                   p.save2[((size_t) k * p.N + i) * p.Q + p.H + j] = Pp[k];
-                                   p.save2[((size_t) k * p.N + i) * p.Q + p.H - 1 - j] = Pm[k];
-                              }
-                         }
+                    for (int k = 0; k < 4; ++k) {
+                         p.save2[((size_t) k * p.N + i) * p.Q + p.H + j] = Pp[k];
+                         p.save2[((size_t) k * p.N + i) * p.Q + p.H - 1 - j] = Pm[k];
                     }
                }
           }
-     // reduce over the 4 lane groups (same angle column), then over the two
-     // waves sharing the columns, then write this block's partial
-#pragma unroll
-     for (int c = 0; c < NW; ++c)
-#pragma unroll
-          for (int b = 0; b < WN; ++b)
-#pragma unroll
-               for (int q = 0; q < 8; ++q) {
-                    double v = ew[c][b][q];
-                    v += __shfl_xor(v, 16);
-                    v += __shfl_xor(v, 32);
-                    ew[c][b][q] = v;
-               }
-     __syncthreads();                    // every wave is done with the stages (sR aliases them)
-     if (wm == 1 && lg == 0) {
-#pragma unroll
-          for (int c = 0; c < NW; ++c)
-#pragma unroll
-               for (int b = 0; b < WN; ++b)
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) sR[((c * WN + b) * 8 + q) * 32 + wn * 16 + l16] = ew[c][b][q];
      }
-     __syncthreads();
-     if (wm == 0 && lg == 0) {
-          double *out = p.part + (size_t) tile * NW * 4 * p.Q;
+     const int nraw = p.nP + p.nX + (HM ? 2 : 0);
+     double *out = p.part + (size_t) tile * nraw * 4 * p.Q;
+     for (int c0 = 0; c0 < nraw; c0 += CAP) {
+          const int c1 = c0 + CAP < nraw ? c0 + CAP : nraw;
+          __syncthreads();               // every wave is done with the stages (or the last flush)
 #pragma unroll
-          for (int b = 0; b < WN; ++b) {
-               const int j = jt0 + wn * 16 * WN + 16 * b + l16;
-               if (j < p.H) {
+          for (int sg = 0; sg < 2; ++sg) {
+               // elements of kind kd (0: P, 1: dP/dx, 2, 3: dP/dRe m, dP/dIm m)
+               // under the weight rows of channels k0 .. k1 - 1
+               auto kind = [&](auto kdc, int k0, int k1) {
+                    constexpr int kd = decltype(kdc)::value;
+                    k0 = k0 < c0 ? c0 : k0;
+                    k1 = k1 > c1 ? c1 : k1;
+                    if (k0 >= k1) return;
+                    double e[4][4];
 #pragma unroll
-                    for (int c = 0; c < NW; ++c)
+                    for (int v = 0; v < 4; ++v) {
+                         const v4d *q = acc[0] + 4 * sg, *d = acc[kd == 0 ? 0 : kd == 1 ? 1 : NB - 1] + 4 * sg;
+                         if constexpr (kd == 0) stokes(q[0][v], q[1][v], q[2][v], q[3][v], e[v]);
+                         else if constexpr (kd < 3)
+                              stokes_tan(q[0][v], q[1][v], q[2][v], q[3][v], d[0][v], d[1][v], d[2][v], d[3][v], e[v]);
+                         else
+                              stokes_tan(q[0][v], q[1][v], q[2][v], q[3][v], -d[1][v], d[0][v], -d[3][v], d[2][v], e[v]);
+                    }
+                    for (int c = k0; c < k1; ++c) {
+                         const double *w = p.W + (kd < 2 ? (size_t) c * Np : 0) + i0;
+                         double r[4] = {0., 0., 0., 0.};
+#pragma unroll
+                         for (int v = 0; v < 4; ++v) {
+                              const double wv = w[4 * v];
+#pragma unroll
+                              for (int k = 0; k < 4; ++k) r[k] += wv * e[v][k];
+                         }
 #pragma unroll
                          for (int k = 0; k < 4; ++k) {
-                              const double vp = ew[c][b][k] + sR[((c * WN + b) * 8 + k) * 32 + wn * 16 + l16];
-                              const double vm = ew[c][b][4 + k] + sR[((c * WN + b) * 8 + 4 + k) * 32 + wn * 16 + l16];
-                              out[((size_t) c * 4 + k) * p.Q + p.H + j] = vp;
-                              out[((size_t) c * 4 + k) * p.Q + p.H - 1 - j] = vm;
+                              r[k] += __shfl_xor(r[k], 16);
+                              r[k] += __shfl_xor(r[k], 32);
                          }
+                         // lane group k stores element k
+                         const double t = lg == 0 ? r[0] : lg == 1 ? r[1] : lg == 2 ? r[2] : r[3];
+                         sh[(c - c0) * CHB + ((4 * sg + lg) * WM + wm) * TN + 16 * wn + l16] = t;
+                    }
+               };
+               kind(std::integral_constant<int, 0>{}, 0, p.nP);
+               if constexpr (HX) kind(std::integral_constant<int, 1>{}, p.nP, p.nP + p.nX);
+               if constexpr (HM) {
+                    kind(std::integral_constant<int, 2>{}, p.nP + p.nX, p.nP + p.nX + 1);
+                    kind(std::integral_constant<int, 3>{}, p.nP + p.nX + 1, p.nP + p.nX + 2);
                }
           }
-     }
-}
-
-// Operand staging of the FP64 contraction without tangent channels
-// (environment LMIE_F64_STAGING, read at every call): 1 (default) direct
-// loads into two LDS buffers on 32 x 32 tiles (angular_f64_dma, 16 x 16 per
-// wave, two workgroups per CU); 0 the loads through registers into one
-// buffer on 64 x 32 tiles (angular_f64).  Measured on the two-mode workload
-// (32768 sizes, 3810 angles): 20.9 against 43.7 ms; the direct loads on
-// 64 x 32 tiles took 26.1 ms with three buffers and 27.0 with two.
-int f64_staging() {
-     const char *e = getenv("LMIE_F64_STAGING");
-     return e && atoi(e) == 0 ? 0 : 1;
-}
-
-// Size tile of the FP64 contraction of a pass: 32 with tangent channels or
-// the direct loads, else 64
-int f64_tile(int n_tan, int staging) { return n_tan > 0 || staging != 0 ? 32 : 64; }
-
-// Size tiles per workgroup of the FP64 contraction: one for the direct-load
-// kernel, four for angular_f64 (each workgroup's partial takes one slot)
-int f64_tiles_per_block(int n_tan, int staging) { return n_tan == 0 && staging != 0 ? 1 : 4; }
-
-// Launch sequence of the contraction for one pass (up to 2 tangent channels
-// and up to 4 weight channels).
-template <int WM, int WN, int NT, int NW>
-int launch_angular(const AngArgs &a, int n_tiles, int staging, hipStream_t s, int *nblk_out) {
-     constexpr int TM = 32 * WM, TN = 32 * WN;
-     (void) TM;
-     const int tpb = f64_tiles_per_block(NT, staging);
-     const int nblk = (n_tiles + tpb - 1) / tpb;
-     AngArgs b = a;
-     b.tiles_per_block = tpb;
-     dim3 grid(a.Hp / TN, nblk);
-     if constexpr (NT == 0) {
-          if constexpr (WM == 1 && WN == 1) {
-               if (staging != 0) hipLaunchKernelGGL((angular_f64_dma<WM, WN, NW, 2, 2>), grid, dim3(256), 0, s, b);
-               else hipLaunchKernelGGL((angular_f64<WM, WN, NT, NW>), grid, dim3(256), 0, s, b);
-          } else {
-               if (staging == 0) hipLaunchKernelGGL((angular_f64<WM, WN, NT, NW>), grid, dim3(256), 0, s, b);
-               else return set_err("internal: FP64 staging %d with %d x %d tiles", staging, TM, TN);
+          __syncthreads();
+          for (int e = threadIdx.x; e < (c1 - c0) * 8 * TN; e += 64 * NW) {
+               const int jc = e % TN, ck = e / TN, k = ck & 7, c = ck >> 3;
+               const double *t = sh + (size_t) c * CHB + k * WM * TN + jc;
+               double s = t[0];
+#pragma unroll
+               for (int m = 1; m < WM; ++m) s += t[m * TN];
+               if (jt0 + jc < p.H)
+                    out[((size_t) (c0 + c) * 4 + (k & 3)) * p.Q + (k < 4 ? p.H + jt0 + jc : p.H - 1 - jt0 - jc)] = s;
           }
-     } else {
-          hipLaunchKernelGGL((angular_f64<WM, WN, NT, NW>), grid, dim3(256), 0, s, b);
-     }
-     HIPCHECK(hipGetLastError());
-     *nblk_out = nblk;
-     return 0;
-}
-
-template <int WM, int WN, int NT>
-int launch_angular_nw(int nw, const AngArgs &a, int n_tiles, int staging, hipStream_t s, int *nblk) {
-     switch (nw) {
-     case 0:
-          if (NT == 0) return set_err("internal: contraction pass without channels");
-          return launch_angular<WM, WN, NT, (NT > 0 ? 0 : 1)>(a, n_tiles, staging, s, nblk);
-     case 1: return launch_angular<WM, WN, NT, 1>(a, n_tiles, staging, s, nblk);
-     case 2: return launch_angular<WM, WN, NT, 2>(a, n_tiles, staging, s, nblk);
-     case 3: return launch_angular<WM, WN, NT, 3>(a, n_tiles, staging, s, nblk);
-     default: return launch_angular<WM, WN, NT, 4>(a, n_tiles, staging, s, nblk);
      }
 }
 
-int launch_coefs(int nt, const CoefArgs &c, hipStream_t s) {
-     dim3 grid(c.Np / 64);
-     switch (nt) {
-     case 1: hipLaunchKernelGGL(mie_coefs<1>, grid, dim3(64), 0, s, c); break;
-     case 2: hipLaunchKernelGGL(mie_coefs<2>, grid, dim3(64), 0, s, c); break;
-     case 3: hipLaunchKernelGGL(mie_coefs<3>, grid, dim3(64), 0, s, c); break;
-     default: hipLaunchKernelGGL(mie_coefs<4>, grid, dim3(64), 0, s, c); break;
-     }
+// Tiles of the FP64 contraction and the size tiles per group of its task list.
+// 32 x 32 tiles on four waves, two stages: three workgroups per CU with one
+// operand set, two with more (the accumulators then take 128 or 192
+// registers).  Measured on the two-mode workload (32768 sizes, 3810 angles, one
+// set) and the gamma mode with tangents of m (16384 sizes, 1922 angles, two
+// sets): 14.7 and 4.3 ms; the same tiles with three stages and two workgroups
+// per CU 15.2 and 4.6; 32 x 64 on eight waves 15.7 and 4.6; 64 x 64 on
+// sixteen waves 15.3.  Groups of 1 or 2 size tiles took 0.3-0.4 ms less than 4
+// or 8, of 16 1 ms more.
+constexpr int F64_TILE = 32, F64_GROUP = 2;
+
+int launch_angular_f64(const F64Args &a, bool hx, bool hm, unsigned ntask, hipStream_t s) {
+     if (!hx && !hm) hipLaunchKernelGGL((angular_f64<2, 2, false, false, 16, 2, 3>), dim3(ntask), dim3(256), 0, s, a);
+     else if (!hm) hipLaunchKernelGGL((angular_f64<2, 2, true, false, 8, 2, 2>), dim3(ntask), dim3(256), 0, s, a);
+     else if (!hx) hipLaunchKernelGGL((angular_f64<2, 2, false, true, 8, 2, 2>), dim3(ntask), dim3(256), 0, s, a);
+     else hipLaunchKernelGGL((angular_f64<2, 2, true, true, 8, 2, 2>), dim3(ntask), dim3(256), 0, s, a);
      HIPCHECK(hipGetLastError());
      return 0;
+}
+
+// Directions from the raw channels: out[o] = sum_t c_t raw[r_t] (r_t < 0: none),
+// each channel 4 Q elements.
+struct ChComb {
+     int r[4];
+     double c[4];
+};
+__global__ __launch_bounds__(256) void combine_channels(const double *raw, int per, const ChComb *comb, double *out) {
+     const int e = blockIdx.x * 256 + threadIdx.x;
+     if (e >= per) return;
+     const ChComb k = comb[blockIdx.y];
+     double s = 0.;
+#pragma unroll
+     for (int t = 0; t < 4; ++t)
+          if (k.r[t] >= 0) s += k.c[t] * raw[(size_t) k.r[t] * per + e];
+     out[(size_t) blockIdx.y * per + e] = s;
 }
 
 // Task list of a tiled contraction over (size tile, column tile) pairs for
@@ -3756,10 +3516,8 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
      // uploads
      if (w->x.get(sizeof(double) * Np) || w->f.get(sizeof(double) * Np) || w->n1.get(sizeof(int) * Np) ||
          w->n2.get(sizeof(int) * Np) || w->kfill.get(sizeof(int) * nt64) || w->ktile32.get(sizeof(int) * nt32) ||
-         w->ktile64.get(sizeof(int) * nt64) || w->dx.get(sizeof(double) * Np * (nt ? nt : 1)) ||
-         w->dm.get(sizeof(double) * 2 * (nt ? nt : 1)) || w->dft.get(sizeof(double) * Np * (nt ? nt : 1)) ||
-         w->dfw.get(sizeof(double) * Np * (nw ? nw : 1)) || w->sx.get(sizeof(double) * Np) ||
-         w->cx.get(sizeof(double) * Np) || w->S.get(sizeof(double) * 4 * Np * (1 + nt)))
+         w->ktile64.get(sizeof(int) * nt64) || w->sx.get(sizeof(double) * Np) ||
+         w->cx.get(sizeof(double) * Np) || w->S.get(sizeof(double) * 4 * Np * (nt ? 4 : 1)))
           return -1;
      // every input of the pipeline goes up in one pinned host-to-device copy
      // and one copy_jobs launch (a dozen small pageable copies cost more host
@@ -3786,16 +3544,50 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
               up.add(w->ktile64.p, kt64.data(), sizeof(int) * nt64))
                return -1;
      }
-     // seed columns zero-padded to Np
-     auto add_padded = [&](Buf &dst, const double *src, int rows) -> int {
-          std::vector<double> pad((size_t) Np * rows, 0.);
-          for (int t = 0; t < rows; ++t) memcpy(pad.data() + (size_t) t * Np, src + (size_t) t * N, sizeof(double) * N);
-          return up.add(dst.p, pad.data(), sizeof(double) * pad.size());
+     // raw channels of the sums over sizes: weight rows of the value (row 0 the
+     // density, then the weight-only directions and the density tangents of the
+     // directions that move x or m), weight rows f dx_i of the value's x
+     // derivative, then its Re m and Im m derivatives under the density
+     // (angular_f64); comb[o] forms direction o from them.
+     std::vector<ChComb> comb(nch, ChComb{{-1, -1, -1, -1}, {1., 1., 1., 1.}});
+     std::vector<double> wrow((size_t) Np, 0.);
+     memcpy(wrow.data(), J->f, sizeof(double) * N);
+     auto add_row = [&](const double *src, const double *by) -> int {   // src (times by), zero-padded to Np
+          const size_t o = wrow.size();
+          wrow.resize(o + Np, 0.);
+          for (int i = 0; i < N; ++i) wrow[o + i] = by ? src[i] * by[i] : src[i];
+          return (int) (o / Np);
      };
-     if (nt && (add_padded(w->dx, J->dx, nt) || add_padded(w->dft, J->df_tan, nt) ||
-                up.add(w->dm.p, J->dm, sizeof(double) * 2 * nt)))
+     auto moves = [&](const double *v) {
+          for (int i = 0; i < N; ++i)
+               if (v[i] != 0.) return true;
+          return false;
+     };
+     bool hx = false, hm = false;
+     comb[0].r[0] = 0;
+     for (int t = 0; t < nw; ++t) comb[1 + nt + t].r[0] = add_row(J->df_wgt + (size_t) t * N, nullptr);
+     for (int t = 0; t < nt; ++t)
+          if (moves(J->df_tan + (size_t) t * N)) comb[1 + t].r[0] = add_row(J->df_tan + (size_t) t * N, nullptr);
+     const int nP = (int) (wrow.size() / Np);
+     for (int t = 0; t < nt; ++t)
+          if (moves(J->dx + (size_t) t * N)) {
+               comb[1 + t].r[1] = add_row(J->dx + (size_t) t * N, J->f);
+               hx = true;
+          }
+     const int nX = (int) (wrow.size() / Np) - nP;
+     for (int t = 0; t < nt; ++t)
+          if (J->dm[2 * t] != 0. || J->dm[2 * t + 1] != 0.) {
+               comb[1 + t].r[2] = nP + nX;
+               comb[1 + t].r[3] = nP + nX + 1;
+               comb[1 + t].c[2] = J->dm[2 * t];
+               comb[1 + t].c[3] = J->dm[2 * t + 1];
+               hm = true;
+          }
+     const int nraw = nP + nX + (hm ? 2 : 0), nb = 1 + hx + hm;
+     const bool tan = hx || hm;
+     if (w->wrow.get(sizeof(double) * wrow.size()) || up.add(w->wrow.p, wrow.data(), sizeof(double) * wrow.size()) ||
+         w->comb.get(sizeof(ChComb) * nch) || (nt && up.add(w->comb.p, comb.data(), sizeof(ChComb) * nch)))
           return -1;
-     if (nw && add_padded(w->dfw, J->df_wgt, nw)) return -1;
      if (Q > 0) {
           // initial guesses of the Gauss roots (host C library)
           if (w->guess.get(sizeof(double) * H)) return -1;
@@ -3804,7 +3596,7 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           if (up.add(w->guess.p, w->hguess.data(), sizeof(double) * H)) return -1;
      }
      // pinned landing area of the results: expansions [2][nch][6][C], then the sums
-     if (w->pres.get(sizeof(double) * ((size_t) nch * 12 * C + 4 * nch))) return -1;
+     if (w->pres.get(sizeof(double) * ((size_t) nch * 12 * C + 4 * nraw))) return -1;
      if (mixed) {
           // the contraction's task list
           xcd_tasks(ms.tm == 64 ? kt64 : kt32, [&](int) { return (H + ms.tn - 1) / ms.tn; }, mix_group(), w->htask);
@@ -3812,18 +3604,22 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
               up.add(w->order.p, w->htask.data(), sizeof(int2) * w->htask.size()))
                return -1;
      }
-     // series dot products: channel 0, then tangent, then weight-only channels
+     if (!mixed && Q > 0) {
+          xcd_tasks(kt32, [&](int) { return (H + F64_TILE - 1) / F64_TILE; }, F64_GROUP, w->htask);
+          if (w->order.get(sizeof(int2) * w->htask.size()) ||
+              up.add(w->order.p, w->htask.data(), sizeof(int2) * w->htask.size()))
+               return -1;
+     }
+     // series dot products of every raw channel
      std::vector<DotJob> dot_jobs;
      {
-          const double *S0 = w->S.as<double>(), *f = w->f.as<double>();
-          for (int q = 0; q < 4; ++q) dot_jobs.push_back(DotJob{f, S0 + (size_t) q * Np, nullptr, nullptr});
-          for (int t = 0; t < nt; ++t)
+          const double *S0 = w->S.as<double>(), *W0 = w->wrow.as<double>();
+          const double *SX = S0 + 4 * (size_t) Np, *SM = S0 + 4 * (size_t) Np * (hx ? 2 : 1);
+          for (int c = 0; c < nraw; ++c)
                for (int q = 0; q < 4; ++q)
-                    dot_jobs.push_back(DotJob{w->dft.as<double>() + (size_t) t * Np, S0 + (size_t) q * Np, f,
-                                              w->S.as<double>() + (size_t) 4 * Np * (1 + t) + (size_t) q * Np});
-          for (int t = 0; t < nw; ++t)
-               for (int q = 0; q < 4; ++q)
-                    dot_jobs.push_back(DotJob{w->dfw.as<double>() + (size_t) t * Np, S0 + (size_t) q * Np, nullptr, nullptr});
+                    dot_jobs.push_back(DotJob{W0 + (c < nP + nX ? (size_t) c * Np : 0),
+                                              (c < nP ? S0 : c < nP + nX ? SX : SM + 4 * (size_t) Np * (c - nP - nX)) +
+                                                   (size_t) q * Np, nullptr, nullptr});
           if (w->dotjobs.get(sizeof(DotJob) * dot_jobs.size()) || w->dots.get(sizeof(double) * dot_jobs.size()) ||
               up.add(w->dotjobs.p, dot_jobs.data(), sizeof(DotJob) * dot_jobs.size()))
                return -1;
@@ -3883,13 +3679,10 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
      return 0;
      };
 
-     // per-size coefficients (passes of up to 4 tangent channels)
-     const size_t plane = (size_t) Kp * Np, srow = (size_t) (n1max + 1) * Np;
-     const int nt_pass = nt < 4 ? nt : 4;
-     if ((!mixed && w->A.get(sizeof(double) * 4 * plane * (1 + nt))) || w->S.get(sizeof(double) * 4 * Np * (1 + nt)) ||
-         (mixed && w->A16.get(sizeof(unsigned short) * 8 * (size_t) Kb * Np * 8)) ||
-         (nt && (w->scrD.get(sizeof(double) * 2 * srow * (1 + nt_pass)) ||
-                 w->scrR.get(sizeof(double) * srow * (1 + nt_pass)))))
+     // per-size coefficients
+     const size_t plane = (size_t) Kp * Np;
+     if ((!mixed && w->A.get(sizeof(double) * 4 * plane * nb)) ||
+         (mixed && w->A16.get(sizeof(unsigned short) * 8 * (size_t) Kb * Np * 8)))
           return -1;
      const int keep = J->keep;
      if (keep) {
@@ -3899,26 +3692,50 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
                return -1;
      }
      tm.mark(LMIE_T_COEFS, 0);
-     if (nt == 0) {
-          // value channel: serial recurrences, parallel terms, per-size sums
+     {
+          // serial recurrences, parallel terms, per-size sums
           int n2max = 0, kfmax = 0;
           for (int i = 0; i < N; ++i) n2max = J->n2[i] > n2max ? J->n2[i] : n2max;
           for (int t = 0; t < nt64; ++t) kfmax = kfill[t] > kfmax ? kfill[t] : kfmax;
           const int n2rows = n2max + 1, ng = kfmax / 8;
           if (w->chD.get(sizeof(double) * 2 * (size_t) n2rows * Np) ||
               w->chPC.get(sizeof(double) * 2 * (size_t) (n1max + 1) * Np) || w->chPS.get(sizeof(double) * Np) ||
-              w->chPart.get(sizeof(double) * 5 * (size_t) (ng > 0 ? ng : 1) * Np))
+              w->chPart.get(sizeof(double) * (5 + 5 * hx + 8 * hm) * (size_t) (ng > 0 ? ng : 1) * Np) ||
+             (tan && (w->chDz.get(sizeof(double) * 2 * (size_t) n2rows * Np) || w->chPQ.get(sizeof(double) * 2 * Np))))
                return -1;
           ChainArgs ca;
           ca.N = N; ca.Np = Np; ca.n1max = n1max; ca.n2rows = n2rows;
           ca.x = w->x.as<double>(); ca.sx = w->sx.as<double>(); ca.cx = w->cx.as<double>();
           ca.n1 = w->n1.as<int>(); ca.n2 = w->n2.as<int>(); ca.mr = J->mr; ca.mi = J->mi;
           ca.d_all = keep; ca.D = w->chD.as<double>(); ca.PC = w->chPC.as<double>(); ca.PS = w->chPS.as<double>();
-          hipLaunchKernelGGL(mie_chains, dim3(Np / 64, 2), dim3(64), 0, s, ca);
+          ca.Dz = w->chDz.as<double>(); ca.PQ = w->chPQ.as<double>();
+          if (tan) hipLaunchKernelGGL(mie_chains<true>, dim3(Np / 64, 2), dim3(64), 0, s, ca);
+          else hipLaunchKernelGGL(mie_chains<false>, dim3(Np / 64, 2), dim3(64), 0, s, ca);
           if (side_tables()) return -1;
           if (w->ftab.get(sizeof(double) * FT_ROWS * (size_t) (n1max + 2))) return -1;
           hipLaunchKernelGGL(order_factors, dim3((n1max + 2 + 255) / 256), dim3(256), 0, s, n1max + 1,
                              w->ftab.as<double>());
+          if (tan) {
+               TanArgs ta;
+               ta.N = N; ta.Np = Np; ta.n1max = n1max; ta.n2rows = n2rows; ta.Kp = Kp; ta.ng = ng;
+               ta.ft = w->ftab.as<double>();
+               ta.x = w->x.as<double>(); ta.n1 = w->n1.as<int>(); ta.kfill = w->kfill.as<int>();
+               ta.mr = J->mr; ta.mi = J->mi; ta.D = w->chD.as<double>(); ta.Dz = w->chDz.as<double>();
+               ta.PC = w->chPC.as<double>(); ta.PS = w->chPS.as<double>(); ta.PQ = w->chPQ.as<double>();
+               for (int b = 0; b < nb; ++b) ta.A[b] = w->A.as<double>() + 4 * plane * b;
+               ta.part = w->chPart.as<double>();
+               const dim3 gt(Np / 64, ng), gs((Np + 31) / 32);
+#define LMIE_TAN(X, M)                                                                                           \
+               do {                                                                                              \
+                    if (ng > 0) hipLaunchKernelGGL((mie_tan_terms<X, M>), gt, dim3(64), 0, s, ta);               \
+                    hipLaunchKernelGGL((mie_tan_sums<X, M>), gs, dim3(256), 0, s, (const double *) w->chPart.as<double>(), N, Np, \
+                                       ng, (const int *) w->n1.as<int>(), w->S.as<double>());                    \
+               } while (0)
+               if (hx && hm) LMIE_TAN(true, true);
+               else if (hx) LMIE_TAN(true, false);
+               else LMIE_TAN(false, true);
+#undef LMIE_TAN
+          } else {
           TermArgs ta;
           ta.N = N; ta.Np = Np; ta.n1max = n1max; ta.n2rows = n2rows; ta.Kp = Kp; ta.Kb = Kb; ta.ng = ng;
           ta.ft = w->ftab.as<double>();
@@ -3936,33 +3753,10 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           }
           hipLaunchKernelGGL(mie_sums, dim3((Np + 31) / 32), dim3(256), 0, s, (const double *) w->chPart.as<double>(), N, Np,
                              ng, (const int *) w->n1.as<int>(), w->S.as<double>(), keep ? w->CB.as<double>() : nullptr);
+          }
           HIPCHECK(hipGetLastError());
           w->n2rows = n2rows;
           w->ng = ng;
-     }
-     if (nt > 0 && side_tables()) return -1;
-     for (int t0 = 0; nt > 0 && t0 < nt; t0 += 4) {
-          CoefArgs c;
-          memset(&c, 0, sizeof c);
-          c.N = N; c.Np = Np; c.n1max = n1max;
-          c.x = w->x.as<double>(); c.sx = w->sx.as<double>(); c.cx = w->cx.as<double>(); c.n1 = w->n1.as<int>(); c.n2 = w->n2.as<int>(); c.kfill = w->kfill.as<int>();
-          c.mr = J->mr; c.mi = J->mi;
-          int k = nt - t0 < 4 ? nt - t0 : 4;
-          if (k < 0) k = 0;
-          c.nt = k;
-          c.dx = w->dx.as<double>() + (size_t) t0 * Np;
-          c.dm = w->dm.as<double>() + 2 * t0;
-          c.scrD = w->scrD.as<double>();
-          c.scrR = w->scrR.as<double>();
-          c.A = w->A.as<double>();
-          c.Kp = Kp;
-          c.S = w->S.as<double>();
-          for (int q = 0; q < k; ++q) {
-               c.At[q] = w->A.as<double>() + 4 * plane * (1 + t0 + q);
-               c.St[q] = w->S.as<double>() + (size_t) 4 * Np * (1 + t0 + q);
-          }
-          c.write_base = t0 == 0;
-          if (launch_coefs(k, c, s)) return -1;
      }
      tm.mark(LMIE_T_COEFS, 1);
 
@@ -3984,38 +3778,10 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
      if (Q > 0) {
           if (w->pf.get(sizeof(double) * (size_t) nch * 4 * Q)) return -1;
           if (J->save_control == 1 && w->save2.get(sizeof(double) * (size_t) 4 * N * Q)) return -1;
-          // pass plan: pass 0 carries channel 0, up to 2 tangent and 3 weight
-          // channels; further passes carry the rest (recomputing the base sums)
-          struct Pass { int ntp, nwp, t0, w0, nblk; size_t off; };
-          std::vector<Pass> plan;
-          size_t tot = 0;
-          const int f64st = f64_staging();
-          for (int td = 0, wd = 0, ps = 0; ps == 0 || td < nt || wd < nw; ++ps) {
-               Pass P;
-               P.ntp = nt - td < 2 ? nt - td : 2;
-               const int base = ps == 0 ? 1 : 0;
-               const int ww = nw - wd < 4 - base ? nw - wd : 4 - base;
-               P.nwp = base + ww;
-               P.t0 = td;
-               P.w0 = wd;
-               const int tpb = f64_tiles_per_block(P.ntp, f64st);
-               P.nblk = ((Np / f64_tile(P.ntp, f64st)) + tpb - 1) / tpb;
-               P.off = tot;
-               tot += (size_t) P.nblk * (P.nwp + P.ntp) * 4 * Q;
-               plan.push_back(P);
-               td += P.ntp;
-               wd += ww;
-          }
-          if (mixed) {
-               plan.resize(1);
-               plan[0].ntp = 0;
-               plan[0].nwp = 1 + nw;
-               plan[0].t0 = plan[0].w0 = 0;
-               plan[0].nblk = Np / ms.tm;
-               plan[0].off = 0;
-               tot = (size_t) plan[0].nblk * plan[0].nwp * 4 * Q;
-          }
-          if (w->part.get(sizeof(double) * tot)) return -1;
+          const int ntile = Np / (mixed ? ms.tm : F64_TILE);
+          if (w->part.get(sizeof(double) * (size_t) ntile * nraw * 4 * Q) ||
+              (nt && w->pfraw.get(sizeof(double) * (size_t) nraw * 4 * Q)))
+               return -1;
           tm.mark(LMIE_T_ANGULAR, 0);
           if (mixed) {
                Mix2Args m;
@@ -4026,7 +3792,7 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
                m.ktile = ms.tm == 64 ? w->ktile64.as<int>() : w->ktile32.as<int>();
                m.task = w->order.as<int2>();
                m.W[0] = w->f.as<double>();
-               for (int q = 0; q < nw; ++q) m.W[1 + q] = w->dfw.as<double>() + (size_t) q * Np;
+               for (int q = 0; q < nw; ++q) m.W[1 + q] = w->wrow.as<double>() + (size_t) (1 + q) * Np;
                m.part = w->part.as<double>();
                const dim3 grid((unsigned) w->htask.size());
                // five split products (three with LMIE_MIX_PRODUCTS=3), in the
@@ -4054,51 +3820,29 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
 #undef LMIE_MIX
                HIPCHECK(hipGetLastError());
           }
-          for (size_t ps = 0; ps < plan.size() && !mixed; ++ps) {
-               Pass &P = plan[ps];
-               AngArgs a;
+          if (!mixed) {
+               F64Args a;
                memset(&a, 0, sizeof a);
                a.Np = Np; a.Kp = Kp; a.Hp = Hp; a.H = H; a.Q = Q; a.N = N;
-               a.A[0] = w->A.as<double>();
-               for (int q = 0; q < P.ntp; ++q) a.A[1 + q] = w->A.as<double>() + 4 * plane * (1 + P.t0 + q);
+               for (int b = 0; b < nb; ++b) a.A[b] = w->A.as<double>() + 4 * plane * b;
                a.Bp = w->Bp.as<double>(); a.Bm = w->Bm.as<double>();
-               a.f = w->f.as<double>();
-               int wi = 0;
-               if (ps == 0) a.W[wi++] = w->f.as<double>();
-               for (int q = 0; wi < P.nwp; ++q) a.W[wi++] = w->dfw.as<double>() + (size_t) (P.w0 + q) * Np;
-               for (int q = 0; q < P.ntp; ++q) a.WT[q] = w->dft.as<double>() + (size_t) (P.t0 + q) * Np;
-               a.part = w->part.as<double>() + P.off;
-               a.save2 = (ps == 0 && J->save_control == 1) ? w->save2.as<double>() : nullptr;
-               a.sst = (ps == 0 && keep) ? w->sst.as<double>() : nullptr;
-               int nblk = 0, rc;
-               if (P.ntp == 0 && f64_tile(0, f64st) == 32) {
-                    a.ktile = w->ktile32.as<int>();
-                    rc = launch_angular_nw<1, 1, 0>(P.nwp, a, Np / 32, f64st, s, &nblk);
-               } else if (P.ntp == 0) {
-                    a.ktile = w->ktile64.as<int>();
-                    rc = launch_angular_nw<2, 1, 0>(P.nwp, a, Np / 64, f64st, s, &nblk);
-               } else {
-                    a.ktile = w->ktile32.as<int>();
-                    rc = P.ntp == 1 ? launch_angular_nw<1, 1, 1>(P.nwp, a, Np / 32, f64st, s, &nblk)
-                                    : launch_angular_nw<1, 1, 2>(P.nwp, a, Np / 32, f64st, s, &nblk);
-               }
-               if (rc) return -1;
-               if (nblk != P.nblk) return set_err("internal: partial block count");
+               a.ktile = w->ktile32.as<int>();
+               a.task = w->order.as<int2>();
+               a.W = w->wrow.as<double>(); a.nP = nP; a.nX = nX;
+               a.part = w->part.as<double>();
+               a.save2 = J->save_control == 1 ? w->save2.as<double>() : nullptr;
+               a.sst = keep ? w->sst.as<double>() : nullptr;
+               if (launch_angular_f64(a, hx, hm, (unsigned) w->htask.size(), s)) return -1;
           }
           tm.mark(LMIE_T_ANGULAR, 1);
           tm.mark(LMIE_T_REDUCE, 0);
-          for (size_t ps = 0; ps < plan.size(); ++ps) {
-               const Pass &P = plan[ps];
-               ChMap map;
-               int c = 0;
-               if (ps == 0) map.g[c++] = 0;
-               for (int q = 0; c < P.nwp; ++q) map.g[c++] = 1 + nt + P.w0 + q;
-               for (int q = 0; q < P.ntp; ++q) map.g[c++] = 1 + P.t0 + q;
-               const int per = (P.nwp + P.ntp) * 4 * Q;
-               hipLaunchKernelGGL(reduce_parts, dim3((per + 31) / 32), dim3(256), 0, s,
-                                  (const double *) (w->part.as<double>() + P.off), P.nblk, P.nwp + P.ntp, Q, map,
+          const int per = nraw * 4 * Q;
+          hipLaunchKernelGGL(reduce_parts, dim3((per + 31) / 32), dim3(256), 0, s, (const double *) w->part.as<double>(),
+                             ntile, nraw, Q, nt ? w->pfraw.as<double>() : w->pf.as<double>());
+          if (nt)
+               hipLaunchKernelGGL(combine_channels, dim3((4 * Q + 255) / 256, nch), dim3(256), 0, s,
+                                  (const double *) w->pfraw.as<double>(), 4 * Q, (const ChComb *) w->comb.as<ChComb>(),
                                   w->pf.as<double>());
-          }
           HIPCHECK(hipGetLastError());
           tm.mark(LMIE_T_REDUCE, 1);
 
@@ -4130,7 +3874,7 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
      tm.mark(LMIE_T_TOTAL, 1);
      // results: through the pinned landing area (the expansions above, the sums here)
      const double *dots = (const double *) w->pres.p + (size_t) nch * 12 * C;
-     HIPCHECK(hipMemcpyAsync((void *) dots, w->dots.p, sizeof(double) * 4 * nch, hipMemcpyDeviceToHost, s));
+     HIPCHECK(hipMemcpyAsync((void *) dots, w->dots.p, sizeof(double) * 4 * nraw, hipMemcpyDeviceToHost, s));
      if (J->save_control == 1 && R->save1)
           for (int q = 0; q < 4; ++q)
                HIPCHECK(hipMemcpyAsync(R->save1 + (size_t) q * N, w->S.as<double>() + (size_t) q * Np,
@@ -4145,7 +3889,12 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           }
      for (int q = 0; q < 4; ++q) R->sums[q] = dots[q];
      for (int c = 1; c < nch; ++c)
-          for (int q = 0; q < 4; ++q) R->sums_ch[4 * (c - 1) + q] = dots[4 * c + q];
+          for (int q = 0; q < 4; ++q) {
+               double v = 0.;
+               for (int t = 0; t < 4; ++t)
+                    if (comb[c].r[t] >= 0) v += comb[c].c[t] * dots[4 * comb[c].r[t] + q];
+               R->sums_ch[4 * (c - 1) + q] = v;
+          }
      const int ids[] = {LMIE_T_TABLES, LMIE_T_COEFS, LMIE_T_ANGULAR, LMIE_T_REDUCE, LMIE_T_EXPAND, LMIE_T_TOTAL};
      tm.collect(ids, Q > 0 ? 6 : 2);
      lmie_gpu_host_time(LMIE_T_HOST_PREP, prep_ms);
@@ -4608,10 +4357,7 @@ int fused_launch(std::vector<FwdCase> &cs, Upload &up, Workspace *L) {
           m.part = w->part.as<double>();
           for (const int2 &t : c.task)
                task.push_back(make_int2(t.x, ((t.x < 0 ? 0 : t.y) & 0xffff) | (int) (k << 16)));
-          ChMap map;
-          memset(&map, 0, sizeof map);
-          map.g[0] = 0;
-          red[k] = reduce_parts_B{w->part.as<double>(), c.nmix, 1, c.Q, map, w->pf.as<double>(),
+          red[k] = reduce_parts_B{w->part.as<double>(), c.nmix, 1, c.Q, w->pf.as<double>(),
                                   (unsigned) (4 * c.Q + 31) / 32, 1};
           for (int gs = 0; gs < 2; ++gs) {
                const unsigned on = (gs ? c.J->calc_gc : c.J->calc_lc) ? 1u : 0u;

@@ -269,3 +269,44 @@ def test_reference_example_program_runs_unchanged(product, tmp_path):
             assert a.shape == e.shape, (b, key)
             scale = np.abs(e).max()
             assert np.all(np.abs(a - e) <= 6e-7 * np.abs(e) + 1e-9 * scale), (b, key)
+
+
+def direction_seeds(kind, rng):
+    """Seed columns: one input each, or 24 random mixtures of all of them
+    (more directions than the contraction's epilogue sums in one round)."""
+    one = lambda names: {k: [1.0 if i == j else 0.0 for j in range(len(names))] for i, k in enumerate(names)}
+    if kind == "x":
+        return one(["lambda", "r1", "r2"])
+    if kind == "m":
+        return one(["mr", "mi"])
+    if kind == "weights":
+        return one(["a1", "a2"])
+    return {k: list(rng.standard_normal(24) * (rng.random(24) < 0.6)) for k in
+            ("lambda", "mr", "mi", "a1", "a2", "r1", "r2")}
+
+
+@pytest.mark.parametrize("kind", ["x", "m", "weights", "mixtures"])
+@pytest.mark.parametrize("n_int2,n_quad,r2", [(1, 1, 0.4), (1, 33, 2.0), (5, 26, 4.0), (3, 97, 9.0)])
+def test_directions_against_the_oracle(product, oracle, kind, n_int2, n_quad, r2):
+    """Tangents of every kind of direction (x, m, weights only, mixtures of
+    all in 24 columns) on grids of 1, 33, 130 and 291 sizes, both expansions
+    and the per-size outputs, against the oracle's differentiated recurrences:
+    1e-12 normwise, the bar of the FP64 path."""
+    rng = np.random.Generator(np.random.PCG64(77))
+    p = dict(dist_type="log_normal", n_int2=n_int2, n_quad=n_quad, calc_gc=1, calc_lc=1, **{"lambda": 0.6}, mr=1.45,
+             mi=0.02, a1=0.3, a2=0.25, r1=0.02, r2=r2, accuracy=-1.0, save_control=1)
+    seeds = direction_seeds(kind, rng)
+    say("case: directions", kind, "sizes", n_int2 * n_quad, "r2", r2)
+    got = lmie.solve(product, p, seeds, "fp64")
+    ref = abi.solve(oracle, p, seeds, n_threads=4)
+    bad = []
+    for k in ("cext", "csca", "cbak", "g", "gc", "lc", "save1", "save2", "cext_l", "csca_l", "cbak_l", "g_l", "gc_l", "lc_l"):
+        a, b = np.asarray(got[k], float), np.asarray(ref[k], float)
+        e = relnorm(a, b)
+        if kind == "weights" and n_int2 * n_quad == 1 and k.endswith("_l"):
+            # the normalised density of one size does not depend on a1, a2:
+            # both sides hold the rounding of an exact zero
+            e = (np.linalg.norm(a) + np.linalg.norm(b)) / np.linalg.norm(np.asarray(ref[k[:-2]], float))
+        if not e <= 1e-12:
+            bad.append((k, e))
+    assert not bad, bad
