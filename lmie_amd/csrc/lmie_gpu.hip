@@ -1,12 +1,13 @@
 // lmie_gpu.hip -- gfx950 kernels of the size-integrated Mie path and the thin C
 // ABI of include/lmie_gpu.h.
 //
-// Forward call (main stream; angle tables on two side streams):
-//   gauss_nodes      Gauss-Legendre angles on [-1, 1]          (misc/rtutil_math.c:231-316)
-//   pitau_table16    split 16-bit pi_n +- tau_n at the positive angles (mixed path)
-//   pitau_table      FP64 pi_n +- tau_n (FP64 path)            (src/lmie_core.c:669-691)
-//   gsf_table        P^{00}, P^{02}, P^{22}, P^{2-2}, P_l       (misc/rtutil_math.c:867-1017)
-//   mie_chains       per size: D_n downward; ratio, psi_n, chi_n (src/lmie_core.c:298-405)
+// Forward call:
+//   front            one launch for what is serial in an order: Gauss-Legendre
+//                    angles (misc/rtutil_math.c:231-316), pi_n +- tau_n at the
+//                    positive angles, split 16-bit or FP64
+//                    (src/lmie_core.c:669-691), P^{00}, P^{02}, P^{22}, P^{2-2},
+//                    P_l (misc/rtutil_math.c:867-1017), and per size D_n
+//                    downward, psi_n, chi_n (src/lmie_core.c:298-405)
 //   mie_terms        per (size, 8 orders): a_n, b_n, contraction operand, series partials
 //                                                              (src/lmie_core.c:453-652)
 //   mie_sums         series per size                          (src/lmie_core.c:537-596)
@@ -217,7 +218,12 @@ __device__ __forceinline__ cd cdiv_nr(cd a, cd b) {
 }
 
 // ---------------------------------------------------------------------------
-// Gauss-Legendre angles: one thread per root.  Newton steps with the
+// The front of a call: everything that is serial in an order and independent of
+// the rest, one wave per role in one launch (kernel front, below): the angle
+// tables and the per-size chains take about the same time (both grow with the
+// largest order), so they share the launch and no stream waits for another.
+//
+// Gauss-Legendre angles: one lane per root.  Newton steps with the
 // second-order correction, stopped at a step <= DBL_EPSILON
 // (misc/rtutil_math.c:73-129); nodes ascending, weights
 // (1 - y^2) 2 / (n P_{n-1}(y'))^2 with y' the last-but-one iterate
@@ -226,235 +232,223 @@ __device__ __forceinline__ cd cdiv_nr(cd a, cd b) {
 // initial guesses come from the host (the C library's cos and tan, as the
 // reference) and every operation here is a separately rounded IEEE operation
 // (no contraction): the rule is the reference's rule bit for bit.
-// The factors j / (j + 1) of the Legendre recurrence come from LDS when the
-// degree fits (the same correctly rounded quotients, computed once per
-// workgroup), else they are divided in the loop.
-constexpr int GAUSS_LDS = 8192;
-
-template <bool TAB>
-__device__ __forceinline__ void gauss_newton(int n, const double *cj, double &y, double &pa, double &pb) {
-#pragma clang fp contract(off)
-     const double dn = (double) n, nn1 = (double) (n * (n + 1));
-     double y0;
-     int it = 0;
-     do {
-          double pm;
-          pa = 1.;
-          pb = 0.;
-#pragma unroll 4
-          for (int j = 0; j < n; ++j) {
-               pm = pb;
-               pb = pa;
-               const double u = __dmul_rn(y, pb);
-               const double c = TAB ? cj[j] : __ddiv_rn((double) j, __dadd_rn((double) j, 1.));
-               pa = __dadd_rn(__dmul_rn(c, __dsub_rn(u, pm)), u);
-          }
-          const double s = __dsub_rn(1., __dmul_rn(y, y));
-          const double d1 = __ddiv_rn(__dmul_rn(dn, __dsub_rn(pb, __dmul_rn(y, pa))), s);
-          const double d2 = __ddiv_rn(__dsub_rn(__dmul_rn(__dmul_rn(2., y), d1), __dmul_rn(nn1, pa)), s);
-          const double h = __ddiv_rn(pa, d1);
-          y0 = y;
-          y = __dsub_rn(y0, __dmul_rn(h, __dadd_rn(1., __ddiv_rn(__dmul_rn(h, d2), __dmul_rn(2., d1)))));
-     } while (fabs(__dsub_rn(y, y0)) > 2.220446049250313e-16 && ++it < 100);
-}
-
-__device__ __forceinline__ void gauss_nodes_body(int n, const double *guess, double *mu, double *w) {
-#pragma clang fp contract(off)
-     __shared__ double cj[GAUSS_LDS];
-     const bool tab = n <= GAUSS_LDS;
-     if (tab) {
-          for (int j = threadIdx.x; j < n; j += blockDim.x) cj[j] = __ddiv_rn((double) j, __dadd_rn((double) j, 1.));
-          __syncthreads();
-     }
-     int i = blockIdx.x * blockDim.x + threadIdx.x;
-     if (i >= (n + 1) / 2) return;
-     double y = guess[i], pa, pb;
-     if (tab) gauss_newton<true>(n, cj, y, pa, pb);
-     else gauss_newton<false>(n, nullptr, y, pa, pb);
-     const double dn = (double) n;
-     double c = __dmul_rn(dn, pb);
-     c = __ddiv_rn(2., __dmul_rn(c, c));
-     const double off = __dmul_rn(1., y);
-     mu[i] = __dsub_rn(0., off);
-     mu[n - 1 - i] = __dadd_rn(0., off);
-     w[i] = w[n - 1 - i] = __dmul_rn(__dsub_rn(1., __dmul_rn(off, y)), c);
-}
-__global__ void gauss_nodes(int n, const double *guess, double *mu, double *w) { gauss_nodes_body(n, guess, mu, w); }
-// Batched form of each kernel used by fused batches (name_b): one launch for
-// all cases, blockIdx.z picks the case, whose own grid (gx, gy blocks) may be
-// smaller than the launch grid; its surplus blocks exit.
-struct gauss_nodes_B {
-     int n;
-     const double *guess;
-     double *mu;
-     double *w;
-     unsigned gx, gy;
-};
-__global__ void gauss_nodes_b(const gauss_nodes_B *cases) {
-     const gauss_nodes_B a = cases[blockIdx.z];
-     if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     gauss_nodes_body(a.n, a.guess, a.mu, a.w);
-}
-
-
-// pi_n +- tau_n at the positive angles mu_{H+j}: one thread per angle, upward
-// recurrences pi_{n+1} = mu pi_n + (n+1)/n (mu pi_n - pi_{n-1}),
-// tau_n = n (mu pi_n - pi_{n-1}) - pi_{n-1} (src/lmie_core.c:669-691).
-__global__ void pitau_table(int H, int Hp, int n1max, int Kp, const double *mu, double *Bp, double *Bm) {
-     // separately rounded operations in the reference's order: the table is
-     // the reference's pi_n, tau_n bit for bit
-#pragma clang fp contract(off)
-     int j = blockIdx.x * blockDim.x + threadIdx.x;
-     if (j >= Hp) return;
-     if (j >= H) {
-          for (int n = 1; n <= Kp; ++n) Bp[(size_t) (n - 1) * Hp + j] = Bm[(size_t) (n - 1) * Hp + j] = 0.;
-          return;
-     }
-     double m = mu[H + j], p0 = 0., p1 = 1.;
-     for (int n = 1; n <= n1max; ++n) {
-          double a1 = m * p1, a2 = a1 - p0;
-          double tau = n * a2 - p0;
-          Bp[(size_t) (n - 1) * Hp + j] = p1 + tau;
-          Bm[(size_t) (n - 1) * Hp + j] = p1 - tau;
-          p0 = p1;
-          p1 = a1 + (n + 1.) / n * a2;
-     }
-     for (int n = n1max + 1; n <= Kp; ++n) Bp[(size_t) (n - 1) * Hp + j] = Bm[(size_t) (n - 1) * Hp + j] = 0.;
-}
-
-// Split 16-bit tables for the mixed path, blocked by 8 orders:
-// [6 planes: (pi+tau) hi, mid, lo, (pi-tau) hi, mid, lo][Kb][Hp][8], value
-// (pi_n +- tau_n) / (n (n+1)) * kSB.  A lane (angle) writes 16 bytes per plane
-// per group of 8 orders; consecutive lanes are consecutive 16-byte chunks.
-// The per-order factors (n+1)/n and kSB/(n(n+1)) come from LDS when n1max
-// fits, else they are divided in the loop.
-constexpr int PITAU_LDS = 4096;
-
-template <class E, bool TAB>
-__device__ __forceinline__ void pitau16_rows(int H, int Hp, int n1max, int Kb, const double *mu, const double *fq,
-                                             const double *fs, unsigned short *B16, int j) {
-     const size_t plane = (size_t) Kb * Hp * 8;
-     const double m = j < H ? mu[H + j] : 0.;
-     double p0 = 0., p1 = 1.;
-     for (int g = 0; g < Kb; ++g) {
-          unsigned short v[B16_PLANES][8];
-          for (int e = 0; e < 8; ++e) {
-               const int n = 8 * g + e + 1;
-               double bp = 0., bm = 0.;
-               if (j < H && n <= n1max) {
-                    const double a1 = m * p1, a2 = a1 - p0;
-                    const double tau = n * a2 - p0;
-                    const double sc = TAB ? fs[n] : kSB / (n * (n + 1.));
-                    bp = (p1 + tau) * sc;
-                    bm = (p1 - tau) * sc;
-                    p0 = p1;
-                    p1 = a1 + (TAB ? fq[n] : (n + 1.) / n) * a2;
-               }
-               split16x3<E>(bp, &v[0][e], &v[1][e], &v[2][e]);
-               split16x3<E>(bm, &v[3][e], &v[4][e], &v[5][e]);
-          }
-          for (int q = 0; q < B16_PLANES; ++q) {
-               v4u w;
-               for (int k = 0; k < 4; ++k) w[k] = (unsigned) v[q][2 * k] | ((unsigned) v[q][2 * k + 1] << 16);
-               *(v4u *) (B16 + q * plane + ((size_t) g * Hp + j) * 8) = w;
-          }
-     }
-}
-
-template <class E>
-__device__ __forceinline__ void pitau_table16_body(int H, int Hp, int n1max, int Kb, const double *mu, unsigned short *B16) {
-     __shared__ double fq[PITAU_LDS + 1], fs[PITAU_LDS + 1];
-     const bool tab = n1max <= PITAU_LDS;
-     if (tab) {
-          for (int n = threadIdx.x + 1; n <= n1max; n += blockDim.x) {
-               fq[n] = (n + 1.) / n;
-               fs[n] = kSB / (n * (n + 1.));
-          }
-          __syncthreads();
-     }
-     const int j = blockIdx.x * blockDim.x + threadIdx.x;
-     if (j >= Hp) return;
-     if (tab) pitau16_rows<E, true>(H, Hp, n1max, Kb, mu, fq, fs, B16, j);
-     else pitau16_rows<E, false>(H, Hp, n1max, Kb, mu, nullptr, nullptr, B16, j);
-}
-template <class E>
-__global__ void pitau_table16(int H, int Hp, int n1max, int Kb, const double *mu, unsigned short *B16) { pitau_table16_body<E>(H, Hp, n1max, Kb, mu, B16); }
-struct pitau_table16_B {
-     int H;
-     int Hp;
-     int n1max;
-     int Kb;
-     const double *mu;
-     unsigned short *B16;
-     unsigned gx, gy;
-};
-template <class E>
-__global__ void pitau_table16_b(const pitau_table16_B *cases) {
-     const pitau_table16_B a = cases[blockIdx.z];
-     if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     pitau_table16_body<E>(a.H, a.Hp, a.n1max, a.Kb, a.mu, a.B16);
-}
-
-
-// Value of lane `lane` (uniform) of a double: a scalar operand for the whole
-// wave.
+// Bound: the Legendre recurrence's chain of four dependent operations (about
+// 38 cycles) per order and Newton step.  Its factors j / (j + 1) are the same
+// in every lane: each lane divides for one order of the next 64 and the steps
+// read them from that lane, so every table wave can run the Newton steps of
+// its own 64 angles and none waits for another.
 __device__ __forceinline__ double readlane_d(double v, int lane) {
+     // value of lane `lane` (uniform) of a double: a scalar operand for the wave
      const unsigned long long u = (unsigned long long) __double_as_longlong(v);
      const unsigned lo = __builtin_amdgcn_readlane((unsigned) u, lane);
      const unsigned hi = __builtin_amdgcn_readlane((unsigned) (u >> 32), lane);
      return __longlong_as_double((long long) (((unsigned long long) hi << 32) | lo));
 }
 
+// y: initial guess in, last iterate out; pb: P_{n-1} at the last-but-one.  The
+// whole wave takes part; a lane that has stopped keeps its values.
+__device__ __forceinline__ void gauss_newton(int n, bool run, double &y, double &pb) {
+#pragma clang fp contract(off)
+     const double dn = (double) n, nn1 = (double) (n * (n + 1));
+     const int lane = threadIdx.x & 63;
+     int it = 0;
+     while (__ballot(run)) {
+          double pa = 1., pm = 0., pc = 0.;
+          auto step = [&](double c) {
+               pm = pc;
+               pc = pa;
+               const double u = y * pc;
+               pa = c * (u - pm) + u;
+          };
+          for (int j0 = 0; j0 < n; j0 += 64) {
+               const double j = j0 + lane, cl = j / (j + 1.);
+               if (n - j0 >= 64) {
+#pragma unroll 16
+                    for (int e = 0; e < 64; ++e) step(readlane_d(cl, e));
+               } else {
+                    for (int e = 0; e < n - j0; ++e) step(readlane_d(cl, e));
+               }
+          }
+          const double s = 1. - y * y;
+          const double d1 = dn * (pc - y * pa) / s;
+          const double d2 = (2. * y * d1 - nn1 * pa) / s;
+          const double h = pa / d1;
+          const double yn = y - h * (1. + h * d2 / (2. * d1));
+          if (run) {
+               run = fabs(yn - y) > 2.220446049250313e-16 && ++it < 100;
+               y = yn;
+               pb = pc;
+          }
+     }
+}
+
+// Roots of the rule of n angles from their guesses: mu[0 .. n), w[0 .. n).
+__device__ __forceinline__ void gauss_role(int n, const double *guess, double *mu, double *w, int block) {
+#pragma clang fp contract(off)
+     const int i = block * 64 + threadIdx.x, nr = (n + 1) / 2;
+     double y = guess[i < nr ? i : nr - 1], pb = 0.;
+     gauss_newton(n, i < nr, y, pb);
+     if (i >= nr) return;
+     double c = (double) n * pb;
+     c = 2. / (c * c);
+     const double off = 1. * y;
+     mu[i] = 0. - off;
+     mu[n - 1 - i] = 0. + off;
+     w[i] = w[n - 1 - i] = (1. - off * y) * c;
+}
+
+// Positive angle j < H of this lane (0 past H): its own Newton steps, or the
+// given angles mu[H + j] without guesses.
+__device__ __forceinline__ double angle_of(int Q, int H, const double *guess, const double *mu, int j) {
+#pragma clang fp contract(off)
+     if (!guess) return j < H ? mu[H + j] : 0.;
+     double y = guess[j < H ? H - 1 - j : 0], pb;
+     gauss_newton(Q, j < H, y, pb);
+     return j < H ? 0. + 1. * y : 0.;
+}
+
+// pi_n +- tau_n at the positive angles mu_{H+j}: one lane per angle, upward
+// recurrences pi_{n+1} = mu pi_n + (n+1)/n (mu pi_n - pi_{n-1}),
+// tau_n = n (mu pi_n - pi_{n-1}) - pi_{n-1} (src/lmie_core.c:669-691), in
+// separately rounded operations in the reference's order: the tables are
+// the reference's pi_n, tau_n bit for bit.  f(n, pi + tau, pi - tau) takes
+// orders 1 .. n1max; quotients (n+1)/n as in gauss_newton.
+template <class F>
+__device__ __forceinline__ void pitau_steps(int n1max, double m, F f) {
+#pragma clang fp contract(off)
+     const int lane = threadIdx.x & 63;
+     double p0 = 0., p1 = 1.;
+     for (int n0 = 1; n0 <= n1max; n0 += 64) {
+          const double nl = n0 + lane, ql = (nl + 1.) / nl;
+          auto step = [&](int e) {
+               const int n = n0 + e;
+               const double a1 = m * p1, a2 = a1 - p0;
+               const double tau = n * a2 - p0;
+               f(n, p1 + tau, p1 - tau);
+               p0 = p1;
+               p1 = a1 + readlane_d(ql, e) * a2;
+          };
+          if (n1max - n0 >= 63) {
+#pragma unroll 8
+               for (int e = 0; e < 64; ++e) step(e);
+          } else {
+               for (int e = 0; e <= n1max - n0; ++e) step(e);
+          }
+     }
+}
+
+// FP64 tables [Kp][Hp], zero rows past n1max and columns past H.
+__device__ __forceinline__ void pitau_role(int H, int Hp, int n1max, int Kp, double m, double *Bp, double *Bm, int j) {
+     const bool live = j < H;
+     pitau_steps(n1max, m, [&](int n, double bp, double bm) {
+          Bp[(size_t) (n - 1) * Hp + j] = live ? bp : 0.;
+          Bm[(size_t) (n - 1) * Hp + j] = live ? bm : 0.;
+     });
+     for (int n = n1max + 1; n <= Kp; ++n) Bp[(size_t) (n - 1) * Hp + j] = Bm[(size_t) (n - 1) * Hp + j] = 0.;
+}
+
+// Split 16-bit tables for the mixed path, blocked by 8 orders:
+// [6 planes: (pi+tau) hi, mid, lo, (pi-tau) hi, mid, lo][Kb][Hb][8], value
+// (pi_n +- tau_n) / (n (n+1)) * kSB.  A lane (angle) writes 16 bytes per plane
+// per group of 8 orders; consecutive lanes are consecutive 16-byte chunks.
+// The splits take eight times the recurrence's own operations, so PITAU_SHARE
+// waves run the recurrence of the same 64 angles and each splits and writes
+// every PITAU_SHARE-th group.
+constexpr int PITAU_SHARE = 8;
+
+template <class E>
+__device__ __forceinline__ void pitau16_role(int H, int Hb, int n1max, int Kb, double m, unsigned short *B16, int j, int share) {
+     const size_t plane = (size_t) Kb * Hb * 8;
+     const int lane = threadIdx.x & 63;
+     const bool live = j < H;
+     double p0 = 0., p1 = 1.;
+     double ql = 1., sl = 0.;
+     for (int g = 0; g < Kb; ++g) {
+          if ((g & 7) == 0) {          // factors of the next 64 orders, one per lane
+               const double n = 8 * g + 1 + lane;
+               ql = (n + 1.) / n;
+               sl = kSB / (n * (n + 1.));
+          }
+          const int e0 = 8 * (g & 7);
+          if ((g & (PITAU_SHARE - 1)) != share) {
+#pragma unroll
+               for (int e = 0; e < 8; ++e) {
+                    const double a1 = m * p1, a2 = a1 - p0;
+                    p0 = p1;
+                    p1 = a1 + readlane_d(ql, e0 + e) * a2;
+               }
+               continue;
+          }
+          unsigned short v[B16_PLANES][8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+               const int n = 8 * g + e + 1;
+               const double a1 = m * p1, a2 = a1 - p0;
+               const double tau = n * a2 - p0, sc = readlane_d(sl, e0 + e);
+               const bool on = live && n <= n1max;
+               split16x3<E>(on ? (p1 + tau) * sc : 0., &v[0][e], &v[1][e], &v[2][e]);
+               split16x3<E>(on ? (p1 - tau) * sc : 0., &v[3][e], &v[4][e], &v[5][e]);
+               p0 = p1;
+               p1 = a1 + readlane_d(ql, e0 + e) * a2;
+          }
+#pragma unroll
+          for (int q = 0; q < B16_PLANES; ++q) {
+               v4u w;
+#pragma unroll
+               for (int k = 0; k < 4; ++k) w[k] = (unsigned) v[q][2 * k] | ((unsigned) v[q][2 * k + 1] << 16);
+               *(v4u *) (B16 + q * plane + ((size_t) g * Hb + j) * 8) = w;
+          }
+     }
+}
+
 // Generalized spherical functions at the positive angles, l = 0 .. C-1, by
 // their three-term recurrences in l (misc/rtutil_math.c:956-1016).  Layout
 // [4][C][Hp] (+ plane 4: P_l for the Legendre expansion,
 // misc/rtutil_math.c:506-513): lanes (angles) store contiguously for every l.
-// The five recurrences are independent: blockIdx.y picks one (0: P00, 1: P02,
-// 2: P22, 3: P2-2, 4: P_l), so five times as many threads run one fifth of the
-// steps.  Columns H .. Hp-1 are written as zeros.
+// The five recurrences are independent, one wave each (FN 0: P00, 1: P02,
+// 2: P22, 3: P2-2, 4: P_l).  Columns H .. Hp-1 are written as zeros.
 // Each step divides the reference's numerator by its divisor d_l (L1, sqrt(L1^2
 // - 4) or L (L1^2 - 4)) in the reference's order of operations; the quotient
 // is q = RN(x y) corrected once, q + y RN(x - q d), with y = RN(1 / d_l):
 // Markstein's correction, which gives the correctly rounded x / d (the IEEE
 // division's bits) when y is the correctly rounded reciprocal and q is
-// within an ulp.  The divisors' reciprocals, the square roots and the
-// Legendre factors (l-1)/l of 64 consecutive l are formed one per lane (in
-// parallel) and each step reads its l's from that lane as scalars, so the
-// dependence chain of a step is the numerator and three operations instead
-// of a full division.
-// FN is the recurrence (a template argument, so a step has no branch on it).
+// within an ulp.  All that a step needs besides the angle (divisor,
+// reciprocal, square roots, polynomials in l) is formed for 64 l at a time, one
+// l per lane, and read back from LDS as broadcasts, ahead of the chain of five
+// dependent operations that bounds the step.
+constexpr int GSF_CST = 6, GSF_USED = 5;   // doubles per l: divisor, reciprocal, three factors
 template <int FN>
-__device__ __forceinline__ void gsf_plane(int H, int Hp, int C, const double *mu, double *P, int j, int lane) {
+__device__ __forceinline__ void gsf_role(int H, int Hp, int C, double m, double *P, int j, double *cst) {
      // separately rounded operations in the reference's order (bitwise the
      // reference's functions)
 #pragma clang fp contract(off)
-     // every lane stays in the loops (its l's are read by the others); the
-     // columns past H run with mu = 0 and store zeros
      const bool live = j < H;
-     const double m = live ? mu[H + j] : 0., m2 = m * m;
+     const int lane = threadIdx.x & 63;
+     const double m2 = m * m;
      double a0 = 0., b0 = 0.;
      for (int l0 = 0; l0 < C; l0 += 64) {
-          // this lane's order l0 + lane: divisor, its reciprocal, square root
-          // (FN 1), Legendre factor (FN 4)
-          double dv = 1., yv = 1., sav = 0.;
           {
                const int lc = l0 + lane;
-               const double L = lc - 1, L1 = lc;
+               const double L = lc - 1, L1 = lc, t = 2. * L + 1.;
+               double d = 1., a = 0., b = 0., c = 0.;
                if constexpr (FN == 4) {
-                    yv = lc >= 2 ? (lc - 1) / (double) lc : 0.;
+                    a = lc >= 2 ? (lc - 1) / (double) lc : 0.;
                } else if (lc >= 3) {
-                    if constexpr (FN == 0) dv = L1;
-                    else if constexpr (FN == 1) {
-                         sav = sqrt(L * L - 4.);
-                         dv = sqrt(L1 * L1 - 4.);
-                    } else dv = L * (L1 * L1 - 4);
-                    yv = 1. / dv;
+                    if constexpr (FN == 0) { d = L1; a = t; b = L; }
+                    else if constexpr (FN == 1) { d = sqrt(L1 * L1 - 4.); a = t; b = sqrt(L * L - 4.); }
+                    else { d = L * (L1 * L1 - 4); a = t * (L * L1); b = L1 * (L * L - 4); c = t * 4; }
                }
+               double *o = cst + GSF_CST * lane;
+               __syncthreads();
+               o[0] = d; o[1] = 1. / d; o[2] = a; o[3] = b; o[4] = c;
+               __syncthreads();
           }
           const int ne = min(64, C - l0);
-          double *row = P + (size_t) l0 * Hp + j;
+          // rows from a uniform pointer, the lane's byte offset a 32-bit register
+          char *row = (char *) (P + (size_t) l0 * Hp);
+          const unsigned oj = (unsigned) j * 8u;
           auto put = [&](int e, double v) {
-               row[(size_t) e * Hp] = live ? v : 0.;
+               *(double *) (row + (size_t) e * Hp * 8 + oj) = v;
                a0 = b0;
                b0 = v;
           };
@@ -464,74 +458,65 @@ __device__ __forceinline__ void gsf_plane(int H, int Hp, int C, const double *mu
           if (l0 == 0) {
                for (int l = 0; l < 3 && l < C; ++l) {
                     double v;
-                    if constexpr (FN == 4) v = l == 0 ? 1. : l == 1 ? m : readlane_d(yv, l) * (m * b0 - a0) + m * b0;
+                    if constexpr (FN == 4) v = l == 0 ? 1. : l == 1 ? m : cst[GSF_CST * l + 2] * (m * b0 - a0) + m * b0;
                     else if (l == 0) v = FN == 0 ? 1. : 0.;
                     else if (l == 1) v = FN == 0 ? m : 0.;
                     else if constexpr (FN == 0) v = (3. * m2 - 1.) / 2.;
                     else if constexpr (FN == 1) v = .25 * sqrt(6.) * (m2 - 1.);
                     else if constexpr (FN == 2) v = .25 * (1. + m) * (1. + m);
                     else v = .25 * (1. - m) * (1. - m);
-                    put(l, v);
+                    put(l, live ? v : 0.);       // the columns past H stay zero from here
                }
                e0 = 3;
           }
-          if constexpr (FN == 4) {
-               // P_l = a (m P_{l-1} - P_{l-2}) + m P_{l-1}, a = (l-1)/l
-               for (int e = e0; e < ne; ++e) {
-                    const double a = readlane_d(yv, e), bb = m * b0;
-                    put(e, a * (bb - a0) + bb);
-               }
-          } else {
-               for (int e = e0; e < ne; ++e) {
-                    const int l = l0 + e;
-                    const double L = l - 1, L1 = l, t = 2. * L + 1.;
-                    const double d = readlane_d(dv, e), y = readlane_d(yv, e);
+          struct Cst { double v[GSF_USED]; };
+          auto load = [&](int e) {
+               Cst s;
+#pragma unroll
+               for (int k = 0; k < GSF_USED; ++k) s.v[k] = cst[GSF_CST * e + k];
+               return s;
+          };
+          auto step = [&](int e, const Cst &s) {
+               if constexpr (FN == 4) {
+                    // P_l = a (m P_{l-1} - P_{l-2}) + m P_{l-1}, a = (l-1)/l
+                    const double bb = m * b0;
+                    put(e, s.v[2] * (bb - a0) + bb);
+               } else {
                     double x;
-                    if constexpr (FN == 0) {
-                         const double da = t * m;
-                         x = da * b0 - L * a0;
-                    } else if constexpr (FN == 1) {
-                         const double da = t * m;
-                         x = da * b0 - readlane_d(sav, e) * a0;
+                    if constexpr (FN < 2) {
+                         const double da = s.v[2] * m;
+                         x = da * b0 - s.v[3] * a0;
                     } else {
-                         const double k4 = t * 4, kb = L1 * (L * L - 4);
-                         const double dc = t * (L * L1) * m;
-                         x = FN == 2 ? (dc - k4) * b0 - kb * a0 : (dc + k4) * b0 - kb * a0;
+                         const double dc = s.v[2] * m;
+                         x = FN == 2 ? (dc - s.v[4]) * b0 - s.v[3] * a0 : (dc + s.v[4]) * b0 - s.v[3] * a0;
                     }
-                    const double q = x * y;
-                    put(e, __builtin_fma(__builtin_fma(-q, d, x), y, q));
+                    const double q = x * s.v[1];
+                    put(e, __builtin_fma(__builtin_fma(-q, s.v[0], x), s.v[1], q));
                }
+          };
+          int e = e0;
+          for (; e < ne && (e & 3); ++e) step(e, load(e));
+          // groups of four, the next group's factors read one group ahead
+          // (past the last one: the buffer's four spare entries)
+          Cst c0[4], c1[4];
+          auto read = [&](Cst *c, int o) {
+#pragma unroll
+               for (int k = 0; k < 4; ++k) c[k] = load(o + k);
+          };
+          auto four = [&](const Cst *c, int o) {
+#pragma unroll
+               for (int k = 0; k < 4; ++k) step(o + k, c[k]);
+          };
+          read(c0, e);
+          for (; e + 8 <= ne; e += 8) {
+               read(c1, e + 4);
+               four(c0, e);
+               read(c0, e + 8);
+               four(c1, e + 4);
           }
+          for (; e < ne; ++e) step(e, load(e));
      }
 }
-__device__ __forceinline__ void gsf_table_body(int H, int Hp, int C, const double *mu, double *T) {
-     const int j = blockIdx.x * blockDim.x + threadIdx.x, fn = blockIdx.y, lane = threadIdx.x & 63;
-     if (j >= Hp) return;
-     double *P = T + (size_t) fn * C * Hp;
-     switch (fn) {
-     case 0: gsf_plane<0>(H, Hp, C, mu, P, j, lane); break;
-     case 1: gsf_plane<1>(H, Hp, C, mu, P, j, lane); break;
-     case 2: gsf_plane<2>(H, Hp, C, mu, P, j, lane); break;
-     case 3: gsf_plane<3>(H, Hp, C, mu, P, j, lane); break;
-     default: gsf_plane<4>(H, Hp, C, mu, P, j, lane); break;
-     }
-}
-__global__ void gsf_table(int H, int Hp, int C, const double *mu, double *T) { gsf_table_body(H, Hp, C, mu, T); }
-struct gsf_table_B {
-     int H;
-     int Hp;
-     int C;
-     const double *mu;
-     double *T;
-     unsigned gx, gy;
-};
-__global__ void gsf_table_b(const gsf_table_B *cases) {
-     const gsf_table_B a = cases[blockIdx.z];
-     if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     gsf_table_body(a.H, a.Hp, a.C, a.mu, a.T);
-}
-
-
 // ---------------------------------------------------------------------------
 // Per-size Mie coefficients.
 //
@@ -575,9 +560,8 @@ __device__ __forceinline__ double rcp_s3(double q) {
 }
 
 // ---------------------------------------------------------------------------
-// Three kernels: mie_chains runs the three recurrences that
-// are serial in n, two threads per size in different waves (the D chain; the
-// ratio chain and then the psi, chi chain); mie_terms forms a_n, b_n, the
+// The front runs the three recurrences that are serial in n, two threads per
+// size in different waves (the D chain; the psi and chi chains); mie_terms forms a_n, b_n, the
 // contraction operand and the partial series sums in parallel, one thread
 // per (size, group of 8 orders); mie_sums adds the partial sums per size.  The
 // serial part is a few operations per order, the parallel part fills the GPU.
@@ -599,48 +583,53 @@ struct ChainArgs {
 // dD_j/dz = c' + (dD_{j+1}/dz + c') / w_j^2 with c' = -(j+1)/z^2, beside the
 // chain of w, which stays the longer dependence.
 template <bool TAN>
-__device__ __forceinline__ void mie_chains_body(ChainArgs p) {
+__device__ __forceinline__ void mie_chain_d(const ChainArgs &p, int i) {
 #pragma clang fp contract(off)
-     const int i = blockIdx.x * blockDim.x + threadIdx.x;
      if (i >= p.N) return;
      const size_t Np = p.Np;
      const double x = p.x[i];
      const int n1 = p.n1[i], n2 = p.n2[i], dtop = p.d_all ? n2 - 1 : n1;
      double2 *Dv = (double2 *) p.D;
-     if (blockIdx.y == 0) {
-          // downward D_j(z) = (j+1)/z - 1 / w_j, w_j = D_{j+1} + (j+1)/z,
-          // D_{n2} = 0.  The chain carries w: w_{j-1} = (2j+1)/z - 1 / w_j,
-          // w_{n2-1} = n2 / z, with 1 / w = conj(w) / |w|^2 (|w| stays between
-          // about 1/|z| and n2/|z|) and each update one fused multiply-add per
-          // component; D_j = (j+1)/z - 1 / w_j is formed beside the chain.  The
-          // recurrence damps its last-bit differences.
-          const cd z = cscale(cmk(p.mr, -p.mi), x), iz = crecip(z);
-          cd w = cscale(iz, (double) n2);
-          cd dz = cmk(0., 0.);
-          const cd iz2 = cmul(iz, iz);
-          for (int j = n2 - 1; j >= 1; --j) {
-               const cd c1 = cscale(iz, j + 1.), e = cscale(iz, 2. * j + 1.);
-               const double q = rcp_s3(__builtin_fma(w.r, w.r, w.i * w.i));
-               if constexpr (TAN) {
-                    const cd dc = cscale(iz2, -(j + 1.)), r = cmk(w.r * q, -w.i * q), r2 = cmul(r, r), t = cadd(dz, dc);
-                    dz = cmk(__builtin_fma(t.r, r2.r, __builtin_fma(-t.i, r2.i, dc.r)),
-                             __builtin_fma(t.r, r2.i, __builtin_fma(t.i, r2.r, dc.i)));
-                    if (j <= dtop) ((double2 *) p.Dz)[j * Np + i] = double2{dz.r, dz.i};
-               }
-               if (j <= dtop)
-                    Dv[j * Np + i] = double2{__builtin_fma(-w.r, q, c1.r), __builtin_fma(w.i, q, c1.i)};
-               w = cmk(__builtin_fma(-w.r, q, e.r), __builtin_fma(w.i, q, e.i));
+     // downward D_j(z) = (j+1)/z - 1 / w_j, w_j = D_{j+1} + (j+1)/z,
+     // D_{n2} = 0.  The chain carries w: w_{j-1} = (2j+1)/z - 1 / w_j,
+     // w_{n2-1} = n2 / z, with 1 / w = conj(w) / |w|^2 (|w| stays between
+     // about 1/|z| and n2/|z|) and each update one fused multiply-add per
+     // component; D_j = (j+1)/z - 1 / w_j is formed beside the chain.  The
+     // recurrence damps its last-bit differences.
+     const cd z = cscale(cmk(p.mr, -p.mi), x), iz = crecip(z);
+     cd w = cscale(iz, (double) n2);
+     cd dz = cmk(0., 0.);
+     const cd iz2 = cmul(iz, iz);
+     for (int j = n2 - 1; j >= 1; --j) {
+          const cd c1 = cscale(iz, j + 1.), e = cscale(iz, 2. * j + 1.);
+          const double q = rcp_s3(__builtin_fma(w.r, w.r, w.i * w.i));
+          if constexpr (TAN) {
+               const cd dc = cscale(iz2, -(j + 1.)), r = cmk(w.r * q, -w.i * q), r2 = cmul(r, r), t = cadd(dz, dc);
+               dz = cmk(__builtin_fma(t.r, r2.r, __builtin_fma(-t.i, r2.i, dc.r)),
+                        __builtin_fma(t.r, r2.i, __builtin_fma(t.i, r2.r, dc.i)));
+               if (j <= dtop) ((double2 *) p.Dz)[j * Np + i] = double2{dz.r, dz.i};
           }
-          return;
+          if (j <= dtop)
+               Dv[j * Np + i] = double2{__builtin_fma(-w.r, q, c1.r), __builtin_fma(w.i, q, c1.i)};
+          w = cmk(__builtin_fma(-w.r, q, e.r), __builtin_fma(w.i, q, e.i));
      }
-     // the other chains in another wave (blockIdx.y = 1), one loop: psi by
-     // Miller's downward recurrence, U_{n1} = 0, U_{n1-1} = 1,
-     // U_{j-1} = (2j+1)/x U_j - U_{j+1}, psi_j = s U_j with s = sin x / U_0 (the
-     // ratios r_j = U_j / U_{j-1} of the reference's ratio chain, whose
-     // product from psi_0 = sin x is the same psi_j), beside the upward
-     // chi_{j+1} = (2j+1)/x chi_j - chi_{j-1}; two independent dependence
-     // chains of two operations per order and no round trip through memory.
-     // U grows downward by at most the decay of psi_j between n1 - 1 and 0.
+}
+
+// The other chains, in another wave, one loop: psi by
+// Miller's downward recurrence, U_{n1} = 0, U_{n1-1} = 1,
+// U_{j-1} = (2j+1)/x U_j - U_{j+1}, psi_j = s U_j with s = sin x / U_0 (the
+// ratios r_j = U_j / U_{j-1} of the reference's ratio chain, whose
+// product from psi_0 = sin x is the same psi_j), beside the upward
+// chi_{j+1} = (2j+1)/x chi_j - chi_{j-1}; two independent dependence
+// chains of two operations per order and no round trip through memory.
+// U grows downward by at most the decay of psi_j between n1 - 1 and 0.
+template <bool TAN>
+__device__ __forceinline__ void mie_chain_psi(const ChainArgs &p, int i) {
+#pragma clang fp contract(off)
+     if (i >= p.N) return;
+     const size_t Np = p.Np;
+     const double x = p.x[i];
+     const int n1 = p.n1[i];
      const size_t ppl = (size_t) (p.n1max + 1) * Np;
      double *U = p.PC, *Chi = p.PC + ppl;
      const double ax = 1. / x, sx = p.sx[i], cx = p.cx[i];
@@ -671,19 +660,6 @@ __device__ __forceinline__ void mie_chains_body(ChainArgs p) {
           p.PQ[Np + i] = q;
      }
 }
-template <bool TAN>
-__global__ __launch_bounds__(64) void mie_chains(ChainArgs p) { mie_chains_body<TAN>(p); }
-struct mie_chains_B {
-     ChainArgs p;
-     unsigned gx, gy;
-};
-__global__ __launch_bounds__(64) void mie_chains_b(const mie_chains_B *cases) {
-     const mie_chains_B a = cases[blockIdx.z];
-     if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     mie_chains_body<false>(a.p);
-}
-
-
 // a_j, b_j (src/lmie_core.c:557-583)
 __device__ __forceinline__ void mie_ab_jx(double jx, cd m, cd im, cd Dj, double psi, double psi0, double chi1,
                                           double chi0, cd *a, cd *b) {
@@ -709,9 +685,8 @@ __device__ __forceinline__ void mie_ab_at(int j, double x, cd m, cd im, cd Dj, d
 // instead of dividing in every lane.
 constexpr int FT_FV4 = 0, FT_FV3M = 1, FT_FV4M = 2, FT_FV3 = 3, FT_ROWS = 4;
 
-__device__ __forceinline__ void order_factors_body(int n, double *ft) {
+__device__ __forceinline__ void order_factors(int n, double *ft, int j) {
 #pragma clang fp contract(off)
-     const int j = blockIdx.x * blockDim.x + threadIdx.x;
      if (j > n) return;
      const size_t ld = (size_t) n + 1;
      const double fv1 = 2. * j + 1.;
@@ -720,18 +695,85 @@ __device__ __forceinline__ void order_factors_body(int n, double *ft) {
      ft[FT_FV4M * ld + j] = j > 1 ? (2. * j - 1.) / ((j - 1.) * j) : 0.;
      ft[FT_FV3 * ld + j] = j > 0 ? (j + 2.) / ((j + 1.) / j) : 0.;
 }
-__global__ void order_factors(int n, double *ft) { order_factors_body(n, ft); }
-struct order_factors_B {
-     int n;
-     double *ft;
-     unsigned gx, gy;
+// One launch for the roles of the front: blocks of one wave, the longest
+// dependence chains first.  Measured at 3810 angles and 32768 sizes (each
+// role launched alone): the Gauss rule 0.26 ms (three Newton steps in its
+// slowest wave), with the expansion tables behind it 0.39 (the tables alone
+// 0.53 before their factors came from LDS), with the split pi/tau tables 0.33
+// (0.28 in one wave before, behind the rule), the chains 0.27 (0.34 with D kept to
+// n2); all of them 0.39-0.42, against five launches on three streams before.  Block ranges (ends): the expansion tables (planes
+// x angle blocks), the pi/tau tables (x PITAU_SHARE split), the Gauss rule, the
+// D chains, the psi and chi chains (heaviest sizes first), the order factors.
+// PK: pi/tau tables, 0 none, 1 FP64, 2 split fp16, 3 split bf16.
+struct FrontArgs {
+     int Q, H, Hp, C, n1max;
+     const double *guess;       // [(Q + 1) / 2] guesses of the roots, or NULL: angles given in mu
+     double *mu, *w;
+     double *T;                 // [planes][C][Hp]
+     int Kp, Kb, Hb;
+     double *Bp, *Bm;           // [Kp][Hp]
+     unsigned short *B16;
+     double *ft;                // order factors over 0 .. n1max + 1
+     ChainArgs ch;
+     unsigned e_gsf, e_pi, e_gauss, e_d, e_psi, e_ft;
+     void plan(int planes, int pk, bool gauss, int tiles, bool factors) {
+          e_gsf = (unsigned) (Hp / 64 * planes);
+          e_pi = e_gsf + (unsigned) (pk == 0 ? 0 : pk == 1 ? Hp / 64 : Hb / 64 * PITAU_SHARE);
+          e_gauss = e_pi + (unsigned) (gauss ? ((Q + 1) / 2 + 63) / 64 : 0);
+          e_d = e_gauss + (unsigned) tiles;
+          e_psi = e_d + (unsigned) tiles;
+          e_ft = e_psi + (unsigned) (factors ? (n1max + 2 + 63) / 64 : 0);
+     }
 };
-__global__ void order_factors_b(const order_factors_B *cases) {
-     const order_factors_B a = cases[blockIdx.z];
-     if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     order_factors_body(a.n, a.ft);
-}
 
+template <int PK, bool TAN>
+__device__ __forceinline__ void front_body(const FrontArgs &p, unsigned b) {
+     __shared__ __align__(16) double cst[68 * GSF_CST];
+     const int lane = threadIdx.x;
+     if (b < p.e_gsf) {
+          const int na = p.Hp / 64, fn = b / na, j = (b % na) * 64 + lane;
+          const double m = angle_of(p.Q, p.H, p.guess, p.mu, j);
+          double *P = p.T + (size_t) fn * p.C * p.Hp;
+          switch (fn) {
+          case 0: gsf_role<0>(p.H, p.Hp, p.C, m, P, j, cst); break;
+          case 1: gsf_role<1>(p.H, p.Hp, p.C, m, P, j, cst); break;
+          case 2: gsf_role<2>(p.H, p.Hp, p.C, m, P, j, cst); break;
+          case 3: gsf_role<3>(p.H, p.Hp, p.C, m, P, j, cst); break;
+          default: gsf_role<4>(p.H, p.Hp, p.C, m, P, j, cst); break;
+          }
+     } else if (b < p.e_pi) {
+          if constexpr (PK == 1) {
+               const int j = (b - p.e_gsf) * 64 + lane;
+               pitau_role(p.H, p.Hp, p.n1max, p.Kp, angle_of(p.Q, p.H, p.guess, p.mu, j), p.Bp, p.Bm, j);
+          } else if constexpr (PK > 1) {
+               const int e = b - p.e_gsf, j = e / PITAU_SHARE * 64 + lane;
+               typedef typename std::conditional<PK == 2, F16, BF16>::type E;
+               pitau16_role<E>(p.H, p.Hb, p.n1max, p.Kb, angle_of(p.Q, p.H, p.guess, p.mu, j), p.B16, j, e % PITAU_SHARE);
+          }
+     } else if (b < p.e_gauss) gauss_role(p.Q, p.guess, p.mu, p.w, b - p.e_pi);
+     else if (b < p.e_d) mie_chain_d<TAN>(p.ch, (int) (p.e_d - 1 - b) * 64 + lane);
+     else if (b < p.e_psi) mie_chain_psi<TAN>(p.ch, (int) (p.e_psi - 1 - b) * 64 + lane);
+     else if (b < p.e_ft) order_factors(p.n1max + 1, p.ft, (int) (b - p.e_psi) * 64 + lane);
+}
+template <int PK, bool TAN>
+__global__ __launch_bounds__(64) void front(FrontArgs p) { front_body<PK, TAN>(p, blockIdx.x); }
+// Batched form of each kernel used by fused batches (name_b): one launch for
+// all cases, blockIdx.z picks the case, whose own grid (gx, gy blocks) may be
+// smaller than the launch grid; its surplus blocks exit.
+template <int PK>
+__global__ __launch_bounds__(64) void front_b(const FrontArgs *cases) { front_body<PK, false>(cases[blockIdx.z], blockIdx.x); }
+
+int launch_front(const FrontArgs &p, int pk, bool tan, hipStream_t s) {
+     const dim3 g(p.e_ft);
+     if (p.e_ft == 0) return 0;
+     if (pk == 0) hipLaunchKernelGGL((front<0, false>), g, dim3(64), 0, s, p);
+     else if (pk == 2) hipLaunchKernelGGL((front<2, false>), g, dim3(64), 0, s, p);
+     else if (pk == 3) hipLaunchKernelGGL((front<3, false>), g, dim3(64), 0, s, p);
+     else if (tan) hipLaunchKernelGGL((front<1, true>), g, dim3(64), 0, s, p);
+     else hipLaunchKernelGGL((front<1, false>), g, dim3(64), 0, s, p);
+     HIPCHECK(hipGetLastError());
+     return 0;
+}
 
 struct TermArgs {
      int N, Np, n1max, n2rows, Kp, Kb, ng;
@@ -740,7 +782,7 @@ struct TermArgs {
      const int *n1;
      const int *kfill;          // [Np / TILE]
      double mr, mi;
-     const double *D, *PC, *PS; // from mie_chains: [n2rows][Np][2] D_j, [2][n1max + 1][Np] U_j and
+     const double *D, *PC, *PS; // from the chains: [n2rows][Np][2] D_j, [2][n1max + 1][Np] U_j and
                                 // chi_j, [Np] s (psi_j = s U_j)
      double *A;                 // FP64 planes [4][Kp][Np] (E = void)
      unsigned short *A16;       // split planes [8][Kb][Np][8] (E = F16 / BF16)
@@ -954,7 +996,7 @@ __global__ __launch_bounds__(256) void mie_sums_b(const mie_sums_B *cases) {
 // Forward tangents of the per-size coefficients.  a_n and b_n depend on the
 // inputs through the size parameter x and, analytically, through the complex
 // m, so the derivatives along x (HX) and along m (HM) give those of every
-// direction.  mie_chains<true> carries dD_j/dz along the D chain; everything
+// direction.  The D chain carries dD_j/dz; everything
 // else is closed per order from the kept D, U and chi:
 //   chi'_j = chi_{j-1} - (j/x) chi_j,
 //   psi'_j = psi_{j-1} - (j/x) psi_j + p psi_j + q chi_j,
@@ -971,7 +1013,7 @@ struct TanArgs {
      const double *x;
      const int *n1, *kfill;
      double mr, mi;
-     const double *D, *Dz, *PC, *PS, *PQ;   // from mie_chains: D_j and dD_j/dz [n2rows][Np][2], U and chi, s, [2][Np] p and q
+     const double *D, *Dz, *PC, *PS, *PQ;   // from the chains: D_j and dD_j/dz [n2rows][Np][2], U and chi, s, [2][Np] p and q
      double *A[3];              // operand planes [4][Kp][Np] of the value, then of d/dx, d/dm as present
      double *part;              // [rows][ng][Np]: the value's se, ss, cb (re, im), sg, then mie_tan_sums's rows
 };
@@ -2315,7 +2357,7 @@ struct RevArgs {
      const int *n1, *n2;
      double mr, mi;
      double im1r, im1i, im2r, im2i;   // 1/m, 1/m^2 (uniform, formed on the host)
-     const double *D, *PC, *PS; // forward recurrences (mie_chains, D up to n2 - 1)
+     const double *D, *PC, *PS; // forward recurrences (the chains, D up to n2 - 1)
      const double *CB;          // [2][Np]
      const double *S;           // series [4][Np]
      const double *bar;         // [4][Kp][Np] f-weighted cotangents (FP64 path), or
@@ -2974,9 +3016,8 @@ struct Download {
 struct Workspace {
      int device = -1;
      hipStream_t stream = nullptr;
-     hipStream_t side = nullptr;     // angle tables, concurrent with the per-size recurrences
-     hipStream_t side2 = nullptr;    // expansion tables, from the Gauss rule on
-     hipEvent_t fork = nullptr, join = nullptr, join2 = nullptr, sums = nullptr, nodes = nullptr, join3 = nullptr;
+     hipStream_t side = nullptr;     // the series sums, beside the contraction
+     hipEvent_t join2 = nullptr, sums = nullptr;
      hipEvent_t uploaded = nullptr;  // a batch case's inputs are on the device (its own stream)
      std::vector<double> hguess;     // host staging of the Gauss root guesses
      std::vector<int2> htask;        // host staging of the contraction task list
@@ -3025,13 +3066,8 @@ int ws_create(int device, Workspace **out) {
      w->device = device;
      HIPCHECK(hipStreamCreateWithFlags(&w->stream, hipStreamNonBlocking));
      HIPCHECK(hipStreamCreateWithFlags(&w->side, hipStreamNonBlocking));
-     HIPCHECK(hipStreamCreateWithFlags(&w->side2, hipStreamNonBlocking));
-     HIPCHECK(hipEventCreateWithFlags(&w->fork, hipEventDisableTiming));
-     HIPCHECK(hipEventCreateWithFlags(&w->join, hipEventDisableTiming));
      HIPCHECK(hipEventCreateWithFlags(&w->join2, hipEventDisableTiming));
      HIPCHECK(hipEventCreateWithFlags(&w->sums, hipEventDisableTiming));
-     HIPCHECK(hipEventCreateWithFlags(&w->nodes, hipEventDisableTiming));
-     HIPCHECK(hipEventCreateWithFlags(&w->join3, hipEventDisableTiming));
      HIPCHECK(hipEventCreateWithFlags(&w->uploaded, hipEventDisableTiming));
      for (auto &e : w->ev) HIPCHECK(hipEventCreate(&e));
      *out = w;
@@ -3628,57 +3664,6 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
      const double prep_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_entry).count();
      tm.mark(LMIE_T_TOTAL, 0);
 
-     // angle tables, on the side streams while the per-size recurrences run
-     // (side_tables, launched after the first per-size kernel)
-     hipStream_t ts = w->side;
-     HIPCHECK(hipEventRecord(w->fork, s));
-     HIPCHECK(hipStreamWaitEvent(ts, w->fork, 0));
-     tm.mark(LMIE_T_TABLES, 0, ts);
-     auto side_tables = [&]() -> int {
-     if (Q > 0) {
-          hipStream_t s = ts;
-          if (w->mu.get(sizeof(double) * Q) || w->w.get(sizeof(double) * Q) ||
-              (!mixed && (w->Bp.get(sizeof(double) * (size_t) Kp * Hp) || w->Bm.get(sizeof(double) * (size_t) Kp * Hp))))
-               return -1;
-          hipLaunchKernelGGL(gauss_nodes, dim3((H + 63) / 64), dim3(64), 0, s, Q, (const double *) w->guess.as<double>(),
-                             w->mu.as<double>(), w->w.as<double>());
-          // the expansion tables on a third stream from here: they run beside
-          // the per-size recurrences rather than beside the contraction
-          if (J->calc_gc || J->calc_lc) {
-               const int planes = J->calc_lc ? 5 : 4;
-               if (w->T.get(sizeof(double) * planes * (size_t) C * Hp)) return -1;
-               HIPCHECK(hipEventRecord(w->nodes, s));
-               HIPCHECK(hipStreamWaitEvent(w->side2, w->nodes, 0));
-               hipLaunchKernelGGL(gsf_table, dim3(Hp / 64, planes), dim3(64), 0, w->side2, H, Hp, C,
-                                  (const double *) w->mu.as<double>(), w->T.as<double>());
-          }
-          HIPCHECK(hipEventRecord(w->join3, w->side2));
-          if (mixed) {
-               if (w->B16.get(sizeof(unsigned short) * B16_PLANES * (size_t) Kb * Hb * 8)) return -1;
-               if (bf16)
-                    hipLaunchKernelGGL(pitau_table16<BF16>, dim3(Hb / 64), dim3(64), 0, s, H, Hb, n1max, Kb,
-                                       (const double *) w->mu.as<double>(), w->B16.as<unsigned short>());
-               else
-                    hipLaunchKernelGGL(pitau_table16<F16>, dim3(Hb / 64), dim3(64), 0, s, H, Hb, n1max, Kb,
-                                       (const double *) w->mu.as<double>(), w->B16.as<unsigned short>());
-               // the mixed contraction needs only the split tables; the FP64
-               // tables below serve the reverse pass, which runs after join2
-               HIPCHECK(hipEventRecord(w->join, s));
-          }
-          if (!mixed) {
-               hipLaunchKernelGGL(pitau_table, dim3(Hp / 64), dim3(64), 0, s, H, Hp, n1max, Kp, w->mu.as<double>(),
-                                  w->Bp.as<double>(), w->Bm.as<double>());
-          }
-          // the FP64 contraction needs the tables above; the expansion tables
-          // below only the expansion
-          if (!mixed) HIPCHECK(hipEventRecord(w->join, s));
-          HIPCHECK(hipGetLastError());
-     }
-     tm.mark(LMIE_T_TABLES, 1, ts);
-     if (Q <= 0) HIPCHECK(hipEventRecord(w->join, ts));
-     return 0;
-     };
-
      // per-size coefficients
      const size_t plane = (size_t) Kp * Np;
      if ((!mixed && w->A.get(sizeof(double) * 4 * plane * nb)) ||
@@ -3709,12 +3694,25 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           ca.n1 = w->n1.as<int>(); ca.n2 = w->n2.as<int>(); ca.mr = J->mr; ca.mi = J->mi;
           ca.d_all = keep; ca.D = w->chD.as<double>(); ca.PC = w->chPC.as<double>(); ca.PS = w->chPS.as<double>();
           ca.Dz = w->chDz.as<double>(); ca.PQ = w->chPQ.as<double>();
-          if (tan) hipLaunchKernelGGL(mie_chains<true>, dim3(Np / 64, 2), dim3(64), 0, s, ca);
-          else hipLaunchKernelGGL(mie_chains<false>, dim3(Np / 64, 2), dim3(64), 0, s, ca);
-          if (side_tables()) return -1;
-          if (w->ftab.get(sizeof(double) * FT_ROWS * (size_t) (n1max + 2))) return -1;
-          hipLaunchKernelGGL(order_factors, dim3((n1max + 2 + 255) / 256), dim3(256), 0, s, n1max + 1,
-                             w->ftab.as<double>());
+          // angle tables, chains and order factors
+          FrontArgs fa;
+          memset(&fa, 0, sizeof fa);
+          fa.Q = Q; fa.H = H; fa.Hp = Hp; fa.C = C; fa.n1max = n1max; fa.Kp = Kp; fa.Kb = Kb; fa.Hb = Hb;
+          const int planes = Q <= 0 ? 0 : J->calc_lc ? 5 : J->calc_gc ? 4 : 0;
+          const int pk = Q <= 0 ? 1 : !mixed ? 1 : bf16 ? 3 : 2;
+          if (w->ftab.get(sizeof(double) * FT_ROWS * (size_t) (n1max + 2)) ||
+              (Q > 0 && (w->mu.get(sizeof(double) * Q) || w->w.get(sizeof(double) * Q))) ||
+              (planes && w->T.get(sizeof(double) * planes * (size_t) C * Hp)) ||
+              (Q > 0 && !mixed && (w->Bp.get(sizeof(double) * (size_t) Kp * Hp) || w->Bm.get(sizeof(double) * (size_t) Kp * Hp))) ||
+              (mixed && w->B16.get(sizeof(unsigned short) * B16_PLANES * (size_t) Kb * Hb * 8)))
+               return -1;
+          fa.guess = w->guess.as<double>(); fa.mu = w->mu.as<double>(); fa.w = w->w.as<double>();
+          fa.T = w->T.as<double>(); fa.Bp = w->Bp.as<double>(); fa.Bm = w->Bm.as<double>();
+          fa.B16 = w->B16.as<unsigned short>(); fa.ft = w->ftab.as<double>(); fa.ch = ca;
+          fa.plan(planes, Q > 0 ? pk : 0, Q > 0, Np / 64, true);
+          tm.mark(LMIE_T_TABLES, 0);
+          if (launch_front(fa, pk, tan, s)) return -1;
+          tm.mark(LMIE_T_TABLES, 1);
           if (tan) {
                TanArgs ta;
                ta.N = N; ta.Np = Np; ta.n1max = n1max; ta.n2rows = n2rows; ta.Kp = Kp; ta.ng = ng;
@@ -3762,8 +3760,9 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
 
      // series sums (jobs uploaded with the inputs)
      {
-          // on the side stream after the angle tables (beside the contraction);
+          // on the side stream (beside the contraction);
           // the main stream joins it (join2) before the expansion
+          hipStream_t ts = w->side;
           HIPCHECK(hipEventRecord(w->sums, s));
           HIPCHECK(hipStreamWaitEvent(ts, w->sums, 0));
           tm.mark(LMIE_T_REDUCE, 0);
@@ -3773,8 +3772,7 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           HIPCHECK(hipEventRecord(w->join2, ts));
      }
 
-     // angular contraction and reduction (after the angle tables)
-     HIPCHECK(hipStreamWaitEvent(s, w->join, 0));
+     // angular contraction and reduction
      if (Q > 0) {
           if (w->pf.get(sizeof(double) * (size_t) nch * 4 * Q)) return -1;
           if (J->save_control == 1 && w->save2.get(sizeof(double) * (size_t) 4 * N * Q)) return -1;
@@ -3846,9 +3844,7 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           HIPCHECK(hipGetLastError());
           tm.mark(LMIE_T_REDUCE, 1);
 
-          // expansion (after the expansion tables)
-          HIPCHECK(hipStreamWaitEvent(s, w->join2, 0));
-          HIPCHECK(hipStreamWaitEvent(s, w->join3, 0));
+          // expansion
           tm.mark(LMIE_T_EXPAND, 0);
           if (w->E.get(sizeof(double) * (size_t) nch * 12 * Hp) || w->coefs.get(sizeof(double) * (size_t) nch * 6 * C))
                return -1;
@@ -3870,7 +3866,6 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           tm.mark(LMIE_T_REDUCE, 1);
      }
      HIPCHECK(hipStreamWaitEvent(s, w->join2, 0));   // the series dots
-     HIPCHECK(hipStreamWaitEvent(s, w->join3, 0));   // the expansion tables
      tm.mark(LMIE_T_TOTAL, 1);
      // results: through the pinned landing area (the expansions above, the sums here)
      const double *dots = (const double *) w->pres.p + (size_t) nch * 12 * C;
@@ -3966,14 +3961,14 @@ int saved_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           w->hguess.resize(H > 0 ? H : 1);
           gauss_guesses(Q, w->hguess.data());
           HIPCHECK(hipMemcpyAsync(w->guess.p, w->hguess.data(), sizeof(double) * H, hipMemcpyHostToDevice, s));
-          hipLaunchKernelGGL(gauss_nodes, dim3((H + 63) / 64), dim3(64), 0, s, Q, (const double *) w->guess.as<double>(),
-                             w->mu.as<double>(), w->w.as<double>());
-          if (J->calc_gc || J->calc_lc) {
-               const int planes = J->calc_lc ? 5 : 4;
-               if (w->T.get(sizeof(double) * planes * (size_t) C * Hp)) return -1;
-               hipLaunchKernelGGL(gsf_table, dim3(Hp / 64, planes), dim3(64), 0, s, H, Hp, C,
-                                  (const double *) w->mu.as<double>(), w->T.as<double>());
-          }
+          FrontArgs fa;
+          memset(&fa, 0, sizeof fa);
+          const int planes = J->calc_lc ? 5 : J->calc_gc ? 4 : 0;
+          if (planes && w->T.get(sizeof(double) * planes * (size_t) C * Hp)) return -1;
+          fa.Q = Q; fa.H = H; fa.Hp = Hp; fa.C = C;
+          fa.guess = w->guess.as<double>(); fa.mu = w->mu.as<double>(); fa.w = w->w.as<double>(); fa.T = w->T.as<double>();
+          fa.plan(planes, 0, true, 0, false);
+          if (launch_front(fa, 0, false, s)) return -1;
      }
      const int per = 4 * (Q + 1);
      hipLaunchKernelGGL(saved_sums, dim3((per + 31) / 32, nch), dim3(256), 0, s, (const double *) W,
@@ -4306,14 +4301,10 @@ int fused_prepare(FwdCase &c, Upload &up) {
 // One launch per kernel over the prepared cases, on the streams of workspace L.
 template <class E>
 int fused_launch(std::vector<FwdCase> &cs, Upload &up, Workspace *L) {
-     hipStream_t s = L->stream, ts = L->side, t2 = L->side2;
+     hipStream_t s = L->stream;
      if (up.flush(L->bup, L->pup, s)) return -1;
      const unsigned n = (unsigned) cs.size();
-     std::vector<mie_chains_B> chains(n);
-     std::vector<gauss_nodes_B> gauss(n);
-     std::vector<gsf_table_B> gsf(n);
-     std::vector<pitau_table16_B> pitau(n);
-     std::vector<order_factors_B> fac(n);
+     std::vector<FrontArgs> fronts(n);
      std::vector<mie_terms_B> terms(n);
      std::vector<mie_sums_B> sums(n);
      std::vector<weighted_dots_B> dots(n);
@@ -4330,14 +4321,13 @@ int fused_launch(std::vector<FwdCase> &cs, Upload &up, Workspace *L) {
           ca.x = w->x.as<double>(); ca.sx = w->sx.as<double>(); ca.cx = w->cx.as<double>();
           ca.n1 = w->n1.as<int>(); ca.n2 = w->n2.as<int>(); ca.mr = c.J->mr; ca.mi = c.J->mi;
           ca.d_all = 1; ca.D = w->chD.as<double>(); ca.PC = w->chPC.as<double>(); ca.PS = w->chPS.as<double>();
-          chains[k] = mie_chains_B{ca, (unsigned) c.Np / 64, 2};
-          gauss[k] = gauss_nodes_B{c.Q, w->guess.as<double>(), w->mu.as<double>(), w->w.as<double>(),
-                                   (unsigned) (c.H + 63) / 64, 1};
-          gsf[k] = gsf_table_B{c.H, c.Hp, c.C, w->mu.as<double>(), w->T.as<double>(), (unsigned) c.Hp / 64,
-                               (unsigned) c.planes};
-          pitau[k] = pitau_table16_B{c.H, c.Hb, c.n1max, c.Kb, w->mu.as<double>(), w->B16.as<unsigned short>(),
-                                     (unsigned) c.Hb / 64, 1};
-          fac[k] = order_factors_B{c.n1max + 1, w->ftab.as<double>(), (unsigned) (c.n1max + 2 + 255) / 256, 1};
+          ca.Dz = ca.PQ = nullptr;
+          FrontArgs &fa = fronts[k];
+          memset(&fa, 0, sizeof fa);
+          fa.Q = c.Q; fa.H = c.H; fa.Hp = c.Hp; fa.C = c.C; fa.n1max = c.n1max; fa.Kp = c.Kp; fa.Kb = c.Kb; fa.Hb = c.Hb;
+          fa.guess = w->guess.as<double>(); fa.mu = w->mu.as<double>(); fa.w = w->w.as<double>();
+          fa.T = w->T.as<double>(); fa.B16 = w->B16.as<unsigned short>(); fa.ft = w->ftab.as<double>(); fa.ch = ca;
+          fa.plan(c.planes, 2, true, c.Np / 64, true);
           TermArgs ta;
           ta.N = c.N; ta.Np = c.Np; ta.n1max = c.n1max; ta.n2rows = c.n2rows; ta.Kp = c.Kp; ta.Kb = c.Kb; ta.ng = c.ng;
           ta.ft = w->ftab.as<double>(); ta.x = w->x.as<double>(); ta.n1 = w->n1.as<int>();
@@ -4370,31 +4360,15 @@ int fused_launch(std::vector<FwdCase> &cs, Upload &up, Workspace *L) {
           }
      }
      BatchBlob b;
-     const size_t o_chains = b.add(chains), o_gauss = b.add(gauss), o_gsf = b.add(gsf), o_pitau = b.add(pitau),
-                  o_fac = b.add(fac), o_terms = b.add(terms), o_sums = b.add(sums), o_dots = b.add(dots),
+     const size_t o_front = b.add(fronts), o_terms = b.add(terms), o_sums = b.add(sums), o_dots = b.add(dots),
                   o_mix = b.add(mix), o_task = b.add(task), o_red = b.add(red), o_rows0 = b.add(rows[0]),
                   o_rows1 = b.add(rows[1]), o_coefs0 = b.add(coefs[0]), o_coefs1 = b.add(coefs[1]);
      if (L->bargs.get(b.h.size())) return -1;
      unsigned char *d = L->bargs.as<unsigned char>();
      HIPCHECK(hipMemcpyAsync(d, b.h.data(), b.h.size(), hipMemcpyHostToDevice, s));
 #define LMIE_B(T, off) ((const T *) (d + (off)))
-     // main stream: per-size recurrences; side streams: the angle tables
-     HIPCHECK(hipEventRecord(L->fork, s));
-     HIPCHECK(hipStreamWaitEvent(ts, L->fork, 0));
-     hipLaunchKernelGGL(mie_chains_b, dim3(max_g(chains, &mie_chains_B::gx), 2, n), dim3(64), 0, s,
-                        LMIE_B(mie_chains_B, o_chains));
-     hipLaunchKernelGGL(gauss_nodes_b, dim3(max_g(gauss, &gauss_nodes_B::gx), 1, n), dim3(64), 0, ts,
-                        LMIE_B(gauss_nodes_B, o_gauss));
-     HIPCHECK(hipEventRecord(L->nodes, ts));
-     HIPCHECK(hipStreamWaitEvent(t2, L->nodes, 0));
-     hipLaunchKernelGGL(gsf_table_b, dim3(max_g(gsf, &gsf_table_B::gx), max_g(gsf, &gsf_table_B::gy), n), dim3(64), 0,
-                        t2, LMIE_B(gsf_table_B, o_gsf));
-     HIPCHECK(hipEventRecord(L->join3, t2));
-     hipLaunchKernelGGL(pitau_table16_b<E>, dim3(max_g(pitau, &pitau_table16_B::gx), 1, n), dim3(64), 0, ts,
-                        LMIE_B(pitau_table16_B, o_pitau));
-     HIPCHECK(hipEventRecord(L->join, ts));
-     hipLaunchKernelGGL(order_factors_b, dim3(max_g(fac, &order_factors_B::gx), 1, n), dim3(256), 0, s,
-                        LMIE_B(order_factors_B, o_fac));
+     hipLaunchKernelGGL((front_b<std::is_same<E, F16>::value ? 2 : 3>), dim3(max_g(fronts, &FrontArgs::e_ft), 1, n), dim3(64),
+                        0, s, LMIE_B(FrontArgs, o_front));
      const unsigned tgy = max_g(terms, &mie_terms_B::gy);
      if (tgy > 0)
           hipLaunchKernelGGL(mie_terms_b<E>, dim3(max_g(terms, &mie_terms_B::gx), tgy, n), dim3(64), 0, s,
@@ -4402,8 +4376,7 @@ int fused_launch(std::vector<FwdCase> &cs, Upload &up, Workspace *L) {
      hipLaunchKernelGGL(mie_sums_b, dim3(max_g(sums, &mie_sums_B::gx), 1, n), dim3(256), 0, s,
                         LMIE_B(mie_sums_B, o_sums));
      hipLaunchKernelGGL(weighted_dots_b, dim3(4, 1, n), dim3(256), 0, s, LMIE_B(weighted_dots_B, o_dots));
-     // contraction after the split tables, one task list for all cases
-     HIPCHECK(hipStreamWaitEvent(s, L->join, 0));
+     // contraction, one task list for all cases
      if (!task.empty())
      {
           const dim3 g((unsigned) task.size());
@@ -4417,8 +4390,7 @@ int fused_launch(std::vector<FwdCase> &cs, Upload &up, Workspace *L) {
      }
      hipLaunchKernelGGL(reduce_parts_b, dim3(max_g(red, &reduce_parts_B::gx), 1, n), dim3(256), 0, s,
                         LMIE_B(reduce_parts_B, o_red));
-     // expansion after the expansion tables: generalized spherical, then Legendre
-     HIPCHECK(hipStreamWaitEvent(s, L->join3, 0));
+     // expansion: generalized spherical, then Legendre
      for (int gs = 1; gs >= 0; --gs) {
           if (max_g(rows[gs], &expand_rows_B::gy) == 0) continue;
           hipLaunchKernelGGL(expand_rows_b, dim3(max_g(rows[gs], &expand_rows_B::gx), 1, n), dim3(64), 0, s,
@@ -5060,7 +5032,6 @@ int forward_one(const lmie_gpu_job *job, lmie_gpu_result *res) {
      int rc = job->save_control == 2 ? saved_impl(job, res, w) : forward_impl(job, res, w);
      if (rc) {
           (void) hipStreamSynchronize(w->side);
-          (void) hipStreamSynchronize(w->side2);
           (void) hipStreamSynchronize(w->stream);
      }
      if (rc == 0 && job->keep) {
@@ -5175,9 +5146,11 @@ int lmie_gpu_gauss_rule(int n, double *x, double *wt, int device) {
      double *d = nullptr;
      HIPCHECK(hipMalloc(&d, sizeof(double) * (g.size() + 2 * (size_t) n)));
      HIPCHECK(hipMemcpy(d, g.data(), sizeof(double) * g.size(), hipMemcpyHostToDevice));
-     hipLaunchKernelGGL(gauss_nodes, dim3(((n + 1) / 2 + 63) / 64), dim3(64), 0, 0, n, (const double *) d,
-                        d + g.size(), d + g.size() + n);
-     HIPCHECK(hipGetLastError());
+     FrontArgs fa;
+     memset(&fa, 0, sizeof fa);
+     fa.Q = n; fa.guess = d; fa.mu = d + g.size(); fa.w = d + g.size() + n;
+     fa.plan(0, 0, true, 0, false);
+     if (launch_front(fa, 0, false, nullptr)) return -1;
      HIPCHECK(hipMemcpy(x, d + g.size(), sizeof(double) * n, hipMemcpyDeviceToHost));
      HIPCHECK(hipMemcpy(wt, d + g.size() + n, sizeof(double) * n, hipMemcpyDeviceToHost));
      HIPCHECK(hipFree(d));
@@ -5188,14 +5161,17 @@ int lmie_gpu_gsf_table(int n_mu, const double *mu, int n_l, double *out, int dev
      if (n_mu < 1 || n_l < 1) return set_err("n_mu < 1 or n_l < 1");
      if (!mu || !out) return set_err("missing argument");
      HIPCHECK(hipSetDevice(device));
-     // gsf_table reads the angles at mu[H + j], j < H, and writes [5][n_l][Hp]
+     // the expansion tables' role reads the angles at mu[H + j], j < H, and writes [5][n_l][Hp]
      const int H = n_mu, Hp = rup(H, 64);
      const size_t tab = (size_t) 5 * n_l * Hp;
      double *d = nullptr;
      HIPCHECK(hipMalloc(&d, sizeof(double) * (2 * (size_t) H + tab)));
      HIPCHECK(hipMemcpy(d + H, mu, sizeof(double) * H, hipMemcpyHostToDevice));
-     hipLaunchKernelGGL(gsf_table, dim3(Hp / 64, 5), dim3(64), 0, 0, H, Hp, n_l, (const double *) d, d + 2 * H);
-     HIPCHECK(hipGetLastError());
+     FrontArgs fa;
+     memset(&fa, 0, sizeof fa);
+     fa.H = H; fa.Hp = Hp; fa.C = n_l; fa.mu = d; fa.T = d + 2 * H;
+     fa.plan(5, 0, false, 0, false);
+     if (launch_front(fa, 0, false, nullptr)) return -1;
      std::vector<double> t(tab);
      HIPCHECK(hipMemcpy(t.data(), d + 2 * H, sizeof(double) * tab, hipMemcpyDeviceToHost));
      HIPCHECK(hipFree(d));
@@ -5207,15 +5183,17 @@ int lmie_gpu_pitau_table(int n_mu, const double *mu, int n, double *bp, double *
      if (n_mu < 1 || n < 1) return set_err("n_mu < 1 or n < 1");
      if (!mu || !bp || !bm) return set_err("missing argument");
      HIPCHECK(hipSetDevice(device));
-     // pitau_table reads the angles at mu[H + j], j < H, and writes [n][Hp] twice
+     // the pi/tau tables' role reads the angles at mu[H + j], j < H, and writes [n][Hp] twice
      const int H = n_mu, Hp = rup(H, 64);
      const size_t tab = (size_t) n * Hp;
      double *d = nullptr;
      HIPCHECK(hipMalloc(&d, sizeof(double) * (2 * (size_t) H + 2 * tab)));
      HIPCHECK(hipMemcpy(d + H, mu, sizeof(double) * H, hipMemcpyHostToDevice));
-     hipLaunchKernelGGL(pitau_table, dim3(Hp / 64), dim3(64), 0, 0, H, Hp, n, n, (const double *) d, d + 2 * H,
-                        d + 2 * H + tab);
-     HIPCHECK(hipGetLastError());
+     FrontArgs fa;
+     memset(&fa, 0, sizeof fa);
+     fa.H = H; fa.Hp = Hp; fa.n1max = fa.Kp = n; fa.mu = d; fa.Bp = d + 2 * H; fa.Bm = d + 2 * H + tab;
+     fa.plan(0, 1, false, 0, false);
+     if (launch_front(fa, 1, false, nullptr)) return -1;
      std::vector<double> t(2 * tab);
      HIPCHECK(hipMemcpy(t.data(), d + 2 * H, sizeof(double) * 2 * tab, hipMemcpyDeviceToHost));
      HIPCHECK(hipFree(d));
