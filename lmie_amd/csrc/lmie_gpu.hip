@@ -15,7 +15,8 @@
 //   angular_mix      S sums on the 16-bit matrix cores (split operands), Stokes in
 //                    FP64, weighted sums per angle            (src/lmie_core.c:658-791)
 //   angular_f64      the same on the FP64 matrix cores
-//   reduce_parts     fixed-order sum of the per-tile partials (src/lmie_schedule.c:109-147)
+//   reduce_channels  fixed-order sums of the per-tile partials and of the series
+//                    (src/lmie_schedule.c:109-147)
 //   expand_*         generalized-spherical / Legendre expansion (misc/rtutil_scat_int.c:20-480)
 //   saved_sums       save_control 2: re-weighting of saved per-size arrays
 //                                                              (src/lmie_schedule.c:1087-1124)
@@ -1196,56 +1197,36 @@ __global__ __launch_bounds__(256) void mie_tan_sums(const double *part, int N, i
 }
 
 // ---------------------------------------------------------------------------
-// Weighted sums over sizes: out[k] = sum_i u_k[i] v_k[i] (+ sum_i u2_k[i] v2_k[i]),
+// Weighted sums over sizes: out[k] = sum_i u_k[i] v_k[i],
 // one workgroup per output, fixed-order tree reduction (deterministic).
 struct DotJob {
-     const double *u, *v, *u2, *v2;
+     const double *u, *v;
 };
 
-__device__ __forceinline__ void weighted_dots_body(const DotJob *jobs, int n, double *out) {
+__device__ __forceinline__ void weighted_dots_body(const DotJob *jobs, int n, double *out, int k) {
      __shared__ double red[256];
-     const DotJob jb = jobs[blockIdx.x];
+     const DotJob jb = jobs[k];
      double s = 0.;
      int i = threadIdx.x;
      // eight elements in flight, added in the order of the plain loop
      for (; i + 7 * 256 < n; i += 8 * 256) {
-          double a[8], b[8], a2[8], b2[8];
+          double a[8], b[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-               a[e] = jb.u ? jb.u[i + 256 * e] : 1.;
+               a[e] = jb.u[i + 256 * e];
                b[e] = jb.v[i + 256 * e];
-               a2[e] = jb.u2 ? jb.u2[i + 256 * e] : 0.;
-               b2[e] = jb.u2 ? jb.v2[i + 256 * e] : 0.;
           }
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-               s += jb.u ? a[e] * b[e] : b[e];
-               if (jb.u2) s += a2[e] * b2[e];
-          }
+          for (int e = 0; e < 8; ++e) s += a[e] * b[e];
      }
-     for (; i < n; i += 256) {
-          s += jb.u ? jb.u[i] * jb.v[i] : jb.v[i];
-          if (jb.u2) s += jb.u2[i] * jb.v2[i];
-     }
+     for (; i < n; i += 256) s += jb.u[i] * jb.v[i];
      red[threadIdx.x] = s;
      __syncthreads();
      for (int w = 128; w > 0; w >>= 1) {
           if ((int) threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
           __syncthreads();
      }
-     if (threadIdx.x == 0) out[blockIdx.x] = red[0];
-}
-__global__ __launch_bounds__(256) void weighted_dots(const DotJob *jobs, int n, double *out) { weighted_dots_body(jobs, n, out); }
-struct weighted_dots_B {
-     const DotJob *jobs;
-     int n;
-     double *out;
-     unsigned gx, gy;
-};
-__global__ __launch_bounds__(256) void weighted_dots_b(const weighted_dots_B *cases) {
-     const weighted_dots_B a = cases[blockIdx.z];
-     if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     weighted_dots_body(a.jobs, a.n, a.out);
+     if (threadIdx.x == 0) out[k] = red[0];
 }
 
 
@@ -2363,13 +2344,13 @@ struct RevArgs {
      const double *bar;         // [4][Kp][Np] f-weighted cotangents (FP64 path), or
      const float *Uf;           // [4][Kq][Np] U = Sbar / f (mixed path; fang from U)
      int Kq;
-     const double *fang;        // [Np] (FP64 path)
+     const double *fang;        // [Np] (FP64 path), or NULL
      double sb0, sb1, sb2, sb3; // cotangents of the raw sums
      double *scan;              // [nch][REV_ROWS][Np]: P, C0, Q, Z0 (re, im), m cotangent (re, im),
                                 // f quadratic form, local x cotangent
-     double *mbar;              // [2][Np]
-     double *fbar;              // [Np]
-     double *xbar;              // [Np] cotangent of x_i, or null (not formed)
+     double *mbar;              // [Np / 64][2] m cotangent (re, im) of 64 sizes
+     double *fbar;              // [N]
+     double *xbar;              // [N] cotangent of x_i, or null (not formed)
 };
 constexpr int REV_ROWS = 12;
 
@@ -2602,14 +2583,9 @@ __device__ __forceinline__ void rev_carry_body(RevArgs p) {
      const int i = blockIdx.x * blockDim.x + threadIdx.x;
      if (i >= p.Np) return;
      const size_t Np = p.Np;
-     if (i >= p.N) {
-          p.mbar[i] = p.mbar[Np + i] = 0.;
-          p.fbar[i] = 0.;
-          if (p.xbar) p.xbar[i] = 0.;
-          return;
-     }
+     const bool live = i < p.N;
      const double x = p.x[i];
-     const int nk = (p.n2[i] - 1 + RCH - 1) / RCH;
+     const int nk = live ? (p.n2[i] - 1 + RCH - 1) / RCH : 0;
      // chain the chunks upward from j = 1 with carry 0
      cd carry = cmk(0., 0.), zb = cmk(0., 0.), mb = cmk(0., 0.);
      double fq = 0., xq = 0.;
@@ -2625,12 +2601,21 @@ __device__ __forceinline__ void rev_carry_body(RevArgs p) {
      }
      mb = cadd(mb, cscale(zb, x));
      // z = m x with m = mr - i mi: the x cotangent of z is Re(conj(m) zbar)
-     if (p.xbar) p.xbar[i] = xq + p.mr * zb.r - p.mi * zb.i;
-     p.mbar[i] = mb.r;
-     p.mbar[Np + i] = mb.i;
+     if (live && p.xbar) p.xbar[i] = xq + p.mr * zb.r - p.mi * zb.i;
+     // the wave's 64 sizes added in a fixed order; the host adds the waves
+#pragma unroll
+     for (int o = 32; o > 0; o >>= 1) {
+          mb.r += __shfl_xor(mb.r, o);
+          mb.i += __shfl_xor(mb.i, o);
+     }
+     if (threadIdx.x == 0) {
+          p.mbar[2 * blockIdx.x] = mb.r;
+          p.mbar[2 * blockIdx.x + 1] = mb.i;
+     }
+     if (!live) return;
      // size-weight cotangent: angular part plus the series part
      const double fser = p.sb0 * p.S[i] + p.sb1 * p.S[Np + i] + p.sb2 * p.S[2 * Np + i] + p.sb3 * p.S[3 * Np + i];
-     p.fbar[i] = (p.Uf ? fq : p.fang[i]) + fser;
+     p.fbar[i] = (p.Uf ? fq : p.fang ? p.fang[i] : 0.) + fser;
 }
 __global__ __launch_bounds__(64) void rev_carry(RevArgs p) { rev_carry_body(p); }
 struct rev_carry_B {
@@ -2644,131 +2629,120 @@ __global__ __launch_bounds__(64) void rev_carry_b(const rev_carry_B *cases) {
 }
 
 
-// Sum of the per-tile partials per (channel, element, angle).
-// Eight lanes per output element, each summing every eighth block, then the
-// eight partials in a fixed order: deterministic, and eight times the
-// threads of a plain per-element loop.
-__device__ __forceinline__ void reduce_parts_body(const double *part, int nblk, int nchp, int Q, double *out) {
-     const int per = nchp * 4 * Q;
-     const int e = blockIdx.x * 32 + (threadIdx.x >> 3), l = threadIdx.x & 7;
-     double s = 0.;
-     if (e < per) {
-          int b = l;
-          for (; b + 56 < nblk; b += 64) {   // eight partials in flight, added in order
-               double t[8];
-#pragma unroll
-               for (int k = 0; k < 8; ++k) t[k] = part[(size_t) (b + 8 * k) * per + e];
-#pragma unroll
-               for (int k = 0; k < 8; ++k) s += t[k];
-          }
-          for (; b < nblk; b += 8) s += part[(size_t) b * per + e];
-     }
-     s += __shfl_xor(s, 1);
-     s += __shfl_xor(s, 2);
-     s += __shfl_xor(s, 4);
-     if (e >= per || l) return;
-     out[e] = s;
-}
-__global__ __launch_bounds__(256) void reduce_parts(const double *part, int nblk, int nchp, int Q, double *out) { reduce_parts_body(part, nblk, nchp, Q, out); }
-struct reduce_parts_B {
-     const double *part;
-     int nblk;
-     int nchp;
-     int Q;
-     double *out;
-     unsigned gx, gy;
+// Directions from the raw channels of the sums over sizes: direction o is
+// sum_t c_t raw[r_t] (r_t < 0: none).
+struct ChComb {
+     int r[4];
+     double c[4];
 };
-__global__ __launch_bounds__(256) void reduce_parts_b(const reduce_parts_B *cases) {
-     const reduce_parts_B a = cases[blockIdx.z];
-     if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     reduce_parts_body(a.part, a.nblk, a.nchp, a.Q, a.out);
+
+// Sum of the per-tile partials per (raw channel, element, angle) and the
+// directions formed from them; the last ndot blocks are the series sums of the
+// raw channels (weighted_dots), which wait for nothing here.  Eight lanes per
+// output element, each summing every eighth tile, then the eight partials in a
+// fixed order: deterministic, and eight times the threads of a plain
+// per-element loop.
+struct ReduceArgs {
+     const double *part;        // [nblk][nraw][4 Q]
+     int nblk, nraw, Q, nch;
+     const ChComb *comb;        // [nch], or NULL: channels as they are
+     double *out;               // [nch][4 Q]
+     const DotJob *jobs;
+     int n, ndot;
+     double *dots;
+     unsigned gx;
+};
+__device__ __forceinline__ void reduce_channels_body(const ReduceArgs &p, unsigned block) {
+     const int per = 4 * p.Q, all = p.nraw * per;
+     const unsigned nred = (unsigned) ((p.nch * per + 31) / 32);
+     if (block >= nred) {
+          if (block < p.gx) weighted_dots_body(p.jobs, p.n, p.dots, (int) (block - nred));
+          return;
+     }
+     const int e = block * 32 + (threadIdx.x >> 3), l = threadIdx.x & 7;
+     const bool live = e < p.nch * per;
+     const int o = live ? e / per : 0, rem = e - o * per;
+     double out = 0.;
+     const int nt = p.comb ? 4 : 1;
+     for (int t = 0; t < nt; ++t) {
+          const int r = !live ? -1 : p.comb ? p.comb[o].r[t] : o;
+          double s = 0.;
+          if (r >= 0) {
+               const double *q = p.part + (size_t) r * per + rem;
+               int b = l;
+               for (; b + 56 < p.nblk; b += 64) {   // eight partials in flight, added in order
+                    double v[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) v[k] = q[(size_t) (b + 8 * k) * all];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) s += v[k];
+               }
+               for (; b < p.nblk; b += 8) s += q[(size_t) b * all];
+          }
+          s += __shfl_xor(s, 1);
+          s += __shfl_xor(s, 2);
+          s += __shfl_xor(s, 4);
+          if (r >= 0) out += p.comb ? p.comb[o].c[t] * s : s;
+     }
+     if (live && l == 0) p.out[e] = out;
 }
+__global__ __launch_bounds__(256) void reduce_channels(ReduceArgs p) { reduce_channels_body(p, blockIdx.x); }
+__global__ __launch_bounds__(256) void reduce_channels_b(const ReduceArgs *cases) { reduce_channels_body(cases[blockIdx.z], blockIdx.x); }
 
 
 // ---------------------------------------------------------------------------
 // Expansion.  For channel c the quadrature-weighted element rows at the
 // mirrored (-) and direct (+) angles of every positive node j:
-//   GSF rows  0..5: F11, F11+F33, F11-F33, F33, F12, F34 at -mu_j
-//            6..11: the same at +mu_j            (misc/rtutil_scat_int.c:173-183)
-//   Legendre 0..5: F11, F11, F33, F33, F12, F34 at -mu_j, 6..11 at +mu_j.
-__device__ __forceinline__ void expand_rows_body(const double *pf, int nch, int Q, int H, int Hp, const double *w, int gsf, double *E) {
-     const int j = blockIdx.x * blockDim.x + threadIdx.x;
-     const int c = blockIdx.y;
-     if (j >= Hp || c >= nch) return;
-     double *Ec = E + (size_t) c * 12 * Hp;
-     if (j >= H) {
-          for (int r = 0; r < 12; ++r) Ec[r * Hp + j] = 0.;
-          return;
-     }
-     const double *P = pf + (size_t) c * 4 * Q;
-     const int ip = H + j, im = H - 1 - j;
-     const double wq = w[ip];
-     for (int s = 0; s < 2; ++s) {
-          const int a = s ? ip : im;
-          const double f11 = P[a] * wq, f33 = P[Q + a] * wq, f12 = P[2 * Q + a] * wq, f34 = P[3 * Q + a] * wq;
-          double *row = Ec + (size_t) 6 * s * Hp;
-          if (gsf) {
-               row[0 * Hp + j] = f11;
-               row[1 * Hp + j] = f11 + f33;
-               row[2 * Hp + j] = f11 - f33;
-               row[3 * Hp + j] = f33;
-          } else {
-               row[0 * Hp + j] = f11;
-               row[1 * Hp + j] = f11;
-               row[2 * Hp + j] = f33;
-               row[3 * Hp + j] = f33;
-          }
-          row[4 * Hp + j] = f12;
-          row[5 * Hp + j] = f34;
-     }
-}
-__global__ void expand_rows(const double *pf, int nch, int Q, int H, int Hp, const double *w, int gsf, double *E) { expand_rows_body(pf, nch, Q, H, Hp, w, gsf, E); }
-struct expand_rows_B {
-     const double *pf;
-     int nch;
-     int Q;
-     int H;
-     int Hp;
-     const double *w;
-     int gsf;
-     double *E;
-     unsigned gx, gy;
-};
-__global__ void expand_rows_b(const expand_rows_B *cases) {
-     const expand_rows_B a = cases[blockIdx.z];
-     if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     expand_rows_body(a.pf, a.nch, a.Q, a.H, a.Hp, a.w, a.gsf, a.E);
-}
-
-
+//   GSF      F11, F11+F33, F11-F33, F33, F12, F34   (misc/rtutil_scat_int.c:173-183)
+//   Legendre F11, F11, F33, F33, F12, F34.
 // One wave per (l, channel): twelve dot products over the positive nodes,
 // folded with (-1)^l for the mirrored half, then the alpha/zeta recombination
-// and the (2l+1)/2 factor (misc/rtutil_scat_int.c:185-213, :436-469).
-__device__ __forceinline__ void expand_coefs_body(const double *T, const double *E, int H, int Hp, int C, int gsf, double *coefs) {
-     const int lane = threadIdx.x & 63;
+// and the (2l+1)/2 factor (misc/rtutil_scat_int.c:185-213, :436-469).  The
+// rows are formed from the elements as they are read (a launch of their own and
+// a third more reads otherwise).
+__device__ __forceinline__ void expand_coefs_body(const double *T, const double *pf, const double *w, int Q, int Hp, int C, int gsf,
+                                                  double *coefs) {
+     const int lane = threadIdx.x & 63, H = Q / 2;
      const int l = blockIdx.x * 4 + (threadIdx.x >> 6);
      const int c = blockIdx.y;
      if (l >= C) return;
      const size_t plane = (size_t) C * Hp;
      const double *P00 = T + (gsf ? 0 : 4 * plane) + (size_t) l * Hp, *P02 = T + plane + (size_t) l * Hp;
      const double *P22 = T + 2 * plane + (size_t) l * Hp, *P2m = T + 3 * plane + (size_t) l * Hp;
-     const double *Ec = E + (size_t) c * 12 * Hp;
+     const double *P = pf + (size_t) c * 4 * Q;
      double d[12];
 #pragma unroll
      for (int r = 0; r < 12; ++r) d[r] = 0.;
      for (int j = lane; j < H; j += 64) {
-          const double p00 = P00[j];
+          const double p00 = P00[j], wq = w[H + j];
+          double e[2][4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+               e[0][k] = P[(size_t) k * Q + H - 1 - j] * wq;
+               e[1][k] = P[(size_t) k * Q + H + j] * wq;
+          }
           if (gsf) {
                const double p02 = P02[j], p22 = P22[j], p2m = P2m[j];
-               d[0] += p00 * Ec[0 * Hp + j];  d[6] += p00 * Ec[6 * Hp + j];
-               d[1] += p2m * Ec[1 * Hp + j];  d[7] += p22 * Ec[7 * Hp + j];
-               d[2] += p22 * Ec[2 * Hp + j];  d[8] += p2m * Ec[8 * Hp + j];
-               d[3] += p00 * Ec[3 * Hp + j];  d[9] += p00 * Ec[9 * Hp + j];
-               d[4] += p02 * Ec[4 * Hp + j];  d[10] += p02 * Ec[10 * Hp + j];
-               d[5] += p02 * Ec[5 * Hp + j];  d[11] += p02 * Ec[11 * Hp + j];
+#pragma unroll
+               for (int s = 0; s < 2; ++s) {
+                    const double f11 = e[s][0], f33 = e[s][1], sum = f11 + f33, dif = f11 - f33;
+                    d[6 * s + 0] += p00 * f11;
+                    d[6 * s + 1] += (s ? p22 : p2m) * sum;
+                    d[6 * s + 2] += (s ? p2m : p22) * dif;
+                    d[6 * s + 3] += p00 * f33;
+                    d[6 * s + 4] += p02 * e[s][2];
+                    d[6 * s + 5] += p02 * e[s][3];
+               }
           } else {
 #pragma unroll
-               for (int r = 0; r < 12; ++r) d[r] += p00 * Ec[r * Hp + j];
+               for (int s = 0; s < 2; ++s) {
+                    d[6 * s + 0] += p00 * e[s][0];
+                    d[6 * s + 1] += p00 * e[s][0];
+                    d[6 * s + 2] += p00 * e[s][1];
+                    d[6 * s + 3] += p00 * e[s][1];
+                    d[6 * s + 4] += p00 * e[s][2];
+                    d[6 * s + 5] += p00 * e[s][3];
+               }
           }
      }
 #pragma unroll
@@ -2795,21 +2769,17 @@ __device__ __forceinline__ void expand_coefs_body(const double *T, const double 
           for (int k = 0; k < 6; ++k) out[(size_t) k * C + l] = e[k] * fl;
      }
 }
-__global__ __launch_bounds__(256) void expand_coefs(const double *T, const double *E, int H, int Hp, int C, int gsf, double *coefs) { expand_coefs_body(T, E, H, Hp, C, gsf, coefs); }
+__global__ __launch_bounds__(256) void expand_coefs(const double *T, const double *pf, const double *w, int Q, int Hp, int C, int gsf, double *coefs) { expand_coefs_body(T, pf, w, Q, Hp, C, gsf, coefs); }
 struct expand_coefs_B {
-     const double *T;
-     const double *E;
-     int H;
-     int Hp;
-     int C;
-     int gsf;
+     const double *T, *pf, *w;
+     int Q, Hp, C, gsf;
      double *coefs;
      unsigned gx, gy;
 };
 __global__ __launch_bounds__(256) void expand_coefs_b(const expand_coefs_B *cases) {
      const expand_coefs_B a = cases[blockIdx.z];
      if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     expand_coefs_body(a.T, a.E, a.H, a.Hp, a.C, a.gsf, a.coefs);
+     expand_coefs_body(a.T, a.pf, a.w, a.Q, a.Hp, a.C, a.gsf, a.coefs);
 }
 
 
@@ -2914,7 +2884,8 @@ struct PinBuf {      // pinned host memory, grown on demand
      }
 };
 
-// Many small copies as one: each job moves n doubles (src NULL: writes zeros).
+// Many small copies as one: each job moves n doubles.  A fused batch sends its
+// results with it from the device straight into each case's pinned landing area.
 struct CopyJob {
      const double *src;
      double *dst;
@@ -2923,130 +2894,44 @@ struct CopyJob {
 __global__ __launch_bounds__(256) void copy_jobs(const CopyJob *jobs) {
      const CopyJob j = jobs[blockIdx.y];
      for (size_t e = (size_t) blockIdx.x * 256 + threadIdx.x; e < j.n; e += (size_t) gridDim.x * 256)
-          j.dst[e] = j.src ? j.src[e] : 0.;
+          j.dst[e] = j.src[e];
 }
 
-// Uploads of a batch gathered into one host-to-device copy and one copy_jobs
-// launch.  Sizes are whole doubles.
-struct Upload {
-     struct Item { size_t off; void *dst; size_t n8; bool zero; };
-     std::vector<unsigned char> h;
-     std::vector<Item> items;
-     int add(void *dst, const void *src, size_t bytes) {
-          if (bytes % 8) return set_err("internal: upload of %zu bytes", bytes);
-          const size_t off = h.size();
-          h.resize(off + bytes);
-          memcpy(h.data() + off, src, bytes);
-          items.push_back(Item{off, dst, bytes / 8, false});
-          return 0;
-     }
-     int zero(void *dst, size_t bytes) {
-          if (bytes % 8) return set_err("internal: fill of %zu bytes", bytes);
-          items.push_back(Item{0, dst, bytes / 8, true});
-          return 0;
-     }
-     // drops what was queued after the given sizes (a case that failed)
-     void rewind(size_t n_items, size_t n_bytes) {
-          items.resize(n_items);
-          h.resize(n_bytes);
-     }
-     int flush(Buf &dev, PinBuf &pin, hipStream_t s) { return flush_all({this}, dev, pin, s); }
-     // the staged uploads of several callers as one copy and one copy_jobs
-     // launch, each one's bytes going straight into the pinned buffer (which
-     // must not be refilled before the copy has run)
-     static int flush_all(const std::vector<const Upload *> &ups, Buf &dev, PinBuf &pin, hipStream_t s) {
-          size_t bytes = 0, n = 0;
-          for (const Upload *u : ups) {
-               bytes += u->h.size();
-               n += u->items.size();
-          }
-          if (n == 0) return 0;
-          if (n > 65535) return set_err("batch of %zu uploads (at most 65535)", n);
-          const size_t data = (bytes + 255) & ~(size_t) 255, total = data + sizeof(CopyJob) * n;
-          if (dev.get(total) || pin.get(total)) return -1;
-          unsigned char *base = dev.as<unsigned char>(), *hp = (unsigned char *) pin.p;
-          CopyJob *jobs = (CopyJob *) (hp + data);
-          size_t off = 0, k = 0;
-          for (const Upload *u : ups) {
-               memcpy(hp + off, u->h.data(), u->h.size());
-               for (const Item &it : u->items)
-                    jobs[k++] = CopyJob{it.zero ? nullptr : (const double *) (base + off + it.off), (double *) it.dst,
-                                        it.n8};
-               off += u->h.size();
-          }
-          HIPCHECK(hipMemcpyAsync(base, hp, total, hipMemcpyHostToDevice, s));
-          hipLaunchKernelGGL(copy_jobs, dim3(32, (unsigned) n), dim3(256), 0, s, (const CopyJob *) (base + data));
-          HIPCHECK(hipGetLastError());
-          return 0;
-     }
-};
-
-// Results of a batch gathered by one copy_jobs launch into one device-to-host
-// copy; flush waits for the stream and scatters into the callers' arrays.
-struct Download {
-     struct Item { const void *src; void *dst; size_t off, n8; };
-     std::vector<Item> items;
-     size_t total = 0;
-     int add(void *dst, const void *src, size_t bytes) {
-          if (bytes % 8) return set_err("internal: download of %zu bytes", bytes);
-          items.push_back(Item{src, dst, total, bytes / 8});
-          total += bytes;
-          return 0;
-     }
-     int flush(Buf &dev, PinBuf &pin, hipStream_t s) {
-          if (items.empty()) return 0;
-          if (items.size() > 65535) return set_err("batch of %zu results (at most 65535)", items.size());
-          const size_t data = (total + 255) & ~(size_t) 255, jb = sizeof(CopyJob) * items.size();
-          if (dev.get(data + jb) || pin.get(data + jb)) return -1;
-          unsigned char *base = dev.as<unsigned char>(), *hp = (unsigned char *) pin.p;
-          CopyJob *jobs = (CopyJob *) (hp + data);
-          for (size_t k = 0; k < items.size(); ++k)
-               jobs[k] = CopyJob{(const double *) items[k].src, (double *) (base + items[k].off), items[k].n8};
-          HIPCHECK(hipMemcpyAsync(base + data, hp + data, jb, hipMemcpyHostToDevice, s));
-          hipLaunchKernelGGL(copy_jobs, dim3(32, (unsigned) items.size()), dim3(256), 0, s,
-                             (const CopyJob *) (base + data));
-          HIPCHECK(hipGetLastError());
-          HIPCHECK(hipMemcpyAsync(hp, base, total, hipMemcpyDeviceToHost, s));
-          HIPCHECK(hipStreamSynchronize(s));
-          for (const Item &it : items) memcpy(it.dst, hp + it.off, 8 * it.n8);
-          return 0;
-     }
+// Place of an input inside a call's uploaded block (Stage).
+struct Ref {
+     void *p = nullptr;
+     template <class T> T *as() const { return (T *) p; }
 };
 
 struct Workspace {
      int device = -1;
      hipStream_t stream = nullptr;
-     hipStream_t side = nullptr;     // the series sums, beside the contraction
-     hipEvent_t join2 = nullptr, sums = nullptr;
      hipEvent_t uploaded = nullptr;  // a batch case's inputs are on the device (its own stream)
-     std::vector<double> hguess;     // host staging of the Gauss root guesses
-     std::vector<int2> htask;        // host staging of the contraction task list
      hipEvent_t ev[2 * LMIE_N_TIMERS + 2];
-     Buf x, sx, cx, f, n1, n2, kfill, ktile32, ktile64;
-     Buf wrow, comb;                // weight rows and directions of the raw channels
-     Buf guess, mu, w, Bp, Bm, B16, A16, T, A, S, part, pfraw, pf, E, coefs, dots, dotjobs, save2, order;
-     std::vector<double> hsc;       // host staging of sin x, cos x
+     // inputs of the last forward call, in finDev (f: the weight rows, row 0 the density)
+     Ref x, sx, cx, f, n1, n2, kfill, ktile32, ktile64, ktile128, comb, guess, dotjobs, order, tasks;
+     std::vector<int2> rtask;       // host copy of tasks: (size tile, order tile) of the reverse contraction
+     Buf mu, w, Bp, Bm, B16, A16, T, A, S, part, pf, res, save2;
      // reverse-pass checkpoint and buffers
-     Buf CB, sst, pfbar, bar, fang, mbar, fbar, gbar, expart;
-     Buf wts, scal, L16, R16, Gf, G16, Uf, tasks;   // mixed reverse pass
+     Buf CB, sst, pfbar, bar, fang, gbar, expart;
+     Buf rres;                      // results: f cotangents [N], x cotangents [N], m cotangents per 64 sizes [Np / 64][2]
+     Buf wts, scal, L16, R16, Gf, G16, Uf;   // mixed reverse pass
      Buf chD, chPC, chPS, chPart, revScan;   // per-size recurrences
      Buf chDz, chPQ;                // and what their tangents need
      Buf ftab;                      // order_factors of the value channel
-     Buf sw, s1, s2;                // save_control 2: channel weights, saved per-size arrays
-     Buf bargs, bup, bdown;         // per-case arguments and staging of a batch launched from here
-     PinBuf pup, pdown;
-     PinBuf pres;                   // pinned landing area of a call's results (one DMA each)
-     Upload fin;                    // a single call's inputs, one copy (forward_impl)
-     Buf finDev;
+     Buf sw, s1, s2, sguess, dots;  // save_control 2: channel weights, saved per-size arrays, guesses, sums
+     Buf bargs;                     // per-case arguments of a batch launched from here
+     PinBuf pargs;
+     PinBuf pres;                   // pinned landing area of a call's results
+     PinBuf pin;                    // pinned staging of the cotangents
+     Buf finDev;                    // a call's inputs, one copy
      PinBuf finPin;
      int home = -1, busy = 0;       // batch slot of this workspace (-1: general pool)
      int n2rows = 0, ng = 0;
-     int ushape = 8, ntask = 0;     // reverse contraction: shape and task count of the pending pass
+     int ushape = 8;                // reverse contraction: shape
      int valid = 0;
      int N = 0, Np = 0, Kp = 0, Hp = 0, H = 0, Q = 0, C = 0, n1max = 0, n2max = 0, calc_gc = 0, calc_lc = 0;
      int mixed = 0, bf16 = 0, Kb = 0, Hb = 0;
-     std::vector<int> kt64, kt128;  // contraction depth per size tile of 64, 128
-     Buf ktile128;
      double mr = 0., mi = 0.;
 };
 
@@ -3065,9 +2950,6 @@ int ws_create(int device, Workspace **out) {
      Workspace *w = new Workspace();
      w->device = device;
      HIPCHECK(hipStreamCreateWithFlags(&w->stream, hipStreamNonBlocking));
-     HIPCHECK(hipStreamCreateWithFlags(&w->side, hipStreamNonBlocking));
-     HIPCHECK(hipEventCreateWithFlags(&w->join2, hipEventDisableTiming));
-     HIPCHECK(hipEventCreateWithFlags(&w->sums, hipEventDisableTiming));
      HIPCHECK(hipEventCreateWithFlags(&w->uploaded, hipEventDisableTiming));
      for (auto &e : w->ev) HIPCHECK(hipEventCreate(&e));
      *out = w;
@@ -3161,7 +3043,7 @@ struct Timer {
 // weight row per raw channel: rows 0 .. nP-1 of W weigh P (the density, its
 // tangents), rows nP .. nP+nX-1 weigh dP/dx (f dx_i of each direction that
 // moves x), and the two last channels are dP/dRe m and dP/dIm m with the
-// weight of row 0.  combine_channels forms the directions from the sums.
+// weight of row 0.  reduce_channels forms the directions from the sums.
 //
 // What bounds it: the FP64 matrix cores (64 cycles per instruction and SIMD).
 // A wave owns one 16 x 16 block with all its sums in registers (8
@@ -3400,23 +3282,6 @@ int launch_angular_f64(const F64Args &a, bool hx, bool hm, unsigned ntask, hipSt
      return 0;
 }
 
-// Directions from the raw channels: out[o] = sum_t c_t raw[r_t] (r_t < 0: none),
-// each channel 4 Q elements.
-struct ChComb {
-     int r[4];
-     double c[4];
-};
-__global__ __launch_bounds__(256) void combine_channels(const double *raw, int per, const ChComb *comb, double *out) {
-     const int e = blockIdx.x * 256 + threadIdx.x;
-     if (e >= per) return;
-     const ChComb k = comb[blockIdx.y];
-     double s = 0.;
-#pragma unroll
-     for (int t = 0; t < 4; ++t)
-          if (k.r[t] >= 0) s += k.c[t] * raw[(size_t) k.r[t] * per + e];
-     out[(size_t) blockIdx.y * per + e] = s;
-}
-
 // Task list of a tiled contraction over (size tile, column tile) pairs for
 // the XCD layout of the chip: the hardware deals workgroup ids round robin
 // over the 8 XCDs, so id 8k + x is the k-th workgroup of XCD x.  Size tiles go
@@ -3505,294 +3370,354 @@ void gauss_guesses(int n, double *g) {
 }
 
 
-int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
-     const auto t_entry = std::chrono::steady_clock::now();
-     const int N = J->n_size, Np = rup(N, 2 * TILE);   // whole tiles of 128 sizes
-     const int n1max = J->n1_max, Q = J->n_qang, C = J->n_coef;
-     const int H = Q / 2, Hp = rup(H > 0 ? H : 1, TILE), Kp = rup(n1max, 32);
-     const int nt = J->n_tan, nw = J->n_wgt, nch = 1 + nt + nw;
+// What the host works out of a forward job before its launches: padded extents,
+// contraction depths, the raw channels of the sums over sizes and the task
+// list of the contraction.
+struct FwdPlan {
+     int N, Np, n1max, Q, C, H, Hp, Kp, Kb, Hb, nt, nw, nch;
+     int mixed, bf16, planes, keep, n2max, n2rows, ng, tm, ntile;
+     // raw channels: weight rows of the value (row 0 the density, then the
+     // weight-only directions and the density tangents of the directions that
+     // move x or m), weight rows f dx_i of the value's x derivative, then its
+     // Re m and Im m derivatives under the density (angular_f64); comb[o] forms
+     // direction o from them
+     int nP, nX, nraw, nb;
+     bool hx, hm;
+     struct Row { const double *src; bool byf; };
+     std::vector<Row> rows;
+     std::vector<ChComb> comb;
+     std::vector<int> kt32, kt64, kt128;
+     std::vector<int2> task;
+};
+
+int plan_forward(const lmie_gpu_job *J, FwdPlan &p) {
+     const int N = J->n_size, n1max = J->n1_max, Q = J->n_qang;
      if (N <= 0) return set_err("no size points");
      if (Q % 2) return set_err("odd n_qang");
-     for (int i = 0; i < N; ++i)
+     p.n2max = 0;
+     for (int i = 0; i < N; ++i) {
           if (J->n1[i] > n1max || J->n1[i] < 1 || J->n2[i] < J->n1[i])
                return set_err("size point %d: order n1 = %d outside [1, %d] (n2 = %d)", i, J->n1[i], n1max, J->n2[i]);
-     hipStream_t s = w->stream;
-     Timer tm{w, g_timing};
-     w->valid = 0;
-     // mixed path: value and weight-only channels on the split 16-bit kernel;
-     // forward tangents and per-size matrix output stay on the FP64 kernel
-     const int mixed = (J->precision == LMIE_PRECISION_MIXED || J->precision == LMIE_PRECISION_MIXED_BF16) &&
-                       nt == 0 && nw <= 3 && J->save_control != 1 && Q > 0;
-     const int bf16 = J->precision == LMIE_PRECISION_MIXED_BF16;
-     const int kgran = mixed ? KM : KC;
-     const int Kb = rup(n1max, KM) / 8;
+          p.n2max = std::max(p.n2max, J->n2[i]);
+     }
+     p.N = N; p.Np = rup(N, 2 * TILE);                 // whole tiles of 128 sizes
+     p.n1max = n1max; p.Q = Q; p.C = J->n_coef; p.H = Q / 2;
+     p.Hp = rup(p.H > 0 ? p.H : 1, TILE); p.Kp = rup(n1max, 32); p.Kb = rup(n1max, KM) / 8;
      // angle padding of the split tables: tiles of 128 angles (whole angle
      // tiles of every contraction shape)
-     const MixShapeInfo ms = mix_shape();
-     const int Hb = rup(H > 0 ? H : 1, 128);
-
-     // host-side tables: per-tile contraction depths
-     const int nt32 = Np / 32, nt64 = Np / 64;
-     std::vector<int> n1h(Np, 0), n2h(Np, 0), kt32(nt32), kt64(nt64), kfill(nt64);
-     for (int i = 0; i < N; ++i) { n1h[i] = J->n1[i]; n2h[i] = J->n2[i]; }
-     for (int t = 0; t < nt32; ++t) {
-          int m = 0;
-          for (int i = t * 32; i < t * 32 + 32; ++i) m = n1h[i] > m ? n1h[i] : m;
-          kt32[t] = rup(m, kgran);
-     }
-     for (int t = 0; t < nt64; ++t) {
-          kt64[t] = kt32[2 * t] > kt32[2 * t + 1] ? kt32[2 * t] : kt32[2 * t + 1];
-          kfill[t] = 0;
-     }
-     // operand rows are zero up to the depth of the 128-size tile (the
-     // reverse contraction runs whole 128-size tiles)
-     std::vector<int> kt128(nt64 / 2);
-     for (int t = 0; t < nt64 / 2; ++t) kt128[t] = std::max(kt64[2 * t], kt64[2 * t + 1]);
-     for (int t = 0; t < nt64; ++t) kfill[t] = kt128[t / 2];
-     // uploads
-     if (w->x.get(sizeof(double) * Np) || w->f.get(sizeof(double) * Np) || w->n1.get(sizeof(int) * Np) ||
-         w->n2.get(sizeof(int) * Np) || w->kfill.get(sizeof(int) * nt64) || w->ktile32.get(sizeof(int) * nt32) ||
-         w->ktile64.get(sizeof(int) * nt64) || w->sx.get(sizeof(double) * Np) ||
-         w->cx.get(sizeof(double) * Np) || w->S.get(sizeof(double) * 4 * Np * (nt ? 4 : 1)))
-          return -1;
-     // every input of the pipeline goes up in one pinned host-to-device copy
-     // and one copy_jobs launch (a dozen small pageable copies cost more host
-     // time than the data)
-     Upload &up = w->fin;
-     up.items.clear();
-     up.h.clear();
-     // x, f zero-padded to Np; sin x, cos x of every size from the host C
-     // library, as the reference (padding 0, 1)
-     w->hsc.assign(4 * (size_t) Np, 0.);
-     {
-          double *hx = w->hsc.data(), *hf = hx + Np, *hs = hf + Np, *hc = hs + Np;
-          for (int i = 0; i < Np; ++i) {
-               hx[i] = i < N ? J->x[i] : 0.;
-               hf[i] = i < N ? J->f[i] : 0.;
-               hs[i] = i < N ? (J->sx ? J->sx[i] : sin(J->x[i])) : 0.;
-               hc[i] = i < N ? (J->cx ? J->cx[i] : cos(J->x[i])) : 1.;
-          }
-          if (up.add(w->x.p, hx, sizeof(double) * Np) || up.add(w->f.p, hf, sizeof(double) * Np) ||
-              up.add(w->sx.p, hs, sizeof(double) * Np) || up.add(w->cx.p, hc, sizeof(double) * Np) ||
-              up.add(w->n1.p, n1h.data(), sizeof(int) * Np) || up.add(w->n2.p, n2h.data(), sizeof(int) * Np) ||
-              up.add(w->kfill.p, kfill.data(), sizeof(int) * nt64) ||
-              up.add(w->ktile32.p, kt32.data(), sizeof(int) * nt32) ||
-              up.add(w->ktile64.p, kt64.data(), sizeof(int) * nt64))
-               return -1;
-     }
-     // raw channels of the sums over sizes: weight rows of the value (row 0 the
-     // density, then the weight-only directions and the density tangents of the
-     // directions that move x or m), weight rows f dx_i of the value's x
-     // derivative, then its Re m and Im m derivatives under the density
-     // (angular_f64); comb[o] forms direction o from them.
-     std::vector<ChComb> comb(nch, ChComb{{-1, -1, -1, -1}, {1., 1., 1., 1.}});
-     std::vector<double> wrow((size_t) Np, 0.);
-     memcpy(wrow.data(), J->f, sizeof(double) * N);
-     auto add_row = [&](const double *src, const double *by) -> int {   // src (times by), zero-padded to Np
-          const size_t o = wrow.size();
-          wrow.resize(o + Np, 0.);
-          for (int i = 0; i < N; ++i) wrow[o + i] = by ? src[i] * by[i] : src[i];
-          return (int) (o / Np);
-     };
+     p.Hb = rup(p.H > 0 ? p.H : 1, 128);
+     p.nt = J->n_tan; p.nw = J->n_wgt; p.nch = 1 + p.nt + p.nw;
+     // mixed path: value and weight-only channels on the split 16-bit kernel;
+     // forward tangents and per-size matrix output stay on the FP64 kernel
+     p.mixed = (J->precision == LMIE_PRECISION_MIXED || J->precision == LMIE_PRECISION_MIXED_BF16) && p.nt == 0 &&
+               p.nw <= 3 && J->save_control != 1 && Q > 0;
+     p.bf16 = J->precision == LMIE_PRECISION_MIXED_BF16;
+     p.planes = Q <= 0 ? 0 : J->calc_lc ? 5 : J->calc_gc ? 4 : 0;
+     p.keep = J->keep;
+     if (p.keep && (p.nt || J->save_control == 1))
+          return set_err("the reverse-pass checkpoint covers the value channel only");
+     // per-tile contraction depths; operand rows are zero up to the depth of
+     // the 128-size tile (the reverse contraction runs whole 128-size tiles)
+     const int gran = p.mixed ? KM : KC, nt32 = p.Np / 32, nt64 = p.Np / 64;
+     p.kt32.assign(nt32, 0);
+     for (int i = 0; i < N; ++i) p.kt32[i / 32] = std::max(p.kt32[i / 32], J->n1[i]);
+     for (int &k : p.kt32) k = rup(k, gran);
+     p.kt64.resize(nt64);
+     p.kt128.resize(nt64 / 2);
+     for (int t = 0; t < nt64; ++t) p.kt64[t] = std::max(p.kt32[2 * t], p.kt32[2 * t + 1]);
+     int kfmax = 0;
+     for (int t = 0; t < nt64 / 2; ++t) kfmax = std::max(kfmax, p.kt128[t] = std::max(p.kt64[2 * t], p.kt64[2 * t + 1]));
+     p.n2rows = p.n2max + 1;
+     p.ng = kfmax / 8;
+     // channels
      auto moves = [&](const double *v) {
           for (int i = 0; i < N; ++i)
                if (v[i] != 0.) return true;
           return false;
      };
-     bool hx = false, hm = false;
-     comb[0].r[0] = 0;
-     for (int t = 0; t < nw; ++t) comb[1 + nt + t].r[0] = add_row(J->df_wgt + (size_t) t * N, nullptr);
-     for (int t = 0; t < nt; ++t)
-          if (moves(J->df_tan + (size_t) t * N)) comb[1 + t].r[0] = add_row(J->df_tan + (size_t) t * N, nullptr);
-     const int nP = (int) (wrow.size() / Np);
-     for (int t = 0; t < nt; ++t)
-          if (moves(J->dx + (size_t) t * N)) {
-               comb[1 + t].r[1] = add_row(J->dx + (size_t) t * N, J->f);
-               hx = true;
-          }
-     const int nX = (int) (wrow.size() / Np) - nP;
-     for (int t = 0; t < nt; ++t)
+     p.rows.assign(1, FwdPlan::Row{J->f, false});
+     p.comb.assign(p.nch, ChComb{{-1, -1, -1, -1}, {1., 1., 1., 1.}});
+     p.comb[0].r[0] = 0;
+     auto row = [&](const double *src, bool byf) { p.rows.push_back(FwdPlan::Row{src, byf}); return (int) p.rows.size() - 1; };
+     for (int t = 0; t < p.nw; ++t) p.comb[1 + p.nt + t].r[0] = row(J->df_wgt + (size_t) t * N, false);
+     for (int t = 0; t < p.nt; ++t)
+          if (moves(J->df_tan + (size_t) t * N)) p.comb[1 + t].r[0] = row(J->df_tan + (size_t) t * N, false);
+     p.nP = (int) p.rows.size();
+     for (int t = 0; t < p.nt; ++t)
+          if (moves(J->dx + (size_t) t * N)) p.comb[1 + t].r[1] = row(J->dx + (size_t) t * N, true);
+     p.nX = (int) p.rows.size() - p.nP;
+     p.hx = p.nX > 0;
+     p.hm = false;
+     for (int t = 0; t < p.nt; ++t)
           if (J->dm[2 * t] != 0. || J->dm[2 * t + 1] != 0.) {
-               comb[1 + t].r[2] = nP + nX;
-               comb[1 + t].r[3] = nP + nX + 1;
-               comb[1 + t].c[2] = J->dm[2 * t];
-               comb[1 + t].c[3] = J->dm[2 * t + 1];
-               hm = true;
+               ChComb &c = p.comb[1 + t];
+               c.r[2] = p.nP + p.nX; c.r[3] = p.nP + p.nX + 1;
+               c.c[2] = J->dm[2 * t]; c.c[3] = J->dm[2 * t + 1];
+               p.hm = true;
           }
-     const int nraw = nP + nX + (hm ? 2 : 0), nb = 1 + hx + hm;
-     const bool tan = hx || hm;
-     if (w->wrow.get(sizeof(double) * wrow.size()) || up.add(w->wrow.p, wrow.data(), sizeof(double) * wrow.size()) ||
-         w->comb.get(sizeof(ChComb) * nch) || (nt && up.add(w->comb.p, comb.data(), sizeof(ChComb) * nch)))
-          return -1;
-     if (Q > 0) {
-          // initial guesses of the Gauss roots (host C library)
-          if (w->guess.get(sizeof(double) * H)) return -1;
-          w->hguess.resize(H > 0 ? H : 1);
-          gauss_guesses(Q, w->hguess.data());
-          if (up.add(w->guess.p, w->hguess.data(), sizeof(double) * H)) return -1;
+     p.nraw = p.nP + p.nX + (p.hm ? 2 : 0);
+     p.nb = 1 + p.hx + p.hm;
+     // the contraction's task list
+     p.task.clear();
+     p.tm = F64_TILE;
+     if (p.mixed) {
+          const MixShapeInfo ms = mix_shape();
+          p.tm = ms.tm;
+          xcd_tasks(ms.tm == 64 ? p.kt64 : p.kt32, [&](int) { return (p.H + ms.tn - 1) / ms.tn; }, mix_group(), p.task);
+     } else if (Q > 0)
+          xcd_tasks(p.kt32, [&](int) { return (p.H + F64_TILE - 1) / F64_TILE; }, F64_GROUP, p.task);
+     p.ntile = p.Np / p.tm;
+     return 0;
+}
+
+// The inputs of a call, laid out in one pinned buffer and sent as one copy; the
+// kernels read them where they land (the pointers of the workspace).  They
+// stay valid until the workspace's next forward call.
+struct Stage {
+     size_t n = 0;
+     std::vector<std::pair<Ref *, size_t>> at;
+     template <class T> void add(Ref &r, size_t count) {
+          at.push_back({&r, n});
+          n = (n + sizeof(T) * count + 255) & ~(size_t) 255;
      }
-     // pinned landing area of the results: expansions [2][nch][6][C], then the sums
-     if (w->pres.get(sizeof(double) * ((size_t) nch * 12 * C + 4 * nraw))) return -1;
-     if (mixed) {
-          // the contraction's task list
-          xcd_tasks(ms.tm == 64 ? kt64 : kt32, [&](int) { return (H + ms.tn - 1) / ms.tn; }, mix_group(), w->htask);
-          if (w->order.get(sizeof(int2) * w->htask.size()) ||
-              up.add(w->order.p, w->htask.data(), sizeof(int2) * w->htask.size()))
-               return -1;
+     // device addresses into the Refs; host(r) is r's place in the pinned copy
+     unsigned char *hp = nullptr;
+     int open(Buf &dev, PinBuf &pin) {
+          if (dev.get(n) || pin.get(n)) return -1;
+          hp = (unsigned char *) pin.p;
+          for (auto &a : at) a.first->p = dev.as<unsigned char>() + a.second;
+          return 0;
      }
-     if (!mixed && Q > 0) {
-          xcd_tasks(kt32, [&](int) { return (H + F64_TILE - 1) / F64_TILE; }, F64_GROUP, w->htask);
-          if (w->order.get(sizeof(int2) * w->htask.size()) ||
-              up.add(w->order.p, w->htask.data(), sizeof(int2) * w->htask.size()))
-               return -1;
+     template <class T> T *host(const Ref &r, const Buf &dev) const { return (T *) (hp + ((unsigned char *) r.p - (unsigned char *) dev.p)); }
+};
+
+int stage_forward(Workspace *w, const lmie_gpu_job *J, const FwdPlan &p, bool batch, hipStream_t s) {
+     const int N = p.N, Np = p.Np;
+     const size_t nrow = p.rows.size();
+     // what the reverse pass needs besides the cotangents goes up with the
+     // forward's inputs: the task list and depths of the reverse contraction
+     std::vector<int2> rtask;
+     if (p.keep && p.mixed) {
+          w->ushape = batch ? 8 : ugemm_waves();       // fused passes run the 128-size shape
+          const std::vector<int> &kts = w->ushape == 2 ? p.kt64 : p.kt128;
+          xcd_tasks(kts, [&](int t) { return (kts[t] + 63) / 64; }, tile_group(), rtask);
      }
+     w->rtask = rtask;
+     Stage st;
+     st.add<double>(w->x, Np); st.add<double>(w->sx, Np); st.add<double>(w->cx, Np);
+     st.add<double>(w->f, nrow * Np);
+     st.add<int>(w->n1, Np); st.add<int>(w->n2, Np);
+     st.add<int>(w->kfill, Np / 64); st.add<int>(w->ktile32, Np / 32); st.add<int>(w->ktile64, Np / 64);
+     st.add<int>(w->ktile128, Np / 64);
+     st.add<ChComb>(w->comb, p.nch); st.add<double>(w->guess, p.H > 0 ? p.H : 1);
+     st.add<DotJob>(w->dotjobs, 4 * (size_t) p.nraw);
+     st.add<int2>(w->order, p.task.size()); st.add<int2>(w->tasks, rtask.size());
+     if (st.open(w->finDev, w->finPin)) return -1;
+     auto h = [&](const Ref &r) { return st.host<double>(r, w->finDev); };
+     // x, f zero-padded to Np; sin x, cos x of every size from the host C
+     // library, as the reference (padding 0, 1)
+     auto pad = [&](double *d, const double *v, double fill) {
+          memcpy(d, v, sizeof(double) * N);
+          for (int i = N; i < Np; ++i) d[i] = fill;
+     };
+     pad(h(w->x), J->x, 0.);
+     double *hs = h(w->sx), *hc = h(w->cx);
+     if (J->sx) pad(hs, J->sx, 0.);
+     else for (int i = 0; i < Np; ++i) hs[i] = i < N ? sin(J->x[i]) : 0.;
+     if (J->cx) pad(hc, J->cx, 1.);
+     else for (int i = 0; i < Np; ++i) hc[i] = i < N ? cos(J->x[i]) : 1.;
+     for (size_t r = 0; r < nrow; ++r) {
+          double *d = h(w->f) + r * Np;
+          pad(d, p.rows[r].src, 0.);
+          if (p.rows[r].byf)
+               for (int i = 0; i < N; ++i) d[i] *= J->f[i];
+     }
+     auto ints = [&](const Ref &r, const int *v, size_t n, size_t cap) {
+          int *d = st.host<int>(r, w->finDev);
+          memcpy(d, v, sizeof(int) * n);
+          for (size_t k = n; k < cap; ++k) d[k] = 0;
+     };
+     ints(w->n1, J->n1, N, Np);
+     ints(w->n2, J->n2, N, Np);
+     ints(w->ktile32, p.kt32.data(), p.kt32.size(), Np / 32);
+     ints(w->ktile64, p.kt64.data(), p.kt64.size(), Np / 64);
+     int *kf = st.host<int>(w->kfill, w->finDev);
+     for (int t = 0; t < Np / 64; ++t) kf[t] = p.kt128[t / 2];
+     const std::vector<int> &kts = p.keep && p.mixed && w->ushape == 2 ? p.kt64 : p.kt128;
+     ints(w->ktile128, kts.data(), kts.size(), Np / 64);
+     memcpy(st.host<ChComb>(w->comb, w->finDev), p.comb.data(), sizeof(ChComb) * p.nch);
+     // initial guesses of the Gauss roots (host C library)
+     if (p.Q > 0) gauss_guesses(p.Q, h(w->guess));
      // series dot products of every raw channel
-     std::vector<DotJob> dot_jobs;
-     {
-          const double *S0 = w->S.as<double>(), *W0 = w->wrow.as<double>();
-          const double *SX = S0 + 4 * (size_t) Np, *SM = S0 + 4 * (size_t) Np * (hx ? 2 : 1);
-          for (int c = 0; c < nraw; ++c)
-               for (int q = 0; q < 4; ++q)
-                    dot_jobs.push_back(DotJob{W0 + (c < nP + nX ? (size_t) c * Np : 0),
-                                              (c < nP ? S0 : c < nP + nX ? SX : SM + 4 * (size_t) Np * (c - nP - nX)) +
-                                                   (size_t) q * Np, nullptr, nullptr});
-          if (w->dotjobs.get(sizeof(DotJob) * dot_jobs.size()) || w->dots.get(sizeof(double) * dot_jobs.size()) ||
-              up.add(w->dotjobs.p, dot_jobs.data(), sizeof(DotJob) * dot_jobs.size()))
-               return -1;
-     }
-     if (up.flush(w->finDev, w->finPin, s)) return -1;
+     DotJob *dj = st.host<DotJob>(w->dotjobs, w->finDev);
+     const double *S0 = w->S.as<double>(), *W0 = w->f.as<double>();
+     const double *SX = S0 + 4 * (size_t) Np, *SM = S0 + 4 * (size_t) Np * (p.hx ? 2 : 1);
+     for (int c = 0; c < p.nraw; ++c)
+          for (int q = 0; q < 4; ++q)
+               *dj++ = DotJob{W0 + (c < p.nP + p.nX ? (size_t) c * Np : 0),
+                              (c < p.nP ? S0 : c < p.nP + p.nX ? SX : SM + 4 * (size_t) Np * (c - p.nP - p.nX)) + (size_t) q * Np};
+     memcpy(st.host<int2>(w->order, w->finDev), p.task.data(), sizeof(int2) * p.task.size());
+     memcpy(st.host<int2>(w->tasks, w->finDev), rtask.data(), sizeof(int2) * rtask.size());
+     HIPCHECK(hipMemcpyAsync(w->finDev.p, w->finPin.p, st.n, hipMemcpyHostToDevice, s));
+     return 0;
+}
+
+// Device buffers of a forward call.
+int alloc_forward(Workspace *w, const lmie_gpu_job *J, const FwdPlan &p) {
+     const size_t Np = p.Np, plane = (size_t) p.Kp * Np, C = p.C, Q = p.Q > 0 ? p.Q : 1, Hp = p.Hp;
+     const bool tan = p.hx || p.hm;
+     if (w->S.get(sizeof(double) * 4 * Np * (1 + p.hx + 2 * p.hm)) ||
+         w->chD.get(sizeof(double) * 2 * (size_t) p.n2rows * Np) || w->chPC.get(sizeof(double) * 2 * (size_t) (p.n1max + 1) * Np) ||
+         w->chPS.get(sizeof(double) * Np) || w->chPart.get(sizeof(double) * (5 + 5 * p.hx + 8 * p.hm) * (size_t) (p.ng > 0 ? p.ng : 1) * Np) ||
+         (tan && (w->chDz.get(sizeof(double) * 2 * (size_t) p.n2rows * Np) || w->chPQ.get(sizeof(double) * 2 * Np))) ||
+         w->ftab.get(sizeof(double) * FT_ROWS * (size_t) (p.n1max + 2)) ||
+         (p.mixed ? w->A16.get(sizeof(unsigned short) * 8 * (size_t) p.Kb * Np * 8) : w->A.get(sizeof(double) * 4 * plane * p.nb)) ||
+         w->res.get(sizeof(double) * ((size_t) p.nch * 12 * C + 4 * p.nraw)) ||
+         w->pres.get(sizeof(double) * ((size_t) p.nch * 12 * C + 4 * p.nraw)) ||
+         (p.keep && w->CB.get(sizeof(double) * 2 * Np)))
+          return -1;
+     if (p.Q <= 0) return 0;
+     if (w->mu.get(sizeof(double) * Q) || w->w.get(sizeof(double) * Q) ||
+         (p.planes && w->T.get(sizeof(double) * p.planes * C * Hp)) ||
+         (p.mixed ? w->B16.get(sizeof(unsigned short) * B16_PLANES * (size_t) p.Kb * p.Hb * 8)
+                  : (w->Bp.get(sizeof(double) * (size_t) p.Kp * Hp) || w->Bm.get(sizeof(double) * (size_t) p.Kp * Hp))) ||
+         w->pf.get(sizeof(double) * (size_t) p.nch * 4 * Q) ||
+         w->part.get(sizeof(double) * (size_t) p.ntile * p.nraw * 4 * Q) ||
+         (p.keep && !p.mixed && w->sst.get(sizeof(double) * 8 * Np * Hp)) ||
+         (J->save_control == 1 && w->save2.get(sizeof(double) * (size_t) 4 * p.N * Q)))
+          return -1;
+     return 0;
+}
+
+// Kernel arguments of the front, the terms and the mixed contraction (shared by
+// the single call and the fused batch).
+void front_args(const Workspace *w, const lmie_gpu_job *J, const FwdPlan &p, FrontArgs &fa) {
+     memset(&fa, 0, sizeof fa);
+     ChainArgs &ca = fa.ch;
+     ca.N = p.N; ca.Np = p.Np; ca.n1max = p.n1max; ca.n2rows = p.n2rows;
+     ca.x = w->x.as<double>(); ca.sx = w->sx.as<double>(); ca.cx = w->cx.as<double>();
+     ca.n1 = w->n1.as<int>(); ca.n2 = w->n2.as<int>(); ca.mr = J->mr; ca.mi = J->mi;
+     ca.d_all = p.keep; ca.D = w->chD.as<double>(); ca.PC = w->chPC.as<double>(); ca.PS = w->chPS.as<double>();
+     ca.Dz = w->chDz.as<double>(); ca.PQ = w->chPQ.as<double>();
+     fa.Q = p.Q; fa.H = p.H; fa.Hp = p.Hp; fa.C = p.C; fa.n1max = p.n1max; fa.Kp = p.Kp; fa.Kb = p.Kb; fa.Hb = p.Hb;
+     fa.guess = w->guess.as<double>(); fa.mu = w->mu.as<double>(); fa.w = w->w.as<double>();
+     fa.T = w->T.as<double>(); fa.Bp = w->Bp.as<double>(); fa.Bm = w->Bm.as<double>();
+     fa.B16 = w->B16.as<unsigned short>(); fa.ft = w->ftab.as<double>();
+     fa.plan(p.planes, p.Q <= 0 ? 0 : p.mixed ? 2 : 1, p.Q > 0, p.Np / 64, true);
+}
+
+void term_args(const Workspace *w, const lmie_gpu_job *J, const FwdPlan &p, TermArgs &ta) {
+     ta.N = p.N; ta.Np = p.Np; ta.n1max = p.n1max; ta.n2rows = p.n2rows; ta.Kp = p.Kp; ta.Kb = p.Kb; ta.ng = p.ng;
+     ta.ft = w->ftab.as<double>();
+     ta.x = w->x.as<double>(); ta.n1 = w->n1.as<int>(); ta.kfill = w->kfill.as<int>();
+     ta.mr = J->mr; ta.mi = J->mi; ta.D = w->chD.as<double>(); ta.PC = w->chPC.as<double>(); ta.PS = w->chPS.as<double>();
+     ta.A = p.mixed ? nullptr : w->A.as<double>();
+     ta.A16 = p.mixed ? w->A16.as<unsigned short>() : nullptr;
+     ta.part = w->chPart.as<double>();
+}
+
+void mix_args(const Workspace *w, const FwdPlan &p, Mix2Args &m) {
+     memset(&m, 0, sizeof m);
+     m.Np = p.Np; m.Kb = p.Kb; m.Hb = p.Hb; m.H = p.H; m.Q = p.Q;
+     m.A16 = w->A16.as<unsigned short>();
+     m.B16 = w->B16.as<unsigned short>();
+     m.ktile = p.tm == 64 ? w->ktile64.as<int>() : w->ktile32.as<int>();
+     m.task = w->order.as<int2>();
+     for (int q = 0; q <= p.nw; ++q) m.W[q] = w->f.as<double>() + (size_t) q * p.Np;
+     m.part = w->part.as<double>();
+}
+
+// Results of a call: the series sums of the raw channels [4 nraw], then the
+// expansions, generalized spherical [nch][6][C] and Legendre [nch][6][C], in
+// one buffer.
+void reduce_args(const Workspace *w, const FwdPlan &p, double *res, ReduceArgs &r) {
+     r.part = w->part.as<double>(); r.nblk = p.ntile; r.nraw = p.nraw; r.Q = p.Q > 0 ? p.Q : 0; r.nch = p.nch;
+     r.comb = p.nt ? w->comb.as<ChComb>() : nullptr;
+     r.out = w->pf.as<double>();
+     r.jobs = w->dotjobs.as<DotJob>(); r.n = p.Np; r.ndot = 4 * p.nraw; r.dots = res;
+     r.gx = (unsigned) ((r.nch * 4 * r.Q + 31) / 32 + r.ndot);
+}
+
+void keep_forward(Workspace *w, const lmie_gpu_job *J, const FwdPlan &p) {
+     w->N = p.N; w->Np = p.Np; w->Kp = p.Kp; w->Hp = p.Hp; w->H = p.H; w->Q = p.Q; w->C = p.C; w->n1max = p.n1max;
+     w->n2max = p.n2max; w->n2rows = p.n2rows; w->ng = p.ng;
+     w->calc_gc = J->calc_gc; w->calc_lc = J->calc_lc; w->mr = J->mr; w->mi = J->mi;
+     w->mixed = p.mixed; w->bf16 = p.bf16; w->Kb = p.Kb; w->Hb = p.Hb;
+}
+
+// Raw sums of every direction from those of the raw channels.
+void unpack_sums(const FwdPlan &p, const double *dots, lmie_gpu_result *R) {
+     for (int q = 0; q < 4; ++q) R->sums[q] = dots[q];
+     for (int c = 1; c < p.nch; ++c)
+          for (int q = 0; q < 4; ++q) {
+               double v = 0.;
+               for (int t = 0; t < 4; ++t)
+                    if (p.comb[c].r[t] >= 0) v += p.comb[c].c[t] * dots[4 * p.comb[c].r[t] + q];
+               R->sums_ch[4 * (c - 1) + q] = v;
+          }
+}
+
+int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
+     const auto t_entry = std::chrono::steady_clock::now();
+     hipStream_t s = w->stream;
+     Timer tm{w, g_timing};
+     w->valid = 0;
+     FwdPlan p;
+     if (plan_forward(J, p) || alloc_forward(w, J, p) || stage_forward(w, J, p, false, s)) return -1;
+     const int N = p.N, Np = p.Np, Q = p.Q, C = p.C, nch = p.nch, keep = p.keep;
+     const bool tan = p.hx || p.hm;
      const double prep_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_entry).count();
      tm.mark(LMIE_T_TOTAL, 0);
 
-     // per-size coefficients
-     const size_t plane = (size_t) Kp * Np;
-     if ((!mixed && w->A.get(sizeof(double) * 4 * plane * nb)) ||
-         (mixed && w->A16.get(sizeof(unsigned short) * 8 * (size_t) Kb * Np * 8)))
-          return -1;
-     const int keep = J->keep;
-     if (keep) {
-          if (nt || J->save_control == 1) return set_err("the reverse-pass checkpoint covers the value channel only");
-          if (w->CB.get(sizeof(double) * 2 * Np) ||
-              (Q > 0 && !mixed && w->sst.get(sizeof(double) * 8 * (size_t) Np * Hp)))
-               return -1;
-     }
+     // angle tables, chains and order factors; terms; per-size sums
      tm.mark(LMIE_T_COEFS, 0);
-     {
-          // serial recurrences, parallel terms, per-size sums
-          int n2max = 0, kfmax = 0;
-          for (int i = 0; i < N; ++i) n2max = J->n2[i] > n2max ? J->n2[i] : n2max;
-          for (int t = 0; t < nt64; ++t) kfmax = kfill[t] > kfmax ? kfill[t] : kfmax;
-          const int n2rows = n2max + 1, ng = kfmax / 8;
-          if (w->chD.get(sizeof(double) * 2 * (size_t) n2rows * Np) ||
-              w->chPC.get(sizeof(double) * 2 * (size_t) (n1max + 1) * Np) || w->chPS.get(sizeof(double) * Np) ||
-              w->chPart.get(sizeof(double) * (5 + 5 * hx + 8 * hm) * (size_t) (ng > 0 ? ng : 1) * Np) ||
-             (tan && (w->chDz.get(sizeof(double) * 2 * (size_t) n2rows * Np) || w->chPQ.get(sizeof(double) * 2 * Np))))
-               return -1;
-          ChainArgs ca;
-          ca.N = N; ca.Np = Np; ca.n1max = n1max; ca.n2rows = n2rows;
-          ca.x = w->x.as<double>(); ca.sx = w->sx.as<double>(); ca.cx = w->cx.as<double>();
-          ca.n1 = w->n1.as<int>(); ca.n2 = w->n2.as<int>(); ca.mr = J->mr; ca.mi = J->mi;
-          ca.d_all = keep; ca.D = w->chD.as<double>(); ca.PC = w->chPC.as<double>(); ca.PS = w->chPS.as<double>();
-          ca.Dz = w->chDz.as<double>(); ca.PQ = w->chPQ.as<double>();
-          // angle tables, chains and order factors
-          FrontArgs fa;
-          memset(&fa, 0, sizeof fa);
-          fa.Q = Q; fa.H = H; fa.Hp = Hp; fa.C = C; fa.n1max = n1max; fa.Kp = Kp; fa.Kb = Kb; fa.Hb = Hb;
-          const int planes = Q <= 0 ? 0 : J->calc_lc ? 5 : J->calc_gc ? 4 : 0;
-          const int pk = Q <= 0 ? 1 : !mixed ? 1 : bf16 ? 3 : 2;
-          if (w->ftab.get(sizeof(double) * FT_ROWS * (size_t) (n1max + 2)) ||
-              (Q > 0 && (w->mu.get(sizeof(double) * Q) || w->w.get(sizeof(double) * Q))) ||
-              (planes && w->T.get(sizeof(double) * planes * (size_t) C * Hp)) ||
-              (Q > 0 && !mixed && (w->Bp.get(sizeof(double) * (size_t) Kp * Hp) || w->Bm.get(sizeof(double) * (size_t) Kp * Hp))) ||
-              (mixed && w->B16.get(sizeof(unsigned short) * B16_PLANES * (size_t) Kb * Hb * 8)))
-               return -1;
-          fa.guess = w->guess.as<double>(); fa.mu = w->mu.as<double>(); fa.w = w->w.as<double>();
-          fa.T = w->T.as<double>(); fa.Bp = w->Bp.as<double>(); fa.Bm = w->Bm.as<double>();
-          fa.B16 = w->B16.as<unsigned short>(); fa.ft = w->ftab.as<double>(); fa.ch = ca;
-          fa.plan(planes, Q > 0 ? pk : 0, Q > 0, Np / 64, true);
-          tm.mark(LMIE_T_TABLES, 0);
-          if (launch_front(fa, pk, tan, s)) return -1;
-          tm.mark(LMIE_T_TABLES, 1);
-          if (tan) {
-               TanArgs ta;
-               ta.N = N; ta.Np = Np; ta.n1max = n1max; ta.n2rows = n2rows; ta.Kp = Kp; ta.ng = ng;
-               ta.ft = w->ftab.as<double>();
-               ta.x = w->x.as<double>(); ta.n1 = w->n1.as<int>(); ta.kfill = w->kfill.as<int>();
-               ta.mr = J->mr; ta.mi = J->mi; ta.D = w->chD.as<double>(); ta.Dz = w->chDz.as<double>();
-               ta.PC = w->chPC.as<double>(); ta.PS = w->chPS.as<double>(); ta.PQ = w->chPQ.as<double>();
-               for (int b = 0; b < nb; ++b) ta.A[b] = w->A.as<double>() + 4 * plane * b;
-               ta.part = w->chPart.as<double>();
-               const dim3 gt(Np / 64, ng), gs((Np + 31) / 32);
-#define LMIE_TAN(X, M)                                                                                           \
-               do {                                                                                              \
-                    if (ng > 0) hipLaunchKernelGGL((mie_tan_terms<X, M>), gt, dim3(64), 0, s, ta);               \
-                    hipLaunchKernelGGL((mie_tan_sums<X, M>), gs, dim3(256), 0, s, (const double *) w->chPart.as<double>(), N, Np, \
-                                       ng, (const int *) w->n1.as<int>(), w->S.as<double>());                    \
-               } while (0)
-               if (hx && hm) LMIE_TAN(true, true);
-               else if (hx) LMIE_TAN(true, false);
-               else LMIE_TAN(false, true);
-#undef LMIE_TAN
-          } else {
-          TermArgs ta;
-          ta.N = N; ta.Np = Np; ta.n1max = n1max; ta.n2rows = n2rows; ta.Kp = Kp; ta.Kb = Kb; ta.ng = ng;
+     FrontArgs fa;
+     front_args(w, J, p, fa);
+     tm.mark(LMIE_T_TABLES, 0);
+     if (launch_front(fa, !p.mixed ? 1 : p.bf16 ? 3 : 2, tan, s)) return -1;
+     tm.mark(LMIE_T_TABLES, 1);
+     const dim3 gt(Np / 64, p.ng), gs((Np + 31) / 32);
+     if (tan) {
+          TanArgs ta;
+          ta.N = N; ta.Np = Np; ta.n1max = p.n1max; ta.n2rows = p.n2rows; ta.Kp = p.Kp; ta.ng = p.ng;
           ta.ft = w->ftab.as<double>();
           ta.x = w->x.as<double>(); ta.n1 = w->n1.as<int>(); ta.kfill = w->kfill.as<int>();
-          ta.mr = J->mr; ta.mi = J->mi; ta.D = w->chD.as<double>(); ta.PC = w->chPC.as<double>();
-          ta.PS = w->chPS.as<double>();
-          ta.A = mixed ? nullptr : w->A.as<double>();
-          ta.A16 = mixed ? w->A16.as<unsigned short>() : nullptr;
+          ta.mr = J->mr; ta.mi = J->mi; ta.D = w->chD.as<double>(); ta.Dz = w->chDz.as<double>();
+          ta.PC = w->chPC.as<double>(); ta.PS = w->chPS.as<double>(); ta.PQ = w->chPQ.as<double>();
+          for (int b = 0; b < p.nb; ++b) ta.A[b] = w->A.as<double>() + 4 * (size_t) p.Kp * Np * b;
           ta.part = w->chPart.as<double>();
-          if (ng > 0) {
-               const dim3 grid(Np / 64, ng);
-               if (!mixed) hipLaunchKernelGGL(mie_terms<void>, grid, dim3(64), 0, s, ta);
-               else if (bf16) hipLaunchKernelGGL(mie_terms<BF16>, grid, dim3(64), 0, s, ta);
-               else hipLaunchKernelGGL(mie_terms<F16>, grid, dim3(64), 0, s, ta);
+#define LMIE_TAN(X, M)                                                                                           \
+          do {                                                                                                   \
+               if (p.ng > 0) hipLaunchKernelGGL((mie_tan_terms<X, M>), gt, dim3(64), 0, s, ta);                  \
+               hipLaunchKernelGGL((mie_tan_sums<X, M>), gs, dim3(256), 0, s, (const double *) w->chPart.as<double>(), N, Np, \
+                                  p.ng, (const int *) w->n1.as<int>(), w->S.as<double>());                       \
+          } while (0)
+          if (p.hx && p.hm) LMIE_TAN(true, true);
+          else if (p.hx) LMIE_TAN(true, false);
+          else LMIE_TAN(false, true);
+#undef LMIE_TAN
+     } else {
+          TermArgs ta;
+          term_args(w, J, p, ta);
+          if (p.ng > 0) {
+               if (!p.mixed) hipLaunchKernelGGL(mie_terms<void>, gt, dim3(64), 0, s, ta);
+               else if (p.bf16) hipLaunchKernelGGL(mie_terms<BF16>, gt, dim3(64), 0, s, ta);
+               else hipLaunchKernelGGL(mie_terms<F16>, gt, dim3(64), 0, s, ta);
           }
-          hipLaunchKernelGGL(mie_sums, dim3((Np + 31) / 32), dim3(256), 0, s, (const double *) w->chPart.as<double>(), N, Np,
-                             ng, (const int *) w->n1.as<int>(), w->S.as<double>(), keep ? w->CB.as<double>() : nullptr);
-          }
-          HIPCHECK(hipGetLastError());
-          w->n2rows = n2rows;
-          w->ng = ng;
+          hipLaunchKernelGGL(mie_sums, gs, dim3(256), 0, s, (const double *) w->chPart.as<double>(), N, Np,
+                             p.ng, (const int *) w->n1.as<int>(), w->S.as<double>(), keep ? w->CB.as<double>() : nullptr);
      }
+     HIPCHECK(hipGetLastError());
      tm.mark(LMIE_T_COEFS, 1);
 
-     // series sums (jobs uploaded with the inputs)
-     {
-          // on the side stream (beside the contraction);
-          // the main stream joins it (join2) before the expansion
-          hipStream_t ts = w->side;
-          HIPCHECK(hipEventRecord(w->sums, s));
-          HIPCHECK(hipStreamWaitEvent(ts, w->sums, 0));
-          tm.mark(LMIE_T_REDUCE, 0);
-          hipLaunchKernelGGL(weighted_dots, dim3(dot_jobs.size()), dim3(256), 0, ts, w->dotjobs.as<DotJob>(), Np,
-                             w->dots.as<double>());
-          HIPCHECK(hipGetLastError());
-          HIPCHECK(hipEventRecord(w->join2, ts));
-     }
-
-     // angular contraction and reduction
+     // angular contraction
      if (Q > 0) {
-          if (w->pf.get(sizeof(double) * (size_t) nch * 4 * Q)) return -1;
-          if (J->save_control == 1 && w->save2.get(sizeof(double) * (size_t) 4 * N * Q)) return -1;
-          const int ntile = Np / (mixed ? ms.tm : F64_TILE);
-          if (w->part.get(sizeof(double) * (size_t) ntile * nraw * 4 * Q) ||
-              (nt && w->pfraw.get(sizeof(double) * (size_t) nraw * 4 * Q)))
-               return -1;
           tm.mark(LMIE_T_ANGULAR, 0);
-          if (mixed) {
+          if (p.mixed) {
                Mix2Args m;
-               memset(&m, 0, sizeof m);
-               m.Np = Np; m.Kb = Kb; m.Hb = Hb; m.H = H; m.Q = Q;
-               m.A16 = w->A16.as<unsigned short>();
-               m.B16 = w->B16.as<unsigned short>();
-               m.ktile = ms.tm == 64 ? w->ktile64.as<int>() : w->ktile32.as<int>();
-               m.task = w->order.as<int2>();
-               m.W[0] = w->f.as<double>();
-               for (int q = 0; q < nw; ++q) m.W[1 + q] = w->wrow.as<double>() + (size_t) (1 + q) * Np;
-               m.part = w->part.as<double>();
-               const dim3 grid((unsigned) w->htask.size());
+               mix_args(w, p, m);
+               const dim3 grid((unsigned) p.task.size());
+               const int nw = p.nw, id = mix_shape().id;
                // five split products (three with LMIE_MIX_PRODUCTS=3), in the
                // shape of LMIE_MIX_SHAPE
 #define LMIE_MIX(E, NP, NWC, S) hipLaunchKernelGGL((angular_mix<E, NP, NWC, S>), grid, dim3(S::NT), 0, s, m)
@@ -3807,99 +3732,71 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
                     else if (mix_products() == 4 && std::is_same<S, MixS3>::value) LMIE_MIX_NW(E, 4, MixS3); \
                     else LMIE_MIX_NW(E, 5, S);                                                          \
                } while (0)
-#define LMIE_MIX_S(S) do { if (bf16) LMIE_MIX_NP(BF16, S); else LMIE_MIX_NP(F16, S); } while (0)
-               if (ms.id == 0) LMIE_MIX_S(MixS0);
-               else if (ms.id == 2) LMIE_MIX_S(MixS2);
-               else if (ms.id == 3) LMIE_MIX_S(MixS3);
+#define LMIE_MIX_S(S) do { if (p.bf16) LMIE_MIX_NP(BF16, S); else LMIE_MIX_NP(F16, S); } while (0)
+               if (id == 0) LMIE_MIX_S(MixS0);
+               else if (id == 2) LMIE_MIX_S(MixS2);
+               else if (id == 3) LMIE_MIX_S(MixS3);
                else LMIE_MIX_S(MixS1);
 #undef LMIE_MIX_S
 #undef LMIE_MIX_NP
 #undef LMIE_MIX_NW
 #undef LMIE_MIX
                HIPCHECK(hipGetLastError());
-          }
-          if (!mixed) {
+          } else {
                F64Args a;
                memset(&a, 0, sizeof a);
-               a.Np = Np; a.Kp = Kp; a.Hp = Hp; a.H = H; a.Q = Q; a.N = N;
-               for (int b = 0; b < nb; ++b) a.A[b] = w->A.as<double>() + 4 * plane * b;
+               a.Np = Np; a.Kp = p.Kp; a.Hp = p.Hp; a.H = p.H; a.Q = Q; a.N = N;
+               for (int b = 0; b < p.nb; ++b) a.A[b] = w->A.as<double>() + 4 * (size_t) p.Kp * Np * b;
                a.Bp = w->Bp.as<double>(); a.Bm = w->Bm.as<double>();
                a.ktile = w->ktile32.as<int>();
                a.task = w->order.as<int2>();
-               a.W = w->wrow.as<double>(); a.nP = nP; a.nX = nX;
+               a.W = w->f.as<double>(); a.nP = p.nP; a.nX = p.nX;
                a.part = w->part.as<double>();
                a.save2 = J->save_control == 1 ? w->save2.as<double>() : nullptr;
                a.sst = keep ? w->sst.as<double>() : nullptr;
-               if (launch_angular_f64(a, hx, hm, (unsigned) w->htask.size(), s)) return -1;
+               if (launch_angular_f64(a, p.hx, p.hm, (unsigned) p.task.size(), s)) return -1;
           }
           tm.mark(LMIE_T_ANGULAR, 1);
-          tm.mark(LMIE_T_REDUCE, 0);
-          const int per = nraw * 4 * Q;
-          hipLaunchKernelGGL(reduce_parts, dim3((per + 31) / 32), dim3(256), 0, s, (const double *) w->part.as<double>(),
-                             ntile, nraw, Q, nt ? w->pfraw.as<double>() : w->pf.as<double>());
-          if (nt)
-               hipLaunchKernelGGL(combine_channels, dim3((4 * Q + 255) / 256, nch), dim3(256), 0, s,
-                                  (const double *) w->pfraw.as<double>(), 4 * Q, (const ChComb *) w->comb.as<ChComb>(),
-                                  w->pf.as<double>());
-          HIPCHECK(hipGetLastError());
-          tm.mark(LMIE_T_REDUCE, 1);
-
-          // expansion
+     }
+     // sums over the size tiles and the series sums, then the expansions
+     double *res = w->res.as<double>(), *land = (double *) w->pres.p;
+     const size_t ndot = 4 * (size_t) p.nraw, nx = (size_t) nch * 6 * C;
+     tm.mark(LMIE_T_REDUCE, 0);
+     ReduceArgs ra;
+     reduce_args(w, p, res, ra);
+     hipLaunchKernelGGL(reduce_channels, dim3(ra.gx), dim3(256), 0, s, ra);
+     HIPCHECK(hipGetLastError());
+     tm.mark(LMIE_T_REDUCE, 1);
+     const bool gc = Q > 0 && J->calc_gc && R->gc_raw, lc = Q > 0 && J->calc_lc && R->lc_raw;
+     if (Q > 0) {
           tm.mark(LMIE_T_EXPAND, 0);
-          if (w->E.get(sizeof(double) * (size_t) nch * 12 * Hp) || w->coefs.get(sizeof(double) * (size_t) nch * 6 * C))
-               return -1;
-          for (int gsf = 1; gsf >= 0; --gsf) {
-               double *dst = gsf ? R->gc_raw : R->lc_raw;
-               if (!(gsf ? J->calc_gc : J->calc_lc) || !dst) continue;
-               double *land = (double *) w->pres.p + (gsf ? 0 : (size_t) nch * 6 * C);
-               hipLaunchKernelGGL(expand_rows, dim3(Hp / 64, nch), dim3(64), 0, s, (const double *) w->pf.as<double>(),
-                                  nch, Q, H, Hp, (const double *) w->w.as<double>(), gsf, w->E.as<double>());
-               hipLaunchKernelGGL(expand_coefs, dim3((C + 3) / 4, nch), dim3(256), 0, s, (const double *) w->T.as<double>(),
-                                  (const double *) w->E.as<double>(), H, Hp, C, gsf, w->coefs.as<double>());
-               HIPCHECK(hipGetLastError());
-               HIPCHECK(hipMemcpyAsync(land, w->coefs.p, sizeof(double) * (size_t) nch * 6 * C, hipMemcpyDeviceToHost, s));
-          }
+          for (int gsf = 1; gsf >= 0; --gsf)
+               if (gsf ? gc : lc)
+                    hipLaunchKernelGGL(expand_coefs, dim3((C + 3) / 4, nch), dim3(256), 0, s, (const double *) w->T.as<double>(),
+                                       (const double *) w->pf.as<double>(), (const double *) w->w.as<double>(), Q, p.Hp, C, gsf,
+                                       res + ndot + (gsf ? 0 : nx));
+          HIPCHECK(hipGetLastError());
           tm.mark(LMIE_T_EXPAND, 1);
           if (J->save_control == 1 && R->save2)
                HIPCHECK(hipMemcpyAsync(R->save2, w->save2.p, sizeof(double) * (size_t) 4 * N * Q, hipMemcpyDeviceToHost, s));
-     } else {
-          tm.mark(LMIE_T_REDUCE, 1);
      }
-     HIPCHECK(hipStreamWaitEvent(s, w->join2, 0));   // the series dots
      tm.mark(LMIE_T_TOTAL, 1);
-     // results: through the pinned landing area (the expansions above, the sums here)
-     const double *dots = (const double *) w->pres.p + (size_t) nch * 12 * C;
-     HIPCHECK(hipMemcpyAsync((void *) dots, w->dots.p, sizeof(double) * 4 * nraw, hipMemcpyDeviceToHost, s));
+     // results: one copy into the pinned landing area
+     HIPCHECK(hipMemcpyAsync(land, res, sizeof(double) * (ndot + (lc ? 2 * nx : gc ? nx : 0)), hipMemcpyDeviceToHost, s));
      if (J->save_control == 1 && R->save1)
           for (int q = 0; q < 4; ++q)
                HIPCHECK(hipMemcpyAsync(R->save1 + (size_t) q * N, w->S.as<double>() + (size_t) q * Np,
                                        sizeof(double) * N, hipMemcpyDeviceToHost, s));
      HIPCHECK(hipStreamSynchronize(s));
-     if (Q > 0)
-          for (int gsf = 1; gsf >= 0; --gsf) {
-               double *dst = gsf ? R->gc_raw : R->lc_raw;
-               if ((gsf ? J->calc_gc : J->calc_lc) && dst)
-                    memcpy(dst, (const double *) w->pres.p + (gsf ? 0 : (size_t) nch * 6 * C),
-                           sizeof(double) * (size_t) nch * 6 * C);
-          }
-     for (int q = 0; q < 4; ++q) R->sums[q] = dots[q];
-     for (int c = 1; c < nch; ++c)
-          for (int q = 0; q < 4; ++q) {
-               double v = 0.;
-               for (int t = 0; t < 4; ++t)
-                    if (comb[c].r[t] >= 0) v += comb[c].c[t] * dots[4 * comb[c].r[t] + q];
-               R->sums_ch[4 * (c - 1) + q] = v;
-          }
-     const int ids[] = {LMIE_T_TABLES, LMIE_T_COEFS, LMIE_T_ANGULAR, LMIE_T_REDUCE, LMIE_T_EXPAND, LMIE_T_TOTAL};
-     tm.collect(ids, Q > 0 ? 6 : 2);
+     if (gc) memcpy(R->gc_raw, land + ndot, sizeof(double) * nx);
+     if (lc) memcpy(R->lc_raw, land + ndot + nx, sizeof(double) * nx);
+     unpack_sums(p, land, R);
+     const int ids[] = {LMIE_T_TABLES, LMIE_T_COEFS, LMIE_T_REDUCE, LMIE_T_TOTAL, LMIE_T_ANGULAR, LMIE_T_EXPAND};
+     tm.collect(ids, Q > 0 ? 6 : 4);
      lmie_gpu_host_time(LMIE_T_HOST_PREP, prep_ms);
      w->valid = 1;
-     w->N = N; w->Np = Np; w->Kp = Kp; w->Hp = Hp; w->H = H; w->Q = Q; w->C = C; w->n1max = n1max;
-     w->n2max = 0;
-     for (int i = 0; i < N; ++i) w->n2max = J->n2[i] > w->n2max ? J->n2[i] : w->n2max;
-     w->calc_gc = J->calc_gc; w->calc_lc = J->calc_lc; w->mr = J->mr; w->mi = J->mi;
-     w->mixed = mixed; w->bf16 = bf16; w->Kb = Kb; w->Hb = Hb; w->kt64 = kt64; w->kt128 = kt128;
-     R->precision = mixed ? J->precision : LMIE_PRECISION_FP64;
+     keep_forward(w, J, p);
+     R->precision = p.mixed ? J->precision : LMIE_PRECISION_FP64;
      return 0;
 }
 
@@ -3942,7 +3839,8 @@ int saved_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
      Timer tm{w, g_timing};
      if (w->sw.get(sizeof(double) * (size_t) nch * N) || w->s1.get(sizeof(double) * 4 * (size_t) N) ||
          (Q > 0 && w->s2.get(sizeof(double) * 4 * (size_t) N * Q)) ||
-         w->pf.get(sizeof(double) * (size_t) nch * 4 * (Q > 0 ? Q : 1)) || w->dots.get(sizeof(double) * 4 * nch))
+         w->pf.get(sizeof(double) * (size_t) nch * 4 * (Q > 0 ? Q : 1)) || w->dots.get(sizeof(double) * 4 * nch) ||
+         w->res.get(sizeof(double) * (size_t) nch * 6 * C))
           return -1;
      double *W = w->sw.as<double>();
      HIPCHECK(hipMemcpyAsync(W, J->f, sizeof(double) * N, hipMemcpyHostToDevice, s));
@@ -3956,17 +3854,17 @@ int saved_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
      tm.mark(LMIE_T_TOTAL, 0);
      if (Q > 0) {
           // Gauss rule and expansion tables (as the forward)
-          if (w->mu.get(sizeof(double) * Q) || w->w.get(sizeof(double) * Q) || w->guess.get(sizeof(double) * H))
+          if (w->mu.get(sizeof(double) * Q) || w->w.get(sizeof(double) * Q) || w->sguess.get(sizeof(double) * H) ||
+              w->pin.get(sizeof(double) * H))
                return -1;
-          w->hguess.resize(H > 0 ? H : 1);
-          gauss_guesses(Q, w->hguess.data());
-          HIPCHECK(hipMemcpyAsync(w->guess.p, w->hguess.data(), sizeof(double) * H, hipMemcpyHostToDevice, s));
+          gauss_guesses(Q, (double *) w->pin.p);
+          HIPCHECK(hipMemcpyAsync(w->sguess.p, w->pin.p, sizeof(double) * H, hipMemcpyHostToDevice, s));
           FrontArgs fa;
           memset(&fa, 0, sizeof fa);
           const int planes = J->calc_lc ? 5 : J->calc_gc ? 4 : 0;
           if (planes && w->T.get(sizeof(double) * planes * (size_t) C * Hp)) return -1;
           fa.Q = Q; fa.H = H; fa.Hp = Hp; fa.C = C;
-          fa.guess = w->guess.as<double>(); fa.mu = w->mu.as<double>(); fa.w = w->w.as<double>(); fa.T = w->T.as<double>();
+          fa.guess = w->sguess.as<double>(); fa.mu = w->mu.as<double>(); fa.w = w->w.as<double>(); fa.T = w->T.as<double>();
           fa.plan(planes, 0, true, 0, false);
           if (launch_front(fa, 0, false, s)) return -1;
      }
@@ -3976,17 +3874,14 @@ int saved_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
                         w->pf.as<double>(), w->dots.as<double>());
      HIPCHECK(hipGetLastError());
      if (Q > 0) {
-          if (w->E.get(sizeof(double) * (size_t) nch * 12 * Hp) || w->coefs.get(sizeof(double) * (size_t) nch * 6 * C))
-               return -1;
           for (int gsf = 1; gsf >= 0; --gsf) {
                double *dst = gsf ? R->gc_raw : R->lc_raw;
                if (!(gsf ? J->calc_gc : J->calc_lc) || !dst) continue;
-               hipLaunchKernelGGL(expand_rows, dim3(Hp / 64, nch), dim3(64), 0, s, (const double *) w->pf.as<double>(),
-                                  nch, Q, H, Hp, (const double *) w->w.as<double>(), gsf, w->E.as<double>());
                hipLaunchKernelGGL(expand_coefs, dim3((C + 3) / 4, nch), dim3(256), 0, s, (const double *) w->T.as<double>(),
-                                  (const double *) w->E.as<double>(), H, Hp, C, gsf, w->coefs.as<double>());
+                                  (const double *) w->pf.as<double>(), (const double *) w->w.as<double>(), Q, Hp, C, gsf,
+                                  w->res.as<double>());
                HIPCHECK(hipGetLastError());
-               HIPCHECK(hipMemcpyAsync(dst, w->coefs.p, sizeof(double) * (size_t) nch * 6 * C, hipMemcpyDeviceToHost, s));
+               HIPCHECK(hipMemcpyAsync(dst, w->res.p, sizeof(double) * (size_t) nch * 6 * C, hipMemcpyDeviceToHost, s));
           }
      }
      tm.mark(LMIE_T_TOTAL, 1);
@@ -4002,40 +3897,78 @@ int saved_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
      return 0;
 }
 
-// Mixed reverse contraction: weights, split tables, G, its split operand and
-// U = G A (Uf, [4][Kq][Np]).
-// Buffers, task list and depth uploads of the mixed reverse contraction, before
-// the timed pipeline (host work and transfers the kernels do not wait on).
-int adjoint_mixed_prepare(Workspace *w, hipStream_t s) {
-     const int Np = w->Np, H = w->H, n1max = w->n1max;
-     const int Kq = rup(n1max, 64), Hq = rup(H, KM);
-     if (rup(n1max, KM) > w->Kb * 8) return set_err("internal: split operand depth");
-     if (w->wts.get(sizeof(double) * 8 * (size_t) Hq) || w->scal.get(sizeof(AdjScal)) ||
-         w->L16.get(sizeof(unsigned short) * 4 * (size_t) Hq * Kq) ||
-         w->R16.get(sizeof(unsigned short) * 16 * (size_t) Hq * Kq) ||
-         w->Gf.get(sizeof(float) * 4 * (size_t) Kq * Kq) || w->G16.get(sizeof(unsigned short) * 12 * (size_t) Kq * Kq) ||
-         w->Uf.get(sizeof(float) * 4 * (size_t) Kq * Np))
+// Buffers of a reverse pass (use_u: through G on the 16-bit matrix cores).
+int alloc_reverse(Workspace *w, bool use_u) {
+     const size_t Np = w->Np, Q = w->Q > 0 ? w->Q : 1, C = w->C > 0 ? w->C : 1;
+     const size_t Kq = rup(w->n1max, 64), Hq = rup(w->H > 0 ? w->H : 1, KM);
+     const size_t nck = (w->C + EXA_L - 1) / EXA_L, nch = (w->n2rows - 1 + RCH - 1) / RCH;
+     if (use_u && rup(w->n1max, KM) > w->Kb * 8) return set_err("internal: split operand depth");
+     const size_t nres = 2 * (size_t) w->N + Np / 32;
+     if (w->pfbar.get(sizeof(double) * 4 * Q) || w->gbar.get(sizeof(double) * 12 * C) || w->pin.get(sizeof(double) * 12 * C) ||
+         w->rres.get(sizeof(double) * nres) || w->pres.get(sizeof(double) * nres) ||
+         w->revScan.get(sizeof(double) * REV_ROWS * (nch > 0 ? nch : 1) * Np) ||
+         (w->Q > 0 && w->expart.get(sizeof(double) * 24 * nck * w->Hp)))
           return -1;
-     // (size tile of 128 or 64, order tile of 64) tasks over the XCDs
-     w->ushape = ugemm_waves();
-     const std::vector<int> &kts = w->ushape == 2 ? w->kt64 : w->kt128;
-     std::vector<int2> task;
-     xcd_tasks(kts, [&](int t) { return (kts[t] + 63) / 64; }, tile_group(), task);
-     w->ntask = (int) task.size();
-     if (w->ktile128.get(sizeof(int) * kts.size())) return -1;
-     HIPCHECK(hipMemcpyAsync(w->ktile128.p, kts.data(), sizeof(int) * kts.size(), hipMemcpyHostToDevice, s));
-     if (!task.empty()) {
-          if (w->tasks.get(sizeof(int2) * task.size())) return -1;
-          HIPCHECK(hipMemcpyAsync(w->tasks.p, task.data(), sizeof(int2) * task.size(), hipMemcpyHostToDevice, s));
-     }
+     if (!use_u)
+          return w->fang.get(sizeof(double) * Np) || w->bar.get(sizeof(double) * 4 * (size_t) w->Kp * Np) ? -1 : 0;
+     return w->wts.get(sizeof(double) * 8 * Hq) || w->scal.get(sizeof(AdjScal)) ||
+                    w->L16.get(sizeof(unsigned short) * 4 * Hq * Kq) || w->R16.get(sizeof(unsigned short) * 16 * Hq * Kq) ||
+                    w->Gf.get(sizeof(float) * 4 * Kq * Kq) || w->G16.get(sizeof(unsigned short) * 12 * Kq * Kq) ||
+                    w->Uf.get(sizeof(float) * 4 * Kq * Np) ? -1 : 0;
+}
+
+// The expansion cotangents through the pinned staging area: gc [6][C] at 0,
+// lc at 6 C of gbar.
+int stage_reverse(Workspace *w, const lmie_gpu_adj_in *in, bool use_gc, bool use_lc, hipStream_t s) {
+     const size_t n = 6 * (size_t) w->C, o = use_gc ? 0 : n, e = use_lc ? 2 * n : n;
+     double *h = (double *) w->pin.p;
+     if (!use_gc && !use_lc) return 0;
+     if (use_gc) memcpy(h, in->gc_bar, sizeof(double) * n);
+     if (use_lc) memcpy(h + n, in->lc_bar, sizeof(double) * n);
+     HIPCHECK(hipMemcpyAsync(w->gbar.as<double>() + o, h + o, sizeof(double) * (e - o), hipMemcpyHostToDevice, s));
      return 0;
 }
 
+// Arguments of the per-size reverse sweep.
+void rev_args(const Workspace *w, const lmie_gpu_adj_in *in, bool xbar, bool use_u, RevArgs &r) {
+     const int nch = (w->n2rows - 1 + RCH - 1) / RCH;
+     r.N = w->N; r.Np = w->Np; r.Kp = w->Kp; r.n1max = w->n1max; r.n2rows = w->n2rows; r.nch = nch;
+     r.ft = w->ftab.as<double>();
+     r.x = w->x.as<double>(); r.f = w->f.as<double>();
+     r.n1 = w->n1.as<int>(); r.n2 = w->n2.as<int>(); r.mr = w->mr; r.mi = w->mi; rev_recips(r);
+     r.D = w->chD.as<double>(); r.PC = w->chPC.as<double>(); r.PS = w->chPS.as<double>();
+     r.CB = w->CB.as<double>(); r.S = w->S.as<double>(); r.bar = use_u ? nullptr : w->bar.as<double>();
+     r.Uf = use_u ? w->Uf.as<float>() : nullptr; r.Kq = rup(w->n1max, 64);
+     r.fang = nullptr;
+     r.sb0 = in->sums_bar[0]; r.sb1 = in->sums_bar[1]; r.sb2 = in->sums_bar[2]; r.sb3 = in->sums_bar[3];
+     r.scan = w->revScan.as<double>();
+     r.fbar = w->rres.as<double>();
+     r.xbar = xbar ? r.fbar + w->N : nullptr;
+     r.mbar = r.fbar + 2 * (size_t) w->N;
+}
+
+// A reverse pass's results out of its landing area.
+void unpack_reverse(const Workspace *w, const double *land, lmie_gpu_adj_out *out) {
+     const size_t N = w->N;
+     memcpy(out->f_bar, land, sizeof(double) * N);
+     if (out->x_bar) memcpy(out->x_bar, land + N, sizeof(double) * N);
+     double mr = 0., mi = 0.;
+     for (int b = 0; b < w->Np / 64; ++b) {
+          mr += land[2 * N + 2 * b];
+          mi += land[2 * N + 2 * b + 1];
+     }
+     // m = mr - i mi: dL/dmr = Re(mbar), dL/dmi = -Im(mbar)
+     out->m_bar[0] = mr;
+     out->m_bar[1] = -mi;
+}
+
+// Mixed reverse contraction: weights, split tables, G, its split operand and
+// U = G A (Uf, [4][Kq][Np]).
 int adjoint_mixed_angular(Workspace *w, hipStream_t s, Timer &tm) {
      const int Np = w->Np, H = w->H, Q = w->Q, n1max = w->n1max;
      const int Kq = rup(n1max, 64), Hq = rup(H, KM);
      const int shape = w->ushape;
-     const unsigned ntask = (unsigned) w->ntask;
+     const unsigned ntask = (unsigned) w->rtask.size();
      if (ntask == 0) {
           HIPCHECK(hipMemsetAsync(w->Uf.p, 0, sizeof(float) * 4 * (size_t) Kq * Np, s));
           return 0;
@@ -4079,35 +4012,17 @@ int adjoint_impl(Workspace *w, const lmie_gpu_adj_in *in, lmie_gpu_adj_out *out)
      const int N = w->N, Np = w->Np, Kp = w->Kp, Hp = w->Hp, H = w->H, Q = w->Q, C = w->C;
      hipStream_t s = w->stream;
      Timer tm{w, g_timing};
-     if (w->pfbar.get(sizeof(double) * 4 * (size_t) (Q > 0 ? Q : 1)) || w->fang.get(sizeof(double) * Np) ||
-         w->mbar.get(sizeof(double) * 2 * Np) || w->fbar.get(sizeof(double) * 2 * Np) ||
-         w->gbar.get(sizeof(double) * 12 * (size_t) (C > 0 ? C : 1)) ||
-         w->bar.get(sizeof(double) * 4 * (size_t) Kp * Np))
-          return -1;
-     const int use_gc = in->gc_bar && w->calc_gc, use_lc = in->lc_bar && w->calc_lc;
-     const int use_u = w->mixed && Q > 0 && (use_gc || use_lc);
-     // the cotangent inputs and the contraction's task list go to the device
-     // before the timed pipeline
-     if (use_u && adjoint_mixed_prepare(w, s)) return -1;
-     {
-          // the m-cotangent sums at the end of the pass
-          DotJob jobs[2] = {{nullptr, w->mbar.as<double>(), nullptr, nullptr},
-                            {nullptr, w->mbar.as<double>() + Np, nullptr, nullptr}};
-          if (w->dotjobs.get(sizeof(jobs)) || w->dots.get(sizeof(double) * 2) ||
-              w->pres.get(sizeof(double) * (2 + 2 * (size_t) N)))
-               return -1;
-          HIPCHECK(hipMemcpyAsync(w->dotjobs.p, jobs, sizeof(jobs), hipMemcpyHostToDevice, s));
-     }
+     const int use_gc = in->gc_bar && w->calc_gc && Q > 0, use_lc = in->lc_bar && w->calc_lc && Q > 0;
+     const int use_u = w->mixed && (use_gc || use_lc);
+     // the cotangents go to the device before the timed pipeline
+     if (alloc_reverse(w, use_u) || stage_reverse(w, in, use_gc, use_lc, s)) return -1;
      double *g = w->gbar.as<double>();
-     if (Q > 0 && use_gc) HIPCHECK(hipMemcpyAsync(g, in->gc_bar, sizeof(double) * 6 * C, hipMemcpyHostToDevice, s));
-     if (Q > 0 && use_lc)
-          HIPCHECK(hipMemcpyAsync(g + 6 * C, in->lc_bar, sizeof(double) * 6 * C, hipMemcpyHostToDevice, s));
+     RevArgs r;
+     rev_args(w, in, out->x_bar != nullptr, use_u, r);
      tm.mark(LMIE_T_TOTAL, 0);
-     HIPCHECK(hipMemsetAsync(w->fang.p, 0, sizeof(double) * Np, s));
      if (Q > 0 && (use_gc || use_lc)) {
           tm.mark(LMIE_T_ADJ_ANGULAR, 0);
           const int nck = (C + EXA_L - 1) / EXA_L;
-          if (w->expart.get(sizeof(double) * 24 * (size_t) nck * Hp)) return -1;
           hipLaunchKernelGGL(expand_adjoint_part, dim3(Hp / 64, nck), dim3(64), 0, s, (const double *) w->T.as<double>(),
                              use_gc ? (const double *) g : nullptr, use_lc ? (const double *) (g + 6 * C) : nullptr,
                              H, Hp, C, w->expart.as<double>());
@@ -4120,6 +4035,7 @@ int adjoint_impl(Workspace *w, const lmie_gpu_adj_in *in, lmie_gpu_adj_out *out)
      } else if (Q > 0 && (use_gc || use_lc)) {
           hipLaunchKernelGGL(fbar_angular, dim3((N + 3) / 4), dim3(256), 0, s, (const double *) w->sst.as<double>(),
                              (const double *) w->pfbar.as<double>(), N, H, Hp, Q, w->fang.as<double>());
+          r.fang = w->fang.as<double>();
           AdjArgs aa;
           aa.Np = Np; aa.Kp = Kp; aa.Hp = Hp; aa.H = H; aa.Q = Q;
           aa.sst = w->sst.as<double>(); aa.pfbar = w->pfbar.as<double>();
@@ -4134,47 +4050,18 @@ int adjoint_impl(Workspace *w, const lmie_gpu_adj_in *in, lmie_gpu_adj_out *out)
           tm.mark(LMIE_T_ADJ_ANGULAR, 1);
      }
      tm.mark(LMIE_T_ADJ_COEFS, 0);
-     const int nch = (w->n2rows - 1 + RCH - 1) / RCH;
-     if (w->revScan.get(sizeof(double) * REV_ROWS * (size_t) (nch > 0 ? nch : 1) * Np)) return -1;
-     RevArgs r;
-     r.N = N; r.Np = Np; r.Kp = Kp; r.n1max = w->n1max; r.n2rows = w->n2rows; r.nch = nch;
-     r.ft = w->ftab.as<double>();
-     r.x = w->x.as<double>(); r.f = w->f.as<double>();
-     r.n1 = w->n1.as<int>(); r.n2 = w->n2.as<int>(); r.mr = w->mr; r.mi = w->mi; rev_recips(r);
-     r.D = w->chD.as<double>(); r.PC = w->chPC.as<double>(); r.PS = w->chPS.as<double>();
-     r.CB = w->CB.as<double>(); r.S = w->S.as<double>(); r.bar = w->bar.as<double>();
-     r.Uf = use_u ? w->Uf.as<float>() : nullptr; r.Kq = rup(w->n1max, 64);
-     r.fang = w->fang.as<double>();
-     r.sb0 = in->sums_bar[0]; r.sb1 = in->sums_bar[1]; r.sb2 = in->sums_bar[2]; r.sb3 = in->sums_bar[3];
-     r.scan = w->revScan.as<double>();
-     r.mbar = w->mbar.as<double>(); r.fbar = w->fbar.as<double>();
-     r.xbar = out->x_bar ? w->fbar.as<double>() + Np : nullptr;
-     if (nch > 0) {
-          if (use_u) hipLaunchKernelGGL(rev_orders<true>, dim3(Np / 64, nch), dim3(64), 0, s, r);
-          else hipLaunchKernelGGL(rev_orders<false>, dim3(Np / 64, nch), dim3(64), 0, s, r);
+     if (r.nch > 0) {
+          if (use_u) hipLaunchKernelGGL(rev_orders<true>, dim3(Np / 64, r.nch), dim3(64), 0, s, r);
+          else hipLaunchKernelGGL(rev_orders<false>, dim3(Np / 64, r.nch), dim3(64), 0, s, r);
      }
      hipLaunchKernelGGL(rev_carry, dim3(Np / 64), dim3(64), 0, s, r);
      HIPCHECK(hipGetLastError());
      tm.mark(LMIE_T_ADJ_COEFS, 1);
-     // sum of the per-size m cotangents; results through the pinned landing area
-     {
-          hipLaunchKernelGGL(weighted_dots, dim3(2), dim3(256), 0, s, (const DotJob *) w->dotjobs.as<DotJob>(), Np,
-                             w->dots.as<double>());
-          HIPCHECK(hipGetLastError());
-          double *land = (double *) w->pres.p;
-          HIPCHECK(hipMemcpyAsync(land, w->dots.p, sizeof(double) * 2, hipMemcpyDeviceToHost, s));
-          HIPCHECK(hipMemcpyAsync(land + 2, w->fbar.p, sizeof(double) * N, hipMemcpyDeviceToHost, s));
-          if (out->x_bar)
-               HIPCHECK(hipMemcpyAsync(land + 2 + N, w->fbar.as<double>() + Np, sizeof(double) * N,
-                                       hipMemcpyDeviceToHost, s));
-          tm.mark(LMIE_T_TOTAL, 1);
-          HIPCHECK(hipStreamSynchronize(s));
-          memcpy(out->f_bar, land + 2, sizeof(double) * N);
-          if (out->x_bar) memcpy(out->x_bar, land + 2 + N, sizeof(double) * N);
-          // m = mr - i mi: dL/dmr = Re(mbar), dL/dmi = -Im(mbar)
-          out->m_bar[0] = land[0];
-          out->m_bar[1] = -land[1];
-     }
+     // results through the pinned landing area
+     tm.mark(LMIE_T_TOTAL, 1);
+     HIPCHECK(hipMemcpyAsync(w->pres.p, w->rres.p, sizeof(double) * (2 * (size_t) N + Np / 32), hipMemcpyDeviceToHost, s));
+     HIPCHECK(hipStreamSynchronize(s));
+     unpack_reverse(w, (const double *) w->pres.p, out);
      const int ids[] = {LMIE_T_ADJ_ANGULAR, LMIE_T_ADJ_COEFS, LMIE_T_TOTAL, LMIE_T_ADJ_GEMM};
      tm.collect(ids, use_u ? 4 : 3);
      return 0;
@@ -4212,9 +4099,7 @@ struct FwdCase {
      const lmie_gpu_job *J;
      lmie_gpu_result *R;
      Workspace *w;
-     int N, Np, n1max, Q, C, H, Hp, Kp, Kb, Hb, nt64, n2rows, ng, planes;
-     int nmix;                      // size tiles of the forward contraction's shape
-     std::vector<int2> task;
+     FwdPlan p;
 };
 
 int fused_forward_ok(const lmie_gpu_job *J) {
@@ -4223,149 +4108,74 @@ int fused_forward_ok(const lmie_gpu_job *J) {
             (J->calc_gc || J->calc_lc);
 }
 
-// Buffers and uploads of one case (the mixed value-channel branch of
-// forward_impl); the uploads are queued on up, no kernels.
-int fused_prepare(FwdCase &c, Upload &up) {
-     const lmie_gpu_job *J = c.J;
-     Workspace *w = c.w;
-     const int N = J->n_size, Np = rup(N, 2 * TILE), n1max = J->n1_max, Q = J->n_qang, C = J->n_coef;
-     const int H = Q / 2, Hp = rup(H, TILE), Kp = rup(n1max, 32), Kb = rup(n1max, KM) / 8,
-               Hb = rup(H, 128);
-     if (N <= 0) return set_err("no size points");
-     for (int i = 0; i < N; ++i)
-          if (J->n1[i] > n1max || J->n1[i] < 1 || J->n2[i] < J->n1[i])
-               return set_err("size point %d: order n1 = %d outside [1, %d] (n2 = %d)", i, J->n1[i], n1max, J->n2[i]);
-     w->valid = 0;
-     const int nt32 = Np / 32, nt64 = Np / 64;
-     std::vector<int> n1h(Np, 0), n2h(Np, 0), kt32(nt32), kt64(nt64), kfill(nt64), kt128(nt64 / 2);
-     for (int i = 0; i < N; ++i) { n1h[i] = J->n1[i]; n2h[i] = J->n2[i]; }
-     for (int t = 0; t < nt32; ++t) {
-          int m = 0;
-          for (int i = t * 32; i < t * 32 + 32; ++i) m = std::max(m, n1h[i]);
-          kt32[t] = rup(m, KM);
-     }
-     for (int t = 0; t < nt64; ++t) kt64[t] = std::max(kt32[2 * t], kt32[2 * t + 1]);
-     for (int t = 0; t < nt64 / 2; ++t) kt128[t] = std::max(kt64[2 * t], kt64[2 * t + 1]);
-     for (int t = 0; t < nt64; ++t) kfill[t] = kt128[t / 2];
-     int n2max = 0, kfmax = 0;
-     for (int i = 0; i < N; ++i) n2max = std::max(n2max, J->n2[i]);
-     for (int t = 0; t < nt64; ++t) kfmax = std::max(kfmax, kfill[t]);
-     const int n2rows = n2max + 1, ng = kfmax / 8, planes = J->calc_lc ? 5 : 4;
-     if (w->x.get(sizeof(double) * Np) || w->f.get(sizeof(double) * Np) || w->n1.get(sizeof(int) * Np) ||
-         w->n2.get(sizeof(int) * Np) || w->kfill.get(sizeof(int) * nt64) || w->ktile32.get(sizeof(int) * nt32) ||
-         w->ktile64.get(sizeof(int) * nt64) || w->sx.get(sizeof(double) * Np) || w->cx.get(sizeof(double) * Np) ||
-         w->guess.get(sizeof(double) * H) || w->mu.get(sizeof(double) * Q) || w->w.get(sizeof(double) * Q) ||
-         w->T.get(sizeof(double) * planes * (size_t) C * Hp) ||
-         w->B16.get(sizeof(unsigned short) * B16_PLANES * (size_t) Kb * Hb * 8) || w->S.get(sizeof(double) * 4 * Np) ||
-         w->A16.get(sizeof(unsigned short) * 8 * (size_t) Kb * Np * 8) || w->CB.get(sizeof(double) * 2 * Np) ||
-         w->chD.get(sizeof(double) * 2 * (size_t) n2rows * Np) ||
-         w->chPC.get(sizeof(double) * 2 * (size_t) (n1max + 1) * Np) || w->chPS.get(sizeof(double) * Np) ||
-         w->chPart.get(sizeof(double) * 5 * (size_t) (ng > 0 ? ng : 1) * Np) ||
-         w->ftab.get(sizeof(double) * FT_ROWS * (size_t) (n1max + 2)) || w->dotjobs.get(sizeof(DotJob) * 4) ||
-         w->dots.get(sizeof(double) * 4) || w->pf.get(sizeof(double) * 4 * (size_t) Q) ||
-         w->part.get(sizeof(double) * (size_t) (Np / 32) * 4 * Q) || w->E.get(sizeof(double) * 12 * (size_t) Hp) ||
-         w->coefs.get(sizeof(double) * 12 * (size_t) C))
-          return -1;
-     // x, f zero-padded to Np; sin x, cos x from the host C library (padding 0, 1)
-     w->hsc.assign(4 * (size_t) Np, 0.);
-     double *hx = w->hsc.data(), *hf = hx + Np, *hs = hf + Np, *hc = hs + Np;
-     for (int i = 0; i < Np; ++i) {
-          hx[i] = i < N ? J->x[i] : 0.;
-          hf[i] = i < N ? J->f[i] : 0.;
-          hs[i] = i < N ? (J->sx ? J->sx[i] : sin(J->x[i])) : 0.;
-          hc[i] = i < N ? (J->cx ? J->cx[i] : cos(J->x[i])) : 1.;
-     }
-     w->hguess.resize(H);
-     gauss_guesses(Q, w->hguess.data());
-     DotJob jobs[4];
-     for (int q = 0; q < 4; ++q) jobs[q] = DotJob{w->f.as<double>(), w->S.as<double>() + (size_t) q * Np, nullptr, nullptr};
-     if (up.add(w->x.p, hx, sizeof(double) * Np) || up.add(w->f.p, hf, sizeof(double) * Np) ||
-         up.add(w->sx.p, hs, sizeof(double) * Np) || up.add(w->cx.p, hc, sizeof(double) * Np) ||
-         up.add(w->n1.p, n1h.data(), sizeof(int) * Np) || up.add(w->n2.p, n2h.data(), sizeof(int) * Np) ||
-         up.add(w->kfill.p, kfill.data(), sizeof(int) * nt64) || up.add(w->ktile32.p, kt32.data(), sizeof(int) * nt32) ||
-         up.add(w->ktile64.p, kt64.data(), sizeof(int) * nt64) ||
-         up.add(w->guess.p, w->hguess.data(), sizeof(double) * H) || up.add(w->dotjobs.p, jobs, sizeof(jobs)))
-          return -1;
-     const MixShapeInfo ms = mix_shape();
-     xcd_tasks(ms.tm == 64 ? kt64 : kt32, [&](int) { return (H + ms.tn - 1) / ms.tn; }, mix_group(), c.task);
-     c.nmix = Np / ms.tm;
-     c.N = N; c.Np = Np; c.n1max = n1max; c.Q = Q; c.C = C; c.H = H; c.Hp = Hp; c.Kp = Kp; c.Kb = Kb; c.Hb = Hb;
-     c.nt64 = nt64; c.n2rows = n2rows; c.ng = ng; c.planes = planes;
-     w->N = N; w->Np = Np; w->Kp = Kp; w->Hp = Hp; w->H = H; w->Q = Q; w->C = C; w->n1max = n1max;
-     w->n2max = n2max; w->calc_gc = J->calc_gc; w->calc_lc = J->calc_lc; w->mr = J->mr; w->mi = J->mi;
-     w->mixed = 1; w->bf16 = J->precision == LMIE_PRECISION_MIXED_BF16; w->Kb = Kb; w->Hb = Hb;
-     w->kt64 = kt64; w->kt128 = kt128; w->n2rows = n2rows; w->ng = ng;
+// Sends a batch's per-case arguments (from pinned memory) and gives their
+// device address.
+int send_args(Workspace *L, const std::vector<unsigned char> &h, hipStream_t s, unsigned char **d) {
+     if (L->bargs.get(h.size()) || L->pargs.get(h.size())) return -1;
+     memcpy(L->pargs.p, h.data(), h.size());
+     HIPCHECK(hipMemcpyAsync(L->bargs.p, L->pargs.p, h.size(), hipMemcpyHostToDevice, s));
+     *d = L->bargs.as<unsigned char>();
      return 0;
 }
 
-// One launch per kernel over the prepared cases, on the streams of workspace L.
+// Buffers and inputs of one case, sent on its own stream; no kernels.
+int fused_prepare(FwdCase &c) {
+     return plan_forward(c.J, c.p) || alloc_forward(c.w, c.J, c.p) || stage_forward(c.w, c.J, c.p, true, c.w->stream) ? -1 : 0;
+}
+
+// A case's results out of its landing area: the series sums, then the
+// expansions.
+void fused_unpack(const FwdCase &c) {
+     const double *land = (const double *) c.w->pres.p;
+     const size_t n = 6 * (size_t) c.p.C;
+     unpack_sums(c.p, land, c.R);
+     if (c.J->calc_gc && c.R->gc_raw) memcpy(c.R->gc_raw, land + 4, sizeof(double) * n);
+     if (c.J->calc_lc && c.R->lc_raw) memcpy(c.R->lc_raw, land + 4 + n, sizeof(double) * n);
+}
+
+// One launch per kernel over the prepared cases, on the stream of workspace L.
 template <class E>
-int fused_launch(std::vector<FwdCase> &cs, Upload &up, Workspace *L) {
+int fused_launch(std::vector<FwdCase *> &cs, Workspace *L) {
      hipStream_t s = L->stream;
-     if (up.flush(L->bup, L->pup, s)) return -1;
      const unsigned n = (unsigned) cs.size();
      std::vector<FrontArgs> fronts(n);
      std::vector<mie_terms_B> terms(n);
      std::vector<mie_sums_B> sums(n);
-     std::vector<weighted_dots_B> dots(n);
      std::vector<Mix2Args> mix(n);
-     std::vector<reduce_parts_B> red(n);
-     std::vector<expand_rows_B> rows[2];
+     std::vector<ReduceArgs> red(n);
      std::vector<expand_coefs_B> coefs[2];
      std::vector<int2> task;
+     std::vector<CopyJob> out(n);
      for (unsigned k = 0; k < n; ++k) {
-          const FwdCase &c = cs[k];
+          const FwdCase &c = *cs[k];
+          const FwdPlan &p = c.p;
           Workspace *w = c.w;
-          ChainArgs ca;
-          ca.N = c.N; ca.Np = c.Np; ca.n1max = c.n1max; ca.n2rows = c.n2rows;
-          ca.x = w->x.as<double>(); ca.sx = w->sx.as<double>(); ca.cx = w->cx.as<double>();
-          ca.n1 = w->n1.as<int>(); ca.n2 = w->n2.as<int>(); ca.mr = c.J->mr; ca.mi = c.J->mi;
-          ca.d_all = 1; ca.D = w->chD.as<double>(); ca.PC = w->chPC.as<double>(); ca.PS = w->chPS.as<double>();
-          ca.Dz = ca.PQ = nullptr;
-          FrontArgs &fa = fronts[k];
-          memset(&fa, 0, sizeof fa);
-          fa.Q = c.Q; fa.H = c.H; fa.Hp = c.Hp; fa.C = c.C; fa.n1max = c.n1max; fa.Kp = c.Kp; fa.Kb = c.Kb; fa.Hb = c.Hb;
-          fa.guess = w->guess.as<double>(); fa.mu = w->mu.as<double>(); fa.w = w->w.as<double>();
-          fa.T = w->T.as<double>(); fa.B16 = w->B16.as<unsigned short>(); fa.ft = w->ftab.as<double>(); fa.ch = ca;
-          fa.plan(c.planes, 2, true, c.Np / 64, true);
-          TermArgs ta;
-          ta.N = c.N; ta.Np = c.Np; ta.n1max = c.n1max; ta.n2rows = c.n2rows; ta.Kp = c.Kp; ta.Kb = c.Kb; ta.ng = c.ng;
-          ta.ft = w->ftab.as<double>(); ta.x = w->x.as<double>(); ta.n1 = w->n1.as<int>();
-          ta.kfill = w->kfill.as<int>(); ta.mr = c.J->mr; ta.mi = c.J->mi; ta.D = w->chD.as<double>();
-          ta.PC = w->chPC.as<double>(); ta.PS = w->chPS.as<double>(); ta.A = nullptr; ta.A16 = w->A16.as<unsigned short>();
-          ta.part = w->chPart.as<double>();
-          terms[k] = mie_terms_B{ta, (unsigned) c.Np / 64, (unsigned) c.ng};
-          sums[k] = mie_sums_B{w->chPart.as<double>(), c.N, c.Np, c.ng, w->n1.as<int>(), w->S.as<double>(),
-                               w->CB.as<double>(), (unsigned) (c.Np + 31) / 32, 1};
-          dots[k] = weighted_dots_B{w->dotjobs.as<DotJob>(), c.Np, w->dots.as<double>(), 4, 1};
-          Mix2Args &m = mix[k];
-          memset(&m, 0, sizeof m);
-          m.Np = c.Np; m.Kb = c.Kb; m.Hb = c.Hb; m.H = c.H; m.Q = c.Q;
-          m.A16 = w->A16.as<unsigned short>(); m.B16 = w->B16.as<unsigned short>();
-          m.ktile = c.nmix == c.Np / 64 ? w->ktile64.as<int>() : w->ktile32.as<int>();
-          m.task = nullptr; m.W[0] = w->f.as<double>();
-          m.part = w->part.as<double>();
-          for (const int2 &t : c.task)
+          front_args(w, c.J, p, fronts[k]);
+          term_args(w, c.J, p, terms[k].p);
+          terms[k].gx = (unsigned) p.Np / 64;
+          terms[k].gy = (unsigned) p.ng;
+          sums[k] = mie_sums_B{w->chPart.as<double>(), p.N, p.Np, p.ng, w->n1.as<int>(), w->S.as<double>(),
+                               w->CB.as<double>(), (unsigned) (p.Np + 31) / 32, 1};
+          mix_args(w, p, mix[k]);
+          mix[k].task = nullptr;
+          for (const int2 &t : p.task)
                task.push_back(make_int2(t.x, ((t.x < 0 ? 0 : t.y) & 0xffff) | (int) (k << 16)));
-          red[k] = reduce_parts_B{w->part.as<double>(), c.nmix, 1, c.Q, w->pf.as<double>(),
-                                  (unsigned) (4 * c.Q + 31) / 32, 1};
+          double *res = w->res.as<double>();
+          const size_t nx = 6 * (size_t) p.C;
+          reduce_args(w, p, res, red[k]);
           for (int gs = 0; gs < 2; ++gs) {
                const unsigned on = (gs ? c.J->calc_gc : c.J->calc_lc) ? 1u : 0u;
-               rows[gs].push_back(expand_rows_B{w->pf.as<double>(), 1, c.Q, c.H, c.Hp, w->w.as<double>(), gs,
-                                                w->E.as<double>(), (unsigned) c.Hp / 64, on});
-               // generalized spherical into coefs[0 .. 6C), Legendre into [6C .. 12C)
-               coefs[gs].push_back(expand_coefs_B{w->T.as<double>(), w->E.as<double>(), c.H, c.Hp, c.C, gs,
-                                                  w->coefs.as<double>() + (gs ? 0 : 6 * (size_t) c.C),
-                                                  (unsigned) (c.C + 3) / 4, on});
+               coefs[gs].push_back(expand_coefs_B{w->T.as<double>(), w->pf.as<double>(), w->w.as<double>(), p.Q, p.Hp, p.C, gs,
+                                                  res + 4 + (gs ? 0 : nx), (unsigned) (p.C + 3) / 4, on});
           }
+          out[k] = CopyJob{res, (double *) w->pres.p, 4 + (c.J->calc_lc ? 2 * nx : nx)};
      }
      BatchBlob b;
-     const size_t o_front = b.add(fronts), o_terms = b.add(terms), o_sums = b.add(sums), o_dots = b.add(dots),
-                  o_mix = b.add(mix), o_task = b.add(task), o_red = b.add(red), o_rows0 = b.add(rows[0]),
-                  o_rows1 = b.add(rows[1]), o_coefs0 = b.add(coefs[0]), o_coefs1 = b.add(coefs[1]);
-     if (L->bargs.get(b.h.size())) return -1;
-     unsigned char *d = L->bargs.as<unsigned char>();
-     HIPCHECK(hipMemcpyAsync(d, b.h.data(), b.h.size(), hipMemcpyHostToDevice, s));
+     const size_t o_front = b.add(fronts), o_terms = b.add(terms), o_sums = b.add(sums),
+                  o_mix = b.add(mix), o_task = b.add(task), o_red = b.add(red),
+                  o_coefs0 = b.add(coefs[0]), o_coefs1 = b.add(coefs[1]), o_out = b.add(out);
+     unsigned char *d;
+     if (send_args(L, b.h, s, &d)) return -1;
 #define LMIE_B(T, off) ((const T *) (d + (off)))
      hipLaunchKernelGGL((front_b<std::is_same<E, F16>::value ? 2 : 3>), dim3(max_g(fronts, &FrontArgs::e_ft), 1, n), dim3(64),
                         0, s, LMIE_B(FrontArgs, o_front));
@@ -4375,7 +4185,6 @@ int fused_launch(std::vector<FwdCase> &cs, Upload &up, Workspace *L) {
                              LMIE_B(mie_terms_B, o_terms));
      hipLaunchKernelGGL(mie_sums_b, dim3(max_g(sums, &mie_sums_B::gx), 1, n), dim3(256), 0, s,
                         LMIE_B(mie_sums_B, o_sums));
-     hipLaunchKernelGGL(weighted_dots_b, dim3(4, 1, n), dim3(256), 0, s, LMIE_B(weighted_dots_B, o_dots));
      // contraction, one task list for all cases
      if (!task.empty())
      {
@@ -4388,33 +4197,21 @@ int fused_launch(std::vector<FwdCase> &cs, Upload &up, Workspace *L) {
           else { if (np == 3) LMIE_MIXB(3, MixS1); else LMIE_MIXB(5, MixS1); }
 #undef LMIE_MIXB
      }
-     hipLaunchKernelGGL(reduce_parts_b, dim3(max_g(red, &reduce_parts_B::gx), 1, n), dim3(256), 0, s,
-                        LMIE_B(reduce_parts_B, o_red));
+     hipLaunchKernelGGL(reduce_channels_b, dim3(max_g(red, &ReduceArgs::gx), 1, n), dim3(256), 0, s,
+                        LMIE_B(ReduceArgs, o_red));
      // expansion: generalized spherical, then Legendre
      for (int gs = 1; gs >= 0; --gs) {
-          if (max_g(rows[gs], &expand_rows_B::gy) == 0) continue;
-          hipLaunchKernelGGL(expand_rows_b, dim3(max_g(rows[gs], &expand_rows_B::gx), 1, n), dim3(64), 0, s,
-                             LMIE_B(expand_rows_B, gs ? o_rows1 : o_rows0));
+          if (max_g(coefs[gs], &expand_coefs_B::gy) == 0) continue;
           hipLaunchKernelGGL(expand_coefs_b, dim3(max_g(coefs[gs], &expand_coefs_B::gx), 1, n), dim3(256), 0, s,
                              LMIE_B(expand_coefs_B, gs ? o_coefs1 : o_coefs0));
-          HIPCHECK(hipGetLastError());
      }
+     hipLaunchKernelGGL(copy_jobs, dim3(8, n), dim3(256), 0, s, LMIE_B(CopyJob, o_out));
 #undef LMIE_B
      HIPCHECK(hipGetLastError());
-     std::vector<double> hd(4 * (size_t) n);
-     Download dn;
-     for (unsigned k = 0; k < n; ++k) {
-          const FwdCase &c = cs[k];
-          const size_t cb = sizeof(double) * 6 * c.C;
-          if ((c.J->calc_gc && c.R->gc_raw && dn.add(c.R->gc_raw, c.w->coefs.p, cb)) ||
-              (c.J->calc_lc && c.R->lc_raw && dn.add(c.R->lc_raw, c.w->coefs.as<double>() + 6 * (size_t) c.C, cb)) ||
-              dn.add(hd.data() + 4 * k, c.w->dots.p, sizeof(double) * 4))
-               return -1;
-     }
-     if (dn.flush(L->bdown, L->pdown, s)) return -1;
-     for (unsigned k = 0; k < n; ++k) {
-          for (int q = 0; q < 4; ++q) cs[k].R->sums[q] = hd[4 * k + q];
-          cs[k].w->valid = 1;
+     HIPCHECK(hipStreamSynchronize(s));
+     for (FwdCase *c : cs) {
+          keep_forward(c->w, c->J, c->p);
+          c->w->valid = 1;
      }
      return 0;
 }
@@ -4424,59 +4221,30 @@ struct RevCase {
      Workspace *w;
      const lmie_gpu_adj_in *in;
      lmie_gpu_adj_out *out;
-     int nck, Kq, Hq, nch, use_gc, use_lc;
-     std::vector<int2> task;
+     int use_gc, use_lc;
 };
 
 int fused_reverse_ok(Workspace *w, const lmie_gpu_adj_in *in) {
      return w->valid && w->mixed && w->Q > 0 && ((in->gc_bar && w->calc_gc) || (in->lc_bar && w->calc_lc));
 }
 
-// Buffers and uploads of one reverse pass (the mixed branch of adjoint_impl),
-// queued on up.
-int fused_rev_prepare(RevCase &c, Upload &up) {
+// Buffers of one reverse pass (the mixed branch of adjoint_impl) and its
+// cotangents in its pinned staging area.
+int fused_rev_prepare(RevCase &c) {
      Workspace *w = c.w;
-     const int Np = w->Np, Hp = w->Hp, H = w->H, Q = w->Q, C = w->C, n1max = w->n1max;
-     const int Kq = rup(n1max, 64), Hq = rup(H, KM);
-     if (rup(n1max, KM) > w->Kb * 8) return set_err("internal: split operand depth");
      c.use_gc = c.in->gc_bar && w->calc_gc;
      c.use_lc = c.in->lc_bar && w->calc_lc;
-     c.nck = (C + EXA_L - 1) / EXA_L;
-     c.Kq = Kq; c.Hq = Hq;
-     c.nch = (w->n2rows - 1 + RCH - 1) / RCH;
-     const size_t nk = w->kt128.size(), nk2 = nk + (nk & 1);   // whole doubles
-     if (w->pfbar.get(sizeof(double) * 4 * (size_t) Q) || w->fang.get(sizeof(double) * Np) ||
-         w->mbar.get(sizeof(double) * 2 * Np) || w->fbar.get(sizeof(double) * 2 * Np) ||
-         w->gbar.get(sizeof(double) * 12 * (size_t) C) ||
-         w->expart.get(sizeof(double) * 24 * (size_t) c.nck * Hp) || w->wts.get(sizeof(double) * 8 * (size_t) Hq) ||
-         w->scal.get(sizeof(AdjScal)) || w->L16.get(sizeof(unsigned short) * 4 * (size_t) Hq * Kq) ||
-         w->R16.get(sizeof(unsigned short) * 16 * (size_t) Hq * Kq) ||
-         w->Gf.get(sizeof(float) * 4 * (size_t) Kq * Kq) ||
-         w->G16.get(sizeof(unsigned short) * 12 * (size_t) Kq * Kq) ||
-         w->Uf.get(sizeof(float) * 4 * (size_t) Kq * Np) ||
-         w->revScan.get(sizeof(double) * REV_ROWS * (size_t) (c.nch > 0 ? c.nch : 1) * Np) ||
-         w->ktile128.get(sizeof(int) * nk2) || w->dotjobs.get(sizeof(DotJob) * 2) || w->dots.get(sizeof(double) * 2))
-          return -1;
-     double *g = w->gbar.as<double>();
-     std::vector<int> kt(w->kt128);
-     kt.resize(nk2, 0);
-     const std::vector<int> &kts = w->kt128;
-     xcd_tasks(kts, [&](int t) { return (kts[t] + 63) / 64; }, tile_group(), c.task);
-     DotJob jobs[2] = {{nullptr, w->mbar.as<double>(), nullptr, nullptr},
-                       {nullptr, w->mbar.as<double>() + Np, nullptr, nullptr}};
-     if ((c.use_gc && up.add(g, c.in->gc_bar, sizeof(double) * 6 * C)) ||
-         (c.use_lc && up.add(g + 6 * C, c.in->lc_bar, sizeof(double) * 6 * C)) ||
-         up.zero(w->fang.p, sizeof(double) * Np) || up.add(w->ktile128.p, kt.data(), sizeof(int) * nk2) ||
-         (c.task.empty() && up.zero(w->Uf.p, sizeof(float) * 4 * (size_t) Kq * Np)) ||
-         up.add(w->dotjobs.p, jobs, sizeof(jobs)))
-          return -1;
+     if (alloc_reverse(w, true)) return -1;
+     double *h = (double *) w->pin.p;
+     const size_t n = 6 * (size_t) w->C;
+     if (c.use_gc) memcpy(h, c.in->gc_bar, sizeof(double) * n);
+     if (c.use_lc) memcpy(h + n, c.in->lc_bar, sizeof(double) * n);
      return 0;
 }
 
 template <class E>
-int fused_rev_launch(std::vector<RevCase> &cs, Upload &up, Workspace *L) {
+int fused_rev_launch(std::vector<RevCase *> &cs, Workspace *L) {
      hipStream_t s = L->stream;
-     if (up.flush(L->bup, L->pup, s)) return -1;
      const unsigned n = (unsigned) cs.size();
      std::vector<expand_adjoint_part_B> epart(n);
      std::vector<expand_adjoint_fin_B> efin(n);
@@ -4488,53 +4256,50 @@ int fused_rev_launch(std::vector<RevCase> &cs, Upload &up, Workspace *L) {
      std::vector<int2> task;
      std::vector<rev_orders_B> ro(n);
      std::vector<rev_carry_B> rc(n);
-     std::vector<weighted_dots_B> dots(n);
+     std::vector<CopyJob> in(n), out(n);
      for (unsigned k = 0; k < n; ++k) {
-          const RevCase &c = cs[k];
+          const RevCase &c = *cs[k];
           Workspace *w = c.w;
           const int H = w->H, Hp = w->Hp, Q = w->Q, C = w->C, Np = w->Np;
+          const int Kq = rup(w->n1max, 64), Hq = rup(H, KM), nck = (C + EXA_L - 1) / EXA_L;
           const double *g = w->gbar.as<double>();
           AdjScal *sc = w->scal.as<AdjScal>();
+          // cotangents from the case's pinned staging area, results into its
+          // landing area
+          const size_t o = c.use_gc ? 0 : 6 * (size_t) C;
+          in[k] = CopyJob{(const double *) w->pin.p + o, w->gbar.as<double>() + o, (c.use_lc ? 12 * (size_t) C : 6 * (size_t) C) - o};
+          out[k] = CopyJob{w->rres.as<double>(), (double *) w->pres.p, 2 * (size_t) w->N + Np / 32};
           epart[k] = expand_adjoint_part_B{w->T.as<double>(), c.use_gc ? g : nullptr, c.use_lc ? g + 6 * C : nullptr,
-                                           H, Hp, C, w->expart.as<double>(), (unsigned) Hp / 64, (unsigned) c.nck};
-          efin[k] = expand_adjoint_fin_B{w->expart.as<double>(), c.nck, w->w.as<double>(), H, Hp, Q,
+                                           H, Hp, C, w->expart.as<double>(), (unsigned) Hp / 64, (unsigned) nck};
+          efin[k] = expand_adjoint_fin_B{w->expart.as<double>(), nck, w->w.as<double>(), H, Hp, Q,
                                          w->pfbar.as<double>(), (unsigned) (H + EXF_J - 1) / EXF_J, 1};
-          wts[k] = adj_weights_B{w->pfbar.as<double>(), H, c.Hq, Q, w->wts.as<double>(), sc, 1, 1};
-          tabs[k] = adj_tables_B{w->B16.as<unsigned short>(), w->Kb, w->Hb, w->wts.as<double>(), H, c.Hq, c.Kq,
+          wts[k] = adj_weights_B{w->pfbar.as<double>(), H, Hq, Q, w->wts.as<double>(), sc, 1, 1};
+          tabs[k] = adj_tables_B{w->B16.as<unsigned short>(), w->Kb, w->Hb, w->wts.as<double>(), H, Hq, Kq,
                                  w->n1max, w->L16.as<unsigned short>(), w->R16.as<unsigned short>(),
-                                 (unsigned) c.Kq / 64, (unsigned) c.Hq / 8};
-          gb[k] = adj_gbuild_B{w->L16.as<unsigned short>(), w->R16.as<unsigned short>(), c.Hq, c.Kq,
-                               w->Gf.as<float>(), sc, (unsigned) c.Kq / 64, (unsigned) c.Kq / 64};
-          gsp[k] = adj_gsplit_B{w->Gf.as<float>(), sc, c.Kq, w->G16.as<unsigned short>(), (unsigned) c.Kq / 64,
-                                (unsigned) c.Kq / 8};
+                                 (unsigned) Kq / 64, (unsigned) Hq / 8};
+          gb[k] = adj_gbuild_B{w->L16.as<unsigned short>(), w->R16.as<unsigned short>(), Hq, Kq,
+                               w->Gf.as<float>(), sc, (unsigned) Kq / 64, (unsigned) Kq / 64};
+          gsp[k] = adj_gsplit_B{w->Gf.as<float>(), sc, Kq, w->G16.as<unsigned short>(), (unsigned) Kq / 64,
+                                (unsigned) Kq / 8};
           UArgs &u = ua[k];
-          u.Np = Np; u.Kb = w->Kb; u.Kq = c.Kq;
+          u.Np = Np; u.Kb = w->Kb; u.Kq = Kq;
           u.A16 = w->A16.as<unsigned short>(); u.G16 = w->G16.as<unsigned short>();
           u.ktile = w->ktile128.as<int>(); u.task = nullptr; u.sc = sc; u.Uf = w->Uf.as<float>();
-          for (const int2 &t : c.task)
+          for (const int2 &t : w->rtask)
                task.push_back(make_int2(t.x, ((t.x < 0 ? 0 : t.y) & 0xffff) | (int) (k << 16)));
           RevArgs r;
-          r.N = w->N; r.Np = Np; r.Kp = w->Kp; r.n1max = w->n1max; r.n2rows = w->n2rows; r.nch = c.nch;
-          r.ft = w->ftab.as<double>(); r.x = w->x.as<double>(); r.f = w->f.as<double>();
-          r.n1 = w->n1.as<int>(); r.n2 = w->n2.as<int>(); r.mr = w->mr; r.mi = w->mi; rev_recips(r);
-          r.D = w->chD.as<double>(); r.PC = w->chPC.as<double>(); r.PS = w->chPS.as<double>();
-          r.CB = w->CB.as<double>(); r.S = w->S.as<double>(); r.bar = nullptr;   // read only without Uf
-          r.Uf = w->Uf.as<float>(); r.Kq = c.Kq; r.fang = w->fang.as<double>();
-          r.sb0 = c.in->sums_bar[0]; r.sb1 = c.in->sums_bar[1]; r.sb2 = c.in->sums_bar[2]; r.sb3 = c.in->sums_bar[3];
-          r.scan = w->revScan.as<double>(); r.mbar = w->mbar.as<double>(); r.fbar = w->fbar.as<double>();
-          r.xbar = c.out->x_bar ? w->fbar.as<double>() + Np : nullptr;
-          ro[k] = rev_orders_B{r, (unsigned) Np / 64, (unsigned) c.nch};
+          rev_args(w, c.in, c.out->x_bar != nullptr, true, r);
+          ro[k] = rev_orders_B{r, (unsigned) Np / 64, (unsigned) r.nch};
           rc[k] = rev_carry_B{r, (unsigned) Np / 64, 1};
-          dots[k] = weighted_dots_B{w->dotjobs.as<DotJob>(), Np, w->dots.as<double>(), 2, 1};
      }
      BatchBlob b;
      const size_t o_ep = b.add(epart), o_ef = b.add(efin), o_w = b.add(wts), o_t = b.add(tabs), o_gb = b.add(gb),
                   o_gs = b.add(gsp), o_u = b.add(ua), o_task = b.add(task), o_ro = b.add(ro), o_rc = b.add(rc),
-                  o_d = b.add(dots);
-     if (L->bargs.get(b.h.size())) return -1;
-     unsigned char *d = L->bargs.as<unsigned char>();
-     HIPCHECK(hipMemcpyAsync(d, b.h.data(), b.h.size(), hipMemcpyHostToDevice, s));
+                  o_in = b.add(in), o_out = b.add(out);
+     unsigned char *d;
+     if (send_args(L, b.h, s, &d)) return -1;
 #define LMIE_B(T, off) ((const T *) (d + (off)))
+     hipLaunchKernelGGL(copy_jobs, dim3(8, n), dim3(256), 0, s, LMIE_B(CopyJob, o_in));
      hipLaunchKernelGGL(expand_adjoint_part_b, dim3(max_g(epart, &expand_adjoint_part_B::gx),
                                                     max_g(epart, &expand_adjoint_part_B::gy), n),
                         dim3(64), 0, s, LMIE_B(expand_adjoint_part_B, o_ep));
@@ -4556,23 +4321,10 @@ int fused_rev_launch(std::vector<RevCase> &cs, Upload &up, Workspace *L) {
                              LMIE_B(rev_orders_B, o_ro));
      hipLaunchKernelGGL(rev_carry_b, dim3(max_g(rc, &rev_carry_B::gx), 1, n), dim3(64), 0, s,
                         LMIE_B(rev_carry_B, o_rc));
-     hipLaunchKernelGGL(weighted_dots_b, dim3(2, 1, n), dim3(256), 0, s, LMIE_B(weighted_dots_B, o_d));
+     hipLaunchKernelGGL(copy_jobs, dim3(8, n), dim3(256), 0, s, LMIE_B(CopyJob, o_out));
 #undef LMIE_B
      HIPCHECK(hipGetLastError());
-     std::vector<double> mb(2 * (size_t) n);
-     Download dn;
-     for (unsigned k = 0; k < n; ++k)
-          if (dn.add(mb.data() + 2 * k, cs[k].w->dots.p, sizeof(double) * 2) ||
-              dn.add(cs[k].out->f_bar, cs[k].w->fbar.p, sizeof(double) * cs[k].w->N) ||
-              (cs[k].out->x_bar &&
-               dn.add(cs[k].out->x_bar, cs[k].w->fbar.as<double>() + cs[k].w->Np, sizeof(double) * cs[k].w->N)))
-               return -1;
-     if (dn.flush(L->bdown, L->pdown, s)) return -1;
-     for (unsigned k = 0; k < n; ++k) {
-          // m = mr - i mi: dL/dmr = Re(mbar), dL/dmi = -Im(mbar)
-          cs[k].out->m_bar[0] = mb[2 * k];
-          cs[k].out->m_bar[1] = -mb[2 * k + 1];
-     }
+     HIPCHECK(hipStreamSynchronize(s));
      return 0;
 }
 
@@ -4593,17 +4345,15 @@ struct Batch {
      std::vector<std::string> err[2];
      int fused_cases[2] = {0, 0};
      // forward cases prepared by their own threads before they arrive
-     // (buffers, host tables and staged uploads), so the thread that runs
-     // the pass only launches
-     std::vector<char> prepped;
+     // (buffers, host tables and inputs), so the thread that runs the pass
+     // only launches; a case takes its results out of its landing area itself
+     std::vector<char> prepped, done[2];
      std::vector<FwdCase> pre;
-     std::vector<Upload> preup;
      std::vector<int> prerc;
      std::vector<std::string> preerr;
      // the same for the reverse pass
      std::vector<char> rprepped;
      std::vector<RevCase> rpre;
-     std::vector<Upload> rpreup;
      std::vector<int> rprerc;
      std::vector<std::string> rpreerr;
 };
@@ -4625,11 +4375,7 @@ void batch_prepare(Batch *b, int k, const lmie_gpu_job *J, lmie_gpu_result *res)
      if (rc == 0) {
           // the case's inputs go up from here, on its own stream, one pinned
           // copy; the launch waits for the event
-          Upload &up = b->preup[k];
-          up.items.clear();
-          up.h.clear();
-          rc = fused_prepare(c, up);
-          if (rc == 0) rc = up.flush(c.w->finDev, c.w->finPin, c.w->stream);
+          rc = fused_prepare(c);
           if (rc == 0 && hipEventRecord(c.w->uploaded, c.w->stream) != hipSuccess)
                rc = set_err("hipEventRecord failed");
           if (rc) {
@@ -4644,44 +4390,32 @@ void batch_prepare(Batch *b, int k, const lmie_gpu_job *J, lmie_gpu_result *res)
 }
 
 // A reverse case of a fused batch prepared on its own thread, before it
-// arrives (fused_rev_prepare).  Its uploads stay staged on the host: the pass
-// sends those of all cases as one copy (a few tens of KB per case; a copy, a
-// scatter launch and an event per case from every case's thread contend for
-// the runtime).
+// arrives (fused_rev_prepare); the pass reads the cotangents from its pinned
+// staging area.
 void batch_rev_prepare(Batch *b, int k, Workspace *w, const lmie_gpu_adj_in *in, lmie_gpu_adj_out *out) {
      g_err[0] = 0;
      RevCase &c = b->rpre[k];
      c.slot = k; c.w = w; c.in = in; c.out = out;
-     Upload &up = b->rpreup[k];
-     up.items.clear();
-     up.h.clear();
      int rc = use_device(w->device);
-     if (rc == 0) rc = fused_rev_prepare(c, up);
+     if (rc == 0) rc = fused_rev_prepare(c);
      b->rprerc[k] = rc;
      b->rpreerr[k] = rc ? g_err : "";
      b->rprepped[k] = 1;
 }
 
 void batch_run_forward(Batch *b) {
-     std::vector<FwdCase> f16, b16;
-     Upload up16, upb;
-     Workspace *L = nullptr;           // the workspace whose streams launch the batch
+     std::vector<FwdCase *> f16, b16;
+     Workspace *L = nullptr;           // the workspace whose stream launches the batch
      for (int k = 0; k < b->n; ++k) {
           if (!b->in[0][k]) continue;
           const lmie_gpu_job *J = b->job[k];
           g_err[0] = 0;
           int rc;
-          if (b->prepped[k] && (b->prerc[k] || J->device != b->device)) {
-               // prepared on another device, or the preparation failed
-               if (b->prerc[k] == 0) {
-                    ws_release(b->pre[k].w);
-                    rc = forward_one(J, b->res[k]);
-               } else {
-                    b->rc[0][k] = b->prerc[k];
-                    b->err[0][k] = b->preerr[k];
-                    continue;
-               }
-          } else if (b->prepped[k]) {
+          if (b->prepped[k] && b->prerc[k]) {
+               b->rc[0][k] = b->prerc[k];
+               b->err[0][k] = b->preerr[k];
+               continue;
+          } else if (b->prepped[k] && J->device == b->device) {
                // its inputs are on the way on its own stream (batch_prepare)
                FwdCase &c = b->pre[k];
                if (!L) L = c.w;
@@ -4693,46 +4427,34 @@ void batch_run_forward(Batch *b) {
                     continue;
                }
                const bool bf = J->precision == LMIE_PRECISION_MIXED_BF16;
-               (bf ? b16 : f16).push_back(std::move(c));
+               (bf ? b16 : f16).push_back(&c);
                continue;
-          } else if (!fused_forward_ok(J) || J->device != b->device) {
-               rc = forward_one(J, b->res[k]);
-          } else {
-               FwdCase c;
-               c.slot = k; c.J = J; c.R = b->res[k]; c.w = nullptr;
-               rc = ws_acquire_home(J->device, k, &c.w);
-               if (rc == 0) {
-                    if (!L) L = c.w;
-                    const bool bf = J->precision == LMIE_PRECISION_MIXED_BF16;
-                    Upload &up = bf ? upb : up16;
-                    const size_t ni = up.items.size(), nb = up.h.size();
-                    rc = fused_prepare(c, up);
-                    if (rc == 0) {
-                         (bf ? b16 : f16).push_back(std::move(c));
-                         continue;
-                    }
-                    up.rewind(ni, nb);
-                    if (c.w != L) ws_release(c.w);
-               }
           }
+          // another device's case, or one that the fused kernels do not cover
+          if (b->prepped[k]) {
+               (void) hipStreamSynchronize(b->pre[k].w->stream);
+               ws_release(b->pre[k].w);
+          }
+          rc = forward_one(J, b->res[k]);
           b->rc[0][k] = rc;
           b->err[0][k] = rc ? g_err : "";
      }
      if (!L) return;
      bool L_kept = false;
      for (int t = 0; t < 2; ++t) {     // one arithmetic type per launch
-          std::vector<FwdCase> &v = t ? b16 : f16;
+          std::vector<FwdCase *> &v = t ? b16 : f16;
           if (v.empty()) continue;
           g_err[0] = 0;
-          const int rc = t ? fused_launch<BF16>(v, upb, L) : fused_launch<F16>(v, up16, L);
+          const int rc = t ? fused_launch<BF16>(v, L) : fused_launch<F16>(v, L);
           if (rc) (void) hipStreamSynchronize(L->stream);
-          for (FwdCase &c : v) {
-               b->rc[0][c.slot] = rc;
-               b->err[0][c.slot] = rc ? g_err : "";
-               c.R->state = rc ? nullptr : c.w;
-               c.R->precision = c.J->precision;
-               if (rc == 0 && c.w == L) L_kept = true;
-               if (rc && c.w != L) ws_release(c.w);
+          for (FwdCase *c : v) {
+               b->rc[0][c->slot] = rc;
+               b->err[0][c->slot] = rc ? g_err : "";
+               b->done[0][c->slot] = rc == 0;
+               c->R->state = rc ? nullptr : c->w;
+               c->R->precision = c->J->precision;
+               if (rc == 0 && c->w == L) L_kept = true;
+               if (rc && c->w != L) ws_release(c->w);
                b->fused_cases[0]++;
           }
      }
@@ -4740,66 +4462,35 @@ void batch_run_forward(Batch *b) {
 }
 
 void batch_run_reverse(Batch *b) {
-     std::vector<RevCase> f16, b16;
-     Upload up16, upb;
-     std::vector<const Upload *> staged;
+     std::vector<RevCase *> f16, b16;
      Workspace *L = nullptr;
      for (int k = 0; k < b->n; ++k) {
           if (!b->in[1][k]) continue;
           Workspace *w = b->ws[k];
           g_err[0] = 0;
-          int rc;
           if (b->rprepped[k] && b->rprerc[k]) {
                b->rc[1][k] = b->rprerc[k];
                b->err[1][k] = b->rpreerr[k];
                continue;
           } else if (b->rprepped[k] && w->device == b->device) {
-               // its uploads are staged (batch_rev_prepare)
-               RevCase &c = b->rpre[k];
                if (!L) L = w;
-               staged.push_back(&b->rpreup[k]);
-               (w->bf16 ? b16 : f16).push_back(std::move(c));
+               (w->bf16 ? b16 : f16).push_back(&b->rpre[k]);
                continue;
-          } else if (!fused_reverse_ok(w, b->ain[k]) || w->device != b->device) {
-               rc = adjoint_one(w, b->ain[k], b->aout[k]);
-          } else {
-               RevCase c;
-               c.slot = k; c.w = w; c.in = b->ain[k]; c.out = b->aout[k];
-               if (!L) L = w;
-               Upload &up = w->bf16 ? upb : up16;
-               const size_t ni = up.items.size(), nb = up.h.size();
-               rc = fused_rev_prepare(c, up);
-               if (rc == 0) {
-                    (w->bf16 ? b16 : f16).push_back(std::move(c));
-                    continue;
-               }
-               up.rewind(ni, nb);
           }
+          const int rc = adjoint_one(w, b->ain[k], b->aout[k]);
           b->rc[1][k] = rc;
           b->err[1][k] = rc ? g_err : "";
      }
-     // every case's uploads in one copy on the launching stream, before
-     // either arithmetic's launches
-     int up_rc = 0;
-     if (L) {
-          g_err[0] = 0;
-          staged.push_back(&up16);
-          staged.push_back(&upb);
-          up_rc = Upload::flush_all(staged, L->bup, L->pup, L->stream);
-          up16.items.clear(); up16.h.clear();
-          upb.items.clear(); upb.h.clear();
-     }
-     const std::string up_err = up_rc ? g_err : "";
      for (int t = 0; t < 2; ++t) {
-          std::vector<RevCase> &v = t ? b16 : f16;
+          std::vector<RevCase *> &v = t ? b16 : f16;
           if (v.empty()) continue;
           g_err[0] = 0;
-          if (up_rc) snprintf(g_err, sizeof g_err, "%s", up_err.c_str());
-          const int rc = up_rc ? up_rc : t ? fused_rev_launch<BF16>(v, upb, L) : fused_rev_launch<F16>(v, up16, L);
+          const int rc = t ? fused_rev_launch<BF16>(v, L) : fused_rev_launch<F16>(v, L);
           if (rc) (void) hipStreamSynchronize(L->stream);
-          for (RevCase &c : v) {
-               b->rc[1][c.slot] = rc;
-               b->err[1][c.slot] = rc ? g_err : "";
+          for (RevCase *c : v) {
+               b->rc[1][c->slot] = rc;
+               b->err[1][c->slot] = rc ? g_err : "";
+               b->done[1][c->slot] = rc == 0;
                b->fused_cases[1]++;
           }
      }
@@ -4844,9 +4535,11 @@ int batch_arrive(int p, const lmie_gpu_job *job, lmie_gpu_result *res, Workspace
      t_phase = p + 1;
      batch_fire(b, p);
      while (b->state[p] != 2) pthread_cond_wait(&b->cv, &b->mu);
-     const int rc = b->rc[p][k];
+     const int rc = b->rc[p][k], done = b->done[p][k];
      const std::string e = b->err[p][k];
      pthread_mutex_unlock(&b->mu);
+     if (done && p == 0) fused_unpack(b->pre[k]);
+     if (done && p == 1) unpack_reverse(w, (const double *) w->pres.p, aout);
      if (rc) return set_err("%s", e.c_str());
      return 0;
 }
@@ -4977,12 +4670,12 @@ void *lmie_gpu_batch_open(int n_case) {
      b->aout.assign(n_case, nullptr);
      b->prepped.assign(n_case, 0);
      b->pre.resize(n_case);
-     b->preup.resize(n_case);
+     b->done[0].assign(n_case, 0);
+     b->done[1].assign(n_case, 0);
      b->prerc.assign(n_case, 0);
      b->preerr.assign(n_case, std::string());
      b->rprepped.assign(n_case, 0);
      b->rpre.resize(n_case);
-     b->rpreup.resize(n_case);
      b->rprerc.assign(n_case, 0);
      b->rpreerr.assign(n_case, std::string());
      return b;
@@ -5031,7 +4724,6 @@ int forward_one(const lmie_gpu_job *job, lmie_gpu_result *res) {
      res->precision = LMIE_PRECISION_FP64;   /* the re-weighting of save_control 2 is FP64 */
      int rc = job->save_control == 2 ? saved_impl(job, res, w) : forward_impl(job, res, w);
      if (rc) {
-          (void) hipStreamSynchronize(w->side);
           (void) hipStreamSynchronize(w->stream);
      }
      if (rc == 0 && job->keep) {
