@@ -880,11 +880,28 @@ static int user_angles(int n_coef, int n_angles, int nd, int ld, double **xc, do
                        double *theta, double **pf, double ***pf_l, int gsf, int device) {
      double dth = 180. / (n_angles - 1);
      for (int i = 0; i < n_angles; ++i) theta[i] = i * dth;
-     if (lmie_gpu_phase_func(1, n_coef, ld, xc[0], n_angles, theta, pf[0], gsf, device))
-          return fail("lmie_gpu_phase_func", lmie_gpu_last_error());
-     if (nd > 0 && lmie_gpu_phase_func(nd, n_coef, ld, xc_l[0][0], n_angles, theta, pf_l[0][0], gsf, device))
-          return fail("lmie_gpu_phase_func", lmie_gpu_last_error());
-     return 0;
+     if (nd <= 0) {
+          if (lmie_gpu_phase_func(1, n_coef, ld, xc[0], n_angles, theta, pf[0], gsf, device))
+               return fail("lmie_gpu_phase_func", lmie_gpu_last_error());
+          return 0;
+     }
+     /* the value's and the tangents' sets in one device call */
+     const size_t rows = (size_t) 6 * (1 + nd);
+     double *x = vec(rows * n_coef), *o = vec(rows * n_angles);
+     int rc = !x || !o ? fail("phase function", "out of memory") : 0;
+     if (!rc) {
+          for (size_t r = 0; r < rows; ++r)
+               memcpy(x + r * n_coef, r < 6 ? xc[0] + r * ld : xc_l[0][0] + (r - 6) * ld, sizeof(double) * n_coef);
+          if (lmie_gpu_phase_func(1 + nd, n_coef, n_coef, x, n_angles, theta, o, gsf, device))
+               rc = fail("lmie_gpu_phase_func", lmie_gpu_last_error());
+     }
+     if (!rc) {
+          memcpy(pf[0], o, sizeof(double) * 6 * n_angles);
+          memcpy(pf_l[0][0], o + (size_t) 6 * n_angles, sizeof(double) * 6 * nd * n_angles);
+     }
+     free(x);
+     free(o);
+     return rc;
 }
 
 /* Everything of lmie_solution2_l for one or several distributions on one grid. */

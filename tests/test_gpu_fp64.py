@@ -310,3 +310,43 @@ def test_directions_against_the_oracle(product, oracle, kind, n_int2, n_quad, r2
         if not e <= 1e-12:
             bad.append((k, e))
     assert not bad, bad
+
+
+@pytest.mark.parametrize("gsf", [1, 0])
+@pytest.mark.parametrize("n_set,n_theta,n_coef", [(1, 1, 1), (1, 2, 2), (3, 63, 3), (4, 64, 4), (5, 65, 63), (9, 130, 64),
+                                                  (2, 181, 67), (13, 200, 130)])
+def test_phase_function_against_plain_sums(product, gsf, n_set, n_theta, n_coef):
+    """The phase function at user angles, at the edges of its blocks (64
+    angles, 4 sets, 64 coefficients), against the recurrences summed in numpy.
+    |P| <= 1 and both sides form them by the same stable recurrences (errors of
+    a few l ulp), so 1e-13 of the sum of magnitudes."""
+    say("case: phase function gsf %d sets %d angles %d coefficients %d" % (gsf, n_set, n_theta, n_coef))
+    rng = np.random.Generator(np.random.PCG64(5))
+    ld = n_coef + 3
+    x = np.ascontiguousarray(rng.standard_normal((n_set, 6, ld)))
+    theta = np.ascontiguousarray(rng.uniform(0.0, 180.0, n_theta))
+    pf = np.full((n_set, 6, n_theta), np.nan)
+    f = product.lmie_gpu_phase_func
+    dp = C.POINTER(C.c_double)
+    f.argtypes = [C.c_int, C.c_int, C.c_int, dp, C.c_int, dp, dp, C.c_int, C.c_int]
+    assert f(n_set, n_coef, ld, x.ctypes.data_as(dp), n_theta, theta.ctypes.data_as(dp), pf.ctypes.data_as(dp), gsf, 0) == 0
+    mu = np.cos(theta * (np.pi / 180.0))
+    P = np.zeros((4, max(n_coef, 3), n_theta))
+    P[0, 0], P[0, 1], P[0, 2] = 1.0, mu, (3 * mu * mu - 1) / 2
+    P[1, 2], P[2, 2], P[3, 2] = np.sqrt(6.0) / 4 * (mu * mu - 1), (1 + mu) ** 2 / 4, (1 - mu) ** 2 / 4
+    for l in range(2, n_coef - 1):
+        u, t = l + 1.0, 2.0 * l + 1
+        P[0, l + 1] = (t * mu * P[0, l] - l * P[0, l - 1]) / u
+        P[1, l + 1] = (t * mu * P[1, l] - np.sqrt(l * l - 4.0) * P[1, l - 1]) / np.sqrt(u * u - 4)
+        for q, s in ((2, -4.0), (3, 4.0)):
+            P[q, l + 1] = ((t * l * u * mu + s * t) * P[q, l] - u * (l * l - 4.0) * P[q, l - 1]) / (l * (u * u - 4))
+    P = P[:, :n_coef]
+    c = x[:, :, :n_coef]
+    if gsf:
+        a, b = (c[:, 1] + c[:, 2]) @ P[2], (c[:, 1] - c[:, 2]) @ P[3]
+        ref = np.stack([c[:, 0] @ P[0], (a + b) / 2, (a - b) / 2, c[:, 3] @ P[0], c[:, 4] @ P[1], c[:, 5] @ P[1]], axis=1)
+    else:
+        ref = c @ P[0]
+        ref[:, 5] *= -1
+    scale = np.abs(c).sum(axis=2).max()
+    assert np.all(np.abs(pf - ref) <= 1e-13 * scale)
