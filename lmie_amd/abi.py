@@ -8,6 +8,7 @@ a checker.  ``solve`` fills an ``lmie_in_data`` from keyword parameters, calls
 arrays before releasing the C-side blocks with ``lmie_out_free``.
 """
 import ctypes as C
+import math
 
 import numpy as np
 
@@ -71,10 +72,14 @@ def bind(lib):
 
 
 def _arr(ptr, shape):
-    n = int(np.prod(shape))
-    if n == 0:
-        return np.zeros(shape)
-    return np.ctypeslib.as_array(ptr, shape=(n,)).reshape(shape).copy()
+    """A copy of the block at ptr: short ones through a list, longer ones as one
+    memmove (an array view of a pointer costs more than either)."""
+    n = math.prod(shape)
+    if n <= 16:
+        return np.array(ptr[:n] if n else [], dtype=np.float64).reshape(shape)
+    a = np.empty(shape)
+    C.memmove(a.ctypes.data, ptr, 8 * n)
+    return a
 
 
 def n_size_points(p):

@@ -38,38 +38,45 @@ static double wall_ms(void) {
 /* ------------------------------------------------------------------------- */
 /* Per-size host loops on a small persistent thread pool (up to 16 threads,
    one parallel region at a time; a caller that finds the pool busy runs its
-   loop alone).  Chunks are static, so every element is computed by the same
-   code as a serial loop would: the results do not depend on the threads. */
+   loop alone).  A region wakes as many workers as its size pays for (waking
+   all fifteen cost 50 us, more than a loop over 4000 sizes), and the caller and
+   whoever is awake take chunks from a counter, so nobody waits for a sleeping
+   worker.  Every element is computed by the same code as a serial loop would:
+   the results do not depend on the threads. */
 typedef void (*par_fn)(void *ctx, int i0, int i1);
 static struct {
      pthread_mutex_t region, lk;
      pthread_cond_t go, done;
-     int started, nthr, gen, pending, n;
+     int started, nthr;
+     int tickets, active;               /* workers still wanted, workers inside (under lk) */
+     int next, n, chunk;                /* next: atomic */
      par_fn fn;
      void *ctx;
 } g_pool = {PTHREAD_MUTEX_INITIALIZER, PTHREAD_MUTEX_INITIALIZER, PTHREAD_COND_INITIALIZER,
-            PTHREAD_COND_INITIALIZER, 0, 0, 0, 0, 0, NULL, NULL};
+            PTHREAD_COND_INITIALIZER, 0, 0, 0, 0, 0, 0, 0, NULL, NULL};
 
-static void pool_chunk(int t, int T, int n, int *i0, int *i1) {
-     *i0 = (int) ((long long) n * t / T);
-     *i1 = (int) ((long long) n * (t + 1) / T);
+static void pool_chunks(par_fn fn, void *ctx, int n, int chunk) {
+     for (;;) {
+          const int i0 = __atomic_fetch_add(&g_pool.next, chunk, __ATOMIC_RELAXED);
+          if (i0 >= n) return;
+          fn(ctx, i0, n - i0 > chunk ? i0 + chunk : n);
+     }
 }
 
 static void *pool_worker(void *arg) {
-     const int t = (int) (intptr_t) arg;
-     int seen = 0;
+     (void) arg;
      pthread_mutex_lock(&g_pool.lk);
      for (;;) {
-          while (g_pool.gen == seen) pthread_cond_wait(&g_pool.go, &g_pool.lk);
-          seen = g_pool.gen;
+          while (g_pool.tickets == 0) pthread_cond_wait(&g_pool.go, &g_pool.lk);
+          g_pool.tickets--;
+          g_pool.active++;
           par_fn fn = g_pool.fn;
           void *ctx = g_pool.ctx;
-          int n = g_pool.n, T = g_pool.nthr + 1, i0, i1;
+          const int n = g_pool.n, chunk = g_pool.chunk;
           pthread_mutex_unlock(&g_pool.lk);
-          pool_chunk(t, T, n, &i0, &i1);
-          if (i1 > i0) fn(ctx, i0, i1);
+          pool_chunks(fn, ctx, n, chunk);
           pthread_mutex_lock(&g_pool.lk);
-          if (--g_pool.pending == 0) pthread_cond_signal(&g_pool.done);
+          if (--g_pool.active == 0) pthread_cond_signal(&g_pool.done);
      }
      return NULL;
 }
@@ -78,10 +85,11 @@ static void *pool_worker(void *arg) {
    and each runs its host loops alone */
 static __thread int g_batch_thread;
 
-/* fn over [0, n) on the pool when n >= min_n (else, on a batch thread or
-   with the pool busy, in the calling thread) */
-static void par_run(int n, par_fn fn, void *ctx, int min_n) {
-     if (n < min_n || g_batch_thread || pthread_mutex_trylock(&g_pool.region) != 0) {
+/* fn over [0, n) in chunks, with one more thread per `grain` elements (in the
+   calling thread alone below two grains, on a batch thread or with the pool
+   busy) */
+static void par_run(int n, par_fn fn, void *ctx, int grain, int chunk) {
+     if (n < 2 * grain || g_batch_thread || pthread_mutex_trylock(&g_pool.region) != 0) {
           fn(ctx, 0, n);
           return;
      }
@@ -92,33 +100,108 @@ static void par_run(int n, par_fn fn, void *ctx, int min_n) {
           int T = nc > 16 ? 16 : (nc < 1 ? 1 : (int) nc);
           for (int t = 1; t < T; ++t) {
                pthread_t th;
-               if (pthread_create(&th, NULL, pool_worker, (void *) (intptr_t) t) != 0) break;
+               if (pthread_create(&th, NULL, pool_worker, NULL) != 0) break;
                pthread_detach(th);
                g_pool.nthr++;
           }
      }
-     const int T = g_pool.nthr + 1;
+     const int want = n / grain - 1 < g_pool.nthr ? n / grain - 1 : g_pool.nthr;
      g_pool.fn = fn;
      g_pool.ctx = ctx;
      g_pool.n = n;
-     g_pool.pending = g_pool.nthr;
-     g_pool.gen++;
-     pthread_cond_broadcast(&g_pool.go);
+     g_pool.chunk = chunk;
+     __atomic_store_n(&g_pool.next, 0, __ATOMIC_RELAXED);
+     g_pool.tickets = want;
+     if (2 * want > g_pool.nthr) pthread_cond_broadcast(&g_pool.go);     /* one call, they start together */
+     else
+          for (int t = 0; t < want; ++t) pthread_cond_signal(&g_pool.go);
      pthread_mutex_unlock(&g_pool.lk);
-     int i0, i1;
-     pool_chunk(0, T, n, &i0, &i1);
-     fn(ctx, i0, i1);
+     pool_chunks(fn, ctx, n, chunk);
      pthread_mutex_lock(&g_pool.lk);
-     while (g_pool.pending > 0) pthread_cond_wait(&g_pool.done, &g_pool.lk);
+     g_pool.tickets = 0;                /* nobody enters any more */
+     while (g_pool.active > 0) pthread_cond_wait(&g_pool.done, &g_pool.lk);
      pthread_mutex_unlock(&g_pool.lk);
      pthread_mutex_unlock(&g_pool.region);
 }
 
-static void par_for(int n, par_fn fn, void *ctx) { par_run(n, fn, ctx, 2048); }
+static void par_for(int n, par_fn fn, void *ctx) { par_run(n, fn, ctx, 1024, 256); }
 
-/* fixed blocks 0 .. nb-1 spread over the pool: each block's result is the
-   same whichever thread runs it */
-static void par_blocks(int nb, par_fn fn, void *ctx) { par_run(nb, fn, ctx, 2); }
+/* fixed blocks 0 .. nb-1 spread over the pool, `work` elements in all: each
+   block's result is the same whichever thread runs it */
+static void par_blocks(int nb, int work, par_fn fn, void *ctx) {
+     const int T = work / 8192 < nb ? work / 8192 : nb;
+     par_run(nb, fn, ctx, T > 1 ? nb / T : nb, 1);
+}
+
+/* ------------------------------------------------------------------------- */
+/* Per-size arrays.  Blocks of 64 KiB and more are kept for the next call (at
+   most 32 of them and 64 MiB; the rest, and all of them when the library is
+   unloaded, go back to the C library): from malloc they come as fresh pages, whose
+   first touch and release cost more than the loops over them. */
+#define BLK_MIN ((size_t) 65536)
+#define BLK_CAP ((size_t) 64 << 20)
+typedef struct { size_t n; char pad[56]; } blk_head;
+static struct {
+     pthread_mutex_t mu;
+     blk_head *b[32];
+     size_t total;
+} g_blk = {PTHREAD_MUTEX_INITIALIZER, {0}, 0};
+
+static void *blk_get(size_t bytes) {
+     blk_head *h = NULL;
+     bytes += sizeof(blk_head);
+     if (bytes >= BLK_MIN) {
+          int best = -1;
+          pthread_mutex_lock(&g_blk.mu);
+          for (int k = 0; k < 32; ++k)
+               if (g_blk.b[k] && g_blk.b[k]->n >= bytes && g_blk.b[k]->n <= 2 * bytes &&
+                   (best < 0 || g_blk.b[k]->n < g_blk.b[best]->n))
+                    best = k;
+          if (best >= 0) {
+               h = g_blk.b[best];
+               g_blk.b[best] = NULL;
+               g_blk.total -= h->n;
+          }
+          pthread_mutex_unlock(&g_blk.mu);
+     }
+     if (!h && (h = malloc(bytes))) h->n = bytes;
+     return h ? (void *) (h + 1) : NULL;
+}
+
+static void blk_put(void *p) {
+     if (!p) return;
+     blk_head *h = (blk_head *) p - 1;
+     if (h->n >= BLK_MIN && h->n <= BLK_CAP / 4) {
+          pthread_mutex_lock(&g_blk.mu);
+          for (int k = 0; k < 32 && h && g_blk.total + h->n <= BLK_CAP; ++k)
+               if (!g_blk.b[k]) {
+                    g_blk.b[k] = h;
+                    g_blk.total += h->n;
+                    h = NULL;
+               }
+          pthread_mutex_unlock(&g_blk.mu);
+     }
+     free(h);
+}
+
+__attribute__((destructor)) static void blk_drop(void) {
+     pthread_mutex_lock(&g_blk.mu);
+     for (int k = 0; k < 32; ++k) {
+          free(g_blk.b[k]);
+          g_blk.b[k] = NULL;
+     }
+     g_blk.total = 0;
+     pthread_mutex_unlock(&g_blk.mu);
+}
+
+/* n doubles, released with blk_put: as they are (every element is written by
+   the caller), or zero */
+static double *raw(size_t n) { return blk_get(sizeof(double) * (n ? n : 1)); }
+static double *zeros(size_t n) {
+     double *p = raw(n);
+     if (p) memset(p, 0, sizeof(double) * (n ? n : 1));
+     return p;
+}
 
 /* ------------------------------------------------------------------------- */
 /* errors: one message per thread; -1 returns leave a breadcrumb like the
@@ -222,9 +305,6 @@ typedef struct {
 
 static double sd(const double *v, int d) { return v ? v[d] : 0.; }
 
-/* n_int equal intervals on [r1, r2] with n_quad nodes each; the map of the
-   [-1, 1] rule onto each interval follows misc/rtutil_math.c:329-387 (the
-   mirrored node sets the offset). */
 /* gl_rule of the last few orders asked for, kept for the next calls (a
    batch of cases builds the same rule once per case). */
 static void gl_rule_cached(int n, double *x, double *w) {
@@ -252,35 +332,38 @@ static void gl_rule_cached(int n, double *x, double *w) {
      pthread_mutex_unlock(&mu);
 }
 
-static void grid_intervals(int n_int, int n_quad, int nd, double r1, double r2,
-                           const double *r1_l, const double *r2_l,
-                           double *qx, double *qw, double *qx_l, double *qw_l) {
-     double *tx = vec(n_quad), *tw = vec(n_quad);
-     gl_rule_cached(n_quad, tx, tw);
-     /* the reference scales the [-1,1] weights by the half-width of each
-        interval with its own weight formula ((half - off*y) * c); on [-1, 1]
-        that is (1 - y^2) * c, as gl_rule computes */
-     double step = (r2 - r1) / n_int;
-     for (int s = 0; s < n_int; ++s) {
-          double lo = r1 + s * step, hi = lo + step;
-          double mid = (lo + hi) / 2., half = (hi - lo) / 2.;
-          for (int i = 0, k = n_quad - 1; i < (n_quad + 1) / 2; ++i, --k) {
-               int a = s * n_quad + i, b = s * n_quad + k;
-               qx[a] = mid - half * tx[k];
-               qx[b] = mid + half * tx[k];
-               qw[a] = qw[b] = tw[i] * half;
-               for (int d = 0; d < nd && (r1_l || r2_l); ++d) {   /* else the tangents stay zero */
-                    double st_l = (sd(r2_l, d) - sd(r1_l, d)) / n_int;
-                    double lo_l = sd(r1_l, d) + s * st_l, hi_l = lo_l + st_l;
-                    double mid_l = (lo_l + hi_l) / 2., half_l = (hi_l - lo_l) / 2.;
-                    qx_l[(size_t) a * nd + d] = mid_l - half_l * tx[k];
-                    qx_l[(size_t) b * nd + d] = mid_l + half_l * tx[k];
-                    qw_l[(size_t) a * nd + d] = qw_l[(size_t) b * nd + d] = tw[i] * half_l;
-               }
+/* n_int equal intervals on [r1, r2] with n_quad nodes each; the map of the
+   [-1, 1] rule onto each interval follows misc/rtutil_math.c:329-387 (the
+   mirrored node sets the offset). */
+typedef struct {
+     int n_int, n_quad, nd, nm, *mv;    /* mv: the nm seeds that move an end; the others' tangents stay zero */
+     double r1, r2;
+     const double *r1_l, *r2_l, *tx, *tw;
+     double *qx, *qw, *qx_l, *qw_l;
+} nodes_t;
+
+/* the nodes i0 .. i1-1 */
+static void nodes_range(const nodes_t *p, int i0, int i1) {
+     const int n = p->n_quad;
+     const double step = (p->r2 - p->r1) / p->n_int;
+     for (int i = i0; i < i1; ++i) {
+          /* the reference scales the [-1,1] weights by the half-width of each
+             interval with its own weight formula ((half - off*y) * c); on [-1, 1]
+             that is (1 - y^2) * c, as gl_rule computes */
+          const int s = i / n, q = i - s * n, up = q >= n / 2, k = up ? q : n - 1 - q;
+          const double lo = p->r1 + s * step, hi = lo + step, mid = (lo + hi) / 2., half = (hi - lo) / 2.;
+          const double off = half * p->tx[k], w = p->tw[n - 1 - k];
+          p->qx[i] = up ? mid + off : mid - off;
+          p->qw[i] = w * half;
+          for (int e = 0; e < p->nm; ++e) {
+               const int d = p->mv[e];
+               const double st_l = (sd(p->r2_l, d) - sd(p->r1_l, d)) / p->n_int;
+               const double lo_l = sd(p->r1_l, d) + s * st_l, hi_l = lo_l + st_l;
+               const double mid_l = (lo_l + hi_l) / 2., half_l = (hi_l - lo_l) / 2., off_l = half_l * p->tx[k];
+               p->qx_l[(size_t) i * p->nd + d] = up ? mid_l + off_l : mid_l - off_l;
+               p->qw_l[(size_t) i * p->nd + d] = w * half_l;
           }
      }
-     free(tx);
-     free(tw);
 }
 
 static int grid_points(int dist, int n_int1, int n_int2, int n_quad) {
@@ -332,11 +415,12 @@ typedef struct {
      int N, nd;
      double *qx, *qw, *nr, *qx_l, *qw_l, *nr_l;    /* [N], [N][nd] */
      double r1, r2, *r1_l, *r2_l, norm, *norm_l;
+     int n_act, *act;                              /* seeds with tangents that are not zero throughout */
 } grid_t;
 
 static void grid_free(grid_t *g) {
-     free(g->qx); free(g->qw); free(g->nr); free(g->qx_l); free(g->qw_l); free(g->nr_l);
-     free(g->r1_l); free(g->r2_l); free(g->norm_l);
+     blk_put(g->qx); blk_put(g->qw); blk_put(g->nr); blk_put(g->qx_l); blk_put(g->qw_l); blk_put(g->nr_l);
+     free(g->r1_l); free(g->r2_l); free(g->norm_l); free(g->act);
 }
 
 /* Grid, number density normalised to unit integral, and tangents along each
@@ -348,15 +432,17 @@ typedef struct {
      const seeds *sv;
      grid_t *g;
      double a[5];
+     nodes_t seg[2];                    /* the grid: its nodes below N1, and from N1 on */
 } dens_ctx;
 
 static void dens_range(void *vp, int i0, int i1) {
      const dens_ctx *dc = vp;
-     const int dist = dc->dist, nd = dc->nd, N1 = dc->N1;
+     const int dist = dc->dist, nd = dc->nd, N1 = dc->N1, na = dc->g->n_act, *act = dc->g->act;
      const seeds *sv = dc->sv;
      grid_t *g = dc->g;
      const double a1 = dc->a[0], a2 = dc->a[1], a3 = dc->a[2], a4 = dc->a[3], a5 = dc->a[4];
-     (void) N1;
+     if (i0 < N1) nodes_range(&dc->seg[0], i0, i1 < N1 ? i1 : N1);
+     if (i1 > N1) nodes_range(&dc->seg[1], (i0 > N1 ? i0 : N1) - N1, i1 - N1);
      for (int i = i0; i < i1; ++i) {
           double r = g->qx[i], lr = log(r), *nl = g->nr_l + (size_t) i * nd;
           const double *xl = g->qx_l + (size_t) i * nd;
@@ -365,7 +451,7 @@ static void dens_range(void *vp, int i0, int i1) {
           case SIZE_DIST_MODIFIED_GAMMA: {
                double b = pow(a2, a3), c = a3 * b, h = pow(r, a3);
                n = pow(r, a1) * exp(-a1 / c * h);
-               for (int d = 0; d < nd; ++d) {
+               for (int e = 0, d; e < na && (d = act[e], 1); ++e) {
                     double s1 = sd(sv->a[0], d), s2 = sd(sv->a[1], d), s3 = sd(sv->a[2], d);
                     double lc = s3 / a3 + s2 * (a3 / a2) + s3 * log(a2);    /* d ln c */
                     double px = xl[d] / r;
@@ -374,22 +460,22 @@ static void dens_range(void *vp, int i0, int i1) {
                break;
           }
           case SIZE_DIST_LOG_NORMAL: {
-               double dv = lr - log(a1), e = dv * dv / (2. * a2);
-               n = exp(-e) / r;
-               for (int d = 0; d < nd; ++d) {
+               double dv = lr - log(a1), ex = dv * dv / (2. * a2);
+               n = exp(-ex) / r;
+               for (int e = 0, d; e < na && (d = act[e], 1); ++e) {
                     double px = xl[d] / r;
-                    nl[d] = n * (-px - (2. * dv * (px - sd(sv->a[0], d) / a1) - e * 2. * sd(sv->a[1], d)) / (2. * a2));
+                    nl[d] = n * (-px - (2. * dv * (px - sd(sv->a[0], d) / a1) - ex * 2. * sd(sv->a[1], d)) / (2. * a2));
                }
                break;
           }
           case SIZE_DIST_POWER_LAW:
                n = 1. / pow(r, 3);
-               for (int d = 0; d < nd; ++d) nl[d] = -n * 3. * xl[d] / r;
+               for (int e = 0, d; e < na && (d = act[e], 1); ++e) nl[d] = -n * 3. * xl[d] / r;
                break;
           case SIZE_DIST_GAMMA: {
                double ab = a1 * a2, pw = (1. - 3. * a2) / a2, rp = pow(r, pw), ex = exp(-r / ab);
                n = rp * ex;
-               for (int d = 0; d < nd; ++d) {
+               for (int e = 0, d; e < na && (d = act[e], 1); ++e) {
                     double ab_l = sd(sv->a[0], d) * a2 + a1 * sd(sv->a[1], d);
                     double pw_l = (-3. * sd(sv->a[1], d) - pw * sd(sv->a[1], d)) / a2;
                     nl[d] = rp * ((xl[d] * (pw / r) + pw_l * lr) + (-xl[d] + r / ab * ab_l) / ab) * ex;
@@ -411,7 +497,7 @@ static void dens_range(void *vp, int i0, int i1) {
                double d2 = lr - log(a3), e2 = d2 * d2 / (2. * a4);
                double o1 = exp(-e1), o2 = exp(-e2), r4 = r * r * r * r;
                n = (o1 + a5 * o2) / r4;
-               for (int d = 0; d < nd; ++d) {
+               for (int e = 0, d; e < na && (d = act[e], 1); ++e) {
                     double px = xl[d] / r;
                     double h1 = ((-px + sd(sv->a[0], d) / a1) * 2. * d1 + e1 * 2. * sd(sv->a[1], d)) * o1 / (2. * a2);
                     double h2 = ((-px + sd(sv->a[2], d) / a3) * 2. * d2 + e2 * 2. * sd(sv->a[3], d)) * o2 / (2. * a4);
@@ -434,12 +520,14 @@ static int grid_build(int dist, int n_int1, int n_int2, int n_quad, const double
      if (N <= 0) return fail("size distribution", "invalid distribution type");
      size_t L = (size_t) N * (nd > 0 ? nd : 1);
      g->N = N; g->nd = nd;
-     g->qx = vec(N); g->qw = vec(N); g->nr = vec(N);
-     g->qx_l = vec(L); g->qw_l = vec(L); g->nr_l = vec(L);
+     g->qx = raw(N); g->qw = raw(N); g->nr = raw(N);
+     if (nd == 0) L = 1;                /* no tangents */
+     g->qx_l = zeros(L); g->qw_l = zeros(L); g->nr_l = zeros(L);
      g->r1_l = vec(nd); g->r2_l = vec(nd); g->norm_l = vec(nd);
+     g->act = calloc(nd + 1, sizeof(int)); g->n_act = 0;
      double *tot_l = vec(nd), tot = 0.;
      if (!g->qx || !g->qw || !g->nr || !g->qx_l || !g->qw_l || !g->nr_l || !g->r1_l || !g->r2_l ||
-         !g->norm_l || !tot_l) {
+         !g->norm_l || !g->act || !tot_l) {
           free(tot_l);
           return fail("size distribution", "out of memory");   /* the caller frees g */
      }
@@ -449,7 +537,10 @@ static int grid_build(int dist, int n_int1, int n_int2, int n_quad, const double
 
      if (dist == SIZE_DIST_MONO) {
           g->r1 = g->r2 = a1;
-          for (int d = 0; d < nd; ++d) { g->r1_l[d] = g->r2_l[d] = 0.; g->qx_l[d] = sd(sv->a[0], d); }
+          for (int d = 0; d < nd; ++d) {
+               g->r1_l[d] = g->r2_l[d] = 0.;
+               if ((g->qx_l[d] = sd(sv->a[0], d)) != 0.) g->act[g->n_act++] = d;
+          }
           g->qx[0] = a1; g->qw[0] = 1.; g->nr[0] = 1.;
           g->norm = 1.;
           free(tot_l);
@@ -466,30 +557,45 @@ static int grid_build(int dist, int n_int1, int n_int2, int n_quad, const double
                g->r2_l[d] = (p * v - u) / (p - q);
           }
      }
-     int N1 = 0;
-     if (dist == SIZE_DIST_MODIFIED_POWER_LAW) {
-          N1 = n_int1 * n_quad;
-          grid_intervals(n_int1, n_quad, nd, 0., g->r1, NULL, g->r1_l, g->qx, g->qw, g->qx_l, g->qw_l);
-          grid_intervals(n_int2, n_quad, nd, g->r1, g->r2, g->r1_l, g->r2_l, g->qx + N1, g->qw + N1,
-                         g->qx_l + (size_t) N1 * nd, g->qw_l + (size_t) N1 * nd);
-     } else
-          grid_intervals(n_int2, n_quad, nd, g->r1, g->r2, g->r1_l, g->r2_l, g->qx, g->qw, g->qx_l, g->qw_l);
-
+     /* a seed is active if it moves the grid or a parameter (the others, m's and
+        lambda's, have zero tangents here) */
+     for (int d = 0; d < nd; ++d) {
+          int on = g->r1_l[d] != 0. || g->r2_l[d] != 0.;
+          for (int q = 0; q < 5; ++q) on |= sd(sv->a[q], d) != 0.;
+          if (on) g->act[g->n_act++] = d;
+     }
      {
-          dens_ctx dc = {dist, nd, N1, sv, g, {a1, a2, a3, a4, a5}};
+          /* nodes and densities in one pass over the pool */
+          const int N1 = dist == SIZE_DIST_MODIFIED_POWER_LAW ? n_int1 * n_quad : 0;
+          double *tx = vec(n_quad), *tw = vec(n_quad);
+          int *mv = calloc(2 * (size_t) nd + 2, sizeof(int));
+          if (!tx || !tw || !mv) {
+               free(tx); free(tw); free(mv); free(tot_l);
+               return fail("size distribution", "out of memory");
+          }
+          gl_rule_cached(n_quad, tx, tw);
+          nodes_t lo = {n_int1, n_quad, nd, 0, mv, 0., g->r1, NULL, g->r1_l, tx, tw, g->qx, g->qw, g->qx_l, g->qw_l};
+          nodes_t hi = {n_int2, n_quad, nd, 0, mv + nd + 1, g->r1, g->r2, g->r1_l, g->r2_l, tx, tw, g->qx + N1, g->qw + N1,
+                        g->qx_l + (size_t) N1 * nd, g->qw_l + (size_t) N1 * nd};
+          for (int d = 0; d < nd; ++d) {
+               if (N1 && g->r1_l[d] != 0.) lo.mv[lo.nm++] = d;
+               if (g->r1_l[d] != 0. || g->r2_l[d] != 0.) hi.mv[hi.nm++] = d;
+          }
+          dens_ctx dc = {dist, nd, N1, sv, g, {a1, a2, a3, a4, a5}, {lo, hi}};
           par_for(N, dens_range, &dc);
+          free(tx); free(tw); free(mv);
      }
      for (int i = 0; i < N; ++i) {
           tot += g->nr[i] * g->qw[i];
           if (dist != SIZE_DIST_EXPONENTIAL)
-               for (int d = 0; d < nd; ++d)
+               for (int e = 0, d; e < g->n_act && (d = g->act[e], 1); ++e)
                     tot_l[d] += g->nr_l[(size_t) i * nd + d] * g->qw[i] + g->nr[i] * g->qw_l[(size_t) i * nd + d];
      }
      g->norm = tot;
      for (int d = 0; d < nd; ++d) g->norm_l[d] = tot_l[d];
      for (int i = 0; i < N; ++i) {
           g->nr[i] /= tot;
-          for (int d = 0; d < nd; ++d)
+          for (int e = 0, d; e < g->n_act && (d = g->act[e], 1); ++e)
                g->nr_l[(size_t) i * nd + d] = (g->nr_l[(size_t) i * nd + d] - g->nr[i] * tot_l[d]) / tot;
      }
      free(tot_l);
@@ -506,7 +612,8 @@ static void grid_stats(const grid_t *g, dstats *s, dstats *sl /* [nd] or NULL */
      for (int i = 0; i < N; ++i) {
           double t = g->nr[i] * g->qx[i] * g->qw[i];
           for (int k = 0; k < 4; ++k) { m[k] += t; t *= g->qx[i]; }
-          for (int d = 0; d < nd; ++d) {
+          for (int e = 0; e < g->n_act; ++e) {
+               const int d = g->act[e];
                size_t o = (size_t) i * nd + d;
                double h = g->qx[i] * g->qw[i] * g->nr_l[o], p = g->nr[i] * g->qw[i] * g->qx_l[o];
                double q = g->nr[i] * g->qx[i] * g->qw_l[o], rp = 1.;
@@ -529,7 +636,8 @@ static void grid_stats(const grid_t *g, dstats *s, dstats *sl /* [nd] or NULL */
      for (int i = 0; i < N; ++i) {
           double dr = g->qx[i] - s->reff, r2w = g->qx[i] * g->qx[i] * g->qw[i];
           v += g->nr[i] * dr * dr * r2w;
-          for (int d = 0; d < nd && sl; ++d) {
+          for (int e = 0; e < g->n_act && sl; ++e) {
+               const int d = g->act[e];
                size_t o = (size_t) i * nd + d;
                vl[d] += g->nr_l[o] * dr * dr * r2w + g->nr[i] *
                         (2. * dr * r2w * (g->qx_l[o] - sl[d].reff) +
@@ -639,15 +747,15 @@ typedef struct {
 } job_mem;
 
 static void job_mem_alloc(job_mem *m, int N, int nd1, int nd2) {
-     m->x = vec(N); m->f = vec(N); m->sx = vec(N); m->cx = vec(N);
-     m->n1 = calloc(N, sizeof(int)); m->n2 = calloc(N, sizeof(int));
-     m->dx = vec((size_t) nd1 * N); m->dm = vec(2 * (size_t) nd1); m->dft = vec((size_t) nd1 * N);
-     m->dfw = vec((size_t) nd2 * N);
+     m->x = raw(N); m->f = raw(N); m->sx = raw(N); m->cx = raw(N);
+     m->n1 = blk_get(sizeof(int) * N); m->n2 = blk_get(sizeof(int) * N);
+     m->dx = raw((size_t) nd1 * N); m->dm = raw(2 * (size_t) nd1); m->dft = raw((size_t) nd1 * N);
+     m->dfw = raw((size_t) nd2 * N);
 }
 
 static void job_mem_free(job_mem *m) {
-     free(m->x); free(m->f); free(m->n1); free(m->n2); free(m->dx); free(m->dm); free(m->dft); free(m->dfw);
-     free(m->sx); free(m->cx);
+     blk_put(m->x); blk_put(m->f); blk_put(m->n1); blk_put(m->n2); blk_put(m->dx); blk_put(m->dm); blk_put(m->dft);
+     blk_put(m->dfw); blk_put(m->sx); blk_put(m->cx);
 }
 
 /* Normalise the expansion of channel c of raw into out (one 6 x n_coef set):
@@ -676,8 +784,8 @@ static int core_run(const core_args *c, core_out *o) {
      o->n_qang = Q; o->n_coef = C;
      memset(&res, 0, sizeof res);
      res.sums_ch = vec((size_t) 4 * (nch - 1));
-     res.gc_raw = c->calc_gc ? vec((size_t) nch * 6 * C) : NULL;
-     res.lc_raw = c->calc_lc ? vec((size_t) nch * 6 * C) : NULL;
+     res.gc_raw = c->calc_gc ? zeros((size_t) nch * 6 * C) : NULL;
+     res.lc_raw = c->calc_lc ? zeros((size_t) nch * 6 * C) : NULL;
      if (c->save_control == 1) {
           *o->save1 = table2(4, c->N);
           *o->save2 = table3(4, c->N, Q > 0 ? Q : 1);
@@ -735,7 +843,7 @@ static int core_run(const core_args *c, core_out *o) {
      if (c->calc_gc) { norm_set(res.gc_raw, 0, C, a, 0., o->gc); rc = truncated_count(o->gc, C, c->accuracy); }
      if (c->calc_lc) { norm_set(res.lc_raw, 0, C, a, 0., o->lc); rc = truncated_count(o->lc, C, c->accuracy); }
 done:
-     free(res.sums_ch); free(res.gc_raw); free(res.lc_raw);
+     free(res.sums_ch); blk_put(res.gc_raw); blk_put(res.lc_raw);
      job_mem_free(&jm);
      return rc;
 }
@@ -1152,6 +1260,9 @@ static int mix_grid(lmie_in_data *const *modes, const double *weight, int n_mode
                     *mix = gk;
                     for (int i = 0; i < gk.N; ++i) mix->nr[i] *= w;
                     for (size_t i = 0; i < (size_t) gk.N * nd; ++i) mix->nr_l[i] *= w;
+                    /* the modes' seeds are different columns: all of them count as active */
+                    if (n_modes > 1)
+                         for (mix->n_act = 0; mix->n_act < nd; ++mix->n_act) mix->act[mix->n_act] = mix->n_act;
                     mix->norm *= w;
                     for (int d = 0; d < nd; ++d) mix->norm_l[d] *= w;
                } else {
@@ -1248,21 +1359,21 @@ struct lmie_adj_ctx {
      double lambda, Csca, g, cext, csca, cbak;
      double *gc, *lc;               /* normalised outputs [6][C] */
      double *w;                     /* mode weights */
-     double **df;                   /* per mode: d (w_k qw_i n_k(r_i)) / d seed, [N][ADJ_SEEDS] */
-     double **dx;                   /* per mode: d x_i / d seed, [N][ADJ_SEEDS] */
+     double **df;                   /* per mode and seed [n_modes][ADJ_SEEDS]: d (w_k qw_i n_k(r_i)) / d seed [N], NULL if zero */
+     double **dx;                   /* the same: d x_i / d seed */
      double *xl;                    /* [N] x_i / lambda */
 };
 
 static void adj_tangents_free(double **v, int n) {
      if (v)
-          for (int k = 0; k < n; ++k) free(v[k]);
+          for (int k = 0; k < n * ADJ_SEEDS; ++k) blk_put(v[k]);
      free(v);
 }
 
 void lmie_adjoint_free(lmie_adj_ctx *ctx) {
      if (!ctx) return;
      lmie_gpu_release(ctx->state);
-     free(ctx->gc); free(ctx->lc); free(ctx->w); free(ctx->xl);
+     free(ctx->gc); free(ctx->lc); free(ctx->w); blk_put(ctx->xl);
      adj_tangents_free(ctx->df, ctx->n_modes);
      adj_tangents_free(ctx->dx, ctx->n_modes);
      free(ctx);
@@ -1283,8 +1394,8 @@ static void *dn_build(void *vp) {
      dn_job *j = vp;
      const lmie_in_data *m0 = j->modes[0];
      const int S = ADJ_SEEDS;
-     j->df = calloc(j->n_modes, sizeof(double *));
-     j->dx = calloc(j->n_modes, sizeof(double *));
+     j->df = calloc((size_t) S * j->n_modes, sizeof(double *));
+     j->dx = calloc((size_t) S * j->n_modes, sizeof(double *));
      for (int k = 0; k < j->n_modes; ++k) {
           const lmie_in_data *m = j->modes[k];
           const double w = j->weight ? j->weight[k] : 1.;
@@ -1295,8 +1406,6 @@ static void *dn_build(void *vp) {
           double a[5] = {m->a1, m->a2, m->a3, m->a4, m->a5};
           grid_t gk;
           memset(&gk, 0, sizeof gk);
-          j->df[k] = vec((size_t) S * j->N);
-          j->dx[k] = vec((size_t) S * j->N);
           /* a seed moves the size parameters only where the forward makes it a
              Mie tangent channel: where it moves the radius range
              (src/lmie_interface.c:327-331), so the mono distribution's a1,
@@ -1304,13 +1413,15 @@ static void *dn_build(void *vp) {
              acts on the weights only, as in the reference's tangents */
           if (grid_build(m->dist_type, m0->n_int1, m0->n_int2, m0->n_quad, a, m0->r1, m0->r2, &sv, &gk) == 0 &&
               gk.N == j->N)
-               for (int i = 0; i < gk.N; ++i)
-                    for (int q = 0; q < S; ++q) {
+               for (int e = 0; e < gk.n_act; ++e) {
+                    const int q = gk.act[e], moves = gk.r1_l[q] != 0. || gk.r2_l[q] != 0.;
+                    double *df = j->df[S * k + q] = raw(j->N), *dx = j->dx[S * k + q] = moves ? raw(j->N) : NULL;
+                    for (int i = 0; df && i < gk.N; ++i) {
                          const size_t o = (size_t) i * S + q;
-                         const int moves = gk.r1_l[q] != 0. || gk.r2_l[q] != 0.;
-                         j->df[k][o] = w * (gk.nr_l[o] * gk.qw[i] + gk.nr[i] * gk.qw_l[o]);
-                         j->dx[k][o] = moves ? 2. * LM_PI * gk.qx_l[o] / j->lambda : 0.;
+                         df[i] = w * (gk.nr_l[o] * gk.qw[i] + gk.nr[i] * gk.qw_l[o]);
+                         if (dx) dx[i] = 2. * LM_PI * gk.qx_l[o] / j->lambda;
                     }
+               }
           grid_free(&gk);
      }
      return NULL;
@@ -1490,7 +1601,7 @@ static int adjoint_forward_run(lmie_in_data *const *modes, const double *weight,
      c->w = vec(n_modes);
      for (int k = 0; k < n_modes; ++k) c->w[k] = weight ? weight[k] : 1.;
      c->df = dj.df; c->dx = dj.dx;
-     c->xl = vec(g.N);
+     c->xl = raw(g.N);
      for (int i = 0; i < g.N; ++i) c->xl[i] = 2. * LM_PI * g.qx[i] / (m0->lambda * m0->lambda);
      grid_free(&g);
      *ctxp = c;
@@ -1525,17 +1636,24 @@ static void grad_block(void *vp, int b0, int b1) {
           const int i0 = (int) ((long long) c->N * b / GRAD_BLOCKS), i1 = (int) ((long long) c->N * (b + 1) / GRAD_BLOCKS);
           for (int q = 0; q < W; ++q) pb[q] = 0.;
           for (int k = 0; k < c->n_modes; ++k)
-               for (int i = i0; i < i1; ++i) {
-                    const double *df = c->df[k] + (size_t) i * S, *dx = c->dx[k] + (size_t) i * S;
-                    for (int q = 0; q < 5; ++q) pb[5 * k + q] += g->f_bar[i] * df[q] + g->x_bar[i] * dx[q];
-                    pb[W - 3] += g->f_bar[i] * df[5];
-                    pb[W - 2] += g->f_bar[i] * df[6];
+               for (int q = 0; q < S; ++q) {
+                    const double *df = c->df[S * k + q], *dx = q < 5 ? c->dx[S * k + q] : NULL;
+                    double t = q < 5 ? 0. : pb[W - 8 + q];
+                    if (df && dx)
+                         for (int i = i0; i < i1; ++i) t += g->f_bar[i] * df[i] + g->x_bar[i] * dx[i];
+                    else if (df)
+                         for (int i = i0; i < i1; ++i) t += g->f_bar[i] * df[i];
+                    pb[q < 5 ? 5 * k + q : W - 8 + q] = t;
                }
-          for (int i = i0; i < i1; ++i) {
-               pb[W - 3] += g->x_bar[i] * c->dx[0][(size_t) i * S + 5];
-               pb[W - 2] += g->x_bar[i] * c->dx[0][(size_t) i * S + 6];
-               pb[W - 1] += g->x_bar[i] * c->xl[i];
+          double lx = 0.;
+          for (int q = 5; q < S; ++q) {
+               const double *dx = c->dx[q];
+               double t = pb[W - 8 + q];
+               for (int i = i0; dx && i < i1; ++i) t += g->x_bar[i] * dx[i];
+               pb[W - 8 + q] = t;
           }
+          for (int i = i0; i < i1; ++i) lx += g->x_bar[i] * c->xl[i];
+          pb[W - 1] = lx;
      }
 }
 
@@ -1570,8 +1688,8 @@ static int adjoint_reverse_run(lmie_adj_ctx *c, const lmie_adj_in *adj, lmie_gra
      sb[1] = s * adj->csca - dot / Csca;
      lmie_gpu_adj_in ain = {sb, gcb, lcb};
      lmie_gpu_adj_out aout;
-     aout.f_bar = vec(c->N);
-     aout.x_bar = vec(c->N);
+     aout.f_bar = zeros(c->N);
+     aout.x_bar = zeros(c->N);
      int rc = lmie_gpu_adjoint(c->state, &ain, &aout);
      if (rc) {
           fail("lmie_gpu_adjoint", lmie_gpu_last_error());
@@ -1585,7 +1703,7 @@ static int adjoint_reverse_run(lmie_adj_ctx *c, const lmie_adj_in *adj, lmie_gra
           /* per fixed block of sizes on the pool, then the blocks in order:
              the sums do not depend on the threads */
           grad_ctx gx = {c, aout.f_bar, aout.x_bar, vec((size_t) GRAD_BLOCKS * (5 * c->n_modes + 3))};
-          par_blocks(GRAD_BLOCKS, grad_block, &gx);
+          par_blocks(GRAD_BLOCKS, c->N * (c->n_modes + 1), grad_block, &gx);
           for (int b = 0; b < GRAD_BLOCKS; ++b) {
                const double *pb = gx.part + (size_t) b * (5 * c->n_modes + 3);
                for (int q = 0; q < 5 * c->n_modes; ++q) gp[q] += pb[q];
@@ -1604,7 +1722,7 @@ static int adjoint_reverse_run(lmie_adj_ctx *c, const lmie_adj_in *adj, lmie_gra
                for (int q = 0; q < 5 * c->n_modes; ++q) grad_modes[q] = gp[q];
           free(gp);
      }
-     free(aout.f_bar); free(aout.x_bar); free(gcb); free(lcb);
+     blk_put(aout.f_bar); blk_put(aout.x_bar); free(gcb); free(lcb);
      return rc ? -1 : 0;
 }
 
