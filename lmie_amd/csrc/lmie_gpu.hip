@@ -233,43 +233,82 @@ __device__ __forceinline__ cd cdiv_nr(cd a, cd b) {
 // initial guesses come from the host (the C library's cos and tan, as the
 // reference) and every operation here is a separately rounded IEEE operation
 // (no contraction): the rule is the reference's rule bit for bit.
-// Bound: the Legendre recurrence's chain of four dependent operations (about
-// 38 cycles) per order and Newton step.  Its factors j / (j + 1) are the same
-// in every lane: each lane divides for one order of the next 64 and the steps
-// read them from that lane, so every table wave can run the Newton steps of
-// its own 64 angles and none waits for another.
-__device__ __forceinline__ double readlane_d(double v, int lane) {
-     // value of lane `lane` (uniform) of a double: a scalar operand for the wave
-     const unsigned long long u = (unsigned long long) __double_as_longlong(v);
-     const unsigned lo = __builtin_amdgcn_readlane((unsigned) u, lane);
-     const unsigned hi = __builtin_amdgcn_readlane((unsigned) (u >> 32), lane);
-     return __longlong_as_double((long long) (((unsigned long long) hi << 32) | lo));
+// Bound: the Legendre recurrence's chain of four dependent operations per order
+// and Newton step.  Its factors j / (j + 1) are the same in every lane: each lane
+// divides for one order of the next 64, and the steps read them back from LDS as
+// broadcasts, ahead of the chain (UniformFactors), so every table wave can run
+// the Newton steps of its own 64 angles and none waits for another.
+// Orders the LDS accesses of one wave: what its lanes wrote before is read after
+// (LDS serves a wave's accesses in order; this keeps the compiler to it).
+__device__ __forceinline__ void wave_lds_fence() {
+     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+     __builtin_amdgcn_wave_barrier();
+}
+
+// Runs step(i, factor(i)) for i = 0 .. n-1 where factor is the same in every lane
+// of the wave: 64 factors at a time, one formed per lane, through two LDS buffers
+// (lds: UF_LDS doubles of the wave), the next 64 formed and the next eight read
+// while the steps run.  (Reading them from the forming lane by v_readlane cost two
+// more issue slots per step inside the dependence chain: the Gauss rule of 3810
+// angles took 0.26 ms.)
+constexpr int UF_ROW = 72, UF_LDS = 2 * UF_ROW;
+template <class G, class F>
+__device__ __forceinline__ void uniform_steps(int n, double *lds, G factor, F step) {
+     const int lane = threadIdx.x & 63;
+     wave_lds_fence();
+     lds[lane] = factor(lane);
+     wave_lds_fence();
+     for (int i0 = 0, c = 0; i0 < n; i0 += 64, c ^= 1) {
+          if (i0 + 64 < n) lds[(c ^ 1) * UF_ROW + lane] = factor(i0 + 64 + lane);
+          wave_lds_fence();
+          const double *t = lds + c * UF_ROW;
+          const int m = min(64, n - i0);
+          double a[8], b[8];          // (read past 64: spare entries, unused)
+          auto read = [&](double *v, int o) {
+#pragma unroll
+               for (int k = 0; k < 8; ++k) v[k] = t[o + k];
+          };
+          auto eight = [&](const double *v, int o) {
+#pragma unroll
+               for (int k = 0; k < 8; ++k) step(i0 + o + k, v[k]);
+          };
+          read(a, 0);
+          int e = 0;
+          for (; e + 16 <= m; e += 16) {
+               read(b, e + 8);
+               eight(a, e);
+               read(a, e + 16);
+               eight(b, e + 8);
+          }
+          if (e + 8 <= m) {
+               read(b, e + 8);
+               eight(a, e);
+               e += 8;
+#pragma unroll
+               for (int k = 0; k < 8; ++k) a[k] = b[k];
+          }
+#pragma unroll
+          for (int k = 0; k < 7; ++k)
+               if (e + k < m) step(i0 + e + k, a[k]);
+          wave_lds_fence();
+     }
 }
 
 // y: initial guess in, last iterate out; pb: P_{n-1} at the last-but-one.  The
 // whole wave takes part; a lane that has stopped keeps its values.
-__device__ __forceinline__ void gauss_newton(int n, bool run, double &y, double &pb) {
+__device__ __forceinline__ void gauss_newton(int n, bool run, double &y, double &pb, double *lds) {
 #pragma clang fp contract(off)
      const double dn = (double) n, nn1 = (double) (n * (n + 1));
-     const int lane = threadIdx.x & 63;
      int it = 0;
      while (__ballot(run)) {
           double pa = 1., pm = 0., pc = 0.;
-          auto step = [&](double c) {
-               pm = pc;
-               pc = pa;
-               const double u = y * pc;
-               pa = c * (u - pm) + u;
-          };
-          for (int j0 = 0; j0 < n; j0 += 64) {
-               const double j = j0 + lane, cl = j / (j + 1.);
-               if (n - j0 >= 64) {
-#pragma unroll 16
-                    for (int e = 0; e < 64; ++e) step(readlane_d(cl, e));
-               } else {
-                    for (int e = 0; e < n - j0; ++e) step(readlane_d(cl, e));
-               }
-          }
+          uniform_steps(n, lds, [](int j) { return (double) j / (j + 1.); },
+                        [&](int, double c) {
+                             pm = pc;
+                             pc = pa;
+                             const double u = y * pc;
+                             pa = c * (u - pm) + u;
+                        });
           const double s = 1. - y * y;
           const double d1 = dn * (pc - y * pa) / s;
           const double d2 = (2. * y * d1 - nn1 * pa) / s;
@@ -284,11 +323,11 @@ __device__ __forceinline__ void gauss_newton(int n, bool run, double &y, double 
 }
 
 // Roots of the rule of n angles from their guesses: mu[0 .. n), w[0 .. n).
-__device__ __forceinline__ void gauss_role(int n, const double *guess, double *mu, double *w, int block) {
+__device__ __forceinline__ void gauss_role(int n, const double *guess, double *mu, double *w, int block, double *lds) {
 #pragma clang fp contract(off)
      const int i = block * 64 + threadIdx.x, nr = (n + 1) / 2;
      double y = guess[i < nr ? i : nr - 1], pb = 0.;
-     gauss_newton(n, i < nr, y, pb);
+     gauss_newton(n, i < nr, y, pb, lds);
      if (i >= nr) return;
      double c = (double) n * pb;
      c = 2. / (c * c);
@@ -300,11 +339,11 @@ __device__ __forceinline__ void gauss_role(int n, const double *guess, double *m
 
 // Positive angle j < H of this lane (0 past H): its own Newton steps, or the
 // given angles mu[H + j] without guesses.
-__device__ __forceinline__ double angle_of(int Q, int H, const double *guess, const double *mu, int j) {
+__device__ __forceinline__ double angle_of(int Q, int H, const double *guess, const double *mu, int j, double *lds) {
 #pragma clang fp contract(off)
      if (!guess) return j < H ? mu[H + j] : 0.;
      double y = guess[j < H ? H - 1 - j : 0], pb;
-     gauss_newton(Q, j < H, y, pb);
+     gauss_newton(Q, j < H, y, pb, lds);
      return j < H ? 0. + 1. * y : 0.;
 }
 
@@ -313,35 +352,26 @@ __device__ __forceinline__ double angle_of(int Q, int H, const double *guess, co
 // tau_n = n (mu pi_n - pi_{n-1}) - pi_{n-1} (src/lmie_core.c:669-691), in
 // separately rounded operations in the reference's order: the tables are
 // the reference's pi_n, tau_n bit for bit.  f(n, pi + tau, pi - tau) takes
-// orders 1 .. n1max; quotients (n+1)/n as in gauss_newton.
+// orders 1 .. n1max.
 template <class F>
-__device__ __forceinline__ void pitau_steps(int n1max, double m, F f) {
+__device__ __forceinline__ void pitau_steps(int n1max, double m, double *lds, F f) {
 #pragma clang fp contract(off)
-     const int lane = threadIdx.x & 63;
      double p0 = 0., p1 = 1.;
-     for (int n0 = 1; n0 <= n1max; n0 += 64) {
-          const double nl = n0 + lane, ql = (nl + 1.) / nl;
-          auto step = [&](int e) {
-               const int n = n0 + e;
-               const double a1 = m * p1, a2 = a1 - p0;
-               const double tau = n * a2 - p0;
-               f(n, p1 + tau, p1 - tau);
-               p0 = p1;
-               p1 = a1 + readlane_d(ql, e) * a2;
-          };
-          if (n1max - n0 >= 63) {
-#pragma unroll 8
-               for (int e = 0; e < 64; ++e) step(e);
-          } else {
-               for (int e = 0; e <= n1max - n0; ++e) step(e);
-          }
-     }
+     uniform_steps(n1max, lds, [](int i) { return (i + 2.) / (i + 1.); },      // (n + 1) / n, n = i + 1
+                   [&](int i, double q) {
+                        const int n = i + 1;
+                        const double a1 = m * p1, a2 = a1 - p0;
+                        const double tau = n * a2 - p0;
+                        f(n, p1 + tau, p1 - tau);
+                        p0 = p1;
+                        p1 = a1 + q * a2;
+                   });
 }
 
 // FP64 tables [Kp][Hp], zero rows past n1max and columns past H.
-__device__ __forceinline__ void pitau_role(int H, int Hp, int n1max, int Kp, double m, double *Bp, double *Bm, int j) {
+__device__ __forceinline__ void pitau_role(int H, int Hp, int n1max, int Kp, double m, double *Bp, double *Bm, int j, double *lds) {
      const bool live = j < H;
-     pitau_steps(n1max, m, [&](int n, double bp, double bm) {
+     pitau_steps(n1max, m, lds, [&](int n, double bp, double bm) {
           Bp[(size_t) (n - 1) * Hp + j] = live ? bp : 0.;
           Bm[(size_t) (n - 1) * Hp + j] = live ? bm : 0.;
      });
@@ -358,25 +388,30 @@ __device__ __forceinline__ void pitau_role(int H, int Hp, int n1max, int Kp, dou
 constexpr int PITAU_SHARE = 8;
 
 template <class E>
-__device__ __forceinline__ void pitau16_role(int H, int Hb, int n1max, int Kb, double m, unsigned short *B16, int j, int share) {
+__device__ __forceinline__ void pitau16_role(int H, int Hb, int n1max, int Kb, double m, unsigned short *B16, int j, int share,
+                                             double *lds) {
      const size_t plane = (size_t) Kb * Hb * 8;
      const int lane = threadIdx.x & 63;
      const bool live = j < H;
      double p0 = 0., p1 = 1.;
-     double ql = 1., sl = 0.;
      for (int g = 0; g < Kb; ++g) {
           if ((g & 7) == 0) {          // factors of the next 64 orders, one per lane
                const double n = 8 * g + 1 + lane;
-               ql = (n + 1.) / n;
-               sl = kSB / (n * (n + 1.));
+               wave_lds_fence();
+               lds[lane] = (n + 1.) / n;
+               lds[UF_ROW + lane] = kSB / (n * (n + 1.));
+               wave_lds_fence();
           }
-          const int e0 = 8 * (g & 7);
+          const double *qs = lds + 8 * (g & 7), *ss = qs + UF_ROW;
+          double q[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) q[e] = qs[e];
           if ((g & (PITAU_SHARE - 1)) != share) {
 #pragma unroll
                for (int e = 0; e < 8; ++e) {
                     const double a1 = m * p1, a2 = a1 - p0;
                     p0 = p1;
-                    p1 = a1 + readlane_d(ql, e0 + e) * a2;
+                    p1 = a1 + q[e] * a2;
                }
                continue;
           }
@@ -385,19 +420,19 @@ __device__ __forceinline__ void pitau16_role(int H, int Hb, int n1max, int Kb, d
           for (int e = 0; e < 8; ++e) {
                const int n = 8 * g + e + 1;
                const double a1 = m * p1, a2 = a1 - p0;
-               const double tau = n * a2 - p0, sc = readlane_d(sl, e0 + e);
+               const double tau = n * a2 - p0, sc = ss[e];
                const bool on = live && n <= n1max;
                split16x3<E>(on ? (p1 + tau) * sc : 0., &v[0][e], &v[1][e], &v[2][e]);
                split16x3<E>(on ? (p1 - tau) * sc : 0., &v[3][e], &v[4][e], &v[5][e]);
                p0 = p1;
-               p1 = a1 + readlane_d(ql, e0 + e) * a2;
+               p1 = a1 + q[e] * a2;
           }
 #pragma unroll
-          for (int q = 0; q < B16_PLANES; ++q) {
+          for (int b = 0; b < B16_PLANES; ++b) {
                v4u w;
 #pragma unroll
-               for (int k = 0; k < 4; ++k) w[k] = (unsigned) v[q][2 * k] | ((unsigned) v[q][2 * k + 1] << 16);
-               *(v4u *) (B16 + q * plane + ((size_t) g * Hb + j) * 8) = w;
+               for (int k = 0; k < 4; ++k) w[k] = (unsigned) v[b][2 * k] | ((unsigned) v[b][2 * k + 1] << 16);
+               *(v4u *) (B16 + b * plane + ((size_t) g * Hb + j) * 8) = w;
           }
      }
 }
@@ -417,16 +452,9 @@ __device__ __forceinline__ void pitau16_role(int H, int Hb, int n1max, int Kb, d
 // reciprocal, square roots, polynomials in l) is formed for 64 l at a time, one
 // l per lane, and read back from LDS as broadcasts, ahead of the chain of five
 // dependent operations that bounds the step.
-// Orders the LDS accesses of one wave: what its lanes wrote before is read after
-// (LDS serves a wave's accesses in order; this keeps the compiler to it).
-__device__ __forceinline__ void wave_lds_fence() {
-     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-     __builtin_amdgcn_wave_barrier();
-}
-
 constexpr int GSF_CST = 6, GSF_USED = 5;   // doubles per l: divisor, reciprocal, three factors
-// The wave's functions go to f(l, value), l = 0 .. C-1 in order, and each 64 l are
-// announced by at(l0); a lane that is not live gets zeros.
+// The wave's functions go to f(l, l odd, value), l = 0 .. C-1 in order, and each 64
+// l are announced by at(l0); a lane that is not live gets zeros.
 template <int FN, class A, class F>
 __device__ __forceinline__ void gsf_steps(int C, double m, bool live, double *cst, A at, F f) {
      // separately rounded operations in the reference's order (bitwise the
@@ -455,8 +483,8 @@ __device__ __forceinline__ void gsf_steps(int C, double m, bool live, double *cs
           }
           const int ne = min(64, C - l0);
           at(l0);
-          auto put = [&](int e, double v) {
-               f(l0 + e, v);
+          auto put = [&](int e, bool odd, double v) {
+               f(l0 + e, odd, v);
                a0 = b0;
                b0 = v;
           };
@@ -473,7 +501,7 @@ __device__ __forceinline__ void gsf_steps(int C, double m, bool live, double *cs
                     else if constexpr (FN == 1) v = .25 * sqrt(6.) * (m2 - 1.);
                     else if constexpr (FN == 2) v = .25 * (1. + m) * (1. + m);
                     else v = .25 * (1. - m) * (1. - m);
-                    put(l, live ? v : 0.);       // dead lanes stay zero from here
+                    put(l, l & 1, live ? v : 0.);       // dead lanes stay zero from here
                }
                e0 = 3;
           }
@@ -484,11 +512,11 @@ __device__ __forceinline__ void gsf_steps(int C, double m, bool live, double *cs
                for (int k = 0; k < GSF_USED; ++k) s.v[k] = cst[GSF_CST * e + k];
                return s;
           };
-          auto step = [&](int e, const Cst &s) {
+          auto step = [&](int e, bool odd, const Cst &s) {
                if constexpr (FN == 4) {
                     // P_l = a (m P_{l-1} - P_{l-2}) + m P_{l-1}, a = (l-1)/l
                     const double bb = m * b0;
-                    put(e, s.v[2] * (bb - a0) + bb);
+                    put(e, odd, s.v[2] * (bb - a0) + bb);
                } else {
                     double x;
                     if constexpr (FN < 2) {
@@ -499,11 +527,11 @@ __device__ __forceinline__ void gsf_steps(int C, double m, bool live, double *cs
                          x = FN == 2 ? (dc - s.v[4]) * b0 - s.v[3] * a0 : (dc + s.v[4]) * b0 - s.v[3] * a0;
                     }
                     const double q = x * s.v[1];
-                    put(e, __builtin_fma(__builtin_fma(-q, s.v[0], x), s.v[1], q));
+                    put(e, odd, __builtin_fma(__builtin_fma(-q, s.v[0], x), s.v[1], q));
                }
           };
           int e = e0;
-          for (; e < ne && (e & 3); ++e) step(e, load(e));
+          for (; e < ne && (e & 3); ++e) step(e, e & 1, load(e));
           // groups of four, the next group's factors read one group ahead
           // (past the last one: the buffer's four spare entries)
           Cst c0[4], c1[4];
@@ -513,7 +541,7 @@ __device__ __forceinline__ void gsf_steps(int C, double m, bool live, double *cs
           };
           auto four = [&](const Cst *c, int o) {
 #pragma unroll
-               for (int k = 0; k < 4; ++k) step(o + k, c[k]);
+               for (int k = 0; k < 4; ++k) step(o + k, k & 1, c[k]);
           };
           read(c0, e);
           for (; e + 8 <= ne; e += 8) {
@@ -522,16 +550,38 @@ __device__ __forceinline__ void gsf_steps(int C, double m, bool live, double *cs
                read(c0, e + 8);
                four(c1, e + 4);
           }
-          for (; e < ne; ++e) step(e, load(e));
+          if (e + 4 <= ne) {
+               read(c1, e + 4);
+               four(c0, e);
+               e += 4;
+#pragma unroll
+               for (int k = 0; k < 4; ++k) c0[k] = c1[k];
+          }
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+               if (e + k < ne) step(e + k, k & 1, c0[k]);
      }
 }
-// One plane of the expansion tables, zero columns past H.
+// One plane of the expansion tables, zero columns past H: rows of two l, [(C + 1) /
+// 2][Hp][2], so a step stores half as often (16 bytes a lane every second l): a
+// wave issues its stores inside the chain (42 ns a step with one per l, 32 with one
+// per two, 3810 l).
 template <int FN>
 __device__ __forceinline__ void gsf_role(int H, int Hp, int C, double m, double *P, int j, double *cst) {
      // rows from a uniform pointer, the lane's byte offset a 32-bit register
-     const unsigned oj = (unsigned) j * 8u;
-     gsf_steps<FN>(C, m, j < H, cst, [](int) {}, [&](int l, double v) { *(double *) ((char *) (P + (size_t) l * Hp) + oj) = v; });
+     const unsigned oj = (unsigned) j * 16u;
+     typedef double d2 __attribute__((ext_vector_type(2)));
+     double held = 0.;
+     auto row = [&](int l) { return (d2 *) ((char *) (P + (size_t) (l >> 1) * 2 * Hp) + oj); };
+     gsf_steps<FN>(C, m, j < H, cst, [](int) {},
+                   [&](int l, bool odd, double v) {
+                        if (odd) *row(l) = d2{held, v};
+                        else held = v;
+                   });
+     if (C & 1) *row(C - 1) = d2{held, 0.};
 }
+// doubles of one plane of the expansion tables
+__host__ __device__ inline size_t gsf_plane(int C, int Hp) { return (size_t) ((C + 1) / 2) * 2 * Hp; }
 
 // ---------------------------------------------------------------------------
 // Per-size Mie coefficients.
@@ -725,7 +775,7 @@ struct FrontArgs {
      int Q, H, Hp, C, n1max;
      const double *guess;       // [(Q + 1) / 2] guesses of the roots, or NULL: angles given in mu
      double *mu, *w;
-     double *T;                 // [planes][C][Hp]
+     double *T;                 // expansion tables, planes of [(C + 1) / 2][Hp][2]
      int Kp, Kb, Hb;
      double *Bp, *Bm;           // [Kp][Hp]
      unsigned short *B16;
@@ -744,12 +794,13 @@ struct FrontArgs {
 
 template <int PK, bool TAN>
 __device__ __forceinline__ void front_body(const FrontArgs &p, unsigned b) {
-     __shared__ __align__(16) double cst[68 * GSF_CST];
+     __shared__ __align__(16) double cst[68 * GSF_CST];      // (also the Newton steps' and pi/tau factors)
+     static_assert(68 * GSF_CST >= UF_LDS, "factor buffers");
      const int lane = threadIdx.x;
      if (b < p.e_gsf) {
           const int na = p.Hp / 64, fn = b / na, j = (b % na) * 64 + lane;
-          const double m = angle_of(p.Q, p.H, p.guess, p.mu, j);
-          double *P = p.T + (size_t) fn * p.C * p.Hp;
+          const double m = angle_of(p.Q, p.H, p.guess, p.mu, j, cst);
+          double *P = p.T + (size_t) fn * gsf_plane(p.C, p.Hp);
           switch (fn) {
           case 0: gsf_role<0>(p.H, p.Hp, p.C, m, P, j, cst); break;
           case 1: gsf_role<1>(p.H, p.Hp, p.C, m, P, j, cst); break;
@@ -760,13 +811,13 @@ __device__ __forceinline__ void front_body(const FrontArgs &p, unsigned b) {
      } else if (b < p.e_pi) {
           if constexpr (PK == 1) {
                const int j = (b - p.e_gsf) * 64 + lane;
-               pitau_role(p.H, p.Hp, p.n1max, p.Kp, angle_of(p.Q, p.H, p.guess, p.mu, j), p.Bp, p.Bm, j);
+               pitau_role(p.H, p.Hp, p.n1max, p.Kp, angle_of(p.Q, p.H, p.guess, p.mu, j, cst), p.Bp, p.Bm, j, cst);
           } else if constexpr (PK > 1) {
                const int e = b - p.e_gsf, j = e / PITAU_SHARE * 64 + lane;
                typedef typename std::conditional<PK == 2, F16, BF16>::type E;
-               pitau16_role<E>(p.H, p.Hb, p.n1max, p.Kb, angle_of(p.Q, p.H, p.guess, p.mu, j), p.B16, j, e % PITAU_SHARE);
+               pitau16_role<E>(p.H, p.Hb, p.n1max, p.Kb, angle_of(p.Q, p.H, p.guess, p.mu, j, cst), p.B16, j, e % PITAU_SHARE, cst);
           }
-     } else if (b < p.e_gauss) gauss_role(p.Q, p.guess, p.mu, p.w, b - p.e_pi);
+     } else if (b < p.e_gauss) gauss_role(p.Q, p.guess, p.mu, p.w, b - p.e_pi, cst);
      else if (b < p.e_d) mie_chain_d<TAN>(p.ch, (int) (p.e_d - 1 - b) * 64 + lane);
      else if (b < p.e_psi) mie_chain_psi<TAN>(p.ch, (int) (p.e_psi - 1 - b) * 64 + lane);
      else if (b < p.e_ft) order_factors(p.n1max + 1, p.ft, (int) (b - p.e_psi) * 64 + lane);
@@ -1623,18 +1674,21 @@ constexpr int EXA_L = 32;
 __device__ __forceinline__ void expand_adjoint_part_body(const double *T, const double *gbar, const double *lbar, int H, int Hp, int C, double *part) {
      const int j = blockIdx.x * blockDim.x + threadIdx.x, ck = blockIdx.y;
      if (j >= Hp) return;
-     const size_t plane = (size_t) C * Hp;
+     typedef double d2 __attribute__((ext_vector_type(2)));
+     const size_t plane = gsf_plane(C, Hp) / 2;
+     const d2 *T2 = (const d2 *) T;
      double Em[6] = {0, 0, 0, 0, 0, 0}, Ep[6] = {0, 0, 0, 0, 0, 0};   // GSF rows
      double Lm[6] = {0, 0, 0, 0, 0, 0}, Lp[6] = {0, 0, 0, 0, 0, 0};   // Legendre rows
      const int l1 = min(C, (ck + 1) * EXA_L);
-     for (int l = ck * EXA_L; l < l1 && j < H; ++l) {
-          const double sl = (l & 1) ? -1. : 1., fl = (2 * l + 1) / 2.;
-          const size_t o = (size_t) l * Hp + j;
+     static_assert(EXA_L % 2 == 0, "whole rows of two l");
+     d2 q00 = {0., 0.}, q02 = q00, q22 = q00, q2m = q00, qpl = q00;
+     auto step = [&](int l, int u) {
+          const double sl = u ? -1. : 1., fl = (2 * l + 1) / 2.;
           if (gbar) {
                double cb[6];
                for (int k = 0; k < 6; ++k) cb[k] = gbar[(size_t) k * C + l] * fl;
                const double e1 = (cb[1] + cb[2]) / 2., e2 = (cb[1] - cb[2]) / 2.;
-               const double p00 = T[o], p02 = T[plane + o], p22 = T[2 * plane + o], p2m = T[3 * plane + o];
+               const double p00 = q00[u], p02 = q02[u], p22 = q22[u], p2m = q2m[u];
                Em[0] += sl * cb[0] * p00;  Ep[0] += cb[0] * p00;
                Em[1] += sl * e1 * p2m;     Ep[1] += e1 * p22;
                Em[2] += sl * e2 * p22;     Ep[2] += e2 * p2m;
@@ -1643,13 +1697,20 @@ __device__ __forceinline__ void expand_adjoint_part_body(const double *T, const 
                Em[5] += sl * cb[5] * p02;  Ep[5] += cb[5] * p02;
           }
           if (lbar) {
-               const double pl = T[4 * plane + o];
+               const double pl = qpl[u];
                for (int k = 0; k < 6; ++k) {
                     const double c = lbar[(size_t) k * C + l] * fl * (k == 5 ? -1. : 1.);
                     Lm[k] += sl * c * pl;
                     Lp[k] += c * pl;
                }
           }
+     };
+     for (int l = ck * EXA_L; l < l1 && j < H; l += 2) {
+          const size_t o = (size_t) (l / 2) * Hp + j;
+          if (gbar) { q00 = T2[o]; q02 = T2[plane + o]; q22 = T2[2 * plane + o]; q2m = T2[3 * plane + o]; }
+          if (lbar) qpl = T2[4 * plane + o];
+          step(l, 0);
+          if (l + 1 < l1) step(l + 1, 1);
      }
      double *out = part + (size_t) ck * 24 * Hp + j;
      for (int k = 0; k < 6; ++k) {
@@ -2710,78 +2771,93 @@ __global__ __launch_bounds__(256) void reduce_channels_b(const ReduceArgs *cases
 // mirrored (-) and direct (+) angles of every positive node j:
 //   GSF      F11, F11+F33, F11-F33, F33, F12, F34   (misc/rtutil_scat_int.c:173-183)
 //   Legendre F11, F11, F33, F33, F12, F34.
-// One wave per (l, channel): twelve dot products over the positive nodes,
-// folded with (-1)^l for the mirrored half, then the alpha/zeta recombination
-// and the (2l+1)/2 factor (misc/rtutil_scat_int.c:185-213, :436-469).  The
-// rows are formed from the elements as they are read (a launch of their own and
-// a third more reads otherwise).
+// One wave per (two l, channel): twelve dot products per l over the positive
+// nodes, folded with (-1)^l for the mirrored half, then the alpha/zeta
+// recombination and the (2l+1)/2 factor (misc/rtutil_scat_int.c:185-213,
+// :436-469).  The rows are formed from the elements as they are read (a launch of
+// their own otherwise), once for both l.
 __device__ __forceinline__ void expand_coefs_body(const double *T, const double *pf, const double *w, int Q, int Hp, int C, int gsf,
                                                   double *coefs) {
      const int lane = threadIdx.x & 63, H = Q / 2;
-     const int l = blockIdx.x * 4 + (threadIdx.x >> 6);
+     const int l0 = 2 * (blockIdx.x * 4 + (threadIdx.x >> 6));
      const int c = blockIdx.y;
-     if (l >= C) return;
-     const size_t plane = (size_t) C * Hp;
-     const double *P00 = T + (gsf ? 0 : 4 * plane) + (size_t) l * Hp, *P02 = T + plane + (size_t) l * Hp;
-     const double *P22 = T + 2 * plane + (size_t) l * Hp, *P2m = T + 3 * plane + (size_t) l * Hp;
+     if (l0 >= C) return;
+     typedef double d2 __attribute__((ext_vector_type(2)));
+     const size_t plane = gsf_plane(C, Hp), row = (size_t) l0 * Hp;
+     const d2 *P00 = (const d2 *) (T + (gsf ? 0 : 4 * plane) + row), *P02 = (const d2 *) (T + plane + row);
+     const d2 *P22 = (const d2 *) (T + 2 * plane + row), *P2m = (const d2 *) (T + 3 * plane + row);
      const double *P = pf + (size_t) c * 4 * Q;
-     double d[12];
+     double d[2][12];
 #pragma unroll
-     for (int r = 0; r < 12; ++r) d[r] = 0.;
+     for (int r = 0; r < 12; ++r) d[0][r] = d[1][r] = 0.;
      for (int j = lane; j < H; j += 64) {
-          const double p00 = P00[j], wq = w[H + j];
+          const d2 q00 = P00[j];
+          const double wq = w[H + j];
           double e[2][4];
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
                e[0][k] = P[(size_t) k * Q + H - 1 - j] * wq;
                e[1][k] = P[(size_t) k * Q + H + j] * wq;
           }
-          if (gsf) {
-               const double p02 = P02[j], p22 = P22[j], p2m = P2m[j];
+          d2 q02 = {0., 0.}, q22 = q02, q2m = q02;
+          if (gsf) { q02 = P02[j]; q22 = P22[j]; q2m = P2m[j]; }
 #pragma unroll
-               for (int s = 0; s < 2; ++s) {
-                    const double f11 = e[s][0], f33 = e[s][1], sum = f11 + f33, dif = f11 - f33;
-                    d[6 * s + 0] += p00 * f11;
-                    d[6 * s + 1] += (s ? p22 : p2m) * sum;
-                    d[6 * s + 2] += (s ? p2m : p22) * dif;
-                    d[6 * s + 3] += p00 * f33;
-                    d[6 * s + 4] += p02 * e[s][2];
-                    d[6 * s + 5] += p02 * e[s][3];
-               }
-          } else {
+          for (int u = 0; u < 2; ++u) {
+               const double p00 = q00[u];
+               if (gsf) {
+                    const double p02 = q02[u], p22 = q22[u], p2m = q2m[u];
 #pragma unroll
-               for (int s = 0; s < 2; ++s) {
-                    d[6 * s + 0] += p00 * e[s][0];
-                    d[6 * s + 1] += p00 * e[s][0];
-                    d[6 * s + 2] += p00 * e[s][1];
-                    d[6 * s + 3] += p00 * e[s][1];
-                    d[6 * s + 4] += p00 * e[s][2];
-                    d[6 * s + 5] += p00 * e[s][3];
+                    for (int s = 0; s < 2; ++s) {
+                         const double f11 = e[s][0], f33 = e[s][1], sum = f11 + f33, dif = f11 - f33;
+                         d[u][6 * s + 0] += p00 * f11;
+                         d[u][6 * s + 1] += (s ? p22 : p2m) * sum;
+                         d[u][6 * s + 2] += (s ? p2m : p22) * dif;
+                         d[u][6 * s + 3] += p00 * f33;
+                         d[u][6 * s + 4] += p02 * e[s][2];
+                         d[u][6 * s + 5] += p02 * e[s][3];
+                    }
+               } else {
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) {
+                         d[u][6 * s + 0] += p00 * e[s][0];
+                         d[u][6 * s + 1] += p00 * e[s][0];
+                         d[u][6 * s + 2] += p00 * e[s][1];
+                         d[u][6 * s + 3] += p00 * e[s][1];
+                         d[u][6 * s + 4] += p00 * e[s][2];
+                         d[u][6 * s + 5] += p00 * e[s][3];
+                    }
                }
           }
      }
 #pragma unroll
-     for (int r = 0; r < 12; ++r) {
-          double s = d[r];
+     for (int u = 0; u < 2; ++u)
 #pragma unroll
-          for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-          d[r] = s;
-     }
+          for (int r = 0; r < 12; ++r) {
+               double s = d[u][r];
+#pragma unroll
+               for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+               d[u][r] = s;
+          }
      if (lane == 0) {
-          const double sl = (l & 1) ? -1. : 1., fl = (2 * l + 1) / 2.;
-          double e[6];
 #pragma unroll
-          for (int k = 0; k < 6; ++k) e[k] = d[k] * sl + d[6 + k];
-          double *out = coefs + (size_t) c * 6 * C;
-          if (gsf) {
-               const double t = e[1];
-               e[1] = (t + e[2]) / 2.;
-               e[2] = (t - e[2]) / 2.;
-          } else {
-               e[5] = -e[5];
+          for (int u = 0; u < 2; ++u) {
+               const int l = l0 + u;
+               if (l >= C) break;
+               const double sl = (l & 1) ? -1. : 1., fl = (2 * l + 1) / 2.;
+               double e[6];
+#pragma unroll
+               for (int k = 0; k < 6; ++k) e[k] = d[u][k] * sl + d[u][6 + k];
+               double *out = coefs + (size_t) c * 6 * C;
+               if (gsf) {
+                    const double t = e[1];
+                    e[1] = (t + e[2]) / 2.;
+                    e[2] = (t - e[2]) / 2.;
+               } else {
+                    e[5] = -e[5];
+               }
+#pragma unroll
+               for (int k = 0; k < 6; ++k) out[(size_t) k * C + l] = e[k] * fl;
           }
-#pragma unroll
-          for (int k = 0; k < 6; ++k) out[(size_t) k * C + l] = e[k] * fl;
      }
 }
 __global__ __launch_bounds__(256) void expand_coefs(const double *T, const double *pf, const double *w, int Q, int Hp, int C, int gsf, double *coefs) { expand_coefs_body(T, pf, w, Q, Hp, C, gsf, coefs); }
@@ -2839,7 +2915,7 @@ __device__ __forceinline__ void phase_sums(int ncoef, int ld, const double *X, i
                }
                wave_lds_fence();
           },
-          [&](int l, double v) {
+          [&](int l, bool, double v) {
                if (FN > 0 && FN < 4 && l < 2) return;     // the functions start at l = 2
                const double *x = xs + (l - base) * NR;
 #pragma unroll
@@ -3642,7 +3718,7 @@ int alloc_forward(Workspace *w, const lmie_gpu_job *J, const FwdPlan &p) {
           return -1;
      if (p.Q <= 0) return 0;
      if (w->mu.get(sizeof(double) * Q) || w->w.get(sizeof(double) * Q) ||
-         (p.planes && w->T.get(sizeof(double) * p.planes * C * Hp)) ||
+         (p.planes && w->T.get(sizeof(double) * p.planes * gsf_plane(p.C, p.Hp))) ||
          (p.mixed ? w->B16.get(sizeof(unsigned short) * B16_PLANES * (size_t) p.Kb * p.Hb * 8)
                   : (w->Bp.get(sizeof(double) * (size_t) p.Kp * Hp) || w->Bm.get(sizeof(double) * (size_t) p.Kp * Hp))) ||
          w->pf.get(sizeof(double) * (size_t) p.nch * 4 * Q) ||
@@ -3836,7 +3912,7 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           tm.mark(LMIE_T_EXPAND, 0);
           for (int gsf = 1; gsf >= 0; --gsf)
                if (gsf ? gc : lc)
-                    hipLaunchKernelGGL(expand_coefs, dim3((C + 3) / 4, nch), dim3(256), 0, s, (const double *) w->T.as<double>(),
+                    hipLaunchKernelGGL(expand_coefs, dim3((C + 7) / 8, nch), dim3(256), 0, s, (const double *) w->T.as<double>(),
                                        (const double *) w->pf.as<double>(), (const double *) w->w.as<double>(), Q, p.Hp, C, gsf,
                                        res + ndot + (gsf ? 0 : nx));
           HIPCHECK(hipGetLastError());
@@ -3926,7 +4002,7 @@ int saved_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           FrontArgs fa;
           memset(&fa, 0, sizeof fa);
           const int planes = J->calc_lc ? 5 : J->calc_gc ? 4 : 0;
-          if (planes && w->T.get(sizeof(double) * planes * (size_t) C * Hp)) return -1;
+          if (planes && w->T.get(sizeof(double) * planes * gsf_plane(C, Hp))) return -1;
           fa.Q = Q; fa.H = H; fa.Hp = Hp; fa.C = C;
           fa.guess = w->sguess.as<double>(); fa.mu = w->mu.as<double>(); fa.w = w->w.as<double>(); fa.T = w->T.as<double>();
           fa.plan(planes, 0, true, 0, false);
@@ -3941,7 +4017,7 @@ int saved_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           for (int gsf = 1; gsf >= 0; --gsf) {
                double *dst = gsf ? R->gc_raw : R->lc_raw;
                if (!(gsf ? J->calc_gc : J->calc_lc) || !dst) continue;
-               hipLaunchKernelGGL(expand_coefs, dim3((C + 3) / 4, nch), dim3(256), 0, s, (const double *) w->T.as<double>(),
+               hipLaunchKernelGGL(expand_coefs, dim3((C + 7) / 8, nch), dim3(256), 0, s, (const double *) w->T.as<double>(),
                                   (const double *) w->pf.as<double>(), (const double *) w->w.as<double>(), Q, Hp, C, gsf,
                                   w->res.as<double>());
                HIPCHECK(hipGetLastError());
@@ -4230,7 +4306,7 @@ int fused_launch(std::vector<FwdCase *> &cs, Workspace *L) {
           for (int gs = 0; gs < 2; ++gs) {
                const unsigned on = (gs ? c.J->calc_gc : c.J->calc_lc) ? 1u : 0u;
                coefs[gs].push_back(expand_coefs_B{w->T.as<double>(), w->pf.as<double>(), w->w.as<double>(), p.Q, p.Hp, p.C, gs,
-                                                  res + 4 + (gs ? 0 : nx), (unsigned) (p.C + 3) / 4, on});
+                                                  res + 4 + (gs ? 0 : nx), (unsigned) (p.C + 7) / 8, on});
           }
           out[k] = CopyJob{res, (double *) w->pres.p, 4 + (c.J->calc_lc ? 2 * nx : nx)};
      }
@@ -4923,9 +4999,9 @@ int lmie_gpu_gsf_table(int n_mu, const double *mu, int n_l, double *out, int dev
      if (n_mu < 1 || n_l < 1) return set_err("n_mu < 1 or n_l < 1");
      if (!mu || !out) return set_err("missing argument");
      HIPCHECK(hipSetDevice(device));
-     // the expansion tables' role reads the angles at mu[H + j], j < H, and writes [5][n_l][Hp]
+     // the expansion tables' role reads the angles at mu[H + j], j < H, and writes 5 planes of rows of two l
      const int H = n_mu, Hp = rup(H, 64);
-     const size_t tab = (size_t) 5 * n_l * Hp;
+     const size_t pl = gsf_plane(n_l, Hp), tab = 5 * pl;
      double *d = nullptr;
      HIPCHECK(hipMalloc(&d, sizeof(double) * (2 * (size_t) H + tab)));
      HIPCHECK(hipMemcpy(d + H, mu, sizeof(double) * H, hipMemcpyHostToDevice));
@@ -4937,7 +5013,10 @@ int lmie_gpu_gsf_table(int n_mu, const double *mu, int n_l, double *out, int dev
      std::vector<double> t(tab);
      HIPCHECK(hipMemcpy(t.data(), d + 2 * H, sizeof(double) * tab, hipMemcpyDeviceToHost));
      HIPCHECK(hipFree(d));
-     for (size_t r = 0; r < (size_t) 5 * n_l; ++r) memcpy(out + r * H, t.data() + r * Hp, sizeof(double) * H);
+     for (int q = 0; q < 5; ++q)
+          for (int l = 0; l < n_l; ++l)
+               for (int j = 0; j < H; ++j)
+                    out[((size_t) q * n_l + l) * H + j] = t[q * pl + ((size_t) (l / 2) * Hp + j) * 2 + (l & 1)];
      return 0;
 }
 
