@@ -763,11 +763,11 @@ __device__ __forceinline__ void order_factors(int n, double *ft, int j) {
 }
 // One launch for the roles of the front: blocks of one wave, the longest
 // dependence chains first.  Measured at 3810 angles and 32768 sizes (each
-// role launched alone): the Gauss rule 0.26 ms (three Newton steps in its
-// slowest wave), with the expansion tables behind it 0.39 (the tables alone
-// 0.53 before their factors came from LDS), with the split pi/tau tables 0.33
-// (0.28 in one wave before, behind the rule), the chains 0.27 (0.34 with D kept to
-// n2); all of them 0.39-0.42, against five launches on three streams before.  Block ranges (ends): the expansion tables (planes
+// role launched alone): the Gauss rule 0.14 ms (three Newton steps in its
+// slowest wave), with the expansion tables behind it 0.27, with the pi/tau tables
+// 0.22 (split: 0.21), the chains 0.27 (0.36 with D kept to n2); all of them 0.31
+// (0.41).  The factors common to a wave taken from its lanes instead of LDS: 0.26,
+// 0.39, 0.36, and 0.39 for all.  Block ranges (ends): the expansion tables (planes
 // x angle blocks), the pi/tau tables (x PITAU_SHARE split), the Gauss rule, the
 // D chains, the psi and chi chains (heaviest sizes first), the order factors.
 // PK: pi/tau tables, 0 none, 1 FP64, 2 split fp16, 3 split bf16.
@@ -1742,7 +1742,10 @@ __global__ __launch_bounds__(64) void expand_adjoint_part_b(const expand_adjoint
 // per (node, row) adding the chunks in order, then the row combinations per
 // node through LDS.
 constexpr int EXF_J = 32;
-__device__ __forceinline__ void expand_adjoint_fin_body(const double *part, int nck, const double *w, int H, int Hp, int Q, double *pfbar) {
+// adjw: the halved combinations that the FP64 reverse contraction takes
+// (AdjArgs::wts), zero up to a whole stage of angles past H, or NULL.
+__device__ __forceinline__ void expand_adjoint_fin_body(const double *part, int nck, const double *w, int H, int Hp, int Q, double *pfbar,
+                                                        double *adjw) {
      __shared__ double sv[24][EXF_J];
      const int jj = threadIdx.x % EXF_J, k = threadIdx.x / EXF_J, j = blockIdx.x * EXF_J + jj;
      double v = 0.;
@@ -1761,7 +1764,12 @@ __device__ __forceinline__ void expand_adjoint_fin_body(const double *part, int 
      }
      sv[k][jj] = v;
      __syncthreads();
-     if (k || j >= H) return;
+     if (k) return;
+     if (j >= H) {
+          if (adjw && j < Hp)
+               for (int r = 0; r < 8; ++r) adjw[(size_t) j * 8 + r] = 0.;
+          return;
+     }
      double vv[24];
      for (int r = 0; r < 24; ++r) vv[r] = sv[r][jj];
      const int ip = H + j, im = H - 1 - j;
@@ -1769,13 +1777,22 @@ __device__ __forceinline__ void expand_adjoint_fin_body(const double *part, int 
      for (int s = 0; s < 2; ++s) {
           const double *E = vv + (s ? 6 : 0), *L = vv + (s ? 18 : 12);
           const int a = s ? ip : im;
-          pfbar[a] = wq * (E[0] + E[1] + E[2] + L[0] + L[1]);
-          pfbar[Q + a] = wq * (E[1] - E[2] + E[3] + L[2] + L[3]);
-          pfbar[2 * Q + a] = wq * (E[4] + L[4]);
-          pfbar[3 * Q + a] = wq * (E[5] + L[5]);
+          const double p0 = wq * (E[0] + E[1] + E[2] + L[0] + L[1]), p1 = wq * (E[1] - E[2] + E[3] + L[2] + L[3]);
+          const double p2 = wq * (E[4] + L[4]), p3 = wq * (E[5] + L[5]);
+          pfbar[a] = p0;
+          pfbar[Q + a] = p1;
+          pfbar[2 * Q + a] = p2;
+          pfbar[3 * Q + a] = p3;
+          if (adjw) {
+               double *o = adjw + (size_t) j * 8 + (s ? 0 : 4);
+               o[0] = .5 * (p0 + p1);
+               o[1] = .5 * (p0 - p1);
+               o[2] = .5 * p2;
+               o[3] = .5 * p3;
+          }
      }
 }
-__global__ __launch_bounds__(24 * EXF_J) void expand_adjoint_fin(const double *part, int nck, const double *w, int H, int Hp, int Q, double *pfbar) { expand_adjoint_fin_body(part, nck, w, H, Hp, Q, pfbar); }
+__global__ __launch_bounds__(24 * EXF_J) void expand_adjoint_fin(const double *part, int nck, const double *w, int H, int Hp, int Q, double *pfbar, double *adjw) { expand_adjoint_fin_body(part, nck, w, H, Hp, Q, pfbar, adjw); }
 struct expand_adjoint_fin_B {
      const double *part;
      int nck;
@@ -1789,18 +1806,19 @@ struct expand_adjoint_fin_B {
 __global__ __launch_bounds__(24 * EXF_J) void expand_adjoint_fin_b(const expand_adjoint_fin_B *cases) {
      const expand_adjoint_fin_B a = cases[blockIdx.z];
      if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     expand_adjoint_fin_body(a.part, a.nck, a.w, a.H, a.Hp, a.Q, a.pfbar);
+     expand_adjoint_fin_body(a.part, a.nck, a.w, a.H, a.Hp, a.Q, a.pfbar, nullptr);
 }
 
 
-// Cotangents of the four complex sums at one (size, angle) from those of the
+// Cotangents of the two complex sums at one (size, angle) from those of the
 // four matrix elements (gradient convention d/dRe + i d/dIm):
 //   sp^ = (p0 + p1) sp/2 - (p2 + i p3) sm/2,  sm^ = (p0 - p1) sm/2 - (p2 - i p3) sp/2,
 // the adjoint of P11 = (|sp|^2 + |sm|^2)/4, P33 = (|sp|^2 - |sm|^2)/4,
-// P12 = -Re(sp sm*)/2, P34 = -Im(sp sm*)/2 (src/lmie_core.c:726-744).
-__device__ __forceinline__ void stokes_adj(double spr, double spi, double smr, double smi, const double pb[4],
+// P12 = -Re(sp sm*)/2, P34 = -Im(sp sm*)/2 (src/lmie_core.c:726-744);
+// w = (p0 + p1)/2, (p0 - p1)/2, p2/2, p3/2.
+__device__ __forceinline__ void stokes_adj(double spr, double spi, double smr, double smi, const double w[4],
                                            double out[4]) {
-     const double a = .5 * (pb[0] + pb[1]), c = .5 * (pb[0] - pb[1]), p2 = .5 * pb[2], p3 = .5 * pb[3];
+     const double a = w[0], c = w[1], p2 = w[2], p3 = w[3];
      out[0] = a * spr - (p2 * smr - p3 * smi);
      out[1] = a * spi - (p2 * smi + p3 * smr);
      out[2] = c * smr - (p2 * spr + p3 * spi);
@@ -1809,15 +1827,18 @@ __device__ __forceinline__ void stokes_adj(double spr, double spi, double smr, d
 
 // Angular part of the size-weight cotangent: fbar_i = sum_{j, +-, k} pfbar_k P_k(i, j),
 // one wave per size point.
-__global__ __launch_bounds__(256) void fbar_angular(const double *sst, const double *pfbar, int N, int H, int Hp,
+__global__ __launch_bounds__(256) void fbar_angular(const double *sst, const double *pfbar, int N, int Np, int H, int Hp,
                                                     int Q, double *fang) {
      const int lane = threadIdx.x & 63;
      const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
      if (i >= N) return;
+     const size_t plane = (size_t) Np * Hp;
      double acc = 0.;
      for (int j = lane; j < H; j += 64) {
-          const double *q = sst + ((size_t) i * Hp + j) * 8;
-          double Pp[4], Pm[4];
+          const double *o = sst + (size_t) i * Hp + j;
+          double q[8], Pp[4], Pm[4];
+#pragma unroll
+          for (int c = 0; c < 8; ++c) q[c] = o[c * plane];
           stokes(q[0], q[1], q[2], q[3], Pp);
           stokes(q[4], q[5], q[6], q[7], Pm);
           for (int k = 0; k < 4; ++k)
@@ -1827,90 +1848,162 @@ __global__ __launch_bounds__(256) void fbar_angular(const double *sst, const dou
      if (lane == 0) fang[i] = acc;
 }
 
+// waits until at most n of this wave's vector memory operations are in
+// flight (vmcnt in bits 3:0 and 15:14) and its LDS reads have returned (lgkmcnt 0, so
+// a barrier behind it frees the buffer they read); expcnt left open
+template <int n>
+__device__ __forceinline__ void wait_vm() {
+     static_assert(n < 64, "vmcnt field");
+     __builtin_amdgcn_s_waitcnt(0x0070 | (n & 15) | ((n >> 4) << 14));
+}
+
 // Transposed angular contraction on FP64 matrix cores: for every size i and
 // order n,
 //   Sbar_n = f_i sum_j [sp^+ (pi+tau)_n + s_n sp^- (pi-tau)_n],
 //   Tbar_n = f_i sum_j [sm^+ (pi-tau)_n + s_n sm^- (pi+tau)_n],
-// K = the positive angles j (16 per LDS stage), the cotangents of the sums
-// formed while staging from the checkpointed sums.  Tile 32 sizes x 32 orders.
+// K = the positive angles.  Both operands lie along K in memory (the checkpointed
+// sums [8][Np][Hp], the tables [Kp][Hp]), so a stage of ADJ_KS = 8 angles is 64
+// bytes a row, filled by direct loads (16 bytes a lane, 16 rows a load).  LDS rows
+// have no padding; the four 16-byte pieces of row r sit at piece ^ (r / 4 & 3)
+// (each lane fetches the piece its place belongs to), so the 16 rows x 2 angles that
+// half a wave reads fall in different banks.  A wave owns 16 sizes x 16 BO orders,
+// 4 sums each; it forms the cotangents of its 16 sizes from the sums and the
+// angle's weights in registers (28 operations for BO x 8 matrix instructions), so
+// no pass over the checkpoint writes them.  Four waves (2 x 2) share a tile of 32
+// sizes and its two stages, one barrier each, one stage ahead; three workgroups
+// per CU.
+// What bounds it: the FP64 matrix cores (64 cycles per instruction and SIMD), at about
+// 85% of the rate of angular_f64 (two modes of 32768 sizes, 3810 angles: 17.8 ms with
+// the passes around it, 14.3 for the same products there): the cotangents' vector
+// operations, and half lines per row and stage.
+constexpr int ADJ_KS = 8;
+
+// Orders per task of the contraction over size tiles of 32 with kt orders each:
+// 64 (three of every four products then share their cotangents with another)
+// unless the tasks of 32 are all resident at once (three workgroups on each of
+// 256 CUs) and leave the fullest CU less to do: it gets ceil(tasks / 256) tasks of
+// one unit, or half as many of two.  Measured, 32 and 64: 1024 sizes of up to 135
+// orders (91 and 53 tasks) 48 and 58 us for the angular part, 3965 of 251 (577, 319)
+// 121 and 134, 2048 of 372 (424, 227) 126 and 122, 4096 of 372 (842, 452) 200 and
+// 184, 16384 of 954 (8063, 4159) 3150 and 2660.  128 orders on eight waves gave
+// the same as 64; stages of 16 angles, which leave one workgroup to a CU, 3040-3650.
+// The kernel before (32 x 32, the checkpoint by size and angle, staged through
+// registers) took 65, 215, 260, 394 and 6490.
+int adj_f64_orders(const std::vector<int> &kt) {
+     int t32 = 0, t64 = 0;
+     for (int k : kt) {
+          t32 += (k + 31) / 32;
+          t64 += (k + 63) / 64;
+     }
+     return t32 <= 3 * 256 && (t32 + 255) / 256 < 2 * ((t64 + 255) / 256) ? 32 : 64;
+}
+
 struct AdjArgs {
-     int Np, Kp, Hp, H, Q;
-     const double *sst;         // [Np][Hp][8]
-     const double *pfbar;       // [4][Q]
+     int Np, Kp, Hp, H;
+     const double *sst;         // [8][Np][Hp]
+     const double *wts;         // [Hp + 8][8]: stokes_adj's w at +mu_j, then at -mu_j
      const double *Bp, *Bm;     // [Kp][Hp]
      const double *f;           // [Np]
-     const int *ktile;          // orders per size tile of 32
+     const int2 *task;          // (size tile, order tile), (-1, -1) none
      double *bar;               // [4][Kp][Np]: Sbar re, im, Tbar re, im
 };
 
-__global__ __launch_bounds__(256) void angular_adj_f64(AdjArgs p) {
-     constexpr int JC = 16, TM = 32, TN = 32, SA = TM + 16, SB = TN + 16;
-     __shared__ double sA[8 * JC * SA];
-     __shared__ double sB[2 * JC * SB];
-     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-     const int wm = wave & 1, wn = wave >> 1;
+template <int BO>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void angular_adj_f64(AdjArgs p) {
+     constexpr int WO = 2, WI = 2, NW = WO * WI, KS = ADJ_KS, TO = 16 * WO * BO, TI = 16 * WI;
+     constexpr int XSTG = 8 * TI * KS, BSTG = 2 * TO * KS, STG = XSTG + BSTG + 128;
+     constexpr int NL = (XSTG + BSTG) / (128 * NW);   // direct loads per wave and stage, and the weights'
+     static_assert((XSTG + BSTG) % (128 * NW) == 0 && XSTG % 128 == 0, "whole 1 KiB loads");
+     __shared__ double sh[2 * STG];
+
+     const int2 tk = p.task[blockIdx.x];
+     if (tk.x < 0) return;
+     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+     const int wo = wave % WO, wi = wave / WO;
      const int l16 = lane & 15, lg = lane >> 4;
-     const int n0 = blockIdx.x * TN, it0 = blockIdx.y * TM;
-     if (n0 >= p.ktile[blockIdx.y]) return;          // whole tile beyond these sizes' orders
-     const size_t Np = p.Np, Hp = p.Hp, plane = (size_t) p.Kp * Np;
-     v4d acc[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
-     const int ncol = wn * 16 + l16;                  // this lane's output order (B column)
-     const double sg = ((n0 + ncol) & 1) ? -1. : 1.;   // s_n, n = n0 + ncol + 1
-     for (int j0 = 0; j0 < p.H; j0 += JC) {
-          __syncthreads();
-          // stage the cotangents of the sums: 32 sizes x 16 angles
-          for (int e = threadIdx.x; e < TM * JC; e += 256) {
-               const int ii = e % TM, jj = e / TM;
-               const int i = it0 + ii, j = j0 + jj;
-               double out[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-               if (j < p.H) {
-                    const double *q = p.sst + ((size_t) i * Hp + j) * 8;
-                    double pb[4], pm[4];
-                    for (int k = 0; k < 4; ++k) {
-                         pb[k] = p.pfbar[k * p.Q + p.H + j];
-                         pm[k] = p.pfbar[k * p.Q + p.H - 1 - j];
-                    }
-                    stokes_adj(q[0], q[1], q[2], q[3], pb, out);      // sp^+, sm^+
-                    stokes_adj(q[4], q[5], q[6], q[7], pm, out + 4);  // sp^-, sm^-
-               }
-               for (int c = 0; c < 8; ++c) sA[(c * JC + jj) * SA + ii] = out[c];
-          }
-          // stage pi +- tau: rows = angles, columns = orders n0 .. n0 + 31
-          for (int e = threadIdx.x; e < TN * JC; e += 256) {
-               const int nn = e % TN, jj = e / TN;
-               const int j = j0 + jj;
-               const size_t o = (size_t) (n0 + nn) * Hp + j;
-               sB[jj * SB + nn] = j < p.H ? p.Bp[o] : 0.;
-               sB[(JC + jj) * SB + nn] = j < p.H ? p.Bm[o] : 0.;
-          }
-          __syncthreads();
+     const int it0 = tk.x * TI, n0 = tk.y * TO;
+     const size_t Np = p.Np, Hp = p.Hp, plane = (size_t) p.Kp * Np, splane = Np * Hp;
+
+     // this lane's source of each of the wave's loads (row, swizzled piece) at
+     // angle 0; rows past the tables are clamped (their orders are not stored)
+     const double *src[NL];
 #pragma unroll
-          for (int ks = 0; ks < JC / 4; ++ks) {
-               const int r = ks * 4 + lg;
-               const int ic = wm * 16 + l16;
-               const double bp = sB[r * SB + ncol], bm = sB[(JC + r) * SB + ncol];
-               const double bps = sg * bp, bms = sg * bm;
-               const double spr = sA[(0 * JC + r) * SA + ic], spi = sA[(1 * JC + r) * SA + ic];
-               const double smr = sA[(2 * JC + r) * SA + ic], smi = sA[(3 * JC + r) * SA + ic];
-               const double qpr = sA[(4 * JC + r) * SA + ic], qpi = sA[(5 * JC + r) * SA + ic];
-               const double qmr = sA[(6 * JC + r) * SA + ic], qmi = sA[(7 * JC + r) * SA + ic];
-               acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(spr, bp, acc[0], 0, 0, 0);
-               acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(qpr, bms, acc[0], 0, 0, 0);
-               acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(spi, bp, acc[1], 0, 0, 0);
-               acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(qpi, bms, acc[1], 0, 0, 0);
-               acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(smr, bm, acc[2], 0, 0, 0);
-               acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(qmr, bps, acc[2], 0, 0, 0);
-               acc[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(smi, bm, acc[3], 0, 0, 0);
-               acc[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(qmi, bps, acc[3], 0, 0, 0);
+     for (int u = 0; u < NL; ++u) {
+          const int e = (wave + NW * u) * 128 + 2 * lane;
+          const int row = (e < XSTG ? e : e - XSTG) / KS, piece = (lane & 3) ^ (row >> 2 & 3);
+          if (e < XSTG) src[u] = p.sst + (row / TI) * splane + (size_t) (it0 + row % TI) * Hp + 2 * piece;
+          else src[u] = (row / TO ? p.Bm : p.Bp) + (size_t) min(n0 + row % TO, p.Kp - 1) * Hp + 2 * piece;
+     }
+     const double *wsrc = p.wts + 2 * lane;
+     auto stage_load = [&](int buf) {
+#pragma unroll
+          for (int u = 0; u < NL; ++u) {
+               __builtin_amdgcn_global_load_lds((const void *) src[u], (lds_ptr) (sh + buf * STG + (wave + NW * u) * 128), 16, 0, 0);
+               src[u] += KS;
+          }
+          // 1 KiB of weights: this stage's 8 angles and the next 8 (unused)
+          if (wave == 0) __builtin_amdgcn_global_load_lds((const void *) wsrc, (lds_ptr) (sh + buf * STG + XSTG + BSTG), 16, 0, 0);
+          wsrc += KS * 8;
+     };
+
+     v4d acc[BO][4];
+#pragma unroll
+     for (int b = 0; b < BO; ++b)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) acc[b][q] = v4d{0., 0., 0., 0.};
+     // s_n of this lane's table rows n0 + ... + l16 (row n holds order n + 1)
+     const unsigned long long sgn = (unsigned long long) (l16 & 1) << 63;
+     auto flip = [&](double v) { return __longlong_as_double((long long) ((unsigned long long) __double_as_longlong(v) ^ sgn)); };
+     // this lane's angle 4 ks + lg of row l16 in a tile of rows
+     const int o0 = l16 * KS + (((lg >> 1) ^ (l16 >> 2 & 3)) << 1) + (lg & 1);
+     const int nst = (p.H + KS - 1) / KS;
+     if (nst > 0) stage_load(0);
+     for (int k = 0; k < nst; ++k) {
+          const int buf = k & 1;
+          wait_vm<0>();                           // this wave's loads of the stage
+          __builtin_amdgcn_s_barrier();           // everyone's; the other buffer is free
+          __asm__ volatile("" ::: "memory");
+          if (k + 1 < nst) stage_load(buf ^ 1);
+          const double *x0 = sh + buf * STG + 16 * wi * KS, *b0 = sh + buf * STG + XSTG + 16 * BO * wo * KS;
+          const double *w0 = sh + buf * STG + XSTG + BSTG + lg * 8;
+#pragma unroll
+          for (int ks = 0; ks < KS / 4; ++ks) {
+               const int o = o0 ^ (4 * ks);       // pieces 0, 1 <-> 2, 3
+               double x[8], wq[8], xp[4], xm[4];
+#pragma unroll
+               for (int c = 0; c < 8; ++c) x[c] = x0[c * TI * KS + o];
+#pragma unroll
+               for (int c = 0; c < 8; ++c) wq[c] = w0[ks * 32 + c];
+               stokes_adj(x[0], x[1], x[2], x[3], wq, xp);          // sp^+, sm^+
+               stokes_adj(x[4], x[5], x[6], x[7], wq + 4, xm);      // sp^-, sm^-
+#pragma unroll
+               for (int b = 0; b < BO; ++b) {
+                    const double bp = b0[16 * b * KS + o], bm = b0[(TO + 16 * b) * KS + o];
+                    const double sbp = flip(bp), sbm = flip(bm);
+                    v4d *q = acc[b];
+                    q[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(bp, xp[0], q[0], 0, 0, 0);
+                    q[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(bp, xp[1], q[1], 0, 0, 0);
+                    q[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(bm, xp[2], q[2], 0, 0, 0);
+                    q[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(bm, xp[3], q[3], 0, 0, 0);
+                    q[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(sbm, xm[0], q[0], 0, 0, 0);
+                    q[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(sbm, xm[1], q[1], 0, 0, 0);
+                    q[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(sbp, xm[2], q[2], 0, 0, 0);
+                    q[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(sbp, xm[3], q[3], 0, 0, 0);
+               }
           }
      }
-     // result rows (sizes) l/16 + 4 v, column (order) l % 16
-     for (int v = 0; v < 4; ++v) {
-          const int i = it0 + wm * 16 + lg + 4 * v;
-          const int n = n0 + ncol;            // row n of the planes holds order n + 1
-          const double fi = p.f[i];
-          for (int c = 0; c < 4; ++c) p.bar[c * plane + (size_t) n * Np + i] = fi * acc[c][v];
-     }
+     // result rows (orders) l / 16 + 4 v, column (size) l % 16
+     const int i = it0 + 16 * wi + l16;
+     const double fi = p.f[i];
+#pragma unroll
+     for (int b = 0; b < BO; ++b)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+               const int n = n0 + 16 * (BO * wo + b) + lg + 4 * v;
+               if (n >= p.Kp) continue;
+#pragma unroll
+               for (int c = 0; c < 4; ++c) p.bar[c * plane + (size_t) n * Np + i] = fi * acc[b][c][v];
+          }
 }
 
 // ---------------------------------------------------------------------------
@@ -3068,7 +3161,7 @@ struct Workspace {
      PinBuf finPin;
      int home = -1, busy = 0;       // batch slot of this workspace (-1: general pool)
      int n2rows = 0, ng = 0;
-     int ushape = 8;                // reverse contraction: shape
+     int ushape = 8;                // reverse contraction: shape (FP64: orders per task)
      int valid = 0;
      int N = 0, Np = 0, Kp = 0, Hp = 0, H = 0, Q = 0, C = 0, n1max = 0, n2max = 0, calc_gc = 0, calc_lc = 0;
      int mixed = 0, bf16 = 0, Kb = 0, Hb = 0;
@@ -3204,16 +3297,8 @@ struct F64Args {
      int nP, nX;
      double *part;              // [size tiles][channels][4][Q]
      double *save2;             // [4][N][Q] per-size matrix (save_control 1) or NULL
-     double *sst;               // reverse-pass checkpoint [Np][Hp][8]: sp+, sm+, sp-, sm- (re, im) or NULL
+     double *sst;               // reverse-pass checkpoint [8][Np][Hp]: sp+, sm+, sp-, sm- (re, im) or NULL
 };
-
-// waits until at most n of this wave's vector memory operations are in
-// flight (vmcnt in bits 3:0 and 15:14; lgkmcnt and expcnt left open)
-template <int n>
-__device__ __forceinline__ void wait_vm() {
-     static_assert(n < 64, "vmcnt field");
-     __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
-}
 
 template <int WM, int WN, bool HX, bool HM, int KS, int ST, int OCC>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OCC))) void angular_f64(F64Args p) {
@@ -3323,9 +3408,9 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
           for (int v = 0; v < 4; ++v) {
                const int i = i0 + 4 * v;
                if (p.sst) {
-                    double *o = p.sst + ((size_t) i * Hp + j) * 8;
+                    double *o = p.sst + (size_t) i * Hp + j;
 #pragma unroll
-                    for (int c = 0; c < 8; ++c) o[c] = acc[0][c][v];
+                    for (int c = 0; c < 8; ++c) o[c * Np * Hp] = acc[0][c][v];
                }
                if (p.save2 && i < p.N && j < p.H) {
                     double Pp[4], Pm[4];
@@ -3641,6 +3726,9 @@ int stage_forward(Workspace *w, const lmie_gpu_job *J, const FwdPlan &p, bool ba
           w->ushape = batch ? 8 : ugemm_waves();       // fused passes run the 128-size shape
           const std::vector<int> &kts = w->ushape == 2 ? p.kt64 : p.kt128;
           xcd_tasks(kts, [&](int t) { return (kts[t] + 63) / 64; }, tile_group(), rtask);
+     } else if (p.keep && p.Q > 0) {
+          w->ushape = adj_f64_orders(p.kt32);
+          xcd_tasks(p.kt32, [&](int t) { return (p.kt32[t] + w->ushape - 1) / w->ushape; }, F64_GROUP, rtask);
      }
      w->rtask = rtask;
      Stage st;
@@ -4050,7 +4138,8 @@ int alloc_reverse(Workspace *w, bool use_u) {
          (w->Q > 0 && w->expart.get(sizeof(double) * 24 * nck * w->Hp)))
           return -1;
      if (!use_u)
-          return w->fang.get(sizeof(double) * Np) || w->bar.get(sizeof(double) * 4 * (size_t) w->Kp * Np) ? -1 : 0;
+          return w->fang.get(sizeof(double) * Np) || w->bar.get(sizeof(double) * 4 * (size_t) w->Kp * Np) ||
+                         w->wts.get(sizeof(double) * 8 * ((size_t) w->Hp + ADJ_KS)) ? -1 : 0;
      return w->wts.get(sizeof(double) * 8 * Hq) || w->scal.get(sizeof(AdjScal)) ||
                     w->L16.get(sizeof(unsigned short) * 4 * Hq * Kq) || w->R16.get(sizeof(unsigned short) * 16 * Hq * Kq) ||
                     w->Gf.get(sizeof(float) * 4 * Kq * Kq) || w->G16.get(sizeof(unsigned short) * 12 * Kq * Kq) ||
@@ -4167,21 +4256,26 @@ int adjoint_impl(Workspace *w, const lmie_gpu_adj_in *in, lmie_gpu_adj_out *out)
                              use_gc ? (const double *) g : nullptr, use_lc ? (const double *) (g + 6 * C) : nullptr,
                              H, Hp, C, w->expart.as<double>());
           hipLaunchKernelGGL(expand_adjoint_fin, dim3((H + EXF_J - 1) / EXF_J), dim3(24 * EXF_J), 0, s, (const double *) w->expart.as<double>(),
-                             nck, (const double *) w->w.as<double>(), H, Hp, Q, w->pfbar.as<double>());
+                             nck, (const double *) w->w.as<double>(), H, Hp, Q, w->pfbar.as<double>(),
+                             w->mixed ? nullptr : w->wts.as<double>());
      }
      if (w->mixed && Q > 0 && (use_gc || use_lc)) {
           if (adjoint_mixed_angular(w, s, tm)) return -1;
           tm.mark(LMIE_T_ADJ_ANGULAR, 1);
      } else if (Q > 0 && (use_gc || use_lc)) {
           hipLaunchKernelGGL(fbar_angular, dim3((N + 3) / 4), dim3(256), 0, s, (const double *) w->sst.as<double>(),
-                             (const double *) w->pfbar.as<double>(), N, H, Hp, Q, w->fang.as<double>());
+                             (const double *) w->pfbar.as<double>(), N, Np, H, Hp, Q, w->fang.as<double>());
           r.fang = w->fang.as<double>();
           AdjArgs aa;
-          aa.Np = Np; aa.Kp = Kp; aa.Hp = Hp; aa.H = H; aa.Q = Q;
-          aa.sst = w->sst.as<double>(); aa.pfbar = w->pfbar.as<double>();
+          aa.Np = Np; aa.Kp = Kp; aa.Hp = Hp; aa.H = H;
+          aa.sst = w->sst.as<double>(); aa.wts = w->wts.as<double>();
           aa.Bp = w->Bp.as<double>(); aa.Bm = w->Bm.as<double>();
-          aa.f = w->f.as<double>(); aa.ktile = w->ktile32.as<int>(); aa.bar = w->bar.as<double>();
-          hipLaunchKernelGGL(angular_adj_f64, dim3(Kp / 32, Np / 32), dim3(256), 0, s, aa);
+          aa.f = w->f.as<double>(); aa.task = w->tasks.as<int2>(); aa.bar = w->bar.as<double>();
+          if (!w->rtask.empty()) {
+               const dim3 g((unsigned) w->rtask.size());
+               if (w->ushape == 64) hipLaunchKernelGGL(angular_adj_f64<2>, g, dim3(256), 0, s, aa);
+               else hipLaunchKernelGGL(angular_adj_f64<1>, g, dim3(256), 0, s, aa);
+          }
           HIPCHECK(hipGetLastError());
           tm.mark(LMIE_T_ADJ_ANGULAR, 1);
      } else {

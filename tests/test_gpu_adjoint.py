@@ -345,3 +345,29 @@ def test_batch_larger_than_one_group(product):
         out, g = lmie.adjoint(product, [cases[k]], None, loss_fn(refs[k], 200 + k), "mixed")
         assert np.array_equal(out_b["gc"], out["gc"]), k
         assert g_b["mr"] == g["mr"] and g_b["a1"] == g["a1"] and g_b["a2"] == g["a2"], k
+
+
+@pytest.mark.parametrize("n_int2,n_quad,r2", [(1, 33, 0.4), (3, 43, 3.0), (1, 129, 6.0), (20, 50, 40.0), (61, 37, 22.0),
+                                              (61, 64, 30.0)])
+def test_fp64_reverse_contraction_at_tile_edges(product, n_int2, n_quad, r2):
+    """The FP64 reverse contraction where its tiles end: 33 to 3904 sizes (one
+    past a tile, odd counts), angles that fill no stage of 8, orders on both of
+    its tile heights (32 orders up to 1000 sizes here, 64 beyond), against the
+    forward tangents contracted with the same random expansion cotangents."""
+    p = dict(FD_CASE, n_int2=n_int2, n_quad=n_quad, r2=r2)
+    say("case: fp64 reverse contraction", n_int2, n_quad, r2)
+    names = ("lambda", "mr", "mi", "a1", "r2")
+    # at x = k pi (3 x 43 to 3.0 has a node at 5 pi) the forward tangents along x
+    # carry a factor 1 / sin x of rounding error, in the reference's ratio chain too
+    # (psi_j from psi_0 = sin x): those directions are no oracle there
+    edges = np.linspace(p["r1"], r2, n_int2 + 1)
+    nodes = np.add.outer(edges[1:] + edges[:-1], np.outer(edges[1:] - edges[:-1], np.polynomial.legendre.leggauss(n_quad)[0])[0]) / 2
+    if np.abs(np.sin(2 * np.pi * nodes / p["lambda"])).min() < 1e-8:
+        names = ("mr", "mi", "a1")
+    eye = np.eye(len(names))
+    tan = lmie.solve(product, p, {k: list(eye[i]) for i, k in enumerate(names)}, "fp64")
+    rng = np.random.Generator(np.random.PCG64(29))
+    cot = {k: rng.standard_normal(tan[k].shape) / np.abs(tan[k]).max(axis=1, keepdims=True) for k in ("gc", "lc")}
+    ref = sum(np.einsum("dkl,kl->d", tan[k + "_l"], cot[k]) for k in ("gc", "lc"))
+    _, g = lmie.adjoint(product, [p], None, lambda o: cot, "fp64")
+    check([g[k] for k in names], ref, TOL["fp64"], "%d x %d" % (n_int2, n_quad))
