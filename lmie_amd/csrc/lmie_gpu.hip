@@ -262,34 +262,40 @@ __device__ __forceinline__ void uniform_steps(int n, double *lds, G factor, F st
           if (i0 + 64 < n) lds[(c ^ 1) * UF_ROW + lane] = factor(i0 + 64 + lane);
           wave_lds_fence();
           const double *t = lds + c * UF_ROW;
-          const int m = min(64, n - i0);
-          double a[8], b[8];          // (read past 64: spare entries, unused)
-          auto read = [&](double *v, int o) {
+          if (n - i0 >= 64) {
+               // (a loop of a constant count: with the remainder in the same loop a step
+               // took a fifth longer)
+               double a[8], b[8];
 #pragma unroll
-               for (int k = 0; k < 8; ++k) v[k] = t[o + k];
-          };
-          auto eight = [&](const double *v, int o) {
+               for (int k = 0; k < 8; ++k) a[k] = t[k];
+               for (int e = 0; e < 64; e += 16) {
 #pragma unroll
-               for (int k = 0; k < 8; ++k) step(i0 + o + k, v[k]);
-          };
-          read(a, 0);
-          int e = 0;
-          for (; e + 16 <= m; e += 16) {
-               read(b, e + 8);
-               eight(a, e);
-               read(a, e + 16);
-               eight(b, e + 8);
+                    for (int k = 0; k < 8; ++k) b[k] = t[e + 8 + k];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) step(i0 + e + k, a[k]);
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) a[k] = t[e + 16 + k];      // (past 64: spare entries, unused)
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) step(i0 + e + 8 + k, b[k]);
+               }
+          } else {
+               const int m = n - i0;
+               double a[8], b[8];
+#pragma unroll
+               for (int k = 0; k < 8; ++k) a[k] = t[k];
+               int e = 0;
+               for (; e + 8 <= m; e += 8) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) b[k] = t[e + 8 + k];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) step(i0 + e + k, a[k]);
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) a[k] = b[k];
+               }
+#pragma unroll
+               for (int k = 0; k < 7; ++k)
+                    if (e + k < m) step(i0 + e + k, a[k]);
           }
-          if (e + 8 <= m) {
-               read(b, e + 8);
-               eight(a, e);
-               e += 8;
-#pragma unroll
-               for (int k = 0; k < 8; ++k) a[k] = b[k];
-          }
-#pragma unroll
-          for (int k = 0; k < 7; ++k)
-               if (e + k < m) step(i0 + e + k, a[k]);
           wave_lds_fence();
      }
 }
@@ -512,26 +518,27 @@ __device__ __forceinline__ void gsf_steps(int C, double m, bool live, double *cs
                for (int k = 0; k < GSF_USED; ++k) s.v[k] = cst[GSF_CST * e + k];
                return s;
           };
-          auto step = [&](int e, bool odd, const Cst &s) {
+          // the factor of the last value, formed one step ahead of its use: a m -+ c
+          auto lead = [&](const Cst &s) {
+               const double da = s.v[2] * m;
+               return FN < 2 || FN == 4 ? da : FN == 2 ? da - s.v[4] : da + s.v[4];
+          };
+          auto step = [&](int e, bool odd, const Cst &s, double da) {
                if constexpr (FN == 4) {
                     // P_l = a (m P_{l-1} - P_{l-2}) + m P_{l-1}, a = (l-1)/l
                     const double bb = m * b0;
                     put(e, odd, s.v[2] * (bb - a0) + bb);
                } else {
-                    double x;
-                    if constexpr (FN < 2) {
-                         const double da = s.v[2] * m;
-                         x = da * b0 - s.v[3] * a0;
-                    } else {
-                         const double dc = s.v[2] * m;
-                         x = FN == 2 ? (dc - s.v[4]) * b0 - s.v[3] * a0 : (dc + s.v[4]) * b0 - s.v[3] * a0;
-                    }
-                    const double q = x * s.v[1];
+                    const double x = da * b0 - s.v[3] * a0, q = x * s.v[1];
                     put(e, odd, __builtin_fma(__builtin_fma(-q, s.v[0], x), s.v[1], q));
                }
           };
+          auto one = [&](int e) {
+               const Cst s = load(e);
+               step(e, e & 1, s, lead(s));
+          };
           int e = e0;
-          for (; e < ne && (e & 3); ++e) step(e, e & 1, load(e));
+          for (; e < ne && (e & 3); ++e) one(e);
           // groups of four, the next group's factors read one group ahead
           // (past the last one: the buffer's four spare entries)
           Cst c0[4], c1[4];
@@ -539,27 +546,24 @@ __device__ __forceinline__ void gsf_steps(int C, double m, bool live, double *cs
 #pragma unroll
                for (int k = 0; k < 4; ++k) c[k] = load(o + k);
           };
-          auto four = [&](const Cst *c, int o) {
+          double da;
+          auto four = [&](const Cst *c, const Cst *n, int o) {
 #pragma unroll
-               for (int k = 0; k < 4; ++k) step(o + k, k & 1, c[k]);
+               for (int k = 0; k < 4; ++k) {
+                    const double d = lead(k < 3 ? c[k + 1] : n[0]);
+                    step(o + k, k & 1, c[k], da);
+                    da = d;
+               }
           };
           read(c0, e);
+          da = lead(c0[0]);
           for (; e + 8 <= ne; e += 8) {
                read(c1, e + 4);
-               four(c0, e);
+               four(c0, c1, e);
                read(c0, e + 8);
-               four(c1, e + 4);
+               four(c1, c0, e + 4);
           }
-          if (e + 4 <= ne) {
-               read(c1, e + 4);
-               four(c0, e);
-               e += 4;
-#pragma unroll
-               for (int k = 0; k < 4; ++k) c0[k] = c1[k];
-          }
-#pragma unroll
-          for (int k = 0; k < 3; ++k)
-               if (e + k < ne) step(e + k, k & 1, c0[k]);
+          for (; e < ne; ++e) one(e);
      }
 }
 // One plane of the expansion tables, zero columns past H: rows of two l, [(C + 1) /
@@ -615,6 +619,28 @@ __device__ __forceinline__ T ld_row(const T *base, int row, size_t Np, unsigned 
      else return v;
 }
 
+// Stores v at element i of row `row` (as ld_row: ioff = i * sizeof(T)).
+template <class T>
+__device__ __forceinline__ void st_row(T *base, int row, size_t Np, unsigned ioff, T v) {
+     typedef typename LdRowType<T>::type L;
+     const unsigned long long a = (unsigned long long) (base + (size_t) row * Np);
+     const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned) a);
+     const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned) (a >> 32));
+     typedef char __attribute__((address_space(1))) *gchar;
+     typedef L __attribute__((address_space(1))) *gL;
+     const gchar rp = (gchar) (((unsigned long long) hi << 32) | lo);
+     if constexpr (std::is_same<T, double2>::value) *(gL) (rp + ioff) = L{v.x, v.y};
+     else *(gL) (rp + ioff) = v;
+}
+
+// Largest and smallest n of the wave's active lanes.
+__device__ __forceinline__ int wave_max(int n) {
+     int r = __builtin_amdgcn_readfirstlane(n);
+     while (const unsigned long long b = __ballot(n > r)) r = __builtin_amdgcn_readlane(n, __builtin_ctzll(b));
+     return r;
+}
+__device__ __forceinline__ int wave_min(int n) { return -wave_max(-n); }
+
 // 1/q from the hardware reciprocal r (about 2^-24 relative) and the series
 // r (1 + e + e^2), e = 1 - q r: three dependent operations after the
 // reciprocal instead of the four of two Newton steps, error e^3 (< 2^-72)
@@ -655,7 +681,8 @@ __device__ __forceinline__ void mie_chain_d(const ChainArgs &p, int i) {
      const size_t Np = p.Np;
      const double x = p.x[i];
      const int n1 = p.n1[i], n2 = p.n2[i], dtop = p.d_all ? n2 - 1 : n1;
-     double2 *Dv = (double2 *) p.D;
+     // (taken once: the arguments of a batch lie in memory that the stores may alias)
+     double2 *const Dv = (double2 *) p.D, *const Dzv = (double2 *) p.Dz;
      // downward D_j(z) = (j+1)/z - 1 / w_j, w_j = D_{j+1} + (j+1)/z,
      // D_{n2} = 0.  The chain carries w: w_{j-1} = (2j+1)/z - 1 / w_j,
      // w_{n2-1} = n2 / z, with 1 / w = conj(w) / |w|^2 (|w| stays between
@@ -663,22 +690,41 @@ __device__ __forceinline__ void mie_chain_d(const ChainArgs &p, int i) {
      // component; D_j = (j+1)/z - 1 / w_j is formed beside the chain.  The
      // recurrence damps its last-bit differences.
      const cd z = cscale(cmk(p.mr, -p.mi), x), iz = crecip(z);
-     cd w = cscale(iz, (double) n2);
-     cd dz = cmk(0., 0.);
-     const cd iz2 = cmul(iz, iz);
-     for (int j = n2 - 1; j >= 1; --j) {
-          const cd c1 = cscale(iz, j + 1.), e = cscale(iz, 2. * j + 1.);
-          const double q = rcp_s3(__builtin_fma(w.r, w.r, w.i * w.i));
-          if constexpr (TAN) {
-               const cd dc = cscale(iz2, -(j + 1.)), r = cmk(w.r * q, -w.i * q), r2 = cmul(r, r), t = cadd(dz, dc);
-               dz = cmk(__builtin_fma(t.r, r2.r, __builtin_fma(-t.i, r2.i, dc.r)),
-                        __builtin_fma(t.r, r2.i, __builtin_fma(t.i, r2.r, dc.i)));
-               if (j <= dtop) ((double2 *) p.Dz)[j * Np + i] = double2{dz.r, dz.i};
+     const cd w0 = cscale(iz, (double) n2), iz2 = cmul(iz, iz);
+     cd w = w0, dz = cmk(0., 0.);
+     // The loop is the wave's (from its largest n2 to 1; a branch on the lane's
+     // own n2 or store range in every step took as long as the chain): down to
+     // the smallest n2 a lane that has not started keeps its first w, and a row is
+     // stored by every lane as soon as one keeps it (rows past a lane's own
+     // range are never read).
+     const int jt = wave_max(n2) - 1, js = wave_max(dtop), jm = min(wave_min(n2), jt + 1);
+     const unsigned oi = (unsigned) i * 16u;
+     auto run = [&](int j0, int j1, auto sel, auto st) {
+          for (int j = j0; j >= j1; --j) {
+               const double fj = j;
+               const cd c1 = cscale(iz, fj + 1.), e = cscale(iz, 2. * fj + 1.);
+               const double q = rcp_s3(__builtin_fma(w.r, w.r, w.i * w.i));
+               const bool on = !sel.value || j < n2;
+               if constexpr (TAN) {
+                    const cd dc = cscale(iz2, -(fj + 1.)), r = cmk(w.r * q, -w.i * q), r2 = cmul(r, r), t = cadd(dz, dc);
+                    const cd d = cmk(__builtin_fma(t.r, r2.r, __builtin_fma(-t.i, r2.i, dc.r)),
+                                     __builtin_fma(t.r, r2.i, __builtin_fma(t.i, r2.r, dc.i)));
+                    dz = on ? d : cmk(0., 0.);
+                    if (st.value) st_row(Dzv, j, Np, oi, double2{dz.r, dz.i});
+               }
+               if (st.value) st_row(Dv, j, Np, oi, double2{__builtin_fma(-w.r, q, c1.r), __builtin_fma(w.i, q, c1.i)});
+               const cd wn = cmk(__builtin_fma(-w.r, q, e.r), __builtin_fma(w.i, q, e.i));
+               w = on ? wn : w0;
           }
-          if (j <= dtop)
-               Dv[j * Np + i] = double2{__builtin_fma(-w.r, q, c1.r), __builtin_fma(w.i, q, c1.i)};
-          w = cmk(__builtin_fma(-w.r, q, e.r), __builtin_fma(w.i, q, e.i));
-     }
+     };
+     const std::true_type yes;
+     const std::false_type no;
+     // (js < jt: the kept rows lie below the largest n2)
+     const int ja = max(jm, js + 1);
+     run(jt, ja, yes, no);
+     if (jm > js) run(jm - 1, js + 1, no, no);
+     else run(min(js, jt), jm, yes, yes);
+     run(min(jm - 1, js), 1, no, yes);
 }
 
 // The other chains, in another wave, one loop: psi by
@@ -700,28 +746,47 @@ __device__ __forceinline__ void mie_chain_psi(const ChainArgs &p, int i) {
      double *U = p.PC, *Chi = p.PC + ppl;
      const double ax = 1. / x, sx = p.sx[i], cx = p.cx[i];
      double ua = 0., ub = 1.;               // U_{j+1}, U_j, starting at j = n1 - 1
-     U[n1 * Np + i] = 0.;
-     U[(n1 - 1) * Np + i] = 1.;
-     double chi0 = cx, chi1 = ax * cx + sx;
-     Chi[i] = chi0;
-     for (int t = 1; t <= n1; ++t) {
-          Chi[t * Np + i] = chi1;
-          const double fv1 = 2. * t + 1.;
-          const double chi2 = fv1 * ax * chi1 - chi0;
-          chi0 = chi1;
-          chi1 = chi2;
-          const int j = n1 - t;
-          if (j >= 1) {
-               const double un = (2. * j + 1.) * ax * ub - ua;
-               U[(j - 1) * Np + i] = un;
-               ua = ub;
-               ub = un;
+     double chi0 = cx, chi1 = ax * cx + sx, chn = 0.;
+     // as the D chain, one loop for the wave: U waits at its start down to the
+     // lane's n1 - 1 (its rows from n1 up are zero), chi runs on past it
+     const int nt = wave_max(n1), nm = nt - wave_min(n1);
+     const unsigned oi = (unsigned) i * 8u;
+     st_row(U, nt, Np, oi, 0.);
+     st_row(Chi, 0, Np, oi, chi0);
+     auto run = [&](int t0, int t1, auto sel) {
+          for (int t = t0; t <= t1; ++t) {
+               const double ft = t;
+               st_row(Chi, t, Np, oi, chi1);
+               if (TAN) chn = t == n1 ? chi1 : chn;
+               const double chi2 = (2. * ft + 1.) * ax * chi1 - chi0;
+               chi0 = chi1;
+               chi1 = chi2;
+               // U_j of j = nt - t, then U_{j-1}
+               const int j = nt - t;
+               if (sel.value) {
+                    const bool on = j < n1;
+                    st_row(U, j, Np, oi, on ? ub : 0.);
+                    const double un = (2. * j + 1.) * ax * ub - ua;
+                    ua = on ? ub : 0.;
+                    ub = on ? un : 1.;
+               } else {
+                    st_row(U, j, Np, oi, ub);
+                    const double un = (2. * j + 1.) * ax * ub - ua;
+                    ua = ub;
+                    ub = un;
+               }
           }
-     }
+     };
+     run(1, nm, std::true_type{});
+     run(nm + 1, nt - 1, std::false_type{});
+     // t = nt: U_0 is there
+     st_row(Chi, nt, Np, oi, chi1);
+     if (TAN) chn = nt == n1 ? chi1 : chn;
+     st_row(U, 0, Np, oi, ub);
      const double s = sx / ub;
      p.PS[i] = s;
-     if constexpr (TAN) {               // chi0 = chi_{n1}, ua = U_1
-          const double q = -s / chi0;
+     if constexpr (TAN) {               // chn = chi_{n1}, ua = U_1
+          const double q = -s / chn;
           p.PQ[i] = (cx - sx * ax + s * ua - q * cx) / sx;
           p.PQ[Np + i] = q;
      }
@@ -765,9 +830,10 @@ __device__ __forceinline__ void order_factors(int n, double *ft, int j) {
 // dependence chains first.  Measured at 3810 angles and 32768 sizes (each
 // role launched alone): the Gauss rule 0.14 ms (three Newton steps in its
 // slowest wave), with the expansion tables behind it 0.27, with the pi/tau tables
-// 0.22 (split: 0.21), the chains 0.27 (0.36 with D kept to n2); all of them 0.31
-// (0.41).  The factors common to a wave taken from its lanes instead of LDS: 0.26,
-// 0.39, 0.36, and 0.39 for all.  Block ranges (ends): the expansion tables (planes
+// 0.22 (split: 0.21), the chains 0.24 (0.31 with D kept to n2; 0.27 and 0.36 with
+// a branch per lane and step); all of them 0.29 (0.36).  The factors common to a
+// wave taken from its lanes instead of LDS: 0.26, 0.39, 0.36, and 0.39 for all.
+// Block ranges (ends): the expansion tables (planes
 // x angle blocks), the pi/tau tables (x PITAU_SHARE split), the Gauss rule, the
 // D chains, the psi and chi chains (heaviest sizes first), the order factors.
 // PK: pi/tau tables, 0 none, 1 FP64, 2 split fp16, 3 split bf16.
