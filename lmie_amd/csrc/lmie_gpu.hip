@@ -8,7 +8,7 @@
 //                    (src/lmie_core.c:669-691), P^{00}, P^{02}, P^{22}, P^{2-2},
 //                    P_l (misc/rtutil_math.c:867-1017), and per size D_n
 //                    downward, psi_n, chi_n (src/lmie_core.c:298-405)
-//   mie_terms        per (size, 8 orders): a_n, b_n, contraction operand, series partials
+//   mie_terms        per (size, 2 or 8 orders): a_n, b_n, contraction operand, series partials
 //                                                              (src/lmie_core.c:453-652)
 //   mie_sums         series per size                          (src/lmie_core.c:537-596)
 //   mie_tan_*        the same with the derivatives along x and m
@@ -655,7 +655,7 @@ __device__ __forceinline__ double rcp_s3(double q) {
 // The front runs the three recurrences that are serial in n, two threads per
 // size in different waves (the D chain; the psi and chi chains); mie_terms forms a_n, b_n, the
 // contraction operand and the partial series sums in parallel, one thread
-// per (size, group of 8 orders); mie_sums adds the partial sums per size.  The
+// per (size, group of 8 or 2 orders); mie_sums adds the partial sums per size.  The
 // serial part is a few operations per order, the parallel part fills the GPU.
 // D_j is kept as a complex pair, one 16-byte element per (order, size), so
 // each step of the D chain stores one element.
@@ -922,7 +922,7 @@ struct TermArgs {
      double *part;              // [5][ng][Np]: se, ss, cb re, cb im, sg of each group
 };
 
-template <class E>
+template <class E, int OPT>
 __device__ __forceinline__ void mie_terms_body(TermArgs p) {
 #pragma clang fp contract(off)
      constexpr bool MIX = !std::is_void<E>::value;
@@ -933,10 +933,11 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
      const size_t ld = (size_t) p.n1max + 2;
      const int kf = p.kfill[i / TILE];
      const int n1 = i < p.N ? p.n1[i] : 0;
-     const int j0 = 8 * g + 1, j1 = min(8 * g + 8, n1);
+     const int j0 = OPT * g + 1, j1 = min(OPT * g + OPT, n1);
      double se = 0., ss = 0., sg = 0.;
      cd cb = cmk(0., 0.);
-     // split operand of the 8 orders, [plane][order pair]; orders past n1 stay 0
+     // split operand of the orders, [plane][order pair]; orders past n1 stay 0
+     static_assert(OPT == 8 || !MIX, "whole groups of the split operand");
      unsigned buf[8][4];
 #pragma unroll
      for (int q = 0; q < 8; ++q)
@@ -953,31 +954,31 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
           const unsigned o8 = (unsigned) i * 8u, o16 = (unsigned) i * 16u;
           const int pmax = p.n1max, dmax = p.n2rows - 1;
           const double sc = p.PS[i], ax = 1. / x;
-          double ps[10], ch[10], dr[9], di[9];   // rows j0 - 2 .. j0 + 7 (psi, chi), j0 - 1 .. j0 + 7 (D)
+          double ps[OPT + 2], ch[OPT + 2], dr[OPT + 1], di[OPT + 1];   // rows j0 - 2 .. j0 + OPT - 1 (psi, chi), j0 - 1 .. (D)
           // U and chi of the group's rows from two seed rows each, by the
           // chains' own steps (the same bits as the stored rows): U downward
-          // from rows j0 + 8, j0 + 7 (U_{n1} = 0, U_{n1-1} = 1 where those rows
+          // from rows j0 + OPT, j0 + OPT - 1 (U_{n1} = 0, U_{n1-1} = 1 where those rows
           // fall inside, as the chain starts), chi upward from rows j0 - 2,
           // j0 - 1 (rows 0 and 1 for the first group).  Rows past a lane's n1
           // are computed from unused values and never used.
           {
-               double u[11];                  // rows j0 - 2 .. j0 + 8
-               u[10] = ld_row(U, min(j0 + 8, pmax), Np, o8);
-               u[9] = ld_row(U, min(j0 + 7, pmax), Np, o8);
+               double u[OPT + 3];             // rows j0 - 2 .. j0 + OPT
+               u[OPT + 2] = ld_row(U, min(j0 + OPT, pmax), Np, o8);
+               u[OPT + 1] = ld_row(U, min(j0 + OPT - 1, pmax), Np, o8);
 #pragma unroll
-               for (int e = 8; e >= 0; --e) {
+               for (int e = OPT; e >= 0; --e) {
                     const int r = j0 - 2 + e, jj = r + 1;
                     const double un = (2. * jj + 1.) * ax * u[e + 1] - u[e + 2];
                     u[e] = r == n1 ? 0. : r == n1 - 1 ? 1. : un;
                }
 #pragma unroll
-               for (int e = 0; e < 10; ++e) ps[e] = sc * u[e];
+               for (int e = 0; e < OPT + 2; ++e) ps[e] = sc * u[e];
                const bool first = j0 == 1;
                ch[0] = first ? 0. : ld_row(Chi, max(j0 - 2, 0), Np, o8);
                ch[1] = ld_row(Chi, j0 - 1, Np, o8);
                ch[2] = first ? ld_row(Chi, 1, Np, o8) : 0.;
 #pragma unroll
-               for (int e = 2; e < 10; ++e) {
+               for (int e = 2; e < OPT + 2; ++e) {
                     const int t = j0 - 2 + e - 1;
                     const double fv1 = 2. * t + 1.;
                     const double c2 = fv1 * ax * ch[e - 1] - ch[e - 2];
@@ -985,7 +986,7 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
                }
           }
 #pragma unroll
-          for (int e = 0; e < 9; ++e) {
+          for (int e = 0; e < OPT + 1; ++e) {
                const double2 v = ld_row(Dv, min(j0 - 1 + e, dmax), Np, o16);
                dr[e] = v.x;
                di[e] = v.y;
@@ -994,9 +995,9 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
           double psi0 = ps[1], chi0 = ch[1];
           if (j0 > 1) mie_ab_at(j0 - 1, x, m, im, cmk(dr[0], di[0]), psi0, ps[0], chi0, ch[0], &ap, &bp);
           double sgn = (j0 & 1) ? -1. : 1.;
-          // the 8 orders unrolled: the split halves land in registers
+          // the orders unrolled: the split halves land in registers
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
+          for (int e = 0; e < OPT; ++e) {
                const int j = j0 + e;
                if (j <= j1) {
                     const double psi = ps[e + 2], chi = ch[e + 2];
@@ -1044,10 +1045,10 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
                }
           }
      } else {
-          for (int r = max(8 * g, n1); r < min(8 * g + 8, kf); ++r)
+          for (int r = max(OPT * g, n1); r < min(OPT * g + OPT, kf); ++r)
                for (int c = 0; c < 4; ++c) p.A[c * plane + (size_t) r * Np + i] = 0.;
      }
-     // mie_sums reads the groups below (n1 + 7) / 8 only
+     // mie_sums reads the groups below (n1 + OPT - 1) / OPT only
      if (j0 > n1) return;
      double *pt = p.part + (size_t) g * Np + i;
      pt[0] = se;
@@ -1056,8 +1057,8 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
      pt[3 * gp] = cb.i;
      pt[4 * gp] = sg;
 }
-template <class E>
-__global__ __launch_bounds__(64) void mie_terms(TermArgs p) { mie_terms_body<E>(p); }
+template <class E, int OPT>
+__global__ __launch_bounds__(64) void mie_terms(TermArgs p) { mie_terms_body<E, OPT>(p); }
 struct mie_terms_B {
      TermArgs p;
      unsigned gx, gy;
@@ -1066,20 +1067,20 @@ template <class E>
 __global__ __launch_bounds__(64) void mie_terms_b(const mie_terms_B *cases) {
      const mie_terms_B a = cases[blockIdx.z];
      if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     mie_terms_body<E>(a.p);
+     mie_terms_body<E, 8>(a.p);
 }
 
 
 // Series per size from the group partials (src/lmie_core.c:586-596): a block
 // of 32 sizes x 8 lanes, lane l adds the groups g = l mod 8, then the eight
 // lane sums are added in a fixed order (deterministic).
-__device__ __forceinline__ void mie_sums_body(const double *part, int N, int Np, int ng, const int *n1, double *S, double *CB) {
+__device__ __forceinline__ void mie_sums_body(const double *part, int N, int Np, int ng, int opt, const int *n1, double *S, double *CB) {
      __shared__ double red[5][8][32];
      const int il = threadIdx.x & 31, l = threadIdx.x >> 5, i = blockIdx.x * 32 + il;
      const size_t gp = (size_t) ng * Np;
      double v[5] = {0., 0., 0., 0., 0.};
      if (i < Np) {
-          const int gn = i < N ? (n1[i] + 7) / 8 : 0;
+          const int gn = i < N ? (n1[i] + opt - 1) / opt : 0;
           for (int g = l; g < gn; g += 8) {
                const double *pt = part + (size_t) g * Np + i;
 #pragma unroll
@@ -1107,7 +1108,7 @@ __device__ __forceinline__ void mie_sums_body(const double *part, int N, int Np,
           CB[Np + i] = cb.i;
      }
 }
-__global__ __launch_bounds__(256) void mie_sums(const double *part, int N, int Np, int ng, const int *n1, double *S, double *CB) { mie_sums_body(part, N, Np, ng, n1, S, CB); }
+__global__ __launch_bounds__(256) void mie_sums(const double *part, int N, int Np, int ng, int opt, const int *n1, double *S, double *CB) { mie_sums_body(part, N, Np, ng, opt, n1, S, CB); }
 struct mie_sums_B {
      const double *part;
      int N;
@@ -1121,7 +1122,7 @@ struct mie_sums_B {
 __global__ __launch_bounds__(256) void mie_sums_b(const mie_sums_B *cases) {
      const mie_sums_B a = cases[blockIdx.z];
      if (blockIdx.x >= a.gx || blockIdx.y >= a.gy) return;
-     mie_sums_body(a.part, a.N, a.Np, a.ng, a.n1, a.S, a.CB);
+     mie_sums_body(a.part, a.N, a.Np, a.ng, 8, a.n1, a.S, a.CB);
 }
 
 
@@ -1136,7 +1137,7 @@ __global__ __launch_bounds__(256) void mie_sums_b(const mie_sums_B *cases) {
 // where psi_j = s U_j is the chain's psi, cut at psi_{n1} = 0: its derivative
 // in x solves the same recurrence up to a solution p psi + q chi, fixed by the
 // cut (psi'_{n1} = 0: q = -psi_{n1-1} / chi_{n1}) and by psi'_0 = cos x.
-// One thread per (size, 8 orders), as mie_terms; the previous order is formed
+// One thread per (size, 8 or 4 orders), as mie_terms; the previous order is formed
 // again for the g series.  Bound: FP64 VALU (about 400 operations per (size,
 // order) with both derivatives) and the operand planes it writes, 32 bytes per
 // (size, order) and operand set.
@@ -1151,14 +1152,14 @@ struct TanArgs {
      double *part;              // [rows][ng][Np]: the value's se, ss, cb (re, im), sg, then mie_tan_sums's rows
 };
 
-template <bool HX, bool HM>
+template <bool HX, bool HM, int OPT>
 __global__ __launch_bounds__(64) void mie_tan_terms(TanArgs p) {
      constexpr int NB = 1 + HX + HM, BM = HX ? 2 : 1;
      const int i = blockIdx.x * 64 + threadIdx.x, g = blockIdx.y;
      const size_t Np = p.Np, plane = (size_t) p.Kp * Np, gp = (size_t) p.ng * Np, ld = (size_t) p.n1max + 2;
      const int kf = p.kfill[i / TILE];
      const int n1 = i < p.N ? p.n1[i] : 0;
-     const int j0 = 8 * g + 1, j1 = min(8 * g + 8, n1);
+     const int j0 = OPT * g + 1, j1 = min(OPT * g + OPT, n1);
      if (j0 <= j1) {
           const double x = p.x[i], ax = 1. / x, sc = p.PS[i], pc = p.PQ[i], qc = p.PQ[Np + i];
           const cd m = cmk(p.mr, -p.mi), im = crecip(m), m2 = cmul(m, m);
@@ -1179,7 +1180,7 @@ __global__ __launch_bounds__(64) void mie_tan_terms(TanArgs p) {
           double se = 0., ss = 0., sg = 0., xe = 0., xs = 0., xg = 0., mg = 0., mgi = 0.;
           cd cb = cmk(0., 0.), xb = cb, me = cb, ms = cb, mb = cb;
           cd ap = cb, bp = cb, axp = cb, bxp = cb, amp = cb, bmp = cb;
-          const int jl = min(8 * g + 8, p.n1max);       // uniform: the group's last row
+          const int jl = min(OPT * g + OPT, p.n1max);       // uniform: the group's last row
           double un = ld_row(U, js, Np, o8), cn = ld_row(Chi, js, Np, o8);
           double2 dn = ld_row(Dv, js, Np, o16), zn = ld_row(Dz, js, Np, o16);
           for (int j = js; j <= jl; ++j) {
@@ -1274,7 +1275,7 @@ __global__ __launch_bounds__(64) void mie_tan_terms(TanArgs p) {
           }
      }
      // operand rows of orders beyond n1 (up to the tile's depth) are zero
-     for (int r = max(8 * g, n1); r < min(8 * g + 8, kf); ++r)
+     for (int r = max(OPT * g, n1); r < min(OPT * g + OPT, kf); ++r)
 #pragma unroll
           for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -1284,32 +1285,44 @@ __global__ __launch_bounds__(64) void mie_tan_terms(TanArgs p) {
 // Series per size from the group partials (as mie_sums): S [4][Np] of the
 // value (ext, sca, |c_bak|^2, asym), then 4 rows of d/dx (HX), then 4 rows
 // each of the derivatives along Re m and Im m (HM).
+// A block of 32 sizes x 32 lanes: every partial of up to 256 orders is in flight
+// at once (with 8 lanes the sum waited for one group after the other: 18.6 us of
+// 4000 sizes of up to 250 orders, 13 rows; now 12.9 of twice the groups, and 90 -> 41
+// us at 16384 sizes to x = 914).  Lane l adds the groups g = l mod 32,
+// the two lanes of a wave add up, then the 16 waves in a fixed order.
 template <bool HX, bool HM>
-__global__ __launch_bounds__(256) void mie_tan_sums(const double *part, int N, int Np, int ng, const int *n1, double *S) {
+__global__ __launch_bounds__(1024) void mie_tan_sums(const double *part, int N, int Np, int ng, int opt, const int *n1, double *S) {
      constexpr int R = 5 + 5 * HX + 8 * HM;
-     __shared__ double red[R][8][32];
+     __shared__ double red[R][16][32];
      const int il = threadIdx.x & 31, l = threadIdx.x >> 5, i = blockIdx.x * 32 + il;
      const size_t gp = (size_t) ng * Np;
      double v[R];
 #pragma unroll
      for (int q = 0; q < R; ++q) v[q] = 0.;
      if (i < Np) {
-          const int gn = i < N ? (n1[i] + 7) / 8 : 0;
-          for (int g = l; g < gn; g += 8) {
+          const int gn = i < N ? (n1[i] + opt - 1) / opt : 0;
+          for (int g = l; g < gn; g += 32) {
                const double *pt = part + (size_t) g * Np + i;
 #pragma unroll
                for (int q = 0; q < R; ++q) v[q] += pt[q * gp];
           }
      }
 #pragma unroll
-     for (int q = 0; q < R; ++q) red[q][l][il] = v[q];
+     for (int q = 0; q < R; ++q) {
+          const double t = v[q] + __shfl_xor(v[q], 32);
+          if (!(l & 1)) red[q][l >> 1][il] = t;
+     }
+     __syncthreads();
+     if (l < R) {
+          double t = red[l][0][il];
+#pragma unroll
+          for (int k = 1; k < 16; ++k) t += red[l][k][il];
+          red[l][0][il] = t;             // (read by this thread only so far)
+     }
      __syncthreads();
      if (l || i >= Np) return;
 #pragma unroll
-     for (int q = 0; q < R; ++q) {
-          v[q] = red[q][0][il];
-          for (int k = 1; k < 8; ++k) v[q] += red[q][k][il];
-     }
+     for (int q = 0; q < R; ++q) v[q] = red[q][0][il];
      const size_t n = Np;
      const cd cb = cmk(v[2], v[3]);
      double *s = S + i;
@@ -3666,7 +3679,7 @@ void gauss_guesses(int n, double *g) {
 // list of the contraction.
 struct FwdPlan {
      int N, Np, n1max, Q, C, H, Hp, Kp, Kb, Hb, nt, nw, nch;
-     int mixed, bf16, planes, keep, n2max, n2rows, ng, tm, ntile;
+     int mixed, bf16, planes, keep, n2max, n2rows, ng, opt, tm, ntile;
      // raw channels: weight rows of the value (row 0 the density, then the
      // weight-only directions and the density tangents of the directions that
      // move x or m), weight rows f dx_i of the value's x derivative, then its
@@ -3719,7 +3732,6 @@ int plan_forward(const lmie_gpu_job *J, FwdPlan &p) {
      int kfmax = 0;
      for (int t = 0; t < nt64 / 2; ++t) kfmax = std::max(kfmax, p.kt128[t] = std::max(p.kt64[2 * t], p.kt64[2 * t + 1]));
      p.n2rows = p.n2max + 1;
-     p.ng = kfmax / 8;
      // channels
      auto moves = [&](const double *v) {
           for (int i = 0; i < N; ++i)
@@ -3748,6 +3760,16 @@ int plan_forward(const lmie_gpu_job *J, FwdPlan &p) {
           }
      p.nraw = p.nP + p.nX + (p.hm ? 2 : 0);
      p.nb = 1 + p.hx + p.hm;
+     // orders per thread of the terms: 8, or fewer where the waves of 8 leave the
+     // chip's 1024 SIMDs mostly idle and a thread's orders in a row are what the
+     // launch takes (every thread forms the order before its first again, so
+     // more threads are more work).  Measured, terms of 8 and of fewer: one size
+     // 9.1 and 5.7 us (2 orders; 12 waves of 8), 1000 sizes of up to 40 orders 8.6
+     // and 5.6 (96), 4096 sizes with tangents 17.3 and 15.0 (4 orders), 4000 of up
+     // to 250 orders 22.3 and 20.8 (2016).
+     const int waves = p.Np / 64 * (kfmax / 8);
+     p.opt = p.mixed ? 8 : p.hx || p.hm ? (waves <= 4096 ? 4 : 8) : waves <= 512 ? 2 : 8;
+     p.ng = kfmax / p.opt;
      // the contraction's task list
      p.task.clear();
      p.tm = F64_TILE;
@@ -3982,9 +4004,10 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           ta.part = w->chPart.as<double>();
 #define LMIE_TAN(X, M)                                                                                           \
           do {                                                                                                   \
-               if (p.ng > 0) hipLaunchKernelGGL((mie_tan_terms<X, M>), gt, dim3(64), 0, s, ta);                  \
-               hipLaunchKernelGGL((mie_tan_sums<X, M>), gs, dim3(256), 0, s, (const double *) w->chPart.as<double>(), N, Np, \
-                                  p.ng, (const int *) w->n1.as<int>(), w->S.as<double>());                       \
+               if (p.ng > 0 && p.opt == 4) hipLaunchKernelGGL((mie_tan_terms<X, M, 4>), gt, dim3(64), 0, s, ta);  \
+               else if (p.ng > 0) hipLaunchKernelGGL((mie_tan_terms<X, M, 8>), gt, dim3(64), 0, s, ta);          \
+               hipLaunchKernelGGL((mie_tan_sums<X, M>), gs, dim3(1024), 0, s, (const double *) w->chPart.as<double>(), N, Np, \
+                                  p.ng, p.opt, (const int *) w->n1.as<int>(), w->S.as<double>());                       \
           } while (0)
           if (p.hx && p.hm) LMIE_TAN(true, true);
           else if (p.hx) LMIE_TAN(true, false);
@@ -3994,12 +4017,13 @@ int forward_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
           TermArgs ta;
           term_args(w, J, p, ta);
           if (p.ng > 0) {
-               if (!p.mixed) hipLaunchKernelGGL(mie_terms<void>, gt, dim3(64), 0, s, ta);
-               else if (p.bf16) hipLaunchKernelGGL(mie_terms<BF16>, gt, dim3(64), 0, s, ta);
-               else hipLaunchKernelGGL(mie_terms<F16>, gt, dim3(64), 0, s, ta);
+               if (!p.mixed && p.opt == 2) hipLaunchKernelGGL((mie_terms<void, 2>), gt, dim3(64), 0, s, ta);
+               else if (!p.mixed) hipLaunchKernelGGL((mie_terms<void, 8>), gt, dim3(64), 0, s, ta);
+               else if (p.bf16) hipLaunchKernelGGL((mie_terms<BF16, 8>), gt, dim3(64), 0, s, ta);
+               else hipLaunchKernelGGL((mie_terms<F16, 8>), gt, dim3(64), 0, s, ta);
           }
           hipLaunchKernelGGL(mie_sums, gs, dim3(256), 0, s, (const double *) w->chPart.as<double>(), N, Np,
-                             p.ng, (const int *) w->n1.as<int>(), w->S.as<double>(), keep ? w->CB.as<double>() : nullptr);
+                             p.ng, p.opt, (const int *) w->n1.as<int>(), w->S.as<double>(), keep ? w->CB.as<double>() : nullptr);
      }
      HIPCHECK(hipGetLastError());
      tm.mark(LMIE_T_COEFS, 1);

@@ -312,6 +312,23 @@ def test_directions_against_the_oracle(product, oracle, kind, n_int2, n_quad, r2
     assert not bad, bad
 
 
+@pytest.mark.parametrize("seeds", [None, {"mr": [1.0]}])
+@pytest.mark.parametrize("n_int2,n_quad,r2", [(1, 2, 0.3), (1, 33, 2.0), (3, 97, 9.0), (8, 127, 24.0)])
+def test_terms_of_every_group_size_against_the_oracle(product, oracle, seeds, n_int2, n_quad, r2):
+    """a_n, b_n and the series by groups of 2, 4 (with tangents) and 8 orders per
+    thread (1016 sizes of up to 290 orders without tangents), last groups partly
+    filled, against the oracle: 1e-12 normwise, the bar of the FP64 path."""
+    p = dict(dist_type="log_normal", n_int2=n_int2, n_quad=n_quad, calc_gc=1, calc_lc=0, **{"lambda": 0.6}, mr=1.45,
+             mi=0.02, a1=0.3, a2=0.25, r1=0.02, r2=r2, accuracy=-1.0, save_control=1)
+    say("case: terms", n_int2 * n_quad, "sizes to", r2, "tangents" if seeds else "")
+    got = lmie.solve(product, p, seeds, "fp64")
+    ref = abi.solve(oracle, p, seeds, n_threads=4)
+    keys = ["cext", "csca", "cbak", "g", "gc", "save1", "save2"] + (["cext_l", "csca_l", "cbak_l", "g_l", "gc_l"] if seeds else [])
+    bad = [(k, relnorm(np.asarray(got[k], float), np.asarray(ref[k], float))) for k in keys]
+    bad = [(k, e) for k, e in bad if not e <= 1e-12]
+    assert not bad, bad
+
+
 @pytest.mark.parametrize("gsf", [1, 0])
 @pytest.mark.parametrize("n_set,n_theta,n_coef", [(1, 1, 1), (1, 2, 2), (3, 63, 3), (4, 64, 4), (5, 65, 63), (9, 130, 64),
                                                   (2, 181, 67), (13, 200, 130)])
