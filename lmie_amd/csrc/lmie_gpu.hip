@@ -2564,7 +2564,7 @@ int ugemm_waves() {
 // Per-size reverse sweep (adjoint of src/lmie_core.c:298-611) over the
 // forward's kept recurrences (D_j up to n2 - 1, psi_j, chi_j, the reciprocals
 // 1 / (D_{j+1} + (j+1)/z)), in two kernels:
-//   rev_orders one thread per (size, chunk of RCH orders j in [1, n2)):
+//   rev_orders one thread per (size, chunk of rch orders j in [1, n2)):
 //              for j <= n1 the cotangents of a_j, b_j from the angular part
 //              (Sbar, Tbar) and the series, through a = (u psi - psi0) /
 //              (u zeta - zeta0), u = D/m + j/x and b (v = m D + j/x), to the
@@ -2577,10 +2577,18 @@ int ugemm_waves() {
 //   rev_carry  one thread per size: chains the chunks, then the per-size totals.
 // Outputs per size: the cotangent of m (re, im as d/dRe + i d/dIm), of f_i and
 // (when asked for) of x_i.
-constexpr int RCH = 64;
+
+// Orders per chunk of rev_orders: 64, or 32 where the waves of 64 would not fill
+// the chip's 1024 SIMDs once (every chunk forms two orders again, and its twelve
+// results go through memory to rev_carry).  Measured, rev_orders + rev_carry: 3965
+// sizes of up to 270 orders (315 waves of 64) 68 + 5 us with 64, 38 + 7 with 32, 28 +
+// 12 with 16; 16384 sizes to x = 914 155 + 12, 145 + 23, 144 + 44; 32768 to 1848
+// 539 + 32, 537 + 61, 565 + 131.  By the case also in a batch, so a case's results are
+// the same bits alone and in one (32 cases of 4000 sizes: 436 + 17, 412 + 27, 413 + 48).
+int rev_chunk(int Np, int n2rows) { return (size_t) (Np / 64) * ((n2rows + 62) / 64) <= 1024 ? 32 : 64; }
 
 struct RevArgs {
-     int N, Np, Kp, n1max, n2rows, nch;
+     int N, Np, Kp, n1max, n2rows, rch, nch;
      const double *ft;          // order_factors rows over 0 .. n1max + 1
      const double *x, *f;
      const int *n1, *n2;
@@ -2662,7 +2670,7 @@ __device__ __forceinline__ void rev_orders_body(RevArgs p) {
      cd P = cmk(1., 0.), C0 = cmk(0., 0.), Q = cmk(0., 0.), Z0 = cmk(0., 0.), mb = cmk(0., 0.);
      double fq = 0., xq = 0.;
      const int n1 = i < p.N ? p.n1[i] : 0, n2 = i < p.N ? p.n2[i] : 0;
-     const int lo = 1 + k * RCH, hi = min(n2, lo + RCH);
+     const int lo = 1 + k * p.rch, hi = min(n2, lo + p.rch);
      if (lo < hi) {
           const double x = p.x[i], f = p.f[i];
           // m, 1/m, 1/m^2 from the arguments: scalar operands, no registers per lane
@@ -2800,7 +2808,7 @@ __device__ __forceinline__ void rev_orders_body(RevArgs p) {
                u0 = v0; u1 = v1; u2 = v2; u3 = v3;
           }
      }
-     // rev_carry reads the chunks below (n2 - 1 + RCH - 1) / RCH only
+     // rev_carry reads the chunks below (n2 - 1 + rch - 1) / rch only
      if (lo >= n2) return;
      if constexpr (UP) {
           const double f = p.f[i];
@@ -2833,7 +2841,7 @@ __device__ __forceinline__ void rev_carry_body(RevArgs p) {
      const size_t Np = p.Np;
      const bool live = i < p.N;
      const double x = p.x[i];
-     const int nk = live ? (p.n2[i] - 1 + RCH - 1) / RCH : 0;
+     const int nk = live ? (p.n2[i] - 1 + p.rch - 1) / p.rch : 0;
      // chain the chunks upward from j = 1 with carry 0
      cd carry = cmk(0., 0.), zb = cmk(0., 0.), mb = cmk(0., 0.);
      double fq = 0., xq = 0.;
@@ -3240,6 +3248,7 @@ struct Workspace {
      PinBuf finPin;
      int home = -1, busy = 0;       // batch slot of this workspace (-1: general pool)
      int n2rows = 0, ng = 0;
+     int rch = 64;                  // reverse pass: orders per chunk (rev_chunk)
      int ushape = 8;                // reverse contraction: shape (FP64: orders per task)
      int valid = 0;
      int N = 0, Np = 0, Kp = 0, Hp = 0, H = 0, Q = 0, C = 0, n1max = 0, n2max = 0, calc_gc = 0, calc_lc = 0;
@@ -3819,6 +3828,7 @@ int stage_forward(Workspace *w, const lmie_gpu_job *J, const FwdPlan &p, bool ba
           xcd_tasks(p.kt32, [&](int t) { return (p.kt32[t] + w->ushape - 1) / w->ushape; }, F64_GROUP, rtask);
      }
      w->rtask = rtask;
+     w->rch = rev_chunk(Np, p.n2rows);
      Stage st;
      st.add<double>(w->x, Np); st.add<double>(w->sx, Np); st.add<double>(w->cx, Np);
      st.add<double>(w->f, nrow * Np);
@@ -4215,11 +4225,13 @@ int saved_impl(const lmie_gpu_job *J, lmie_gpu_result *R, Workspace *w) {
      return 0;
 }
 
+int rev_chunks(const Workspace *w) { return (w->n2rows - 1 + w->rch - 1) / w->rch; }
+
 // Buffers of a reverse pass (use_u: through G on the 16-bit matrix cores).
 int alloc_reverse(Workspace *w, bool use_u) {
      const size_t Np = w->Np, Q = w->Q > 0 ? w->Q : 1, C = w->C > 0 ? w->C : 1;
      const size_t Kq = rup(w->n1max, 64), Hq = rup(w->H > 0 ? w->H : 1, KM);
-     const size_t nck = (w->C + EXA_L - 1) / EXA_L, nch = (w->n2rows - 1 + RCH - 1) / RCH;
+     const size_t nck = (w->C + EXA_L - 1) / EXA_L, nch = rev_chunks(w);
      if (use_u && rup(w->n1max, KM) > w->Kb * 8) return set_err("internal: split operand depth");
      const size_t nres = 2 * (size_t) w->N + Np / 32;
      if (w->pfbar.get(sizeof(double) * 4 * Q) || w->gbar.get(sizeof(double) * 12 * C) || w->pin.get(sizeof(double) * 12 * C) ||
@@ -4250,7 +4262,8 @@ int stage_reverse(Workspace *w, const lmie_gpu_adj_in *in, bool use_gc, bool use
 
 // Arguments of the per-size reverse sweep.
 void rev_args(const Workspace *w, const lmie_gpu_adj_in *in, bool xbar, bool use_u, RevArgs &r) {
-     const int nch = (w->n2rows - 1 + RCH - 1) / RCH;
+     const int nch = rev_chunks(w);
+     r.rch = w->rch;
      r.N = w->N; r.Np = w->Np; r.Kp = w->Kp; r.n1max = w->n1max; r.n2rows = w->n2rows; r.nch = nch;
      r.ft = w->ftab.as<double>();
      r.x = w->x.as<double>(); r.f = w->f.as<double>();
