@@ -276,13 +276,13 @@ def main():
     mixed = a.path.startswith("mixed")
     peak = PEAK["bf16"] if mixed else PEAK["fp64"]
     # dominant kernel: forward contraction, or the reverse contraction U = G A
-    kern = {"angular_mix" if mixed else "angular_f64_dma": (8.0 * nq * units, ang_ms)}
+    kern = {"angular_mix" if mixed else "angular_f64": (8.0 * nq * units, ang_ms)}
     # matrix products issued per algorithmic product: the forward contraction
     # splits the size operand in two parts and the angle operand in three and
     # takes five of their products (three or four with LMIE_MIX_PRODUCTS=3 or
     # 4); the reverse contraction takes three (two parts of each operand)
     issued = {"angular_mix": {"3": 3.0, "4": 4.0}.get(os.environ.get("LMIE_MIX_PRODUCTS", ""), 5.0),
-              "adj_ugemm": 3.0, "angular_f64_dma": 1.0}
+              "adj_ugemm": 3.0, "angular_f64": 1.0}
     if mixed and a.path.endswith("-adjoint") and stages.get("adj_gemm", 0) > 0:
         kern["adj_ugemm"] = (24.0 * float(np.sum(n1s * n1s)), stages["adj_gemm"])
     kname = max(kern, key=lambda k: kern[k][1])
@@ -293,7 +293,7 @@ def main():
     if ref_dt is not None:
         f64_ms = ref_stages["angular"]
         f64_roof_ms = 8.0 * nq * units / PEAK["fp64"] * 1e3
-        fp64_angular = {"kernel": "angular_f64_dma", "ms": f64_ms, "roofline_ms": f64_roof_ms,
+        fp64_angular = {"kernel": "angular_f64", "ms": f64_ms, "roofline_ms": f64_roof_ms,
                         "frac": f64_roof_ms / f64_ms,
                         # an FP64 forward whose contraction ran at the FP64 matrix
                         # peak (its other stages as measured), against this step

@@ -221,8 +221,10 @@ int lmie_last_precision(void);
    LMIE_T_HOST_* and LMIE_T_CALL entries are host wall-clock times of the
    same call. */
 enum lmie_timer {
-     LMIE_T_TABLES = 0,    /* Gauss nodes + angular and expansion tables  */
-     LMIE_T_COEFS,         /* per-size recurrences, a_n/b_n, series        */
+     LMIE_T_TABLES = 0,    /* Gauss nodes, angular and expansion tables and
+                              the per-size chains (one launch)           */
+     LMIE_T_COEFS,         /* per-size recurrences, a_n/b_n, series (the
+                              tables' launch included)                   */
      LMIE_T_ANGULAR,       /* angular contraction (dominant kernel)        */
      LMIE_T_REDUCE,        /* reductions over sizes                        */
      LMIE_T_EXPAND,        /* expansion into coefficients                  */
