@@ -1750,7 +1750,8 @@ void angular_mix_b(const Mix2Args *cases, const int2 *task) {
 // partials [chunk][24][Hp]), then the fixed-order sum over chunks.
 constexpr int EXA_L = 32;
 
-__device__ __forceinline__ void expand_adjoint_part_body(const double *T, const double *gbar, const double *lbar, int H, int Hp, int C, double *part) {
+template <bool G, bool L>
+__device__ __forceinline__ void expand_adjoint_part_of(const double *T, const double *gbar, const double *lbar, int H, int Hp, int C, double *part) {
      const int j = blockIdx.x * blockDim.x + threadIdx.x, ck = blockIdx.y;
      if (j >= Hp) return;
      typedef double d2 __attribute__((ext_vector_type(2)));
@@ -1763,7 +1764,7 @@ __device__ __forceinline__ void expand_adjoint_part_body(const double *T, const 
      d2 q00 = {0., 0.}, q02 = q00, q22 = q00, q2m = q00, qpl = q00;
      auto step = [&](int l, int u) {
           const double sl = u ? -1. : 1., fl = (2 * l + 1) / 2.;
-          if (gbar) {
+          if constexpr (G) {
                double cb[6];
                for (int k = 0; k < 6; ++k) cb[k] = gbar[(size_t) k * C + l] * fl;
                const double e1 = (cb[1] + cb[2]) / 2., e2 = (cb[1] - cb[2]) / 2.;
@@ -1775,7 +1776,7 @@ __device__ __forceinline__ void expand_adjoint_part_body(const double *T, const 
                Em[4] += sl * cb[4] * p02;  Ep[4] += cb[4] * p02;
                Em[5] += sl * cb[5] * p02;  Ep[5] += cb[5] * p02;
           }
-          if (lbar) {
+          if constexpr (L) {
                const double pl = qpl[u];
                for (int k = 0; k < 6; ++k) {
                     const double c = lbar[(size_t) k * C + l] * fl * (k == 5 ? -1. : 1.);
@@ -1784,12 +1785,25 @@ __device__ __forceinline__ void expand_adjoint_part_body(const double *T, const 
                }
           }
      };
-     for (int l = ck * EXA_L; l < l1 && j < H; l += 2) {
+     auto load = [&](int l) {
           const size_t o = (size_t) (l / 2) * Hp + j;
-          if (gbar) { q00 = T2[o]; q02 = T2[plane + o]; q22 = T2[2 * plane + o]; q2m = T2[3 * plane + o]; }
-          if (lbar) qpl = T2[4 * plane + o];
-          step(l, 0);
-          if (l + 1 < l1) step(l + 1, 1);
+          if constexpr (G) { q00 = T2[o]; q02 = T2[plane + o]; q22 = T2[2 * plane + o]; q2m = T2[3 * plane + o]; }
+          if constexpr (L) qpl = T2[4 * plane + o];
+     };
+     if (j < H) {
+          int l = ck * EXA_L;
+          // four pairs' loads in flight (a pair at a time waited for memory 16 times a
+          // chunk: 17.5 us of 255 nodes and 510 l, now 11.3; 32 cases 37 and 29)
+#pragma unroll 4
+          for (; l + 2 <= l1; l += 2) {
+               load(l);
+               step(l, 0);
+               step(l + 1, 1);
+          }
+          if (l < l1) {
+               load(l);
+               step(l, 0);
+          }
      }
      double *out = part + (size_t) ck * 24 * Hp + j;
      for (int k = 0; k < 6; ++k) {
@@ -1798,6 +1812,13 @@ __device__ __forceinline__ void expand_adjoint_part_body(const double *T, const 
           out[(size_t) (12 + k) * Hp] = Lm[k];
           out[(size_t) (18 + k) * Hp] = Lp[k];
      }
+}
+// (the kinds of cotangents as template arguments: no branch in the loop, so the
+// loads of several l are in flight)
+__device__ __forceinline__ void expand_adjoint_part_body(const double *T, const double *gbar, const double *lbar, int H, int Hp, int C, double *part) {
+     if (gbar && lbar) expand_adjoint_part_of<true, true>(T, gbar, lbar, H, Hp, C, part);
+     else if (gbar) expand_adjoint_part_of<true, false>(T, gbar, lbar, H, Hp, C, part);
+     else expand_adjoint_part_of<false, true>(T, gbar, lbar, H, Hp, C, part);
 }
 __global__ __launch_bounds__(64) void expand_adjoint_part(const double *T, const double *gbar, const double *lbar, int H, int Hp, int C, double *part) { expand_adjoint_part_body(T, gbar, lbar, H, Hp, C, part); }
 struct expand_adjoint_part_B {
