@@ -4582,8 +4582,11 @@ struct RevCase {
      int use_gc, use_lc;
 };
 
+// (fused passes run the 128-size shape; a state whose forward ran alone with
+// LMIE_UGEMM_WAVES=2 holds the tasks and depths of 64-size tiles)
 int fused_reverse_ok(Workspace *w, const lmie_gpu_adj_in *in) {
-     return w->valid && w->mixed && w->Q > 0 && ((in->gc_bar && w->calc_gc) || (in->lc_bar && w->calc_lc));
+     return w->valid && w->mixed && w->ushape != 2 && w->Q > 0 &&
+            ((in->gc_bar && w->calc_gc) || (in->lc_bar && w->calc_lc));
 }
 
 // Buffers of one reverse pass (the mixed branch of adjoint_impl) and its
