@@ -727,6 +727,23 @@ __device__ __forceinline__ void mie_chain_d(const ChainArgs &p, int i) {
      run(min(jm - 1, js), 1, no, yes);
 }
 
+// Quotients f / x by 1/x in two parts (two operations).  1/x rounded once is the same
+// relative shift of x in every step of a chain: near x = 950 it cost psi 4e-14 of its
+// largest value and psi' 2e-13, 25 times that 1e-2 from x = k pi, against 4e-15, 1e-14 and
+// the same factor now (the reference's ratio chain: 4e-15, 3e-13).
+struct OverX {
+     double hi, lo;
+     __device__ __forceinline__ explicit OverX(double x) {
+#pragma clang fp contract(off)
+          hi = 1. / x;
+          lo = __builtin_fma(-x, hi, 1.) * hi;
+     }
+     __device__ __forceinline__ double operator()(double f) const {
+#pragma clang fp contract(off)
+          return __builtin_fma(f, hi, f * lo);
+     }
+};
+
 // The other chains, in another wave, one loop: psi by
 // Miller's downward recurrence, U_{n1} = 0, U_{n1-1} = 1,
 // U_{j-1} = (2j+1)/x U_j - U_{j+1}, psi_j = s U_j with s = sin x / U_0 (the
@@ -744,9 +761,10 @@ __device__ __forceinline__ void mie_chain_psi(const ChainArgs &p, int i) {
      const int n1 = p.n1[i];
      const size_t ppl = (size_t) (p.n1max + 1) * Np;
      double *U = p.PC, *Chi = p.PC + ppl;
-     const double ax = 1. / x, sx = p.sx[i], cx = p.cx[i];
+     const OverX over(x);
+     const double sx = p.sx[i], cx = p.cx[i];
      double ua = 0., ub = 1.;               // U_{j+1}, U_j, starting at j = n1 - 1
-     double chi0 = cx, chi1 = ax * cx + sx, chn = 0.;
+     double chi0 = cx, chi1 = over.hi * cx + sx, chn = 0.;
      // as the D chain, one loop for the wave: U waits at its start down to the
      // lane's n1 - 1 (its rows from n1 up are zero), chi runs on past it
      const int nt = wave_max(n1), nm = nt - wave_min(n1);
@@ -758,7 +776,7 @@ __device__ __forceinline__ void mie_chain_psi(const ChainArgs &p, int i) {
                const double ft = t;
                st_row(Chi, t, Np, oi, chi1);
                if (TAN) chn = t == n1 ? chi1 : chn;
-               const double chi2 = (2. * ft + 1.) * ax * chi1 - chi0;
+               const double chi2 = over(2. * ft + 1.) * chi1 - chi0;
                chi0 = chi1;
                chi1 = chi2;
                // U_j of j = nt - t, then U_{j-1}
@@ -766,12 +784,12 @@ __device__ __forceinline__ void mie_chain_psi(const ChainArgs &p, int i) {
                if (sel.value) {
                     const bool on = j < n1;
                     st_row(U, j, Np, oi, on ? ub : 0.);
-                    const double un = (2. * j + 1.) * ax * ub - ua;
+                    const double un = over(2. * j + 1.) * ub - ua;
                     ua = on ? ub : 0.;
                     ub = on ? un : 1.;
                } else {
                     st_row(U, j, Np, oi, ub);
-                    const double un = (2. * j + 1.) * ax * ub - ua;
+                    const double un = over(2. * j + 1.) * ub - ua;
                     ua = ub;
                     ub = un;
                }
@@ -787,7 +805,7 @@ __device__ __forceinline__ void mie_chain_psi(const ChainArgs &p, int i) {
      p.PS[i] = s;
      if constexpr (TAN) {               // chn = chi_{n1}, ua = U_1
           const double q = -s / chn;
-          p.PQ[i] = (cx - sx * ax + s * ua - q * cx) / sx;
+          p.PQ[i] = (cx - sx * over.hi + s * ua - q * cx) / sx;
           p.PQ[Np + i] = q;
      }
 }
@@ -953,7 +971,8 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
           const double *U = p.PC, *Chi = p.PC + (size_t) (p.n1max + 1) * Np;
           const unsigned o8 = (unsigned) i * 8u, o16 = (unsigned) i * 16u;
           const int pmax = p.n1max, dmax = p.n2rows - 1;
-          const double sc = p.PS[i], ax = 1. / x;
+          const double sc = p.PS[i];
+          const OverX over(x);
           double ps[OPT + 2], ch[OPT + 2], dr[OPT + 1], di[OPT + 1];   // rows j0 - 2 .. j0 + OPT - 1 (psi, chi), j0 - 1 .. (D)
           // U and chi of the group's rows from two seed rows each, by the
           // chains' own steps (the same bits as the stored rows): U downward
@@ -968,7 +987,7 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
 #pragma unroll
                for (int e = OPT; e >= 0; --e) {
                     const int r = j0 - 2 + e, jj = r + 1;
-                    const double un = (2. * jj + 1.) * ax * u[e + 1] - u[e + 2];
+                    const double un = over(2. * jj + 1.) * u[e + 1] - u[e + 2];
                     u[e] = r == n1 ? 0. : r == n1 - 1 ? 1. : un;
                }
 #pragma unroll
@@ -981,7 +1000,7 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
                for (int e = 2; e < OPT + 2; ++e) {
                     const int t = j0 - 2 + e - 1;
                     const double fv1 = 2. * t + 1.;
-                    const double c2 = fv1 * ax * ch[e - 1] - ch[e - 2];
+                    const double c2 = over(fv1) * ch[e - 1] - ch[e - 2];
                     if (e > 2 || !first) ch[e] = c2;
                }
           }
