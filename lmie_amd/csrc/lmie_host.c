@@ -746,11 +746,12 @@ typedef struct {
      int *n1, *n2;
 } job_mem;
 
-static void job_mem_alloc(job_mem *m, int N, int nd1, int nd2) {
+static int job_mem_alloc(job_mem *m, int N, int nd1, int nd2) {
      m->x = raw(N); m->f = raw(N); m->sx = raw(N); m->cx = raw(N);
      m->n1 = blk_get(sizeof(int) * N); m->n2 = blk_get(sizeof(int) * N);
      m->dx = raw((size_t) nd1 * N); m->dm = raw(2 * (size_t) nd1); m->dft = raw((size_t) nd1 * N);
      m->dfw = raw((size_t) nd2 * N);
+     return m->x && m->f && m->sx && m->cx && m->n1 && m->n2 && m->dx && m->dm && m->dft && m->dfw ? 0 : -1;
 }
 
 static void job_mem_free(job_mem *m) {
@@ -778,7 +779,10 @@ static int core_run(const core_args *c, core_out *o) {
      job_mem jm;
      lmie_gpu_job job;
      lmie_gpu_result res;
-     job_mem_alloc(&jm, c->N, c->nd1, c->nd2);
+     if (job_mem_alloc(&jm, c->N, c->nd1, c->nd2)) {
+          job_mem_free(&jm);
+          return fail("lmie_core_solution", "out of memory");
+     }
      fill_job(c, &job, jm.x, jm.f, jm.n1, jm.n2, jm.dx, jm.dm, jm.dft, jm.dfw, jm.sx, jm.cx);
      int C = job.n_coef, Q = job.n_qang, rc = -1;
      o->n_qang = Q; o->n_coef = C;
@@ -786,9 +790,20 @@ static int core_run(const core_args *c, core_out *o) {
      res.sums_ch = vec((size_t) 4 * (nch - 1));
      res.gc_raw = c->calc_gc ? zeros((size_t) nch * 6 * C) : NULL;
      res.lc_raw = c->calc_lc ? zeros((size_t) nch * 6 * C) : NULL;
+     double *rs_l = vec((size_t) 4 * (nd ? nd : 1));
+     if (!res.sums_ch || (c->calc_gc && !res.gc_raw) || (c->calc_lc && !res.lc_raw) || !rs_l) {
+          fail("lmie_core_solution", "out of memory");
+          goto done;
+     }
      if (c->save_control == 1) {
           *o->save1 = table2(4, c->N);
           *o->save2 = table3(4, c->N, Q > 0 ? Q : 1);
+          if (!*o->save1 || !*o->save2) {
+               free(*o->save1); free(*o->save2);
+               *o->save1 = NULL; *o->save2 = NULL;
+               fail("lmie_core_solution", "out of memory");
+               goto done;
+          }
           res.save1 = (*o->save1)[0];
           res.save2 = (*o->save2)[0][0];
      }
@@ -812,7 +827,6 @@ static int core_run(const core_args *c, core_out *o) {
      o->state = res.state;
      g_last_precision = res.precision;
      /* per-channel raw tangent sums -> seed order */
-     double *rs_l = vec((size_t) 4 * (nd ? nd : 1));
      for (int t = 0; t < c->nd1; ++t)
           for (int q = 0; q < 4; ++q) rs_l[4 * c->idx1[t] + q] = res.sums_ch[4 * t + q];
      for (int t = 0; t < c->nd2; ++t)
@@ -834,7 +848,6 @@ static int core_run(const core_args *c, core_out *o) {
           if (c->calc_gc) { norm_set(res.gc_raw, ch, C, a, al, o->gc_l[d]); o->gc_l[d][0][0] = 0.; }
           if (c->calc_lc) { norm_set(res.lc_raw, ch, C, a, al, o->lc_l[d]); o->lc_l[d][0][0] = 0.; }
      }
-     free(rs_l);
      *o->g = G / Csca * 2.;
      *o->cext = Cext * s;
      *o->csca = Csca * s;
@@ -843,6 +856,7 @@ static int core_run(const core_args *c, core_out *o) {
      if (c->calc_gc) { norm_set(res.gc_raw, 0, C, a, 0., o->gc); rc = truncated_count(o->gc, C, c->accuracy); }
      if (c->calc_lc) { norm_set(res.lc_raw, 0, C, a, 0., o->lc); rc = truncated_count(o->lc, C, c->accuracy); }
 done:
+     free(rs_l);
      free(res.sums_ch); blk_put(res.gc_raw); blk_put(res.lc_raw);
      job_mem_free(&jm);
      return rc;
@@ -1387,7 +1401,8 @@ typedef struct {
      const double *weight;
      int n_modes, N;
      double lambda;
-     double **df, **dx;
+     double **df, **dx;             /* NULL rows: proved zero */
+     int bad;                       /* set if an array could not be had */
 } dn_job;
 
 static void *dn_build(void *vp) {
@@ -1396,7 +1411,8 @@ static void *dn_build(void *vp) {
      const int S = ADJ_SEEDS;
      j->df = calloc((size_t) S * j->n_modes, sizeof(double *));
      j->dx = calloc((size_t) S * j->n_modes, sizeof(double *));
-     for (int k = 0; k < j->n_modes; ++k) {
+     j->bad = !j->df || !j->dx;
+     for (int k = 0; k < j->n_modes && !j->bad; ++k) {
           const lmie_in_data *m = j->modes[k];
           const double w = j->weight ? j->weight[k] : 1.;
           double e[ADJ_SEEDS][ADJ_SEEDS];
@@ -1411,17 +1427,19 @@ static void *dn_build(void *vp) {
              (src/lmie_interface.c:327-331), so the mono distribution's a1,
              whose node moves with r1, r2 held (misc/rtutil_size_dist.c:267-290),
              acts on the weights only, as in the reference's tangents */
-          if (grid_build(m->dist_type, m0->n_int1, m0->n_int2, m0->n_quad, a, m0->r1, m0->r2, &sv, &gk) == 0 &&
-              gk.N == j->N)
-               for (int e = 0; e < gk.n_act; ++e) {
-                    const int q = gk.act[e], moves = gk.r1_l[q] != 0. || gk.r2_l[q] != 0.;
-                    double *df = j->df[S * k + q] = raw(j->N), *dx = j->dx[S * k + q] = moves ? raw(j->N) : NULL;
-                    for (int i = 0; df && i < gk.N; ++i) {
-                         const size_t o = (size_t) i * S + q;
-                         df[i] = w * (gk.nr_l[o] * gk.qw[i] + gk.nr[i] * gk.qw_l[o]);
-                         if (dx) dx[i] = 2. * LM_PI * gk.qx_l[o] / j->lambda;
-                    }
+          /* (the forward built the same grid: only its memory can be missing here) */
+          j->bad = grid_build(m->dist_type, m0->n_int1, m0->n_int2, m0->n_quad, a, m0->r1, m0->r2, &sv, &gk) != 0 ||
+                   gk.N != j->N;
+          for (int e = 0; e < gk.n_act && !j->bad; ++e) {
+               const int q = gk.act[e], moves = gk.r1_l[q] != 0. || gk.r2_l[q] != 0.;
+               double *df = j->df[S * k + q] = raw(j->N), *dx = j->dx[S * k + q] = moves ? raw(j->N) : NULL;
+               j->bad = !df || (moves && !dx);
+               for (int i = 0; !j->bad && i < gk.N; ++i) {
+                    const size_t o = (size_t) i * S + q;
+                    df[i] = w * (gk.nr_l[o] * gk.qw[i] + gk.nr[i] * gk.qw_l[o]);
+                    if (dx) dx[i] = 2. * LM_PI * gk.qx_l[o] / j->lambda;
                }
+          }
           grid_free(&gk);
      }
      return NULL;
@@ -1554,13 +1572,14 @@ static int adjoint_forward_run(lmie_in_data *const *modes, const double *weight,
      /* the number density tangents of the modes (for the reverse pass) on a
         helper thread while the forward runs on the GPU: started once the
         host's own per-size loops are done, so the two do not share the cores */
-     dn_job dj = {modes, weight, n_modes, g.N, m0->lambda, NULL, NULL};
+     dn_job dj = {modes, weight, n_modes, g.N, m0->lambda, NULL, NULL, 0};
      dn_start st;
      memset(&st, 0, sizeof st);
      st.job = &dj;
      run_flags rf = {m0->calc_gc, m0->calc_lc, 0, 0, 0, m0->lambda, m0->mr, m0->mi, m0->accuracy, 1,
                      dn_launch, &st};
      core_out keep;
+     memset(&keep, 0, sizeof keep);
      double zero = 0.;
      rc = solve_grid(&rf, &g, &zero, &zero, &zero, opts, &out->n_coef, &out->r1, &out->r2,
                      &out->norm, &out->reff, &out->veff, &out->gavg, &out->vavg, &out->ravg,
@@ -1572,36 +1591,44 @@ static int adjoint_forward_run(lmie_in_data *const *modes, const double *weight,
      else if (st.running) pthread_join(st.th, NULL);
      else if (!st.done && rc == 0) dn_build(&dj);     /* not started (cannot happen on success) */
      lmie_gpu_host_time(LMIE_T_HOST_WAIT, wall_ms() - tw);
-     if (rc) {
+     lmie_adj_ctx *c = rc || dj.bad ? NULL : calloc(1, sizeof *c);
+     if (!c) {
+          if (!rc) fail("lmie_adjoint_forward", "out of memory");
+          if (keep.state) lmie_gpu_release(keep.state);
           adj_tangents_free(dj.df, n_modes);
           adj_tangents_free(dj.dx, n_modes);
           grid_free(&g);
           if (alloc_out) out_release(out);
           return -1;
      }
-     lmie_adj_ctx *c = calloc(1, sizeof *c);
      c->state = keep.state;
      c->n_modes = n_modes; c->N = g.N; c->C = keep.n_coef;
      c->calc_gc = m0->calc_gc; c->calc_lc = m0->calc_lc;
      c->lambda = m0->lambda; c->Csca = keep.sums[1]; c->g = out->g;
      c->cext = out->cext; c->csca = out->csca; c->cbak = out->cbak;
+     c->df = dj.df; c->dx = dj.dx;
+     c->gc = c->calc_gc ? vec((size_t) 6 * c->C) : NULL;
+     c->lc = c->calc_lc ? vec((size_t) 6 * c->C) : NULL;
+     c->w = vec(n_modes);
+     c->xl = raw(g.N);
+     if ((c->calc_gc && !c->gc) || (c->calc_lc && !c->lc) || !c->w || !c->xl) {
+          lmie_adjoint_free(c);
+          grid_free(&g);
+          if (alloc_out) out_release(out);
+          return fail("lmie_adjoint_forward", "out of memory");
+     }
      /* the caller's blocks may be wider than the coefficient count (alloc_out
         = 0 with a larger max_coef): rows are copied with their own stride, and
         the cotangents are read with the same stride */
      if (c->calc_gc) {
           c->ld_gc = (size_t) (out->gc[1] - out->gc[0]);
-          c->gc = vec((size_t) 6 * c->C);
           for (int k = 0; k < 6; ++k) memcpy(c->gc + (size_t) k * c->C, out->gc[k], sizeof(double) * c->C);
      }
      if (c->calc_lc) {
           c->ld_lc = (size_t) (out->lc[1] - out->lc[0]);
-          c->lc = vec((size_t) 6 * c->C);
           for (int k = 0; k < 6; ++k) memcpy(c->lc + (size_t) k * c->C, out->lc[k], sizeof(double) * c->C);
      }
-     c->w = vec(n_modes);
      for (int k = 0; k < n_modes; ++k) c->w[k] = weight ? weight[k] : 1.;
-     c->df = dj.df; c->dx = dj.dx;
-     c->xl = raw(g.N);
      for (int i = 0; i < g.N; ++i) c->xl[i] = 2. * LM_PI * g.qx[i] / (m0->lambda * m0->lambda);
      grid_free(&g);
      *ctxp = c;
@@ -1666,9 +1693,19 @@ static int adjoint_reverse_run(lmie_adj_ctx *c, const lmie_adj_in *adj, lmie_gra
      sb[2] = s * adj->cbak / (2. * 4. * LM_PI);
      sb[3] = 2. * adj->g / Csca;
      double dot = adj->g * c->g;
-     double *gcb = NULL, *lcb = NULL;
-     if (adj->gc && c->calc_gc) {
-          gcb = vec((size_t) 6 * C);
+     /* everything the pass needs, before it runs */
+     const int W = 5 * c->n_modes + 3, use_gc = adj->gc && c->calc_gc, use_lc = adj->lc && c->calc_lc;
+     double *gcb = use_gc ? vec((size_t) 6 * C) : NULL, *lcb = use_lc ? vec((size_t) 6 * C) : NULL;
+     double *gp = vec((size_t) 5 * c->n_modes), *part = vec((size_t) GRAD_BLOCKS * W);
+     lmie_gpu_adj_out aout;
+     aout.f_bar = zeros(c->N);
+     aout.x_bar = zeros(c->N);
+     if ((use_gc && !gcb) || (use_lc && !lcb) || !gp || !part || !aout.f_bar || !aout.x_bar) {
+          free(gcb); free(lcb); free(gp); free(part);
+          blk_put(aout.f_bar); blk_put(aout.x_bar);
+          return fail("lmie_adjoint_reverse", "out of memory");
+     }
+     if (use_gc) {
           for (int k = 0; k < 6; ++k)
                for (int l = 0; l < C; ++l) {
                     const double v = adj->gc[k * c->ld_gc + l];
@@ -1676,8 +1713,7 @@ static int adjoint_reverse_run(lmie_adj_ctx *c, const lmie_adj_in *adj, lmie_gra
                     dot += v * c->gc[k * C + l];
                }
      }
-     if (adj->lc && c->calc_lc) {
-          lcb = vec((size_t) 6 * C);
+     if (use_lc) {
           for (int k = 0; k < 6; ++k)
                for (int l = 0; l < C; ++l) {
                     const double v = adj->lc[k * c->ld_lc + l];
@@ -1687,9 +1723,6 @@ static int adjoint_reverse_run(lmie_adj_ctx *c, const lmie_adj_in *adj, lmie_gra
      }
      sb[1] = s * adj->csca - dot / Csca;
      lmie_gpu_adj_in ain = {sb, gcb, lcb};
-     lmie_gpu_adj_out aout;
-     aout.f_bar = zeros(c->N);
-     aout.x_bar = zeros(c->N);
      int rc = lmie_gpu_adjoint(c->state, &ain, &aout);
      if (rc) {
           fail("lmie_gpu_adjoint", lmie_gpu_last_error());
@@ -1699,19 +1732,18 @@ static int adjoint_reverse_run(lmie_adj_ctx *c, const lmie_adj_in *adj, lmie_gra
           /* a_p of mode k moves f_i through n_k (and, for grids set by the
              parameters, the nodes and weights); r1 and r2 move the shared grid
              of every mode: its weights and densities per mode, its nodes once */
-          double *gp = vec((size_t) 5 * c->n_modes), gr[2] = {0., 0.}, lx = 0.;
+          double gr[2] = {0., 0.}, lx = 0.;
           /* per fixed block of sizes on the pool, then the blocks in order:
              the sums do not depend on the threads */
-          grad_ctx gx = {c, aout.f_bar, aout.x_bar, vec((size_t) GRAD_BLOCKS * (5 * c->n_modes + 3))};
+          grad_ctx gx = {c, aout.f_bar, aout.x_bar, part};
           par_blocks(GRAD_BLOCKS, c->N * (c->n_modes + 1), grad_block, &gx);
           for (int b = 0; b < GRAD_BLOCKS; ++b) {
-               const double *pb = gx.part + (size_t) b * (5 * c->n_modes + 3);
+               const double *pb = part + (size_t) b * W;
                for (int q = 0; q < 5 * c->n_modes; ++q) gp[q] += pb[q];
                gr[0] += pb[5 * c->n_modes];
                gr[1] += pb[5 * c->n_modes + 1];
                lx += pb[5 * c->n_modes + 2];
           }
-          free(gx.part);
           /* lambda: x_i = 2 pi r_i / lambda, and cext, csca, cbak carry
              lambda^2 / (2 pi) (src/lmie_schedule.c:1158-1199) */
           grad->lambda = 2. / c->lambda * (adj->cext * c->cext + adj->csca * c->csca + adj->cbak * c->cbak) - lx;
@@ -1720,9 +1752,8 @@ static int adjoint_reverse_run(lmie_adj_ctx *c, const lmie_adj_in *adj, lmie_gra
           grad->a1 = gp[0]; grad->a2 = gp[1]; grad->a3 = gp[2]; grad->a4 = gp[3]; grad->a5 = gp[4];
           if (grad_modes)
                for (int q = 0; q < 5 * c->n_modes; ++q) grad_modes[q] = gp[q];
-          free(gp);
      }
-     blk_put(aout.f_bar); blk_put(aout.x_bar); free(gcb); free(lcb);
+     blk_put(aout.f_bar); blk_put(aout.x_bar); free(gcb); free(lcb); free(gp); free(part);
      return rc ? -1 : 0;
 }
 
