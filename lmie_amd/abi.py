@@ -75,6 +75,8 @@ def _arr(ptr, shape):
     """A copy of the block at ptr: short ones through a list, longer ones as one
     memmove (an array view of a pointer costs more than either)."""
     n = math.prod(shape)
+    if n and not ptr:
+        raise ValueError("NULL output block")
     if n <= 16:
         return np.array(ptr[:n] if n else [], dtype=np.float64).reshape(shape)
     a = np.empty(shape)
