@@ -184,12 +184,6 @@ __device__ __forceinline__ cd cdiv(cd a, cd b) {
      return cd{(a.r * t + a.i) / d, (a.i * t - a.r) / d};
 }
 __device__ __forceinline__ cd crecip(cd b) { return cdiv(cd{1., 0.}, b); }
-// 1/b = conj(b) / |b|^2 with one division, for divisors well inside the
-// range (|b|^2 neither overflows nor underflows)
-__device__ __forceinline__ cd crecip_fast(cd b) {
-     const double q = 1. / (b.r * b.r + b.i * b.i);
-     return cd{b.r * q, -b.i * q};
-}
 // 1/q from the hardware reciprocal and two Newton steps (about 1 ulp; no
 // special-value handling), for the dependence chains of the recurrences
 __device__ __forceinline__ double rcp_nr(double q) {
@@ -1490,16 +1484,12 @@ struct Mix2Args {
 //   1: 64 x 64, four waves (one per SIMD), separate corrections, 2 x 56 KiB
 //   2: 32 x 64, four waves, separate corrections, 2 x 40 KiB, two workgroups per CU
 //   3: 64 x 64, eight waves (two per SIMD), separate corrections, 2 x 56 KiB
-// DT > 0: every stage also touches each 128-byte line of the stage DT + 1
-// ahead (one 4-byte direct load per line into a scratch slot of LDS that is
-// never read), so that line is in L2 when its stage is loaded; the stage loads
-// then wait for an L2 hit instead of a trip to memory.
 constexpr int MIX_G = KM / 8;
 constexpr int MIX_SHAPE_DEFAULT = 3;
-struct MixS0 { static constexpr int NT = 512, TM = 64, TN = 128, WM = 2, WN = 4, MA = 2, NB = 2, ST = 2, OCC = 1, DT = 0; static constexpr bool SEP = false; };
-struct MixS1 { static constexpr int NT = 256, TM = 64, TN = 64, WM = 2, WN = 2, MA = 2, NB = 2, ST = 2, OCC = 1, DT = 0; static constexpr bool SEP = true; };
-struct MixS2 { static constexpr int NT = 256, TM = 32, TN = 64, WM = 2, WN = 2, MA = 1, NB = 2, ST = 2, OCC = 2, DT = 0; static constexpr bool SEP = true; };
-struct MixS3 { static constexpr int NT = 512, TM = 64, TN = 64, WM = 4, WN = 2, MA = 1, NB = 2, ST = 2, OCC = 1, DT = 0; static constexpr bool SEP = true; };
+struct MixS0 { static constexpr int NT = 512, TM = 64, TN = 128, WM = 2, WN = 4, MA = 2, NB = 2, ST = 2, OCC = 1; static constexpr bool SEP = false; };
+struct MixS1 { static constexpr int NT = 256, TM = 64, TN = 64, WM = 2, WN = 2, MA = 2, NB = 2, ST = 2, OCC = 1; static constexpr bool SEP = true; };
+struct MixS2 { static constexpr int NT = 256, TM = 32, TN = 64, WM = 2, WN = 2, MA = 1, NB = 2, ST = 2, OCC = 2; static constexpr bool SEP = true; };
+struct MixS3 { static constexpr int NT = 512, TM = 64, TN = 64, WM = 4, WN = 2, MA = 1, NB = 2, ST = 2, OCC = 1; static constexpr bool SEP = true; };
 template <class S> constexpr int mix_sa() { return 8 * MIX_G * S::TM; }              // v4u of A per stage
 template <class S> constexpr int mix_sb() { return B16_PLANES * MIX_G * S::TN; }     // v4u of B per stage
 // direct loads one wave issues per stage (its vmcnt events)
@@ -1513,33 +1503,6 @@ typedef __attribute__((address_space(3))) void *lds_ptr;
 // the B rows of the angle tile, cut into segments of at most 64 columns of 16
 // bytes; wave w takes segments w, w + NT / 64, ...  Each segment is one direct
 // load (lane l: column l of the segment).
-// lines a stage touches, and direct loads per wave for them
-template <class S> constexpr int mix_touch_lines() { return 8 * MIX_G * S::TM / 8 + B16_PLANES * MIX_G * S::TN / 8; }
-template <class S> constexpr int mix_touch_loads() { return (mix_touch_lines<S>() + S::NT - 1) / S::NT; }
-
-// Touch of stage c: thread tid loads one dword of lines tid, tid + NT, ...
-// (the last load of a thread repeats a line when the count is not a multiple)
-template <class S>
-__device__ __forceinline__ void mix_stage_touch(const Mix2Args &p, unsigned *sink, int c, int it0, int jt0, int tid) {
-     constexpr int LA = 8 * MIX_G * S::TM / 8, L = mix_touch_lines<S>();
-     const size_t Np = p.Np, Hb = p.Hb;
-     const size_t pA = (size_t) p.Kb * Np * 8, pB = (size_t) p.Kb * Hb * 8;
-#pragma unroll
-     for (int t = 0; t < mix_touch_loads<S>(); ++t) {
-          int li = tid + S::NT * t;
-          li = li < L ? li : L - 1;
-          const unsigned short *src;
-          if (li < LA) {
-               const int row = li / (S::TM / 8), seg = li % (S::TM / 8), q = row / MIX_G, g = row % MIX_G;
-               src = p.A16 + q * pA + ((size_t) (c * MIX_G + g) * Np + it0 + 8 * seg) * 8;
-          } else {
-               const int lb = li - LA, row = lb / (S::TN / 8), seg = lb % (S::TN / 8), q = row / MIX_G, g = row % MIX_G;
-               src = p.B16 + q * pB + ((size_t) (c * MIX_G + g) * Hb + jt0 + 8 * seg) * 8;
-          }
-          __builtin_amdgcn_global_load_lds((const void *) src, (lds_ptr) sink, 4, 0, 0);
-     }
-}
-
 template <class S>
 __device__ __forceinline__ void mix_stage_load(const Mix2Args &p, v4u *sA, v4u *sB, int c, int it0, int jt0,
                                                int wave, int lane) {
@@ -1592,9 +1555,8 @@ template <class E, int NP, int NW, class S>
 __device__ __forceinline__ void angular_mix_body(const Mix2Args &p, int2 tk) {
      constexpr int NT = S::NT, TM = S::TM, TN = S::TN, G = MIX_G, MA = S::MA, NB = S::NB, ST = S::ST;
      constexpr int SA = mix_sa<S>(), SB = mix_sb<S>();
-     __shared__ v4u lds[ST * (SA + SB) + (S::DT > 0 ? 16 : 0)];
+     __shared__ v4u lds[ST * (SA + SB)];
      static_assert(sizeof(lds) >= sizeof(double) * S::WM * 4 * 8 * TN, "epilogue buffer");
-     unsigned *sink = (unsigned *) (lds + ST * (SA + SB));   // touch loads land here (never read)
      static_assert(S::WM * 16 * MA == TM && S::WN * 16 * NB == TN && S::WM * S::WN == NT / 64, "wave grid");
 
      if (tk.x < 0) return;
@@ -1637,17 +1599,11 @@ __device__ __forceinline__ void angular_mix_body(const Mix2Args &p, int2 tk) {
 #pragma unroll
      for (int c = 0; c < ST - 1; ++c)
           if (c < nch) mix_stage_load<S>(p, sA(c), sB(c), c, it0, jt0, wave, lane);
-     if constexpr (S::DT > 0)
-          if (nch > 0) mix_stage_touch<S>(p, sink, min(ST - 1 + S::DT, nch - 1), it0, jt0, threadIdx.x);
      for (int c = 0; c < nch; ++c) {
           const int buf = c % ST;
-          // this wave's rows of stage c have landed (the younger stages may
-          // still be in flight); after the barrier every wave's have, and
-          // every wave is done with stage c - 1
-          // (the touch loads issued after them may stay in flight)
-          if constexpr (S::DT > 0) __builtin_amdgcn_s_waitcnt(0x0F70 | mix_touch_loads<S>());
-          else if (ST == 3 && c + 1 < nch) __builtin_amdgcn_s_waitcnt(0x0F70 | mix_loads<S>());
-          else __builtin_amdgcn_s_waitcnt(0);
+          // this wave's rows of stage c have landed; after the barrier every
+          // wave's have, and every wave is done with stage c - 1
+          __builtin_amdgcn_s_waitcnt(0);
           // the plain barrier: each wave has waited for its own rows above, and
           // a workgroup fence here would also wait for the younger stages
           __builtin_amdgcn_s_barrier();
@@ -1656,8 +1612,6 @@ __device__ __forceinline__ void angular_mix_body(const Mix2Args &p, int2 tk) {
                const int nb = (c + ST - 1) % ST;
                mix_stage_load<S>(p, sA(nb), sB(nb), c + ST - 1, it0, jt0, wave, lane);
           }
-          if constexpr (S::DT > 0)
-               mix_stage_touch<S>(p, sink, min(c + ST + S::DT, nch - 1), it0, jt0, threadIdx.x);
           // B fragments of the angle blocks: (pi+tau) h/m/l, (pi-tau) h/m/l
           v4u bp[NB][3], bm[NB][3];
 #pragma unroll
@@ -3287,7 +3241,7 @@ struct Workspace {
      Buf phIn, phOut;               // phase function: coefficients and angles, elements
      PinBuf finPin;
      int home = -1, busy = 0;       // batch slot of this workspace (-1: general pool)
-     int n2rows = 0, ng = 0;
+     int n2rows = 0;
      int rch = 64;                  // reverse pass: orders per chunk (rev_chunk)
      int ushape = 8;                // reverse contraction: shape (FP64: orders per task)
      int valid = 0;
@@ -3410,7 +3364,7 @@ struct Timer {
 // A wave owns one 16 x 16 block with all its sums in registers (8
 // accumulators per operand set); WM x WN waves share an LDS tile of 16 WM
 // sizes x 16 WN angles, filled by direct loads (global_load_lds_dwordx4, 64
-// lanes x 16 bytes straight into LDS) ST - 1 stages of KS orders ahead, one
+// lanes x 16 bytes straight into LDS) one stage of KS orders ahead, one
 // barrier per stage; a wave waits only for its own loads of the stage.  The
 // products' LDS reads are 16 consecutive doubles per lane group, so rows need
 // no padding.  (size tile, angle tile) tasks come from a host-built list dealt
@@ -3428,16 +3382,15 @@ struct F64Args {
      double *sst;               // reverse-pass checkpoint [8][Np][Hp]: sp+, sm+, sp-, sm- (re, im) or NULL
 };
 
-template <int WM, int WN, bool HX, bool HM, int KS, int ST, int OCC>
+template <int WM, int WN, bool HX, bool HM, int KS, int OCC>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OCC))) void angular_f64(F64Args p) {
      constexpr int NB = 1 + HX + HM, NW = WM * WN, TM = 16 * WM, TN = 16 * WN;
      constexpr int ASTG = NB * 4 * KS * TM, STG = ASTG + 2 * KS * TN;
      constexpr int NL = STG / (128 * NW);             // direct loads per wave and stage
      static_assert(STG % (128 * NW) == 0 && ASTG % 128 == 0 && KS % 4 == 0, "whole 1 KiB loads");
-     static_assert(ST >= 2 && ST <= 4 && NL * (ST - 2) < 64, "stages");
      constexpr int CHB = 8 * WM * TN;                 // epilogue buffer per channel
-     constexpr int CAP = ST * STG / CHB;              // channels per flush
-     __shared__ double sh[ST * STG];
+     constexpr int CAP = 2 * STG / CHB;               // channels per flush
+     __shared__ double sh[2 * STG];
 
      const int2 tk = p.task[blockIdx.x];
      if (tk.x < 0) return;
@@ -3485,22 +3438,16 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
      // s_n of this lane's orders (k0 + 4 ks + lg + 1: alternate lane groups)
      const unsigned long long sgn = (unsigned long long) (lg & 1) << 63;
      auto flip = [&](double v) { return __longlong_as_double((long long) ((unsigned long long) __double_as_longlong(v) ^ sgn)); };
-#pragma unroll
-     for (int k = 0; k < ST - 1; ++k)
-          if (k < nch) stage_load(k);
-     int buf = 0, nbuf = ST - 1;
+     if (nch > 0) stage_load(0);
+     int buf = 0;
      for (int kc = 0; kc < nch; ++kc) {
-          // this wave's loads of the stage have landed (they complete in order;
-          // the younger stages stay in flight), then everyone's; every wave is
-          // also done with the buffer of stage kc - 1, which takes stage
-          // kc + ST - 1
-          const int young = nch - 1 - kc;
-          if (ST >= 4 && young >= 2) wait_vm<NL * (ST >= 4 ? 2 : 0)>();
-          else if (ST >= 3 && young >= 1) wait_vm<NL>();
-          else wait_vm<0>();
+          // this wave's loads of the stage have landed, then everyone's; every
+          // wave is also done with the buffer of stage kc - 1, which takes
+          // stage kc + 1
+          wait_vm<0>();
           __builtin_amdgcn_s_barrier();
           __asm__ volatile("" ::: "memory");
-          if (kc + ST - 1 < nch) stage_load(nbuf);
+          if (kc + 1 < nch) stage_load(buf ^ 1);
           const double *a0 = sh + buf * STG + lg * TM + 16 * wm + l16;
           const double *b0 = sh + buf * STG + ASTG + lg * TN + 16 * wn + l16;
 #pragma unroll
@@ -3523,8 +3470,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
                     q[7] = __builtin_amdgcn_mfma_f64_16x16x4f64(Ti, sbp, q[7], 0, 0, 0);
                }
           }
-          buf = buf + 1 == ST ? 0 : buf + 1;
-          nbuf = nbuf + 1 == ST ? 0 : nbuf + 1;
+          buf ^= 1;
      }
 
      // epilogue: Stokes elements, weighted sums over this wave's 16 sizes (four
@@ -3627,10 +3573,10 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
 constexpr int F64_TILE = 32, F64_GROUP = 2;
 
 int launch_angular_f64(const F64Args &a, bool hx, bool hm, unsigned ntask, hipStream_t s) {
-     if (!hx && !hm) hipLaunchKernelGGL((angular_f64<2, 2, false, false, 16, 2, 3>), dim3(ntask), dim3(256), 0, s, a);
-     else if (!hm) hipLaunchKernelGGL((angular_f64<2, 2, true, false, 8, 2, 2>), dim3(ntask), dim3(256), 0, s, a);
-     else if (!hx) hipLaunchKernelGGL((angular_f64<2, 2, false, true, 8, 2, 2>), dim3(ntask), dim3(256), 0, s, a);
-     else hipLaunchKernelGGL((angular_f64<2, 2, true, true, 8, 2, 2>), dim3(ntask), dim3(256), 0, s, a);
+     if (!hx && !hm) hipLaunchKernelGGL((angular_f64<2, 2, false, false, 16, 3>), dim3(ntask), dim3(256), 0, s, a);
+     else if (!hm) hipLaunchKernelGGL((angular_f64<2, 2, true, false, 8, 2>), dim3(ntask), dim3(256), 0, s, a);
+     else if (!hx) hipLaunchKernelGGL((angular_f64<2, 2, false, true, 8, 2>), dim3(ntask), dim3(256), 0, s, a);
+     else hipLaunchKernelGGL((angular_f64<2, 2, true, true, 8, 2>), dim3(ntask), dim3(256), 0, s, a);
      HIPCHECK(hipGetLastError());
      return 0;
 }
@@ -4006,7 +3952,7 @@ void reduce_args(const Workspace *w, const FwdPlan &p, double *res, ReduceArgs &
 
 void keep_forward(Workspace *w, const lmie_gpu_job *J, const FwdPlan &p) {
      w->N = p.N; w->Np = p.Np; w->Kp = p.Kp; w->Hp = p.Hp; w->H = p.H; w->Q = p.Q; w->C = p.C; w->n1max = p.n1max;
-     w->n2max = p.n2max; w->n2rows = p.n2rows; w->ng = p.ng;
+     w->n2max = p.n2max; w->n2rows = p.n2rows;
      w->calc_gc = J->calc_gc; w->calc_lc = J->calc_lc; w->mr = J->mr; w->mi = J->mi;
      w->mixed = p.mixed; w->bf16 = p.bf16; w->Kb = p.Kb; w->Hb = p.Hb;
 }
