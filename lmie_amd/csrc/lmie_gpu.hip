@@ -803,8 +803,8 @@ __device__ __forceinline__ void mie_chain_psi(const ChainArgs &p, int i) {
           p.PQ[Np + i] = q;
      }
 }
-// a_j, b_j (src/lmie_core.c:557-583)
-__device__ __forceinline__ void mie_ab_jx(double jx, cd m, cd im, cd Dj, double psi, double psi0, double chi1,
+// a_j, b_j (src/lmie_core.c:557-583), jx = j / x
+__device__ __forceinline__ void mie_ab(double jx, cd m, cd im, cd Dj, double psi, double psi0, double chi1,
                                           double chi0, cd *a, cd *b) {
 #pragma clang fp contract(off)
      const cd zj = cmk(psi, chi1), zjm = cmk(psi0, chi0);
@@ -814,11 +814,6 @@ __device__ __forceinline__ void mie_ab_jx(double jx, cd m, cd im, cd Dj, double 
      const cd nb = csub(cscale(v, psi), cmk(psi0, 0.)), db = csub(cmul(v, zj), zjm);
      *a = cdiv_nr(na, da);
      *b = cdiv_nr(nb, db);
-}
-// a_j, b_j of size parameter x (jx = j / x)
-__device__ __forceinline__ void mie_ab_at(int j, double x, cd m, cd im, cd Dj, double psi, double psi0, double chi1,
-                                          double chi0, cd *a, cd *b) {
-     mie_ab_jx(j / x, m, im, Dj, psi, psi0, chi1, chi0, a, b);
 }
 
 // Size-independent factors of order j (the reference's expressions, so the
@@ -956,7 +951,10 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
 #pragma unroll
           for (int k = 0; k < 4; ++k) buf[q][k] = 0u;
      if (j0 <= j1) {
-          const double x = p.x[i];
+          // (quotients by x, j/x of the terms among them, from OverX: two operations
+          // where an IEEE division takes ten; with divisions for j/x the two-mode
+          // workload's 32768 sizes took 412 us, now 384)
+          const OverX over(p.x[i]);
           const cd m = cmk(p.mr, -p.mi), im = crecip(m);
           // the group's rows are the same in every lane: the D rows are all
           // loaded at once (rows clamped to the array; those past a lane's
@@ -966,7 +964,6 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
           const unsigned o8 = (unsigned) i * 8u, o16 = (unsigned) i * 16u;
           const int pmax = p.n1max, dmax = p.n2rows - 1;
           const double sc = p.PS[i];
-          const OverX over(x);
           double ps[OPT + 2], ch[OPT + 2], dr[OPT + 1], di[OPT + 1];   // rows j0 - 2 .. j0 + OPT - 1 (psi, chi), j0 - 1 .. (D)
           // U and chi of the group's rows from two seed rows each, by the
           // chains' own steps (the same bits as the stored rows): U downward
@@ -1006,7 +1003,7 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
           }
           cd ap = cmk(0., 0.), bp = cmk(0., 0.);
           double psi0 = ps[1], chi0 = ch[1];
-          if (j0 > 1) mie_ab_at(j0 - 1, x, m, im, cmk(dr[0], di[0]), psi0, ps[0], chi0, ch[0], &ap, &bp);
+          if (j0 > 1) mie_ab(over(j0 - 1.), m, im, cmk(dr[0], di[0]), psi0, ps[0], chi0, ch[0], &ap, &bp);
           double sgn = (j0 & 1) ? -1. : 1.;
           // the orders unrolled: the split halves land in registers
 #pragma unroll
@@ -1015,7 +1012,7 @@ __device__ __forceinline__ void mie_terms_body(TermArgs p) {
                if (j <= j1) {
                     const double psi = ps[e + 2], chi = ch[e + 2];
                     cd a, b;
-                    mie_ab_at(j, x, m, im, cmk(dr[e + 1], di[e + 1]), psi, psi0, chi, chi0, &a, &b);
+                    mie_ab(over((double) j), m, im, cmk(dr[e + 1], di[e + 1]), psi, psi0, chi, chi0, &a, &b);
                     const double fv1 = 2. * j + 1.;
                     se += fv1 * (a.r + b.r);
                     ss += fv1 * (cabs2(a) + cabs2(b));
