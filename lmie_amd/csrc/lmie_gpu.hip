@@ -230,7 +230,7 @@ __device__ __forceinline__ cd cdiv_nr(cd a, cd b) {
 // Bound: the Legendre recurrence's chain of four dependent operations per order
 // and Newton step.  Its factors j / (j + 1) are the same in every lane: each lane
 // divides for one order of the next 64, and the steps read them back from LDS as
-// broadcasts, ahead of the chain (UniformFactors), so every table wave can run
+// broadcasts, ahead of the chain (uniform_steps), so every table wave can run
 // the Newton steps of its own 64 angles and none waits for another.
 // Orders the LDS accesses of one wave: what its lanes wrote before is read after
 // (LDS serves a wave's accesses in order; this keeps the compiler to it).
@@ -722,9 +722,10 @@ __device__ __forceinline__ void mie_chain_d(const ChainArgs &p, int i) {
 }
 
 // Quotients f / x by 1/x in two parts (two operations).  1/x rounded once is the same
-// relative shift of x in every step of a chain: near x = 950 it cost psi 4e-14 of its
-// largest value and psi' 2e-13, 25 times that 1e-2 from x = k pi, against 4e-15, 1e-14 and
-// the same factor now (the reference's ratio chain: 4e-15, 3e-13).
+// relative shift of x in every step of a chain: at x = 300 pi + 0.8 it cost psi 4e-14
+// of its largest value and psi' 2e-13, at 300 pi + 0.01 4e-12 and 1e-9; now 4e-15, 9e-15 and
+// 2e-13, 4e-11 (the reference's ratio chain: 4e-15, 3e-13 and 2e-13, 4e-11: near x = k pi psi
+// keeps its loss eps / sin x from psi_0 = sin x, and psi' eps / sin^2 x).
 struct OverX {
      double hi, lo;
      __device__ __forceinline__ explicit OverX(double x) {
@@ -3565,7 +3566,10 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
 // set) and the gamma mode with tangents of m (16384 sizes, 1922 angles, two
 // sets): 14.7 and 4.3 ms; the same tiles with three stages and two workgroups
 // per CU 15.2 and 4.6; 32 x 64 on eight waves 15.7 and 4.6; 64 x 64 on
-// sixteen waves 15.3.  Groups of 1 or 2 size tiles took 0.3-0.4 ms less than 4
+// sixteen waves 15.3.  The instance with both derivative sets (192 accumulator
+// registers, the loads' 64-bit sources beside them) spills 112 registers, the
+// other three none; one workgroup per CU without the spill took 0.171-0.175 ms
+// where it takes 0.135 (2257 sizes, 512 angles).  Groups of 1 or 2 size tiles took 0.3-0.4 ms less than 4
 // or 8, of 16 1 ms more.
 constexpr int F64_TILE = 32, F64_GROUP = 2;
 
@@ -5106,7 +5110,7 @@ int lmie_gpu_phase_func(int n_set, int n_coef, int ld, const double *coefs, int 
 
 // Staging of lmie_gpu_phase_func_static: the coefficients, the angles and the
 // phase function of one call, in one file-scope device array in place of the
-// three device blocks lmie_gpu_phase_func allocates per call.  Every GPU the
+// workspace buffers that lmie_gpu_phase_func grows as its calls do.  Every GPU the
 // library runs on holds its own copy of the array (16 MiB) until the process
 // ends.  In host code the name `scratch` is not a device address: the address
 // of each device's copy is taken once (hipGetSymbolAddress, with that device

@@ -134,7 +134,7 @@ static void par_blocks(int nb, int work, par_fn fn, void *ctx) {
 }
 
 /* ------------------------------------------------------------------------- */
-/* Per-size arrays.  Blocks of 64 KiB and more are kept for the next call (at
+/* Per-size arrays.  Blocks of 64 KiB to 16 MiB are kept for the next call (at
    most 32 of them and 64 MiB; the rest, and all of them when the library is
    unloaded, go back to the C library): from malloc they come as fresh pages, whose
    first touch and release cost more than the loops over them. */

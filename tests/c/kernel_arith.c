@@ -3,21 +3,21 @@
  * kernels rely on (lmie_amd/csrc/lmie_gpu.hip), in IEEE double with
  * separately rounded operations and the C library's correctly rounded fma:
  *
- *  1. gsf_table's quotients: with y = RN(1/d) and q = RN(x y), the corrected
+ *  1. the expansion tables' quotients: with y = RN(1/d) and q = RN(x y), the corrected
  *     q + y RN(x - q d) equals the IEEE quotient RN(x/d) bit for bit
  *     (Markstein's theorem), for the divisors of the generalized spherical
  *     function recurrences (l, sqrt(l^2 - 4), (l-1)(l^2 - 4)) and numerators
  *     of every size the recurrences produce, plus random pairs.
- *  2. mie_chains' psi: Miller's downward recurrence U_{n1} = 0, U_{n1-1} = 1,
+ *  2. the psi chain: Miller's downward recurrence U_{n1} = 0, U_{n1-1} = 1,
  *     U_{j-1} = (2j+1)/x U_j - U_{j+1}, normalised by sin x / U_0, is the same
  *     function as the reference's ratio chain r_j = 1/((2j+1)/x - r_{j+1}),
  *     r_{n1} = 0, and product psi_j = sin x r_1 ... r_j (src/lmie_core.c:
  *     298-330): the two agree to rounding over x from 1e-3 to 2000, near
  *     x = k pi to the conditioning of the normalisation, which both share.
- *  3. mie_chains' reciprocal refinement r (1 + e + e^2), e = 1 - q r, from a
+ *  3. the D chain's reciprocal refinement r (1 + e + e^2), e = 1 - q r, from a
  *     starting reciprocal off by up to 2^-23 (the hardware's is good to about
  *     2^-24.6): within one ulp of 1/q.
- *  4. mie_chains' D chain carried as w_j = D_{j+1} + (j+1)/z,
+ *  4. the D chain carried as w_j = D_{j+1} + (j+1)/z,
  *     w_{j-1} = (2j+1)/z - conj(w_j) / |w_j|^2, D_j = (j+1)/z - conj(w_j) / |w_j|^2,
  *     against the reference's D_j = (j+1)/z - 1 / (D_{j+1} + (j+1)/z) with
  *     Smith's complex division (src/lmie_core.c:386-405): the same D_j to
@@ -80,7 +80,7 @@ static int miller(void) {
           for (int j = n1 - 1; j >= 1; --j) r[j] = 1. / ((2. * j + 1.) / x - r[j + 1]);
           pr[0] = sin(x);
           for (int j = 1; j <= n1; ++j) pr[j] = r[j] * pr[j - 1];
-          /* Miller's form, as mie_chains */
+          /* Miller's form (1/x rounded once here; the kernel's quotients: tangent_quad.c) */
           const double ax = 1. / x;
           double ua = 0., ub = 1.;
           pm[n1] = 0.;

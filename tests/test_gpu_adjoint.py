@@ -358,7 +358,7 @@ def test_fp64_reverse_contraction_at_tile_edges(product, n_int2, n_quad, r2):
     say("case: fp64 reverse contraction", n_int2, n_quad, r2)
     names = ("lambda", "mr", "mi", "a1", "r2")
     # at x = k pi (3 x 43 to 3.0 has a node at 5 pi) the forward tangents along x
-    # carry a factor 1 / sin x of rounding error, in the reference's ratio chain too
+    # carry eps / sin^2 x of rounding error, in the reference's ratio chain too
     # (psi_j from psi_0 = sin x): those directions are no oracle there
     edges = np.linspace(p["r1"], r2, n_int2 + 1)
     nodes = np.add.outer(edges[1:] + edges[:-1], np.outer(edges[1:] - edges[:-1], np.polynomial.legendre.leggauss(n_quad)[0])[0]) / 2

@@ -54,7 +54,7 @@ def test_gauss_rule_is_bitwise_the_reference_rule(product, oracle, n):
 
 
 def test_gsf_tables_are_bitwise_the_oracle_functions(product, oracle):
-    """The expansion tables of the angle kernels (gsf_table: each division a
+    """The expansion tables of the angle kernels (front's expansion role: each division a
     corrected product) equal the oracle's generalized spherical functions,
     computed with plain IEEE divisions in the reference's order, bit for bit,
     and P_l its Legendre recurrence; at the nodes of a 3810-point rule, at
@@ -91,7 +91,7 @@ def test_gsf_tables_are_bitwise_the_oracle_functions(product, oracle):
 
 
 def test_pitau_tables_are_bitwise_the_oracle_functions(product, oracle):
-    """The FP64 angle tables (pitau_table: pi_n + tau_n, pi_n - tau_n) equal
+    """The FP64 angle tables (front's role: pi_n + tau_n, pi_n - tau_n) equal
     the oracle's pi_n, tau_n recurrence in the reference's order, added and
     subtracted, bit for bit; at 95 angles (nodes, 0, +-1, random), n <= 1905."""
     n, q = 1905, 3810
